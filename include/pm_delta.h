@@ -320,11 +320,15 @@ size_t pm_delta_bwd_workspace_bytes(int B, int T, int H, int D, int in_dtype);
  * Arguments as pm_delta_bwd, plus g (B, T, H) fp32, the forward's log-gates,
  * and gg (B, T, H) fp32, dL/dg.  With P_t = alpha_t S_{t-1}, per token in
  * reverse: y = P_t w, dL/dg_t = <G - beta_t k_t w^T, P_t>, G <- alpha_t (G -
- * beta_t k_t w^T), the other gradients as pm_delta_bwd's.  Runs the
- * per-token fp32 kernels (any D <= 256, fp32 or bf16 q/k/v); each 8-token
- * checkpoint block is recomputed forward from its start state, never walked
- * back (which would divide by alpha).  Path 2 (chunked backward required)
- * returns PM_E_UNSUPPORTED.  workspace: pm_gated_delta_bwd_workspace_bytes.
+ * beta_t k_t w^T), the other gradients as pm_delta_bwd's.  fp32 arithmetic
+ * for fp32 and bf16 q/k/v alike, by one of two paths:
+ *   - D in {64, 128}, T >= 16, H * D <= 2^24, 16-byte aligned q, k, v, go, gv
+ *     and workspace: chunks of 16 tokens on fp32 MFMA;
+ *   - otherwise (any D <= 256), and under path 1: the per-token kernels; each
+ *     8-token checkpoint block is recomputed forward from its start state.
+ * Neither walks the state back (which would divide by alpha).  Path 2 (the
+ * bf16 chunked backward required) returns PM_E_UNSUPPORTED.  workspace:
+ * pm_gated_delta_bwd_workspace_bytes, enough for either path.
  */
 int pm_gated_delta_bwd(const void* q, const void* k, const void* v, const float* beta,
                        const float* g, const float* s0, const float* go, const float* gs, float* gq,
@@ -341,9 +345,9 @@ size_t pm_gated_delta_bwd_workspace_bytes(int B, int T, int H, int D, int in_dty
  * code for it).  Arguments as pm_gated_delta_bwd, with g and gg (B, T, H, D) fp32.
  * With P_t = Diag(alpha_t) S_{t-1}, per token in reverse: y = P_t w,
  * dL/dg_t[d] = <G_P[d, :], P_t[d, :]> with G_P = G - beta_t k_t w^T, and
- * G <- Diag(alpha_t) G_P; the other gradients as pm_delta_bwd's.  The per-token fp32
- * kernels (any D <= 256, fp32 or bf16 q/k/v), each 8-token checkpoint block
- * recomputed forward from its start state.  Path 2 returns PM_E_UNSUPPORTED.
+ * G <- Diag(alpha_t) G_P; the other gradients as pm_delta_bwd's.  The two paths of
+ * pm_gated_delta_bwd (the chunked one also needs g 16-byte aligned).  Path 2 returns
+ * PM_E_UNSUPPORTED.
  * workspace: pm_kda_delta_bwd_workspace_bytes.
  */
 int pm_kda_delta_bwd(const void* q, const void* k, const void* v, const float* beta,

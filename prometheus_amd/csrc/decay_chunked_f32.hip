@@ -1,0 +1,1161 @@
+// decay_chunked_f32.hip — K10: the rules with a decay (a log-gate per token and head, or
+// one per key channel) in chunked form on fp32 MFMA (v_mfma_f32_16x16x4f32), reverse mode,
+// D in {64, 128}, fixed-length batches, fp32 or bf16 q/k/v.  Every product is fp32 x fp32
+// with fp32 accumulation, as in the per-token kernels (delta_bwd.hip).
+//
+// Per token, alpha_t = exp(g_t) (a d_k-vector; constant over d_k for the per-head gate):
+//   P_t = Diag(alpha_t) S_{t-1},  u_t = v_t - P_t^T k_t,  S_t = P_t + beta_t k_t u_t^T,
+//   o_t = q_t S_t.
+// Per chunk of C = 16 tokens with start state S, F_t = prod_{j <= t} alpha_j and
+// E_s = prod_{j > s} alpha_j inside the chunk, gC = F_{C-1}, and
+// D_ts = prod_{s < j <= t} alpha_j (all per channel):
+//   K^ = K F,  Q^ = Q F,  K- = K E,
+//   A'_ts = sum_d k_t k_s D_ts (s < t),  P_ts = sum_d q_t k_s D_ts (s <= t),
+//   T = (I + diag(beta) A')^-1,  T'' = -T diag(beta),  X = K^ S - V,  U = T'' X,
+//   S' = Diag(gC) S + K-^T U,  O = Q^ S + P U.
+// Reverse, given G = dL/dS' and dO (dP = lower_incl(dO U^T), dA = -strict_lower(W U^T)):
+//   W  = T^T (K- G + P^T dO),  dV = diag(beta) W
+//   dS = Diag(gC) G + Q^^T dO - K^^T diag(beta) W
+//   dQ_t = F_t (dO S^T)_t + sum_s dP_ts k_s D_ts
+//   dK_t = -beta_t F_t (W S^T)_t + E_t (U G^T)_t + sum_{s<t} beta_t dA_ts k_s D_ts
+//          + sum_{r>t} beta_r dA_rt k_r D_rt + sum_{r>=t} dP_rt q_r D_rt
+//   dbeta_t = W_t . V_t - K^_t . (W S^T)_t + sum_s dA_ts A'_ts
+//   dg_j = sum_{t>=j} (Q^ dO S^T - K^ beta W S^T)_t + sum_{s<j} (K- U G^T)_s
+//          + gC <S, G>_rows + sum_{t>=j, s<j} x_ts,
+// x_ts the pair term dP_ts q_t k_s D_ts + beta_t dA_ts k_t k_s D_ts.
+//
+// Decays without exponents of differences.  D_ts is never formed as exp(G_t - G_s) (whose
+// difference of prefix sums loses what a strong decay elsewhere in the chunk adds to both)
+// nor as a quotient.  The strictly lower pairs (t, s) split over four levels h = 1, 2, 4, 8
+// by the highest bit in which t and s differ: at level h, t lies in the upper and s in the
+// lower half of one aligned block of 2h tokens, and
+//   D_ts = F^h_t E^h_s,
+// F^h the inclusive prefix product of alpha inside the aligned block of h tokens and E^h
+// the exclusive suffix product.  Both are products of at most 8 alphas, at most 1 for
+// g <= 0 and exact to rounding for any g, and each level is one masked matrix product:
+// A' = sum_h mask_h((K F^h) (K E^h)^T).  The last level's F and E are the chunk's own.
+//
+// Launches:
+//   K10p (prep, one wave per (b, h, chunk)): K^, K-, Q^, T'', T, P, A', gC, beta.
+//   K10s (one workgroup of eight waves per (b, h, 32 columns of d_v)): the state recurrence
+//     forwards (U per token, S at every span start) beside the G recurrence backwards (W
+//     and dV per token, G at every span end, dS0).
+//   K10c (one workgroup of D/16 waves per (b, h, span of 8 chunks)): the span forwards from
+//     its start state (dQ, dbeta, dK and dg but for what depends on G), then backwards from
+//     its end gradient (the rest).  S cannot be walked back as the ungated backward does
+//     (that divides by gC), hence the two walks.
+
+#include <type_traits>
+
+#include "pm_cdna4.h"
+#include "pm_f32mfma.h"
+#include "pm_internal.h"
+
+namespace pm {
+namespace {
+
+constexpr int kSpan = 8;  // chunks per span (128 tokens)
+
+__device__ __forceinline__ f32x4_t ld4(const unsigned char* p) { return *reinterpret_cast<const f32x4_t*>(p); }
+__device__ __forceinline__ void st4(unsigned char* p, f32x4_t x) { *reinterpret_cast<f32x4_t*>(p) = x; }
+__device__ __forceinline__ void fence() { __builtin_amdgcn_sched_barrier(0); }
+constexpr f32x4_t kZero4 = {0.f, 0.f, 0.f, 0.f};
+
+// One chunk's record (floats): T''^T, T, P, A'^T as accumulator registers, then gC (D) and
+// beta (16), padded to a multiple of 64 (copied 256 bytes an instruction).
+template <int D>
+struct DecRec {
+    static constexpr int T2 = 0, TA = 256, PA = 512, AT = 768, GB = 1024, GBN = D + 64;
+    static constexpr int FLOATS = GB + GBN;
+};
+
+// Lane (g, r)'s operand reads of a swizzled tile of 16 fp32 rows (f32_chunk): row(b, i) =
+// X[r][16 i + 4 g ..] and col(b, e, i) = X[4 g + e][16 i + r].  The swizzle splits into a
+// part that depends on i mod 4 and a constant one: (4 i + x) ^ (4 y + z) = 4 (i ^ y) + (x ^ z)
+// for x, z < 4, and y < 4 leaves i's upper bit alone, so 13 registers address every read.
+template <int D>
+struct TileIdx {
+    int rb, rx[4], cb[4], cx[4];  // byte offsets
+    __device__ __forceinline__ TileIdx(int r, int g) {
+        rb = 16 * (r * (D / 4) + (g ^ (r & 3)));
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            rx[k] = 64 * (k ^ (r >> 2));
+            cb[k] = 16 * ((4 * g + k) * (D / 4) + ((r >> 2) ^ k)) + 4 * (r & 3);
+            cx[k] = 64 * (k ^ g);
+        }
+    }
+    __device__ __forceinline__ f32x4_t row(const unsigned char* b, int i) const {
+        return ld4(b + rb + rx[i & 3] + 256 * (i >> 2));
+    }
+    __device__ __forceinline__ float col(const unsigned char* b, int e, int i) const {
+        return *reinterpret_cast<const float*>(b + cb[e] + cx[i & 3] + 256 * (i >> 2));
+    }
+    // col for an i known only at run time (g: the lane's group)
+    __device__ __forceinline__ float colw(const unsigned char* b, int e, int i, int g) const {
+        return *reinterpret_cast<const float*>(b + cb[e] + 64 * (i ^ g));
+    }
+};
+// One element, and four consecutive ones, of a row through a range-checked buffer (byte
+// offsets off; zeros past the range)
+template <typename InT>
+__device__ __forceinline__ float buf_el(__amdgpu_buffer_rsrc_t rs, unsigned elem) {
+    if constexpr (sizeof(InT) == 2)
+        return __uint_as_float(static_cast<unsigned>(__builtin_amdgcn_raw_buffer_load_b16(rs, elem * 2, 0, 0)) << 16);
+    else
+        return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, elem * 4, 0, 0));
+}
+template <typename InT>
+__device__ __forceinline__ f32x4_t buf_el4(__amdgpu_buffer_rsrc_t rs, unsigned elem) {
+    if constexpr (sizeof(InT) == 2)
+        return widen4(__builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(rs, elem * 2, 0, 0)));
+    else
+        return __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rs, elem * 4, 0, 0));
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp_mov(float x) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, false));
+}
+// 4 bytes per lane buffer -> LDS (lane L's at lds_dst + 4 L), as dma16_asm
+__device__ __forceinline__ void dma4_asm(__amdgpu_buffer_rsrc_t rs, const void* lds_dst, unsigned voffset) {
+    const unsigned m0 = uniform(lds_addr(lds_dst));
+    __asm__ volatile("buffer_load_dword %0, %1, 0 offen lds" ::"v"(voffset), "s"(rs), "{m0}"(m0) : "memory");
+}
+// Ordering of this wave's own LDS accesses for the compiler (the hardware keeps a wave's
+// LDS operations in order)
+__device__ __forceinline__ void wave_lds_fence() { __asm__ volatile("" ::: "memory"); }
+
+// ---------------------------------------------------------------- K10p
+// Lane (r, g) = (lane & 15, lane >> 4) holds token r at d = 16 j + 4 g + v: the A and the B
+// operand of products contracting over d.  MFMA-bound: 4 levels x 2 products of 16 x 16 x D
+// (256 MFMAs at D = 128; a per-head gate needs the two Gram products only once, since its
+// D_ts does not depend on d).
+template <int D, typename InT, bool CHAN>
+__global__ __launch_bounds__(256) void dec_prep_kernel(
+    const InT* __restrict__ q, const InT* __restrict__ k, const float* __restrict__ beta,
+    const float* __restrict__ gate, int T, int H, int n_ch, long n_items, float* __restrict__ kh_ws,
+    float* __restrict__ kb_ws, float* __restrict__ qh_ws, float* __restrict__ rec_ws) {
+    // a per-channel gate takes 64 channels at a time (five values per channel and token live
+    // in registers); a per-head one needs all of them before its levels
+    constexpr int NH = CHAN ? D / 64 : 1, NJ = D / 16 / NH, NF = CHAN ? NJ : 1, NV = CHAN ? 4 : 1;
+    using R = DecRec<D>;
+    constexpr int TILE = kC16 * D * 4, TR = 16 * 17 * 4;
+    __shared__ __attribute__((aligned(16))) unsigned char smem[4 * (TILE + TR)];
+    const int lane = threadIdx.x & 63;
+    const int w = static_cast<int>(uniform(threadIdx.x >> 6));
+    const long item = static_cast<long>(blockIdx.x) * 4 + w;
+    if (item >= n_items) return;  // (waves are independent: no barrier below)
+    unsigned char* tile = smem + w * (TILE + TR);
+    float* tr = reinterpret_cast<float*>(tile + TILE);
+    const int pair = static_cast<int>(item / n_ch), c = static_cast<int>(item % n_ch);
+    const int seq = pair / H, h = pair % H;
+    const int base = c * kC16, clen = min(kC16, T - base);
+    const size_t tok0 = static_cast<size_t>(seq) * T + base;
+    const int r = lane & 15, g = lane >> 4;
+    const size_t tstride = static_cast<size_t>(H) * D;
+    const size_t row0 = tok0 * tstride + static_cast<size_t>(h) * D;
+    const unsigned n_el = static_cast<unsigned>((clen - 1) * tstride + D), n_hd = static_cast<unsigned>((clen - 1) * H + 1);
+    float* const kh = kh_ws + static_cast<size_t>(item) * kC16 * D;
+    float* const kb = kb_ws + static_cast<size_t>(item) * kC16 * D;
+    float* const qh = qh_ws + static_cast<size_t>(item) * kC16 * D;
+    float* const rec = rec_ws + static_cast<size_t>(item) * R::FLOATS;
+
+    const __amdgpu_buffer_rsrc_t rb = make_rsrc(beta + tok0 * H + h, n_hd * 4);
+    const float bc = buf_el<float>(rb, static_cast<unsigned>(r * H));
+    f32x4_t bt;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) bt[v] = buf_el<float>(rb, static_cast<unsigned>((4 * g + v) * H));
+
+    f32x4_t A = kZero4, P = kZero4;
+    float qk = 0.f;  // q_r . k_r, P's diagonal
+#pragma unroll
+    for (int hf = 0; hf < NH; ++hf) {
+        f32x4_t kf[NJ], qf[NJ];
+        float al[NF][NV];  // alpha of token r (rows past the end read g = 0: alpha = 1)
+        {
+            const __amdgpu_buffer_rsrc_t rk = make_rsrc(k + row0, n_el * sizeof(InT));
+            const __amdgpu_buffer_rsrc_t rq = make_rsrc(q + row0, n_el * sizeof(InT));
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const unsigned el = static_cast<unsigned>(r * tstride + 16 * (hf * NJ + j) + 4 * g);
+                kf[j] = buf_el4<InT>(rk, el);
+                qf[j] = buf_el4<InT>(rq, el);
+            }
+            if constexpr (CHAN) {
+                const __amdgpu_buffer_rsrc_t rg = make_rsrc(gate + row0, n_el * 4);
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) {
+                    const f32x4_t x = buf_el4<float>(rg, static_cast<unsigned>(r * tstride + 16 * (hf * NJ + j) + 4 * g));
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) al[j][v] = expf(x[v]);
+                }
+            } else {
+                al[0][0] = expf(buf_el<float>(make_rsrc(gate + tok0 * H + h, n_hd * 4), static_cast<unsigned>(r * H)));
+            }
+        }
+        // the levels: F, E and the block's product tot, of aligned blocks of h = 1, 2, 4, 8 tokens
+        float F[NF][NV], E[NF][NV], tot[NF][NV];
+#pragma unroll
+        for (int j = 0; j < NF; ++j)
+#pragma unroll
+            for (int v = 0; v < NV; ++v) F[j][v] = tot[j][v] = al[j][v], E[j][v] = 1.f;
+        auto fac = [](const float (&x)[NF][NV], int j, int v) { return CHAN ? x[CHAN ? j : 0][CHAN ? v : 0] : x[0][0]; };
+        f32x4_t gk = kZero4, gq = kZero4;  // per-head gate: K K^T and Q K^T
+        if constexpr (!CHAN) {
+            f32x4_t aa[4] = {kZero4, kZero4, kZero4, kZero4}, pa[4] = {kZero4, kZero4, kZero4, kZero4};
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    aa[v] = mfma4(kf[j][v], kf[j][v], aa[v]);
+                    pa[v] = mfma4(qf[j][v], kf[j][v], pa[v]);
+                }
+            gk = (aa[0] + aa[1]) + (aa[2] + aa[3]);
+            gq = (pa[0] + pa[1]) + (pa[2] + pa[3]);
+        }
+        auto level = [&](auto HB) __attribute__((always_inline)) {
+            constexpr int hb = decltype(HB)::value, hh = 1 << hb;
+            f32x4_t a4 = gk, p4 = gq;
+            if constexpr (CHAN) {
+                f32x4_t aa[4] = {kZero4, kZero4, kZero4, kZero4}, pa[4] = {kZero4, kZero4, kZero4, kZero4};
+#pragma unroll
+                for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const float rr = kf[j][v] * E[j][v];
+                        aa[v] = mfma4(kf[j][v] * F[j][v], rr, aa[v]);
+                        pa[v] = mfma4(qf[j][v] * F[j][v], rr, pa[v]);
+                    }
+                a4 = (aa[0] + aa[1]) + (aa[2] + aa[3]);
+                p4 = (pa[0] + pa[1]) + (pa[2] + pa[3]);
+            }
+            // entry (t, s) = (4 g + v, r) belongs to this level: t > s, highest differing bit hb
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int t = 4 * g + v;
+                const bool in = ((t ^ r) >> hb) == 1 && t > r;
+                float d = 1.f;
+                if constexpr (!CHAN) d = __shfl(F[0][0], t) * E[0][0];
+                A[v] += in ? d * a4[v] : 0.f;
+                P[v] += in ? d * p4[v] : 0.f;
+            }
+            constexpr int CTRL = hb == 0 ? 0xB1 : hb == 1 ? 0x4E : hb == 2 ? 0x141 : 0x140;
+            const bool up = (r & hh) != 0;
+#pragma unroll
+            for (int j = 0; j < NF; ++j)
+#pragma unroll
+                for (int v = 0; v < NV; ++v) {
+                    const float sib = dpp_mov<CTRL>(tot[j][v]);  // the other half's product
+                    F[j][v] *= up ? sib : 1.f;
+                    E[j][v] *= up ? 1.f : sib;
+                    tot[j][v] *= sib;
+                }
+        };
+        level(std::integral_constant<int, 0>{});
+        level(std::integral_constant<int, 1>{});
+        level(std::integral_constant<int, 2>{});
+        level(std::integral_constant<int, 3>{});
+        // K^, K- as swizzled row tiles; Q^ in operand order (below); gC
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            f32x4_t x, y, z, gc;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                qk = fmaf(qf[j][v], kf[j][v], qk);
+                x[v] = kf[j][v] * fac(F, j, v);
+                y[v] = kf[j][v] * fac(E, j, v);
+                z[v] = qf[j][v] * fac(F, j, v);
+                gc[v] = fac(tot, j, v);
+            }
+            const int o = 4 * f32_chunk<D>(r, 4 * (hf * NJ + j) + g);
+            *reinterpret_cast<f32x4_t*>(kh + o) = x;
+            *reinterpret_cast<f32x4_t*>(kb + o) = y;
+            st4(tile + 4 * o, z);
+            if (r == 0) *reinterpret_cast<f32x4_t*>(rec + R::GB + 16 * (hf * NJ + j) + 4 * g) = gc;
+        }
+    }
+    qk += __shfl_xor(qk, 16);
+    qk += __shfl_xor(qk, 32);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) P[v] = (4 * g + v == r) ? qk : P[v];
+    if (g == 0) rec[R::GB + D + r] = bc;
+    // A'^T through LDS
+#pragma unroll
+    for (int v = 0; v < 4; ++v) tr[(4 * g + v) * 17 + r] = A[v];
+    wave_lds_fence();
+    f32x4_t At;  // A'[r][4 g + v]
+#pragma unroll
+    for (int v = 0; v < 4; ++v) At[v] = tr[r * 17 + 4 * g + v];
+    const TileIdx<D> ix(r, g);
+    // Q^ as the A operand of Q^^T dO: [m][lane][e] = Q^[4 g + e][16 m + r]
+#pragma unroll
+    for (int m = 0; m < D / 16; ++m) {
+        f32x4_t x;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = ix.col(tile, e, m);
+        *reinterpret_cast<f32x4_t*>(qh + 4 * (64 * m + lane)) = x;
+    }
+
+    // T = (I + diag(beta) A')^-1 = (I+N)(I+N^2)(I+N^4)(I+N^8), N = -diag(beta) A' (N^16 = 0)
+    f32x4_t N, Nt, eye;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        N[v] = -bt[v] * A[v];
+        Nt[v] = -bc * At[v];
+        eye[v] = 4 * g + v == r ? 1.f : 0.f;
+    }
+    const f32x4_t N2 = mm16(Nt, N), N2t = mm16(N, Nt);
+    const f32x4_t N4 = mm16(N2t, N2), N4t = mm16(N2, N2t);
+    const f32x4_t N8 = mm16(N4t, N4);
+    const f32x4_t F1t = mm16(eye + N2, eye + Nt);
+    const f32x4_t F2t = mm16(eye + N4, F1t);
+    const f32x4_t Tt = mm16(eye + N8, F2t);   // T^T
+    const f32x4_t Ta = mm16(F2t, eye + N8);   // T
+    f32x4_t tw;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) tw[v] = -bt[v] * Tt[v];
+    *reinterpret_cast<f32x4_t*>(rec + R::T2 + 4 * lane) = tw;
+    *reinterpret_cast<f32x4_t*>(rec + R::TA + 4 * lane) = Ta;
+    *reinterpret_cast<f32x4_t*>(rec + R::PA + 4 * lane) = P;
+    *reinterpret_cast<f32x4_t*>(rec + R::AT + 4 * lane) = At;
+}
+
+// ---------------------------------------------------------------- K10s
+// Eight waves: 0, 1 the state recurrence (16 columns of S each), 3 its copies; 6, 7 the
+// gradient recurrence (16 columns of G each), 5 its copies and the stores of W and dV; 2
+// and 4 form Q^^T dO for waves 7 and 6 one chunk ahead, from Q^ in operand order straight
+// into registers.  Waves w and w + 4 share a SIMD, so the four chains take one each.  The
+// two recurrences walk the chunks in opposite directions and share the workgroup's barriers
+// (one per chunk); each keeps three chunk buffers, one in use, one landed, one landing.
+template <int D>
+struct DsGeo {
+    static constexpr int NT = D / 16, NI = kC16 * D * 4 / 1024, TILE = kC16 * D * 4;
+    static constexpr int NB = 3;
+    // state half: K^, K- rows, T''^T, V columns of each chain wave, gC
+    static constexpr int H_KH = 0, H_KB = TILE, H_T = 2 * TILE, H_V = H_T + 1024, H_G = H_V + 2048;
+    static constexpr int HBUF = H_G + D * 4;
+    static constexpr int H_NCP = 2 * NI + 3 + D / 64;
+    // gradient half: K^, K- rows, dO columns, T, P, gC and beta
+    static constexpr int S_KH = 0, S_KB = TILE, S_O = 2 * TILE, S_T = S_O + 2048, S_P = S_T + 1024, S_G = S_P + 1024;
+    static constexpr int SBUF = S_G + DecRec<D>::GBN * 4;
+    static constexpr int S_NCP = 2 * NI + 4 + DecRec<D>::GBN / 64;
+    static constexpr int S_NST = 4;  // W and dV stores per chunk
+    static constexpr int OFF_S = NB * HBUF;
+    static constexpr int OFF_H = OFF_S + NB * SBUF;           // 2 slots x 2 chains: Q^^T dO
+    static constexpr int OFF_W = OFF_H + 4 * NT * 1024;       // 2 slots x 2 chains: W, beta
+    static constexpr int WSLOT = 1024 + 64;
+    static constexpr int BYTES = OFF_W + 4 * WSLOT;
+    static_assert(BYTES <= 160 * 1024 && S_NCP + S_NST <= 63 && H_NCP <= 63, "LDS / vmcnt");
+    static_assert(HBUF % 16 == 0 && SBUF % 16 == 0, "alignment");
+};
+
+template <int D, typename InT>
+__global__ __launch_bounds__(512) void dec_sweep_kernel(
+    const InT* __restrict__ v, const float* __restrict__ s0, const float* __restrict__ go,
+    const float* __restrict__ gs, float* __restrict__ gv, float* __restrict__ gs0, const float* __restrict__ kh,
+    const float* __restrict__ kb, const float* __restrict__ qh, const float* __restrict__ rec,
+    float* __restrict__ w_out, float* __restrict__ u_out, float* __restrict__ s_hist, float* __restrict__ g_hist,
+    int n_pairs, int T, int H, int n_ch, int n_span) {
+    using G = DsGeo<D>;
+    using R = DecRec<D>;
+    constexpr int NT = G::NT, NI = G::NI, NB = G::NB, n_tiles = D / 32;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    // XCD-aware placement: the n_tiles workgroups of a pair share bid % 8
+    const int bid = blockIdx.x, xcd = bid & 7, bslot = bid >> 3;
+    const int tile = bslot % n_tiles, pair = (bslot / n_tiles) * 8 + xcd;
+    if (pair >= n_pairs || n_ch <= 0) return;
+    const int seq = pair / H, h = pair % H;
+    const size_t tok0 = static_cast<size_t>(seq) * T;
+    const int col0 = tile * 32;
+    const int w = static_cast<int>(uniform(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int r = lane & 15, g = lane >> 4;
+    const size_t tstride = static_cast<size_t>(H) * D;
+    const size_t sbase = static_cast<size_t>(pair) * D * D;
+    const size_t item0 = static_cast<size_t>(pair) * n_ch;
+    const TileIdx<D> ix(r, g);
+
+    auto hbuf = [=](int c) { return smem + (c % NB) * G::HBUF; };
+    auto sbuf = [=](int c) { return smem + G::OFF_S + (c % NB) * G::SBUF; };
+    auto hslot = [=](int c, int which) { return smem + G::OFF_H + ((c & 1) * 2 + which) * NT * 1024; };
+    auto wslot = [=](int c, int which) { return smem + G::OFF_W + ((c & 1) * 2 + which) * G::WSLOT; };
+    auto row0_of = [=](int c, int col) { return (tok0 + c * kC16) * tstride + static_cast<size_t>(h) * D + col; };
+    auto els_of = [=](int c, int cols) {  // elements from a column block's first row to its last row's end
+        return static_cast<unsigned>((min(kC16, T - c * kC16) - 1) * tstride + cols);
+    };
+    auto copy_tile = [=](const float* ws, int c, unsigned char* dst) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc(ws + (item0 + c) * kC16 * D, G::TILE);
+        unsigned char* d0 = uniform_ptr(dst);
+#pragma unroll
+        for (int i = 0; i < NI; ++i) dma16_asm(rs, d0 + 1024 * i, static_cast<unsigned>(1024 * i + 16 * lane));
+    };
+
+    if (w < 2) {
+        // ============ the state recurrence: S columns col0 + 16 w + [0, 16) ============
+        const int ecol = col0 + 16 * w + r;
+        f32x4_t S[NT];
+#pragma unroll
+        for (int m = 0; m < NT; ++m)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                S[m][e] = s0 ? s0[sbase + static_cast<size_t>(16 * m + 4 * g + e) * D + ecol] : 0.f;
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), seen by the compiler: no wait for S0 in the loop
+        lds_barrier();                       // B0
+        float kt[4][NT];  // K-^T operand of chunk i - 1: K-[4 g + e][16 m + r]
+        f32x4_t gc[NT], Up = kZero4;
+        for (int i = 0; i < n_ch; ++i) {
+            const unsigned char* b = hbuf(i);
+            f32x4_t kf[NT], vr;
+#pragma unroll
+            for (int m = 0; m < NT; ++m) kf[m] = ix.row(b + G::H_KH, m);
+            const InT* Vf = reinterpret_cast<const InT*>(b + G::H_V + 1024 * w);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) vr[e] = to_f32<InT>(Vf[(4 * g + e) * 16 + r]);
+            const f32x4_t tt = ld4(b + G::H_T + 16 * lane);
+            fence();
+            // S = Diag(gC) S + K-^T U of chunk i - 1
+            if (i > 0) {
+#pragma unroll
+                for (int m = 0; m < NT; ++m) S[m] = gc[m] * S[m];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int m = 0; m < NT; ++m) S[m] = mfma4(kt[e][m], Up[e], S[m]);
+            }
+            if (i % kSpan == 0) {
+                float* hp = s_hist + ((static_cast<size_t>(pair) * n_span + i / kSpan) * NT + col0 / 16 + w) * NT * 256;
+#pragma unroll
+                for (int m = 0; m < NT; ++m) *reinterpret_cast<f32x4_t*>(hp + m * 256 + 4 * lane) = S[m];
+            }
+            fence();
+            // X = K^ S - V, U = T'' X
+            f32x4_t xa[4] = {-vr, kZero4, kZero4, kZero4};
+#pragma unroll
+            for (int m = 0; m < NT; ++m)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) xa[e] = mfma4(kf[m][e], S[m][e], xa[e]);
+            const f32x4_t X = (xa[0] + xa[1]) + (xa[2] + xa[3]);
+            Up = mm16(tt, X);
+            // U's rows (U^T = X^T T''^T): lane (g, r) holds U[r][col0 + 16 w + 4 g ..]
+            const f32x4_t Ut = mm16(X, tt);
+            *reinterpret_cast<f32x4_t*>(u_out + (item0 + i) * kC16 * D +
+                                        4 * f32_chunk<D>(r, (col0 + 16 * w) / 4 + g)) = Ut;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int m = 0; m < NT; ++m) kt[e][m] = ix.col(b + G::H_KB, e, m);
+#pragma unroll
+            for (int m = 0; m < NT; ++m) gc[m] = ld4(b + G::H_G + 4 * (16 * m + 4 * g));
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), seen by the compiler
+            lds_barrier();
+        }
+        lds_barrier();
+    } else if (w == 3) {
+        // ============ the state half's copies, two chunks ahead ============
+        auto copies = [=](int c) __attribute__((always_inline)) {
+            unsigned char* b = hbuf(c);
+            const float* rc = rec + (item0 + c) * R::FLOATS;
+            copy_tile(kh, c, b + G::H_KH);
+            copy_tile(kb, c, b + G::H_KB);
+            dma16_asm(make_rsrc(rc + R::T2, 1024), uniform_ptr(b + G::H_T), static_cast<unsigned>(16 * lane));
+            constexpr int LPR = 16 * sizeof(InT) / 16;  // lanes per row of 16 columns
+#pragma unroll
+            for (int j = 0; j < 2; ++j)  // (bf16: lanes 32 .. 63 address rows past the chunk and read zeros)
+                dma16_asm(make_rsrc(v + row0_of(c, col0 + 16 * j), els_of(c, 16) * sizeof(InT)),
+                          uniform_ptr(b + G::H_V + 1024 * j),
+                          static_cast<unsigned>((lane / LPR) * tstride * sizeof(InT) + 16 * (lane % LPR)));
+            const __amdgpu_buffer_rsrc_t rg = make_rsrc(rc + R::GB, D * 4);
+#pragma unroll
+            for (int j = 0; j < D / 64; ++j)
+                dma4_asm(rg, uniform_ptr(b + G::H_G + 256 * j), static_cast<unsigned>(256 * j + 4 * lane));
+        };
+        copies(0);
+        if (n_ch > 1) {
+            copies(1);
+            wait_vm_n<G::H_NCP>();
+        } else {
+            wait_vm_n<0>();
+        }
+        lds_barrier();  // B0
+        for (int i = 0; i < n_ch; ++i) {
+            if (i + 2 < n_ch) {
+                copies(i + 2);
+                wait_vm_n<G::H_NCP>();
+            } else {
+                wait_vm_n<0>();
+            }
+            lds_barrier();
+        }
+        lds_barrier();
+    } else if (w == 2 || w == 4) {
+        // ============ Q^^T dO of chunk n_ch - 1 - i for the gradient chain cw ============
+        const int cw = w == 4 ? 0 : 1;
+        f32x4_t qn[NT];
+        auto fetch = [&](int c) __attribute__((always_inline)) {
+            const float* qp = qh + (item0 + c) * kC16 * D + 4 * lane;
+#pragma unroll
+            for (int m = 0; m < NT; ++m) qn[m] = *reinterpret_cast<const f32x4_t*>(qp + 256 * m);
+        };
+        fetch(n_ch - 1);
+        lds_barrier();  // B0
+        for (int i = 0; i < n_ch; ++i) {
+            const int ch = n_ch - 1 - i;
+            f32x4_t qc[NT];
+#pragma unroll
+            for (int m = 0; m < NT; ++m) qc[m] = qn[m];
+            if (ch > 0) fetch(ch - 1);
+            const float* Of = reinterpret_cast<const float*>(sbuf(ch) + G::S_O + 1024 * cw);
+            f32x4_t dOc;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dOc[e] = Of[(4 * g + e) * 16 + r];
+            f32x4_t hq[NT];
+#pragma unroll
+            for (int m = 0; m < NT; ++m) hq[m] = kZero4;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int m = 0; m < NT; ++m) hq[m] = mfma4(qc[m][e], dOc[e], hq[m]);
+            unsigned char* slot = hslot(ch, cw);
+#pragma unroll
+            for (int m = 0; m < NT; ++m) st4(slot + 1024 * m + 16 * lane, hq[m]);
+            lds_barrier();
+        }
+        lds_barrier();
+    } else if (w == 5) {
+        // ============ the gradient half's copies, and its stores one chunk behind ============
+        auto copies = [=](int c) __attribute__((always_inline)) {
+            unsigned char* b = sbuf(c);
+            const float* rc = rec + (item0 + c) * R::FLOATS;
+            copy_tile(kh, c, b + G::S_KH);
+            copy_tile(kb, c, b + G::S_KB);
+#pragma unroll
+            for (int j = 0; j < 2; ++j)  // a null dO reads zeros (a zero-length range)
+                dma16_asm(make_rsrc(go ? go + row0_of(c, col0 + 16 * j) : go, go ? els_of(c, 16) * 4 : 0u),
+                          uniform_ptr(b + G::S_O + 1024 * j),
+                          static_cast<unsigned>((lane >> 2) * tstride * 4 + 16 * (lane & 3)));
+            dma16_asm(make_rsrc(rc + R::TA, 1024), uniform_ptr(b + G::S_T), static_cast<unsigned>(16 * lane));
+            dma16_asm(make_rsrc(rc + R::PA, 1024), uniform_ptr(b + G::S_P), static_cast<unsigned>(16 * lane));
+            const __amdgpu_buffer_rsrc_t rg = make_rsrc(rc + R::GB, R::GBN * 4);
+#pragma unroll
+            for (int j = 0; j < R::GBN / 64; ++j)
+                dma4_asm(rg, uniform_ptr(b + G::S_G + 256 * j), static_cast<unsigned>(256 * j + 4 * lane));
+        };
+        copies(n_ch - 1);
+        if (n_ch > 1) {
+            copies(n_ch - 2);
+            wait_vm_n<G::S_NCP>();
+        } else {
+            wait_vm_n<0>();
+        }
+        lds_barrier();  // B0
+        for (int i = 0; i <= n_ch + 1; ++i) {
+            const bool cp = n_ch - 3 - i >= 0, st = i >= 2;
+            if (cp) copies(n_ch - 3 - i);
+            if (st) {
+                const int cs = n_ch - i + 1;  // the chunk the chains ran in iteration i - 1
+                const int t = lane >> 2, p = lane & 3;
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const float* ws = reinterpret_cast<const float*>(wslot(cs, j));
+                    const float bt = ws[256 + t];
+                    f32x4_t x;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) x[e] = ws[4 * (16 * (t >> 2) + 4 * p + e) + (t & 3)];
+                    *reinterpret_cast<f32x4_t*>(w_out + (item0 + cs) * kC16 * D +
+                                                4 * f32_chunk<D>(t, (col0 + 16 * j) / 4 + p)) = x;
+                    __builtin_amdgcn_raw_buffer_store_b128(
+                        __builtin_bit_cast(u32x4_t, x * bt),
+                        make_rsrc(gv + row0_of(cs, col0 + 16 * j), els_of(cs, 16) * 4),
+                        static_cast<unsigned>((t * tstride + 4 * p) * 4), 0, 0);
+                }
+            }
+            if (i <= n_ch) {
+                // chunk n_ch - 2 - i has landed (the next iteration's); the newest copies and
+                // this iteration's stores may be in flight
+                if (n_ch - 2 - i >= 0) {
+                    if (cp && st) wait_vm_n<G::S_NCP + G::S_NST>();
+                    else if (cp) wait_vm_n<G::S_NCP>();
+                    else wait_vm_n<0>();
+                }
+                lds_barrier();
+            }
+        }
+    } else {
+        // ============ the gradient recurrence: G columns col0 + 16 cw + [0, 16) ============
+        const int cw = w - 6;
+        const int ecol = col0 + 16 * cw + r;
+        f32x4_t Gm[NT];
+#pragma unroll
+        for (int m = 0; m < NT; ++m)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                Gm[m][e] = gs ? gs[sbase + static_cast<size_t>(16 * m + 4 * g + e) * D + ecol] : 0.f;
+        __builtin_amdgcn_s_waitcnt(0x0F70);
+        lds_barrier();  // B0
+        // Iteration i runs chunk n_ch - i from operands read in iteration i - 1 (its buffer has
+        // landed by then); only Q^^T dO is read in iteration i
+        f32x4_t kf[NT], gc[NT], dOc = kZero4, ta = kZero4, b4 = kZero4, pp = kZero4;
+        float kt[4][NT];
+        for (int i = 0; i <= n_ch; ++i) {
+            if (i >= 1) {
+                const int c = n_ch - i;
+                if (c == n_ch - 1 || c % kSpan == kSpan - 1) {
+                    float* hp = g_hist + ((static_cast<size_t>(pair) * n_span + c / kSpan) * NT + col0 / 16 + cw) * NT * 256;
+#pragma unroll
+                    for (int m = 0; m < NT; ++m) *reinterpret_cast<f32x4_t*>(hp + m * 256 + 4 * lane) = Gm[m];
+                }
+                f32x4_t hq[NT];
+#pragma unroll
+                for (int m = 0; m < NT; ++m) hq[m] = ld4(hslot(c, cw) + 1024 * m + 16 * lane);
+                // Y = K- G, dU = Y + P^T dO, W = T^T dU
+                f32x4_t ya[4] = {kZero4, kZero4, kZero4, kZero4};
+#pragma unroll
+                for (int m = 0; m < NT; ++m)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) ya[e] = mfma4(kf[m][e], Gm[m][e], ya[e]);
+                const f32x4_t dU = mm16(pp, dOc, (ya[0] + ya[1]) + (ya[2] + ya[3]));
+                const f32x4_t W = mm16(ta, dU);
+                const f32x4_t nbW = -(W * b4);
+                st4(wslot(c, cw) + 16 * lane, W);
+                if (r == 0) st4(wslot(c, cw) + 1024 + 16 * g, b4);
+                // G = Diag(gC) G + Q^^T dO - K^^T diag(beta) W
+#pragma unroll
+                for (int m = 0; m < NT; ++m) Gm[m] = gc[m] * Gm[m] + hq[m];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int m = 0; m < NT; ++m) Gm[m] = mfma4(kt[e][m], nbW[e], Gm[m]);
+            }
+            if (i < n_ch) {
+                const unsigned char* b = sbuf(n_ch - 1 - i);
+#pragma unroll
+                for (int m = 0; m < NT; ++m) kf[m] = ix.row(b + G::S_KB, m);
+                const float* Of = reinterpret_cast<const float*>(b + G::S_O + 1024 * cw);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) dOc[e] = Of[(4 * g + e) * 16 + r];
+                ta = ld4(b + G::S_T + 16 * lane);
+                pp = ld4(b + G::S_P + 16 * lane);
+                b4 = ld4(b + G::S_G + 4 * D + 16 * g);
+#pragma unroll
+                for (int m = 0; m < NT; ++m) gc[m] = ld4(b + G::S_G + 4 * (16 * m + 4 * g));
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int m = 0; m < NT; ++m) kt[e][m] = ix.col(b + G::S_KH, e, m);
+            }
+            lds_barrier();
+        }
+#pragma unroll
+        for (int m = 0; m < NT; ++m)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) gs0[sbase + static_cast<size_t>(16 * m + 4 * g + e) * D + ecol] = Gm[m][e];
+    }
+}
+
+// ---------------------------------------------------------------- K10c
+// Wave w owns rows 16 w + [0, 16) of d: lane (g, r) holds S^T and G^T [16 i + 4 g + e][16 w + r]
+// in tile i, and of each chunk's tokens 4 g + e the values at d = 16 w + r (k, q, v, alpha
+// from global memory, one chunk ahead), from which it forms its decay factors: its own four
+// alphas give F^4 and E^4, two lane exchanges the levels 8 and 16.  The pairs (t, s) of
+// levels 8 and 4 are masked matrix products over the chunk's tokens, those inside a lane's
+// four tokens plain arithmetic.
+template <int D>
+struct DcGeo {
+    static constexpr int NW = D / 16, NT = D / 16, NI = kC16 * D * 4 / 1024, TILE = kC16 * D * 4;
+    static constexpr int B_O = 0, B_W = TILE, B_U = 2 * TILE, BUF = 3 * TILE;  // dO, W, U rows
+    static constexpr int NC = 3 * NI;                        // copies per chunk
+    static constexpr int OFF_PP = 2 * BUF;                   // per wave: dO U^T, W U^T parts [t][s]
+    static constexpr int OFF_TR = OFF_PP + NW * 2048;        // totals dP, diag(beta) dA as rows [t][s]
+    static constexpr int OFF_TC = OFF_TR + 2048;             // ... as columns [s][t], stride 20
+    static constexpr int OFF_DB = OFF_TC + 2 * 16 * 20 * 4;  // dbeta parts: 2 slots x NW x 16
+    static constexpr int OFF_EC = OFF_DB + 2 * NW * 64;      // per chunk of the span: sum_t of dg's own terms, D
+    static constexpr int OFF_GG = OFF_EC + kSpan * D * 4;    // per-head gate: dg parts, chunk x wave x 16
+    static constexpr int OFF_MID = OFF_GG + kSpan * NW * 64;  // S^T in mid-span
+    static constexpr int BYTES = OFF_MID + NW * NT * 1024;
+    static_assert(BYTES <= 160 * 1024, "LDS");
+};
+
+template <int D, typename InT, bool CHAN>
+__global__ __launch_bounds__(D * 4) void dec_span_kernel(
+    const InT* __restrict__ q, const InT* __restrict__ k, const InT* __restrict__ v, const float* __restrict__ gate,
+    const float* __restrict__ go, const float* __restrict__ rec, const float* __restrict__ s_hist,
+    const float* __restrict__ g_hist, const float* __restrict__ w_in, const float* __restrict__ u_in,
+    float* __restrict__ gq, float* __restrict__ gk, float* __restrict__ gbeta, float* __restrict__ gg, int T, int H,
+    int n_ch, int n_span) {
+    using G = DcGeo<D>;
+    using R = DecRec<D>;
+    constexpr int NW = G::NW, NT = G::NT;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int pair = blockIdx.x / n_span, span = blockIdx.x % n_span;
+    const int seq = pair / H, h = pair % H;
+    const int c0 = span * kSpan, nm = min(kSpan, n_ch - c0);  // chunks of this span
+    const size_t tok0 = static_cast<size_t>(seq) * T + static_cast<size_t>(c0) * kC16;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = static_cast<int>(uniform(static_cast<unsigned>(tid >> 6)));
+    const int r = lane & 15, g = lane >> 4;
+    const size_t tstride = static_cast<size_t>(H) * D;
+    const size_t item0 = static_cast<size_t>(pair) * n_ch + c0;
+    const TileIdx<D> ix(r, g);
+
+    auto buf = [=](int m) { return smem + (m & 1) * G::BUF; };
+    auto clen_of = [=](int m) { return min(kC16, T - (c0 + m) * kC16); };
+    auto row0_of = [=](int m, int col) { return (tok0 + m * kC16) * tstride + static_cast<size_t>(h) * D + col; };
+    // copy number x of chunk m (one branch per source); wave w issues x = w, w + NW, ...
+    auto issue = [=](int m) __attribute__((always_inline)) {
+        unsigned char* b = buf(m);
+#pragma unroll
+        for (int n = 0; n < G::NC / NW; ++n) {
+            const int x = w + n * NW, which = x / G::NI, i = x % G::NI;
+            if (which == 0) {
+                // dO rows, swizzled here; a null dO reads zeros (a zero-length range)
+                const int ch = 64 * i + lane, t = ch / (D / 4), p = (ch % (D / 4)) ^ t;
+                const unsigned nb = static_cast<unsigned>(((clen_of(m) - 1) * tstride + D) * 4);
+                dma16_asm(make_rsrc(go ? go + row0_of(m, 0) : go, go ? nb : 0u), uniform_ptr(b + G::B_O + 1024 * i),
+                          static_cast<unsigned>(t * tstride * 4 + 16 * p));
+            } else if (which == 1) {
+                dma16_asm(make_rsrc(w_in + (item0 + m) * kC16 * D, G::TILE), uniform_ptr(b + G::B_W + 1024 * i),
+                          static_cast<unsigned>(1024 * i + 16 * lane));
+            } else {
+                dma16_asm(make_rsrc(u_in + (item0 + m) * kC16 * D, G::TILE), uniform_ptr(b + G::B_U + 1024 * i),
+                          static_cast<unsigned>(1024 * i + 16 * lane));
+            }
+        }
+    };
+    constexpr int kMine = G::NC / NW;  // copies each wave issues per chunk
+    static_assert(G::NC % NW == 0, "copies divide over the waves");
+
+    // this lane's tokens of a chunk, as loaded (tokens past the end read zeros)
+    struct Own {
+        f32x4_t k, q, x, lg, b4;  // x: v (forwards) or the gradient so far of k (backwards)
+        f32x4_t y;                // backwards: the gradient so far of the gate
+        float br;
+    };
+    auto load_own = [=](int m, bool fwd) __attribute__((always_inline)) {
+        Own o;
+        const int clen = clen_of(m);
+        const unsigned nel = static_cast<unsigned>((clen - 1) * tstride + 16);
+        const size_t r0 = row0_of(m, 16 * w);
+        const __amdgpu_buffer_rsrc_t rk = make_rsrc(k + r0, nel * sizeof(InT)), rq = make_rsrc(q + r0, nel * sizeof(InT));
+        const __amdgpu_buffer_rsrc_t rv = make_rsrc(v + r0, nel * sizeof(InT)), rgk = make_rsrc(gk + r0, nel * 4);
+        const __amdgpu_buffer_rsrc_t rg = CHAN ? make_rsrc(gate + r0, nel * 4)
+                                               : make_rsrc(gate + (tok0 + m * kC16) * H + h,
+                                                           static_cast<unsigned>(((clen - 1) * H + 1) * 4));
+        const __amdgpu_buffer_rsrc_t rgg = make_rsrc(CHAN ? gg + r0 : gg, CHAN ? nel * 4 : 0u);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const unsigned el = static_cast<unsigned>((4 * g + e) * tstride + r);
+            o.k[e] = buf_el<InT>(rk, el);
+            o.q[e] = buf_el<InT>(rq, el);
+            o.lg[e] = buf_el<float>(rg, CHAN ? el : static_cast<unsigned>((4 * g + e) * H));
+            o.x[e] = fwd ? buf_el<InT>(rv, el) : buf_el<float>(rgk, el);
+            o.y[e] = (CHAN && !fwd) ? buf_el<float>(rgg, el) : 0.f;
+        }
+        const float* rc = rec + (item0 + m) * R::FLOATS + R::GB + D;
+        o.b4 = *reinterpret_cast<const f32x4_t*>(rc + 4 * g);
+        o.br = rc[r];
+        return o;
+    };
+    // decay factors of this lane's four tokens at d = 16 w + r
+    struct Dec {
+        f32x4_t al, F4, E4, F8, E8, F, E;
+        float gc;
+    };
+    auto decays = [=](f32x4_t lg) __attribute__((always_inline)) {
+        Dec x;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x.al[e] = expf(lg[e]);
+        x.F4[0] = x.al[0];
+#pragma unroll
+        for (int e = 1; e < 4; ++e) x.F4[e] = x.F4[e - 1] * x.al[e];
+        x.E4[3] = 1.f;
+        x.E4[2] = x.al[3];
+        x.E4[1] = x.al[2] * x.E4[2];
+        x.E4[0] = x.al[1] * x.E4[1];
+        const float s4 = __shfl_xor(x.F4[3], 16);  // the sibling block's product
+        x.F8 = (g & 1) ? x.F4 * s4 : x.F4;
+        x.E8 = (g & 1) ? x.E4 : x.E4 * s4;
+        const float t8 = x.F4[3] * s4, s8 = __shfl_xor(t8, 32);
+        x.F = (g & 2) ? x.F8 * s8 : x.F8;
+        x.E = (g & 2) ? x.E8 : x.E8 * s8;
+        x.gc = t8 * s8;
+        return x;
+    };
+    // sums over the 16 tokens of a lane's column (4 own, 4 lane groups), all groups equal
+    auto col_total = [=](f32x4_t x) __attribute__((always_inline)) {
+        float s = (x[0] + x[1]) + (x[2] + x[3]);
+        s += __shfl_xor(s, 16);
+        s += __shfl_xor(s, 32);
+        return s;
+    };
+
+    // S^T at the span's start, by rows of d, gathered from the column-block layout: S[16 w +
+    // r][16 i + 4 g + e] is in column block i, tile w, lane 16 (r >> 2) + 4 g + e, register r & 3
+    f32x4_t St[NT];
+    {
+        const float* sp = s_hist + (static_cast<size_t>(pair) * n_span + span) * D * D;
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                St[i][e] = sp[(static_cast<size_t>(i) * NT + w) * 256 + 4 * (16 * (r >> 2) + 4 * g + e) + (r & 3)];
+    }
+    issue(0);
+    if (nm > 1) issue(1);
+    Own own = load_own(0, true);
+    wait_vm_n<0>();
+    lds_barrier();
+
+    // ================ forwards ================
+    // S^T at the end of chunk kSpan / 2 - 1, kept for the way back (this wave's own)
+    unsigned char* const mid = smem + G::OFF_MID + w * NT * 1024 + 16 * lane;
+    for (int m = 0; m < nm; ++m) {
+        const unsigned char* b = buf(m);
+        if (m == kSpan / 2) {
+#pragma unroll
+            for (int i = 0; i < NT; ++i) st4(mid + 1024 * i, St[i]);
+        }
+        // dO S^T, W S^T, and this wave's parts of dO U^T and W U^T
+        f32x4_t qa[2] = {kZero4, kZero4}, wa[2] = {kZero4, kZero4}, pp = kZero4, pa = kZero4;
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+            const f32x4_t dor = ix.row(b + G::B_O, i);
+            const f32x4_t wrw = ix.row(b + G::B_W, i);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                qa[e & 1] = mfma4(dor[e], St[i][e], qa[e & 1]);
+                wa[e & 1] = mfma4(wrw[e], St[i][e], wa[e & 1]);
+            }
+            if (i == w) {
+                const f32x4_t ur = ix.row(b + G::B_U, i);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    pp = mfma4(ur[e], dor[e], pp);  // (U dO^T)[4 g + v][r] = (dO U^T)[r][4 g + v]
+                    pa = mfma4(ur[e], wrw[e], pa);
+                }
+            }
+        }
+        unsigned char* part = smem + G::OFF_PP + w * 2048;
+        st4(part + 16 * (4 * r + g), pp);
+        st4(part + 1024 + 16 * (4 * r + g), pa);
+        f32x4_t wj;  // W at this lane's columns 16 w + r of d_v
+#pragma unroll
+        for (int e = 0; e < 4; ++e) wj[e] = ix.colw(b + G::B_W, e, w, g);
+        const f32x4_t kk = own.k, qq = own.q, b4 = own.b4;
+        const float br = own.br;
+        const Dec x = decays(own.lg);
+        const f32x4_t khat = kk * x.F, kbar = kk * x.E;
+        // S^T = gC S^T + U^T K-
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+            float uc[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) uc[e] = ix.col(b + G::B_U, e, i);
+            St[i] = St[i] * x.gc;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) St[i] = mfma4(uc[e], kbar[e], St[i]);
+        }
+        const f32x4_t dQh = qa[0] + qa[1];          // dO S^T [4 g + v][16 w + r]
+        const f32x4_t WS = wa[0] + wa[1];           // W S^T
+        const f32x4_t kdk = -(b4 * WS);             // dL/dK^
+        {
+            // this wave's part of W.V - K^ . W S^T per token 4 g + v
+            f32x4_t s = wj * own.x - khat * WS;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[e] = row16_sum(s[e]);
+            if (r == 0) st4(smem + G::OFF_DB + ((m & 1) * NW + w) * 64 + 16 * g, s);
+        }
+        lds_barrier();  // Y: the parts are in LDS; every wave is done reading chunk m's rows
+        if (m + 2 < nm) issue(m + 2);
+        for (int z = tid; z < 512; z += NW * 64) {
+            const int mat = z >> 8, t = (z >> 4) & 15, s = z & 15;
+            float sum = 0.f;
+#pragma unroll
+            for (int ww = 0; ww < NW; ++ww)
+                sum += reinterpret_cast<const float*>(smem + G::OFF_PP + ww * 2048 + mat * 1024)[16 * t + s];
+            const float val = mat == 0 ? (s <= t ? sum : 0.f) : (s < t ? -sum : 0.f);
+            reinterpret_cast<float*>(smem + G::OFF_TR + mat * 1024)[16 * t + s] = val;
+            reinterpret_cast<float*>(smem + G::OFF_TC + mat * 1280)[20 * s + t] = val;
+        }
+        // chunk m + 1's copies have landed; chunk m + 2's may be in flight
+        if (m + 2 < nm) wait_vm_n<kMine>();
+        else wait_vm_n<0>();
+        lds_barrier();  // Z: totals in LDS, chunk m + 1 in its buffer
+        if (m + 1 < nm) own = load_own(m + 1, true);
+        const f32x4_t dpr = ld4(smem + G::OFF_TR + 16 * (4 * r + g));            // dP[r][4 g ..]
+        const f32x4_t dar = ld4(smem + G::OFF_TR + 1024 + 16 * (4 * r + g));     // dA[r][4 g ..]
+        const f32x4_t dpc = ld4(smem + G::OFF_TC + 4 * (20 * r + 4 * g));        // dP[4 g ..][r]
+        const f32x4_t dac = ld4(smem + G::OFF_TC + 1280 + 4 * (20 * r + 4 * g)); // dA[4 g ..][r]
+        // pairs between blocks of four tokens: rows (t = r, s = 4 g + e) and columns (s = r,
+        // t = 4 g + e) of each level's mask; dA' = diag(beta) dA
+        const int rb = r >> 2;
+        const bool r8 = r >= 8 && g < 2, c8 = r < 8 && g >= 2;
+        const bool r4 = (rb & 1) && g == rb - 1, c4 = !(rb & 1) && g == rb + 1;
+        const f32x4_t ke8 = kk * x.E8, kf8 = kk * x.F8, qf8 = qq * x.F8;
+        const f32x4_t ke4 = kk * x.E4, kf4 = kk * x.F4, qf4 = qq * x.F4;
+        f32x4_t zq8 = kZero4, zk8 = kZero4, zc8 = kZero4, zq4 = kZero4, zk4 = kZero4, zc4 = kZero4;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float a = dpr[e], bb = br * dar[e], cc = dpc[e], dd = dac[e] * b4[e];
+            zq8 = mfma4(r8 ? a : 0.f, ke8[e], zq8);
+            zk8 = mfma4(r8 ? bb : 0.f, ke8[e], zk8);
+            zc8 = mfma4(c8 ? cc : 0.f, qf8[e], zc8);
+            zq4 = mfma4(r4 ? a : 0.f, ke4[e], zq4);
+            zk4 = mfma4(r4 ? bb : 0.f, ke4[e], zk4);
+            zc4 = mfma4(c4 ? cc : 0.f, qf4[e], zc4);
+            zc8 = mfma4(c8 ? dd : 0.f, kf8[e], zc8);
+            zc4 = mfma4(c4 ? dd : 0.f, kf4[e], zc4);
+        }
+        f32x4_t pq = x.F8 * zq8 + x.F4 * zq4, pk = x.F8 * zk8 + x.F4 * zk4, pc = x.E8 * zc8 + x.E4 * zc4;
+        // pairs inside this lane's four tokens
+        f32x4_t dg;
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            const f32x4_t dp = ld4(smem + G::OFF_TR + 16 * (4 * (4 * g + a) + g));         // dP[4 g + a][4 g ..]
+            const f32x4_t da = ld4(smem + G::OFF_TR + 1024 + 16 * (4 * (4 * g + a) + g));  // dA[4 g + a][4 g ..]
+            dg[a] = dp[a];
+            float f = 1.f;  // D of (a, s)
+#pragma unroll
+            for (int s = a - 1; s >= 0; --s) {
+                f *= x.al[s + 1];
+                const float ws = kk[s] * f, ab = b4[a] * da[s];
+                pq[a] = fmaf(dp[s], ws, pq[a]);
+                pk[a] = fmaf(ab, ws, pk[a]);
+                pc[s] = fmaf(fmaf(dp[s], qq[a], ab * kk[a]), f, pc[s]);
+            }
+        }
+        // the gate: own terms and pair terms, summed over the tokens at and after each
+        const f32x4_t own_t = qq * (x.F * dQh) + khat * kdk;
+        const f32x4_t pair_t = qq * pq + kk * (pk - pc);
+        const float ec = col_total(own_t);
+        if (g == 0) reinterpret_cast<float*>(smem + G::OFF_EC)[m * D + 16 * w + r] = ec;
+        f32x4_t suf = own_t + pair_t;
+        suf[2] += suf[3];
+        suf[1] += suf[2];
+        suf[0] += suf[1];
+        {
+            const float t4 = suf[0], s4 = __shfl_xor(t4, 16);  // the sibling block's sum
+            const float t8 = t4 + s4, s8 = __shfl_xor(t8, 32);
+            suf += ((g & 1) ? 0.f : s4) + ((g & 2) ? 0.f : s8);
+        }
+        const f32x4_t dQ = x.F * dQh + pq + dg * kk;
+        const f32x4_t dK = x.F * kdk + (pk + pc) + dg * qq;
+        {
+            const unsigned nb = static_cast<unsigned>(((clen_of(m) - 1) * tstride + 16) * 4);
+            const size_t r0 = row0_of(m, 16 * w);
+            const __amdgpu_buffer_rsrc_t rq = make_rsrc(gq + r0, nb), rk = make_rsrc(gk + r0, nb);
+            const __amdgpu_buffer_rsrc_t rgg = make_rsrc(CHAN ? gg + r0 : gg, CHAN ? nb : 0u);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const unsigned off = static_cast<unsigned>(((4 * g + e) * tstride + r) * 4);
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dQ[e]), rq, off, 0, 0);
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dK[e]), rk, off, 0, 0);
+                if constexpr (CHAN) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(suf[e]), rgg, off, 0, 0);
+            }
+        }
+        if constexpr (!CHAN) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) suf[e] = row16_sum(suf[e]);
+            if (r == 0) st4(smem + G::OFF_GG + (m * NW + w) * 64 + 16 * g, suf);
+        }
+        if (w == 0) {
+            // dbeta_t = W_t . V_t - K^_t . (W S^T)_t + sum_s dA_ts A'_ts, t = r
+            const f32x4_t at = *reinterpret_cast<const f32x4_t*>(rec + (item0 + m) * R::FLOATS + R::AT + 4 * lane);
+            float s = dar[0] * at[0] + dar[1] * at[1] + dar[2] * at[2] + dar[3] * at[3];
+            s += __shfl_xor(s, 16);
+            s += __shfl_xor(s, 32);
+            float wx = 0.f;
+#pragma unroll
+            for (int ww = 0; ww < NW; ++ww)
+                wx += reinterpret_cast<const float*>(smem + G::OFF_DB + ((m & 1) * NW + ww) * 64)[r];
+            if (g == 0 && r < clen_of(m)) gbeta[(tok0 + m * kC16 + r) * H + h] = wx + s;
+        }
+    }
+
+    // ================ backwards ================
+    // (the last two chunks are still in their buffers; this wave's own stores of gk and gg are
+    // read back below, after the wait)
+    f32x4_t Gt[NT];
+    {
+        const float* gp = g_hist + (static_cast<size_t>(pair) * n_span + span) * D * D;
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                Gt[i][e] = gp[(static_cast<size_t>(i) * NT + w) * 256 + 4 * (16 * (r >> 2) + 4 * g + e) + (r & 3)];
+    }
+    wait_vm_n<0>();
+    own = load_own(nm - 1, false);
+    float hs = 0.f;  // <S, G> of row 16 w + r at the end of the chunk
+    for (int m = nm - 1; m >= 0; --m) {
+        const unsigned char* b = buf(m);
+        if (m == nm - 1 || m == kSpan / 2 - 1) {
+            // from the states themselves at two places of a span, so that the sums carried
+            // along the chunks span 64 tokens at most
+            f32x4_t s = kZero4;
+            if (m == nm - 1) {
+#pragma unroll
+                for (int i = 0; i < NT; ++i) s += St[i] * Gt[i];
+            } else {
+#pragma unroll
+                for (int i = 0; i < NT; ++i) s += ld4(mid + 1024 * i) * Gt[i];
+            }
+            hs = col_total(s);
+        }
+        // U G^T
+        f32x4_t ka[2] = {kZero4, kZero4};
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+            const f32x4_t ur = ix.row(b + G::B_U, i);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) ka[e & 1] = mfma4(ur[e], Gt[i][e], ka[e & 1]);
+        }
+        const Dec x = decays(own.lg);
+        const f32x4_t khat = own.k * x.F, qhat = own.q * x.F;
+        // G^T = gC G^T + dO^T Q^ - (diag(beta) W)^T K^
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+            float dc[4], wc[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                dc[e] = ix.col(b + G::B_O, e, i);
+                wc[e] = -own.b4[e] * ix.col(b + G::B_W, e, i);
+            }
+            Gt[i] = Gt[i] * x.gc;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                Gt[i] = mfma4(dc[e], qhat[e], Gt[i]);
+                Gt[i] = mfma4(wc[e], khat[e], Gt[i]);
+            }
+        }
+        const f32x4_t dKb = x.E * (ka[0] + ka[1]);  // dL/dK- scaled: dK's part
+        const f32x4_t ct = own.k * dKb;             // K- . dL/dK- per token
+        const f32x4_t dK = own.x + dKb;
+        const float tot = col_total(ct);
+        const float sg = hs - tot;                  // gC <S, G> of the chunk
+        hs = sg + reinterpret_cast<const float*>(smem + G::OFF_EC)[m * D + 16 * w + r];
+        // dg: gC <S, G> plus the sums over the tokens before each
+        f32x4_t pre;
+        pre[0] = 0.f;
+        pre[1] = ct[0];
+        pre[2] = pre[1] + ct[1];
+        pre[3] = pre[2] + ct[2];
+        {
+            const float t4 = pre[3] + ct[3], s4 = __shfl_xor(t4, 16);
+            const float t8 = t4 + s4, s8 = __shfl_xor(t8, 32);
+            pre += sg + (((g & 1) ? s4 : 0.f) + ((g & 2) ? s8 : 0.f));
+        }
+        {
+            const unsigned nb = static_cast<unsigned>(((clen_of(m) - 1) * tstride + 16) * 4);
+            const size_t r0 = row0_of(m, 16 * w);
+            const __amdgpu_buffer_rsrc_t rk = make_rsrc(gk + r0, nb);
+            const __amdgpu_buffer_rsrc_t rgg = make_rsrc(CHAN ? gg + r0 : gg, CHAN ? nb : 0u);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const unsigned off = static_cast<unsigned>(((4 * g + e) * tstride + r) * 4);
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dK[e]), rk, off, 0, 0);
+                if constexpr (CHAN)
+                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(own.y[e] + pre[e]), rgg, off, 0, 0);
+            }
+        }
+        if constexpr (!CHAN) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) pre[e] = row16_sum(pre[e]);
+            unsigned char* p = smem + G::OFF_GG + (m * NW + w) * 64 + 16 * g;
+            if (r == 0) st4(p, ld4(p) + pre);
+        }
+        // chunk m - 1's copies have landed (they are older than this chunk's four gk stores)
+        if (m >= 1) {
+            wait_vm_n<4>();
+            lds_barrier();
+            if (m >= 2) issue(m - 2);
+            own = load_own(m - 1, false);
+        }
+    }
+    if constexpr (!CHAN) {
+        lds_barrier();
+        for (int z = tid; z < nm * kC16; z += NW * 64) {
+            const int m = z >> 4, t = z & 15;
+            float s = 0.f;
+#pragma unroll
+            for (int ww = 0; ww < NW; ++ww)
+                s += reinterpret_cast<const float*>(smem + G::OFF_GG + (m * NW + ww) * 64)[t];
+            if (t < clen_of(m)) gg[(tok0 + z) * H + h] = s;
+        }
+    }
+}
+
+// The dynamic-LDS limit is a per-device function attribute, set once per device and kernel.
+template <auto KERN>
+hipError_t set_lds(int bytes) {
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    static bool done[64] = {};
+    if (dev >= 0 && dev < 64 && done[dev]) return hipSuccess;
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(KERN), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (e == hipSuccess && dev >= 0 && dev < 64) done[dev] = true;
+    return e;
+}
+
+struct DecBwdWs {
+    size_t kh, kb, qh, rec, s_hist, g_hist, w, u, bytes;
+};
+DecBwdWs dec_bwd_ws(long n_pairs, int T, int D) {
+    const size_t n_ch = static_cast<size_t>((T + kC16 - 1) / kC16), n_span = (n_ch + kSpan - 1) / kSpan;
+    const size_t np = static_cast<size_t>(n_pairs), tile = np * n_ch * kC16 * D * 4;
+    const size_t rec = np * n_ch * (D == 128 ? DecRec<128>::FLOATS : DecRec<64>::FLOATS) * 4;
+    auto al = [](size_t x) { return (x + 255) & ~static_cast<size_t>(255); };
+    DecBwdWs w;
+    w.kh = 0;
+    w.kb = al(w.kh + tile);
+    w.qh = al(w.kb + tile);
+    w.rec = al(w.qh + tile);
+    w.s_hist = al(w.rec + rec);
+    w.g_hist = al(w.s_hist + np * n_span * D * D * 4);
+    w.w = al(w.g_hist + np * n_span * D * D * 4);
+    w.u = al(w.w + tile);
+    w.bytes = al(w.u + tile);
+    return w;
+}
+
+template <int D, typename InT, bool CHAN>
+hipError_t launch_t(const BwdArgs& a, hipStream_t st) {
+    const int n_ch = (a.T + kC16 - 1) / kC16, n_span = (n_ch + kSpan - 1) / kSpan;
+    const DecBwdWs o = dec_bwd_ws(a.n_pairs, a.T, D);
+    unsigned char* base = reinterpret_cast<unsigned char*>(a.workspace);
+    auto at = [&](size_t off) { return reinterpret_cast<float*>(base + off); };
+    const InT *q = static_cast<const InT*>(a.q), *k = static_cast<const InT*>(a.k), *v = static_cast<const InT*>(a.v);
+    hipError_t e = set_lds<dec_sweep_kernel<D, InT>>(DsGeo<D>::BYTES);
+    if (e != hipSuccess) return e;
+    if ((e = set_lds<dec_span_kernel<D, InT, CHAN>>(DcGeo<D>::BYTES)) != hipSuccess) return e;
+    const long n_items = static_cast<long>(a.n_pairs) * n_ch;
+    hipLaunchKernelGGL((dec_prep_kernel<D, InT, CHAN>), dim3(static_cast<unsigned>((n_items + 3) / 4)), dim3(256), 0, st,
+                       q, k, a.beta, a.g, a.T, a.H, n_ch, n_items, at(o.kh), at(o.kb), at(o.qh), at(o.rec));
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    const int slots = (a.n_pairs + 7) / 8;
+    hipLaunchKernelGGL((dec_sweep_kernel<D, InT>), dim3(static_cast<unsigned>(slots * (D / 32) * 8)), dim3(512),
+                       DsGeo<D>::BYTES, st, v, a.s0, a.go, a.gs, a.gv, a.gs0, at(o.kh), at(o.kb), at(o.qh), at(o.rec),
+                       at(o.w), at(o.u), at(o.s_hist), at(o.g_hist), a.n_pairs, a.T, a.H, n_ch, n_span);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    hipLaunchKernelGGL((dec_span_kernel<D, InT, CHAN>), dim3(static_cast<unsigned>(a.n_pairs * n_span)), dim3(D * 4),
+                       DcGeo<D>::BYTES, st, q, k, v, a.g, a.go, at(o.rec), at(o.s_hist), at(o.g_hist), at(o.w), at(o.u),
+                       a.gq, a.gk, a.gbeta, a.gg, a.T, a.H, n_ch, n_span);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+size_t decay_bwd_ws_bytes(long n_pairs, int T, int D) { return dec_bwd_ws(n_pairs, T, D).bytes; }
+
+hipError_t launch_decay_bwd(const BwdArgs& a, hipStream_t st) {
+    if (a.n_pairs == 0 || a.T == 0) return hipSuccess;
+    if (!f32_bwd_supported(a.D, a.H)) return hipErrorInvalidValue;
+    auto go = [&](auto DD) {
+        constexpr int D = decltype(DD)::value;
+        if (a.per_channel)
+            return a.in_bf16 ? launch_t<D, uint16_t, true>(a, st) : launch_t<D, float, true>(a, st);
+        return a.in_bf16 ? launch_t<D, uint16_t, false>(a, st) : launch_t<D, float, false>(a, st);
+    };
+    return a.D == 128 ? go(std::integral_constant<int, 128>{}) : go(std::integral_constant<int, 64>{});
+}
+
+}  // namespace pm

@@ -10,6 +10,7 @@
 //   K7    delta_chunked_f32.hip     chunked forward on fp32 MFMA, fp32 inputs
 //   K8    kda_chunked.hip           chunked forward with a decay per key channel
 //   K9    delta_chunked_f32_bwd.hip chunked reverse mode on fp32 MFMA, fp32 inputs
+//   K10   decay_chunked_f32.hip     chunked reverse mode of the gated rules on fp32 MFMA
 // Mirrors the checks of kernels/__init__.py:308-338 (shapes), :613-614 and
 // :676-677 (chunk >= 1); shapes arrive as integers, so the Python layer
 // (prometheus_amd/kernels) raises KernelError for the tensor-level checks
@@ -341,6 +342,17 @@ bool bwd_chunked_f32(int H, int D, int in_dtype) {
     return g_path != 1 && in_dtype == PM_DTYPE_F32 && pm::f32_bwd_supported(D, H);
 }
 
+// ... and the chunked fp32 backward of the rules with a decay (K10) for either input type
+// with D in {64, 128}, from one full chunk of 16 tokens on: below, the two are level (T = 8:
+// 40 us both, launches); from there the chunked form is never slower and gains with T
+// (1 to 256 pairs, D = 64 and 128: T = 16 34-61 against 40-142 us, T = 96 56-179 against
+// 119-623 us).  Only under the default path (2 refuses gated backwards, 1 asks for the
+// per-token kernels).
+constexpr int kDecayMinT = 16;
+bool bwd_decay_chunked(int T, int H, int D) {
+    return g_path == 0 && T >= kDecayMinT && pm::f32_bwd_supported(D, H);
+}
+
 // gm: 0 ungated, 1 gated (a log-gate per token and head), 2 per-channel gated (KDA)
 size_t bwd_ws_bytes(int B, int T, int H, int D, int in_dtype, int gm = 0) {
     const long n_pairs = static_cast<long>(B) * H;
@@ -349,8 +361,8 @@ size_t bwd_ws_bytes(int B, int T, int H, int D, int in_dtype, int gm = 0) {
     return sizeof(float) * pm::bwd_workspace_floats(n_pairs, T, D, gm);
 }
 
-// Common backward dispatch; g != NULL: a gated variant (per-token kernels, gg out), with
-// per_channel its KDA form (g and gg (B, T, H, D)).
+// Common backward dispatch; g != NULL: a gated variant (K10 or the per-token kernels, gg
+// out, the per-token kernels' workspace either way: it holds K10's), with per_channel its KDA form (g and gg (B, T, H, D)).
 int backward(const void* q, const void* k, const void* v, const float* beta, const float* g,
              const float* s0, const float* go, const float* gs, float* gq, float* gk, float* gv,
              float* gbeta, float* gg, float* gs0, int B, int T, int H, int D, int in_dtype,
@@ -398,6 +410,12 @@ int backward(const void* q, const void* k, const void* v, const float* beta, con
     a.g = g;
     a.gg = gg;
     a.per_channel = per_channel;
+    if (gated && n_tok > 0 && bwd_decay_chunked(T, H, D) && aligned(q, 16) && aligned(k, 16) && aligned(v, 16) &&
+        (!go || aligned(go, 16)) && aligned(gv, 16) && (!per_channel || aligned(g, 16)) && aligned(workspace, 16) &&
+        pm::decay_bwd_ws_bytes(n_pairs, T, D) <= need) {
+        hipError_t e = pm::launch_decay_bwd(a, static_cast<hipStream_t>(stream));
+        return e == hipSuccess ? 0 : hip_fail(e, "chunked decay backward launch");
+    }
     hipError_t e = chunked16   ? pm::launch_bwd_chunked(a, static_cast<hipStream_t>(stream))
                    : chunked32 ? pm::launch_bwd_chunked_f32(a, static_cast<hipStream_t>(stream))
                                : pm::launch_bwd(a, static_cast<hipStream_t>(stream));

@@ -210,6 +210,13 @@ hipError_t launch_f32_hist_sweep(const BwdArgs& a, const float* t2, const float*
                                  float* g_hist, float* u_out, hipStream_t st);
 hipError_t launch_bwd_chunked_f32(const BwdArgs& a, hipStream_t st);
 
+// K10 (decay_chunked_f32.hip): the reverse mode of the rules with a decay (a.g, a.gg,
+// a.per_channel) in chunked form on fp32 MFMA, fp32 or bf16 q/k/v, f32_bwd_supported(D, H);
+// a.workspace holds decay_bwd_ws_bytes bytes; q, k, v, go, gv, g (per channel) and
+// workspace 16-byte aligned.
+size_t decay_bwd_ws_bytes(long n_pairs, int T, int D);
+hipError_t launch_decay_bwd(const BwdArgs& a, hipStream_t st);
+
 // Zero fill (used instead of hipMemsetAsync so callers may graph-capture).
 hipError_t launch_fill_zero(float* p, size_t n, hipStream_t st);
 hipError_t launch_copy_f32(float* dst, const float* src, size_t n, hipStream_t st);

@@ -607,10 +607,11 @@ def _gated_forward(q, k, v, beta, g, state, out_dtype, per_channel=False):
 def chunked_gated_delta_rule_bwd(residual: _GatedDeltaResidual, grads):
     """Backward of the gated VJP pair: ``grads = (go, gs)`` as ``chunked_delta_rule_bwd``
     (either may be None). Returns ``(gq, gk, gv, gbeta, gg, gstate)``, fp32, shaped like
-    ``q, k, v, beta, g, state0``. Runs the per-token fp32 reverse-mode kernels
-    (``pm_gated_delta_bwd``) for every dtype and head dimension up to 256: with P_t =
-    exp(g_t) S_{t-1}, dL/dg_t = <G - beta_t k_t w^T, P_t> and G <- exp(g_t) (G - beta_t
-    k_t w^T), the other gradients as in the ungated backward."""
+    ``q, k, v, beta, g, state0``. fp32 arithmetic for every dtype (``pm_gated_delta_bwd``):
+    in chunks on fp32 MFMA for head dimension 64 or 128 from 16 tokens on, token by token
+    otherwise (head dimension up to 256). With P_t = exp(g_t) S_{t-1}, dL/dg_t = <G -
+    beta_t k_t w^T, P_t> and G <- exp(g_t) (G - beta_t k_t w^T), the other gradients as in
+    the ungated backward."""
     return _gated_bwd(residual, grads, per_channel=False)
 
 
@@ -618,7 +619,7 @@ def chunked_kda_rule_bwd(residual: _GatedDeltaResidual, grads):
     """Backward of ``chunked_kda_rule_fwd``: as ``chunked_gated_delta_rule_bwd`` with g
     and gg (batch, seq, heads, dim). With P_t = Diag(exp(g_t)) S_{t-1}, dL/dg_t[d] =
     <G_P[d, :], P_t[d, :]> (G_P = G - beta_t k_t w^T) and G <- Diag(exp(g_t)) G_P
-    (``pm_kda_delta_bwd``, the per-token fp32 kernels, head dimension up to 256)."""
+    (``pm_kda_delta_bwd``, the same two paths)."""
     return _gated_bwd(residual, grads, per_channel=True)
 
 

@@ -1,0 +1,97 @@
+"""GPU tests of the chunked fp32 backward of the rules with a decay (gated and KDA, D in
+{64, 128}, from 16 tokens) against the fp64 oracles at the fp32 bounds, at the edges of its
+16-token chunks and its spans of chunks, and against the per-token kernels that every other
+call runs."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import gated_oracle as gref
+from prometheus_amd import _native, kernels, synth
+from tests.parity import assert_f32_parity
+
+pytestmark = pytest.mark.gpu
+
+NAMES = ("gq", "gk", "gv", "gbeta", "gg", "gstate")
+
+
+def _dev(x):
+    return None if x is None else torch.from_numpy(np.ascontiguousarray(x, dtype=np.float32)).cuda()
+
+
+def _case(shape, seed, chan, dtype="fp32", scale=0.3, state=True):
+    x = synth.fwd_inputs(shape, seed=seed, dtype=dtype, s0_std=0.05 if state else None)
+    rng = np.random.default_rng(seed + 1)
+    b, t, h, d = shape
+    g = (-scale * np.abs(rng.standard_normal(shape if chan else shape[:3]))).astype(np.float32)
+    go = rng.standard_normal(shape).astype(np.float32)
+    gs = (rng.standard_normal((b, h, d, d)) * 0.05).astype(np.float32)
+    return x, g, go, gs
+
+
+def _bwd(x, g, go, gs, chan):
+    def qkv(name):
+        bits = getattr(x, name + "_bits")
+        if bits is None:
+            return _dev(getattr(x, name))
+        return torch.from_numpy(bits.view(np.int16)).view(torch.bfloat16).cuda()
+
+    b, _, h, d = x.q.shape
+    s0 = _dev(x.s0) if x.s0 is not None else torch.zeros((b, h, d, d), device="cuda")
+    gd = g if isinstance(g, torch.Tensor) else _dev(g)
+    res = kernels._GatedDeltaResidual(q=qkv("q"), k=qkv("k"), v=qkv("v"), beta=_dev(x.beta), g=gd, state0=s0, chunk=64)
+    f = kernels.chunked_kda_rule_bwd if chan else kernels.chunked_gated_delta_rule_bwd
+    return [t.cpu().numpy() for t in f(res, (_dev(go), _dev(gs)))]
+
+
+def _check(x, g, go, gs, chan, what):
+    got = _bwd(x, g, go, gs, chan)
+    exp = (gref.kda_vjp if chan else gref.gated_vjp)(x.q, x.k, x.v, x.beta, g, go, gs, x.s0)
+    for name, a, e in zip(NAMES, got, exp):
+        assert_f32_parity(a, e, f"{what} {name}", scaled=True)
+
+
+@pytest.mark.parametrize("chan", [False, True])
+@pytest.mark.parametrize("t,d", [(16, 128), (17, 64), (31, 64), (64, 128), (127, 64), (128, 128), (129, 64), (273, 128)])
+def test_edges_of_chunks_and_spans(t, d, chan):
+    """Whole and partial chunks, one chunk up to several spans, with and without a state."""
+    x, g, go, gs = _case((1, t, 3, d), t + d + chan, chan, state=t % 2 == 0)
+    _check(x, g, go, gs, chan, f"T{t} D{d}")
+
+
+@pytest.mark.parametrize("chan", [False, True])
+def test_bf16_inputs_in_fp32_arithmetic(chan):
+    x, g, go, gs = _case((2, 145, 2, 128), 7, chan, dtype="bf16")
+    _check(x, g, go, gs, chan, "bf16")
+
+
+def test_decays_of_every_strength_side_by_side():
+    """Channels that forget everything (alpha 0 and 1e-9), that keep everything (g = 0), that
+    grow a little, and one strong decay in the middle of a chunk before weak ones: no factor
+    is formed from a difference or quotient that the strong one would spoil."""
+    x, g, go, gs = _case((1, 90, 2, 64), 17, True, scale=0.05)
+    g[..., 0], g[..., 1], g[..., 2], g[..., 3] = -np.inf, -20.0, 0.0, 0.02
+    g[:, 37, :, 8:24] = -60.0
+    _check(x, g, go, gs, True, "mixed decays")
+
+
+@pytest.mark.parametrize("chan", [False, True])
+def test_against_the_per_token_kernels(chan):
+    """Missing cotangents, several pairs per XCD slot, bitwise repeatable; a gate tensor that
+    is not 16-byte aligned keeps its (per-token or chunked) route and its result."""
+    shape = (3, 200, 5, 64)
+    x, g, go, gs = _case(shape, 29, chan)
+    for cot in ((go, gs), (None, gs), (go, None)):
+        got = _bwd(x, g, *cot, chan)
+        again = _bwd(x, g, *cot, chan)
+        off = torch.empty(g.size + 1, device="cuda")[1:].copy_(_dev(g).flatten()).view(g.shape)
+        shifted = _bwd(x, off, *cot, chan)
+        with _native.use_knobs(1, 0):
+            ref = _bwd(x, g, *cot, chan)
+        for name, a, b, c, e in zip(NAMES, got, again, shifted, ref):
+            np.testing.assert_array_equal(a, b, err_msg=name)
+            assert_f32_parity(a, e, name, scaled=True)
+            assert_f32_parity(c, e, f"shifted gate {name}", scaled=True)
