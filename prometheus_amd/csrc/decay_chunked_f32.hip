@@ -40,7 +40,7 @@
 //   K10s (one workgroup of eight waves per (b, h, 32 columns of d_v)): the state recurrence
 //     forwards (U per token, S at every span start) beside the G recurrence backwards (W
 //     and dV per token, G at every span end, dS0).
-//   K10c (one workgroup of D/16 waves per (b, h, span of 8 chunks)): the span forwards from
+//   K10c (one workgroup of D/16 waves per (b, h, span of 2 to 8 chunks)): the span forwards from
 //     its start state (dQ, dbeta, dK and dg but for what depends on G), then backwards from
 //     its end gradient (the rest).  S cannot be walked back as the ungated backward does
 //     (that divides by gC), hence the two walks.
@@ -54,7 +54,7 @@
 namespace pm {
 namespace {
 
-constexpr int kSpan = 8;  // chunks per span (128 tokens)
+constexpr int kSpan = 8;  // chunks per span (128 tokens) at most
 
 __device__ __forceinline__ f32x4_t ld4(const unsigned char* p) { return *reinterpret_cast<const f32x4_t*>(p); }
 __device__ __forceinline__ void st4(unsigned char* p, f32x4_t x) { *reinterpret_cast<f32x4_t*>(p) = x; }
@@ -91,7 +91,10 @@ struct TileIdx {
     __device__ __forceinline__ float col(const unsigned char* b, int e, int i) const {
         return *reinterpret_cast<const float*>(b + cb[e] + cx[i & 3] + 256 * (i >> 2));
     }
-    // col for an i known only at run time (g: the lane's group)
+    // row and col for an i known only at run time
+    __device__ __forceinline__ f32x4_t roww(const unsigned char* b, int i, int r) const {
+        return ld4(b + rb + 64 * (i ^ (r >> 2)));
+    }
     __device__ __forceinline__ float colw(const unsigned char* b, int e, int i, int g) const {
         return *reinterpret_cast<const float*>(b + cb[e] + 64 * (i ^ g));
     }
@@ -322,10 +325,10 @@ __global__ __launch_bounds__(256) void dec_prep_kernel(
 
 // ---------------------------------------------------------------- K10s
 // Eight waves: 0, 1 the state recurrence (16 columns of S each), 3 its copies; 6, 7 the
-// gradient recurrence (16 columns of G each), 5 its copies and the stores of W and dV; 2
-// and 4 form Q^^T dO for waves 7 and 6 one chunk ahead, from Q^ in operand order straight
-// into registers.  Waves w and w + 4 share a SIMD, so the four chains take one each.  The
-// two recurrences walk the chunks in opposite directions and share the workgroup's barriers
+// gradient recurrence (16 columns of G each), 5 its copies and the stores of W and dV; 2, 3
+// and 4 form Q^^T dO for waves 6 and 7 one chunk ahead.  Waves w and w + 4 share a SIMD, so
+// the four chains take one each, and the 64 products of Q^^T dO a chunk spread over three of
+// them (a chain's 72 products are dense: a helper's delay it one for one).  The two recurrences walk the chunks in opposite directions and share the workgroup's barriers
 // (one per chunk); each keeps three chunk buffers, one in use, one landed, one landing.
 template <int D>
 struct DsGeo {
@@ -355,7 +358,7 @@ __global__ __launch_bounds__(512) void dec_sweep_kernel(
     const float* __restrict__ gs, float* __restrict__ gv, float* __restrict__ gs0, const float* __restrict__ kh,
     const float* __restrict__ kb, const float* __restrict__ qh, const float* __restrict__ rec,
     float* __restrict__ w_out, float* __restrict__ u_out, float* __restrict__ s_hist, float* __restrict__ g_hist,
-    int n_pairs, int T, int H, int n_ch, int n_span) {
+    int n_pairs, int T, int H, int n_ch, int n_span, int span_len) {
     using G = DsGeo<D>;
     using R = DecRec<D>;
     constexpr int NT = G::NT, NI = G::NI, NB = G::NB, n_tiles = D / 32;
@@ -389,6 +392,31 @@ __global__ __launch_bounds__(512) void dec_sweep_kernel(
         for (int i = 0; i < NI; ++i) dma16_asm(rs, d0 + 1024 * i, static_cast<unsigned>(1024 * i + 16 * lane));
     };
 
+    // Q^^T dO, tiles m0 .. m0 + N - 1 (rows 16 m .. of d): Q^ in operand order straight into
+    // registers, dO of the chain's columns from the gradient half's buffer, into its slot
+    constexpr int NA = NT * 5 / 8, NC = NT - NA;
+    auto fetch_q = [=](int c, int m0, auto& x) __attribute__((always_inline)) {
+        const float* qp = qh + (item0 + c) * kC16 * D + 256 * m0 + 4 * lane;
+#pragma unroll
+        for (unsigned m = 0; m < sizeof(x) / 16; ++m) x[m] = *reinterpret_cast<const f32x4_t*>(qp + 256 * m);
+    };
+    auto qtdo = [=](int c, int cw, int m0, auto& x) __attribute__((always_inline)) {
+        constexpr unsigned N = sizeof(x) / 16;
+        const float* Of = reinterpret_cast<const float*>(sbuf(c) + G::S_O + 1024 * cw);
+        f32x4_t dOc, hq[N];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) dOc[e] = Of[(4 * g + e) * 16 + r];
+#pragma unroll
+        for (unsigned m = 0; m < N; ++m) hq[m] = kZero4;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (unsigned m = 0; m < N; ++m) hq[m] = mfma4(x[m][e], dOc[e], hq[m]);
+        unsigned char* slot = hslot(c, cw) + 1024 * m0 + 16 * lane;
+#pragma unroll
+        for (unsigned m = 0; m < N; ++m) st4(slot + 1024 * m, hq[m]);
+    };
+
     if (w < 2) {
         // ============ the state recurrence: S columns col0 + 16 w + [0, 16) ============
         const int ecol = col0 + 16 * w + r;
@@ -399,52 +427,63 @@ __global__ __launch_bounds__(512) void dec_sweep_kernel(
             for (int e = 0; e < 4; ++e)
                 S[m][e] = s0 ? s0[sbase + static_cast<size_t>(16 * m + 4 * g + e) * D + ecol] : 0.f;
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), seen by the compiler: no wait for S0 in the loop
+        __builtin_amdgcn_s_setprio(3);       // the chains bound the chunk: first on their SIMD's MFMA pipe
         lds_barrier();                       // B0
-        float kt[4][NT];  // K-^T operand of chunk i - 1: K-[4 g + e][16 m + r]
-        f32x4_t gc[NT], Up = kZero4;
+        // One iteration: S += K-^T U of the last chunk (its K-^T operand kt was read an iteration
+        // ago), then X and U of this one.  Every LDS read sits right behind one product (fenced:
+        // a 16x16x4 product holds the MFMA pipe for 32 cycles, in which the wave issues its
+        // reads for free, while a group of reads between products holds the products up); the
+        // decay Diag(gC) S falls into the latency of U's short products.
+        f32x4_t Up = kZero4;
+        float kt[4][NT] = {};  // K-^T operand: K-[4 g + e][16 m + r]
+        auto rd_kt = [&](const unsigned char* b, int e, int m) __attribute__((always_inline)) {
+            kt[e][m] = ix.col(b + G::H_KB, e, m);  // (tiles m and m + 4: one paired read)
+            kt[e][m + NT / 2] = ix.col(b + G::H_KB, e, m + NT / 2);
+        };
         for (int i = 0; i < n_ch; ++i) {
             const unsigned char* b = hbuf(i);
-            f32x4_t kf[NT], vr;
-#pragma unroll
-            for (int m = 0; m < NT; ++m) kf[m] = ix.row(b + G::H_KH, m);
             const InT* Vf = reinterpret_cast<const InT*>(b + G::H_V + 1024 * w);
+            f32x4_t kf[NT], gc[NT], vr, tt;
+            // (kt starts as zeros; kt[e] is read anew behind its products)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) vr[e] = to_f32<InT>(Vf[(4 * g + e) * 16 + r]);
-            const f32x4_t tt = ld4(b + G::H_T + 16 * lane);
-            fence();
-            // S = Diag(gC) S + K-^T U of chunk i - 1
-            if (i > 0) {
+            for (int e = 0; e < 4; ++e)
 #pragma unroll
-                for (int m = 0; m < NT; ++m) S[m] = gc[m] * S[m];
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-#pragma unroll
-                    for (int m = 0; m < NT; ++m) S[m] = mfma4(kt[e][m], Up[e], S[m]);
-            }
-            if (i % kSpan == 0) {
-                float* hp = s_hist + ((static_cast<size_t>(pair) * n_span + i / kSpan) * NT + col0 / 16 + w) * NT * 256;
+                for (int m = 0; m < NT; ++m) {
+                    S[m] = mfma4(kt[e][m], Up[e], S[m]);
+                    if (e == 0) kf[m] = ix.row(b + G::H_KH, m);
+                    if (e > 0 && m < NT / 2) rd_kt(b, e - 1, m);
+                    if (e == 1 && m >= NT / 2 && m < NT / 2 + 2) {
+                        vr[2 * (m - NT / 2)] = to_f32<InT>(Vf[(4 * g + 2 * (m - NT / 2)) * 16 + r]);
+                        vr[2 * (m - NT / 2) + 1] = to_f32<InT>(Vf[(4 * g + 2 * (m - NT / 2) + 1) * 16 + r]);
+                    }
+                    if (e == 2 && m == NT - 1) tt = ld4(b + G::H_T + 16 * lane);
+                    fence();
+                }
+            if ((i & (span_len - 1)) == 0) {
+                float* hp = s_hist + ((static_cast<size_t>(pair) * n_span + i / span_len) * NT + col0 / 16 + w) * NT * 256;
 #pragma unroll
                 for (int m = 0; m < NT; ++m) *reinterpret_cast<f32x4_t*>(hp + m * 256 + 4 * lane) = S[m];
             }
-            fence();
             // X = K^ S - V, U = T'' X
             f32x4_t xa[4] = {-vr, kZero4, kZero4, kZero4};
 #pragma unroll
             for (int m = 0; m < NT; ++m)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) xa[e] = mfma4(kf[m][e], S[m][e], xa[e]);
+                for (int e = 0; e < 4; ++e) {
+                    xa[e] = mfma4(kf[m][e], S[m][e], xa[e]);
+                    const int n = 4 * m + e;
+                    if (n < NT / 2) rd_kt(b, 3, n);
+                    if (n >= NT / 2 && n < NT / 2 + NT) gc[n - NT / 2] = ld4(b + G::H_G + 4 * (16 * (n - NT / 2) + 4 * g));
+                    fence();
+                }
             const f32x4_t X = (xa[0] + xa[1]) + (xa[2] + xa[3]);
             Up = mm16(tt, X);
             // U's rows (U^T = X^T T''^T): lane (g, r) holds U[r][col0 + 16 w + 4 g ..]
             const f32x4_t Ut = mm16(X, tt);
+#pragma unroll
+            for (int m = 0; m < NT; ++m) S[m] = gc[m] * S[m];
             *reinterpret_cast<f32x4_t*>(u_out + (item0 + i) * kC16 * D +
                                         4 * f32_chunk<D>(r, (col0 + 16 * w) / 4 + g)) = Ut;
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int m = 0; m < NT; ++m) kt[e][m] = ix.col(b + G::H_KB, e, m);
-#pragma unroll
-            for (int m = 0; m < NT; ++m) gc[m] = ld4(b + G::H_G + 4 * (16 * m + 4 * g));
             __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), seen by the compiler
             lds_barrier();
         }
@@ -475,48 +514,38 @@ __global__ __launch_bounds__(512) void dec_sweep_kernel(
         } else {
             wait_vm_n<0>();
         }
+        // ... and the remaining tiles of both chains' Q^^T dO, ahead of the copies (the compiler,
+        // which does not see the copies, waits for all of them where it waits for Q^)
+        f32x4_t qc[NC];
+        fetch_q(n_ch - 1, NA, qc);
         lds_barrier();  // B0
         for (int i = 0; i < n_ch; ++i) {
+            const int ch = n_ch - 1 - i;
+            qtdo(ch, 0, NA, qc);
+            qtdo(ch, 1, NA, qc);
             if (i + 2 < n_ch) {
                 copies(i + 2);
                 wait_vm_n<G::H_NCP>();
             } else {
                 wait_vm_n<0>();
             }
+            if (ch > 0) fetch_q(ch - 1, NA, qc);
             lds_barrier();
         }
         lds_barrier();
     } else if (w == 2 || w == 4) {
-        // ============ Q^^T dO of chunk n_ch - 1 - i for the gradient chain cw ============
+        // ============ Q^^T dO of chunk n_ch - 1 - i, tiles [0, NA) of the gradient chain cw ============
         const int cw = w == 4 ? 0 : 1;
-        f32x4_t qn[NT];
-        auto fetch = [&](int c) __attribute__((always_inline)) {
-            const float* qp = qh + (item0 + c) * kC16 * D + 4 * lane;
-#pragma unroll
-            for (int m = 0; m < NT; ++m) qn[m] = *reinterpret_cast<const f32x4_t*>(qp + 256 * m);
-        };
-        fetch(n_ch - 1);
+        f32x4_t qn[NA];
+        fetch_q(n_ch - 1, 0, qn);
         lds_barrier();  // B0
         for (int i = 0; i < n_ch; ++i) {
             const int ch = n_ch - 1 - i;
-            f32x4_t qc[NT];
+            f32x4_t qc[NA];
 #pragma unroll
-            for (int m = 0; m < NT; ++m) qc[m] = qn[m];
-            if (ch > 0) fetch(ch - 1);
-            const float* Of = reinterpret_cast<const float*>(sbuf(ch) + G::S_O + 1024 * cw);
-            f32x4_t dOc;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) dOc[e] = Of[(4 * g + e) * 16 + r];
-            f32x4_t hq[NT];
-#pragma unroll
-            for (int m = 0; m < NT; ++m) hq[m] = kZero4;
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int m = 0; m < NT; ++m) hq[m] = mfma4(qc[m][e], dOc[e], hq[m]);
-            unsigned char* slot = hslot(ch, cw);
-#pragma unroll
-            for (int m = 0; m < NT; ++m) st4(slot + 1024 * m + 16 * lane, hq[m]);
+            for (int m = 0; m < NA; ++m) qc[m] = qn[m];
+            if (ch > 0) fetch_q(ch - 1, 0, qn);
+            qtdo(ch, cw, 0, qc);
             lds_barrier();
         }
         lds_barrier();
@@ -590,58 +619,87 @@ __global__ __launch_bounds__(512) void dec_sweep_kernel(
             for (int e = 0; e < 4; ++e)
                 Gm[m][e] = gs ? gs[sbase + static_cast<size_t>(16 * m + 4 * g + e) * D + ecol] : 0.f;
         __builtin_amdgcn_s_waitcnt(0x0F70);
+        __builtin_amdgcn_s_setprio(3);
         lds_barrier();  // B0
-        // Iteration i runs chunk n_ch - i from operands read in iteration i - 1 (its buffer has
-        // landed by then); only Q^^T dO is read in iteration i
-        f32x4_t kf[NT], gc[NT], dOc = kZero4, ta = kZero4, b4 = kZero4, pp = kZero4;
-        float kt[4][NT];
-        for (int i = 0; i <= n_ch; ++i) {
-            if (i >= 1) {
-                const int c = n_ch - i;
-                if (c == n_ch - 1 || c % kSpan == kSpan - 1) {
-                    float* hp = g_hist + ((static_cast<size_t>(pair) * n_span + c / kSpan) * NT + col0 / 16 + cw) * NT * 256;
+        // One iteration runs chunk c from operands read an iteration ago (its buffer had landed
+        // by then; only Q^^T dO is read here) and reads chunk c - 1's behind its products, as
+        // the state chain does; the decay and Q^^T dO enter G in the latency of dU and W.
+        f32x4_t kf[NT], gc[NT], dOc, ta, b4, pp;
+        float kt[4][NT];  // K^^T operand: K^[4 g + e][16 m + r]
+        auto rd_kt = [&](const unsigned char* b, int e, int m) __attribute__((always_inline)) {
+            kt[e][m] = ix.col(b + G::S_KH, e, m);
+            kt[e][m + NT / 2] = ix.col(b + G::S_KH, e, m + NT / 2);
+        };
+        auto rd_gc = [&](const unsigned char* b, int m) __attribute__((always_inline)) {
+            gc[m] = ld4(b + G::S_G + 4 * (16 * m + 4 * g));
+        };
+        auto rd_do = [&](const unsigned char* b, int e) __attribute__((always_inline)) {
+            return reinterpret_cast<const float*>(b + G::S_O + 1024 * cw)[(4 * g + e) * 16 + r];
+        };
+        {
+            const unsigned char* b = sbuf(n_ch - 1);
 #pragma unroll
-                    for (int m = 0; m < NT; ++m) *reinterpret_cast<f32x4_t*>(hp + m * 256 + 4 * lane) = Gm[m];
+            for (int m = 0; m < NT; ++m) {
+                kf[m] = ix.row(b + G::S_KB, m);
+                rd_gc(b, m);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                dOc[e] = rd_do(b, e);
+#pragma unroll
+                for (int m = 0; m < NT / 2; ++m) rd_kt(b, e, m);
+            }
+            ta = ld4(b + G::S_T + 16 * lane);
+            pp = ld4(b + G::S_P + 16 * lane);
+            b4 = ld4(b + G::S_G + 4 * D + 16 * g);
+            lds_barrier();  // iteration 0: Q^^T dO of chunk n_ch - 1
+        }
+        for (int c = n_ch - 1; c >= 0; --c) {
+            if (c == n_ch - 1 || ((c + 1) & (span_len - 1)) == 0) {
+                float* hp = g_hist + ((static_cast<size_t>(pair) * n_span + c / span_len) * NT + col0 / 16 + cw) * NT * 256;
+#pragma unroll
+                for (int m = 0; m < NT; ++m) *reinterpret_cast<f32x4_t*>(hp + m * 256 + 4 * lane) = Gm[m];
+            }
+            const unsigned char* bn = sbuf(max(c - 1, 0));  // (chunk 0 reads its own buffer again, unused)
+            const unsigned char* hs = hslot(c, cw) + 16 * lane;
+            f32x4_t hq[NT], dOn, tn, pn, bn4;
+            // Y = K- G, dU = Y + P^T dO, W = T^T dU
+            f32x4_t ya[4] = {kZero4, kZero4, kZero4, kZero4};
+#pragma unroll
+            for (int m = 0; m < NT; ++m)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    ya[e] = mfma4(kf[m][e], Gm[m][e], ya[e]);
+                    if (e == 0) hq[m] = ld4(hs + 1024 * m);
+                    if (e == 1 && m > 0) kf[m - 1] = ix.row(bn + G::S_KB, m - 1);
+                    if (e == 2 && m < 4) dOn[m] = rd_do(bn, m);
+                    if (e == 3 && m == 0) tn = ld4(bn + G::S_T + 16 * lane);
+                    if (e == 3 && m == 1) pn = ld4(bn + G::S_P + 16 * lane);
+                    if (e == 3 && m == 2) bn4 = ld4(bn + G::S_G + 4 * D + 16 * g);
+                    fence();
                 }
-                f32x4_t hq[NT];
+            kf[NT - 1] = ix.row(bn + G::S_KB, NT - 1);
+            const f32x4_t dU = mm16(pp, dOc, (ya[0] + ya[1]) + (ya[2] + ya[3]));
 #pragma unroll
-                for (int m = 0; m < NT; ++m) hq[m] = ld4(hslot(c, cw) + 1024 * m + 16 * lane);
-                // Y = K- G, dU = Y + P^T dO, W = T^T dU
-                f32x4_t ya[4] = {kZero4, kZero4, kZero4, kZero4};
+            for (int m = 0; m < NT; ++m) Gm[m] = gc[m] * Gm[m] + hq[m];
+            const f32x4_t W = mm16(ta, dU);
+            const f32x4_t nbW = -(W * b4);
+            st4(wslot(c, cw) + 16 * lane, W);
+            if (r == 0) st4(wslot(c, cw) + 1024 + 16 * g, b4);
+            // G = Diag(gC) G + Q^^T dO - K^^T diag(beta) W
 #pragma unroll
-                for (int m = 0; m < NT; ++m)
+            for (int e = 0; e < 4; ++e)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) ya[e] = mfma4(kf[m][e], Gm[m][e], ya[e]);
-                const f32x4_t dU = mm16(pp, dOc, (ya[0] + ya[1]) + (ya[2] + ya[3]));
-                const f32x4_t W = mm16(ta, dU);
-                const f32x4_t nbW = -(W * b4);
-                st4(wslot(c, cw) + 16 * lane, W);
-                if (r == 0) st4(wslot(c, cw) + 1024 + 16 * g, b4);
-                // G = Diag(gC) G + Q^^T dO - K^^T diag(beta) W
+                for (int m = 0; m < NT; ++m) {
+                    Gm[m] = mfma4(kt[e][m], nbW[e], Gm[m]);
+                    if (e == 0) rd_gc(bn, m);
+                    if (e > 0 && m < NT / 2) rd_kt(bn, e - 1, m);
+                    fence();
+                }
 #pragma unroll
-                for (int m = 0; m < NT; ++m) Gm[m] = gc[m] * Gm[m] + hq[m];
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-#pragma unroll
-                    for (int m = 0; m < NT; ++m) Gm[m] = mfma4(kt[e][m], nbW[e], Gm[m]);
-            }
-            if (i < n_ch) {
-                const unsigned char* b = sbuf(n_ch - 1 - i);
-#pragma unroll
-                for (int m = 0; m < NT; ++m) kf[m] = ix.row(b + G::S_KB, m);
-                const float* Of = reinterpret_cast<const float*>(b + G::S_O + 1024 * cw);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) dOc[e] = Of[(4 * g + e) * 16 + r];
-                ta = ld4(b + G::S_T + 16 * lane);
-                pp = ld4(b + G::S_P + 16 * lane);
-                b4 = ld4(b + G::S_G + 4 * D + 16 * g);
-#pragma unroll
-                for (int m = 0; m < NT; ++m) gc[m] = ld4(b + G::S_G + 4 * (16 * m + 4 * g));
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-#pragma unroll
-                    for (int m = 0; m < NT; ++m) kt[e][m] = ix.col(b + G::S_KH, e, m);
-            }
+            for (int m = 0; m < NT / 2; ++m) rd_kt(bn, 3, m);
+            dOc = dOn, ta = tn, pp = pn, b4 = bn4;
+            __builtin_amdgcn_s_waitcnt(0xC07F);
             lds_barrier();
         }
 #pragma unroll
@@ -680,14 +738,14 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
     const float* __restrict__ go, const float* __restrict__ rec, const float* __restrict__ s_hist,
     const float* __restrict__ g_hist, const float* __restrict__ w_in, const float* __restrict__ u_in,
     float* __restrict__ gq, float* __restrict__ gk, float* __restrict__ gbeta, float* __restrict__ gg, int T, int H,
-    int n_ch, int n_span) {
+    int n_ch, int n_span, int span_len) {
     using G = DcGeo<D>;
     using R = DecRec<D>;
     constexpr int NW = G::NW, NT = G::NT;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int pair = blockIdx.x / n_span, span = blockIdx.x % n_span;
     const int seq = pair / H, h = pair % H;
-    const int c0 = span * kSpan, nm = min(kSpan, n_ch - c0);  // chunks of this span
+    const int c0 = span * span_len, nm = min(span_len, n_ch - c0);  // chunks of this span
     const size_t tok0 = static_cast<size_t>(seq) * T + static_cast<size_t>(c0) * kC16;
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = static_cast<int>(uniform(static_cast<unsigned>(tid >> 6)));
@@ -726,7 +784,7 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
     // this lane's tokens of a chunk, as loaded (tokens past the end read zeros)
     struct Own {
         f32x4_t k, q, x, lg, b4;  // x: v (forwards) or the gradient so far of k (backwards)
-        f32x4_t y;                // backwards: the gradient so far of the gate
+        f32x4_t y;                // forwards: A'[r][4 g ..]; backwards: the gradient so far of the gate
         float br;
     };
     auto load_own = [=](int m, bool fwd) __attribute__((always_inline)) {
@@ -747,11 +805,12 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
             o.q[e] = buf_el<InT>(rq, el);
             o.lg[e] = buf_el<float>(rg, CHAN ? el : static_cast<unsigned>((4 * g + e) * H));
             o.x[e] = fwd ? buf_el<InT>(rv, el) : buf_el<float>(rgk, el);
-            o.y[e] = (CHAN && !fwd) ? buf_el<float>(rgg, el) : 0.f;
+            if (!fwd) o.y[e] = CHAN ? buf_el<float>(rgg, el) : 0.f;
         }
-        const float* rc = rec + (item0 + m) * R::FLOATS + R::GB + D;
-        o.b4 = *reinterpret_cast<const f32x4_t*>(rc + 4 * g);
-        o.br = rc[r];
+        const float* rc = rec + (item0 + m) * R::FLOATS;
+        if (fwd) o.y = *reinterpret_cast<const f32x4_t*>(rc + R::AT + 4 * lane);
+        o.b4 = *reinterpret_cast<const f32x4_t*>(rc + R::GB + D + 4 * g);
+        o.br = rc[R::GB + D + r];
         return o;
     };
     // decay factors of this lane's four tokens at d = 16 w + r
@@ -805,57 +864,103 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
     lds_barrier();
 
     // ================ forwards ================
-    // S^T at the end of chunk kSpan / 2 - 1, kept for the way back (this wave's own)
+    // S^T at the end of the span's first half, kept for the way back (this wave's own)
     unsigned char* const mid = smem + G::OFF_MID + w * NT * 1024 + 16 * lane;
     for (int m = 0; m < nm; ++m) {
         const unsigned char* b = buf(m);
-        if (m == kSpan / 2) {
+        Own next = own;  // the next chunk's values, loaded a whole chunk ahead
+        if (m + 1 < nm) next = load_own(m + 1, true);
+        if (m == span_len / 2) {
 #pragma unroll
             for (int i = 0; i < NT; ++i) st4(mid + 1024 * i, St[i]);
         }
-        // dO S^T, W S^T, and this wave's parts of dO U^T and W U^T
+        // dO S^T, W S^T, and this wave's parts of dO U^T and W U^T.  (Operand reads go two
+        // tiles ahead of their products, fenced: left to itself the compiler reads each right
+        // before its use and waits out the LDS latency.)
         f32x4_t qa[2] = {kZero4, kZero4}, wa[2] = {kZero4, kZero4}, pp = kZero4, pa = kZero4;
-#pragma unroll
-        for (int i = 0; i < NT; ++i) {
-            const f32x4_t dor = ix.row(b + G::B_O, i);
-            const f32x4_t wrw = ix.row(b + G::B_W, i);
+        {
+            f32x4_t dor[NT], wrw[NT];
+            const f32x4_t uw = ix.roww(b + G::B_U, w, r), dw = ix.roww(b + G::B_O, w, r), ww = ix.roww(b + G::B_W, w, r);
+            auto rd = [&](int i) __attribute__((always_inline)) {
+                dor[i] = ix.row(b + G::B_O, i);
+                wrw[i] = ix.row(b + G::B_W, i);
+            };
+            rd(0);
+            fence();
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                qa[e & 1] = mfma4(dor[e], St[i][e], qa[e & 1]);
-                wa[e & 1] = mfma4(wrw[e], St[i][e], wa[e & 1]);
+                pp = mfma4(uw[e], dw[e], pp);  // (U dO^T)[4 g + v][r] = (dO U^T)[r][4 g + v]
+                pa = mfma4(uw[e], ww[e], pa);
             }
-            if (i == w) {
-                const f32x4_t ur = ix.row(b + G::B_U, i);
+            rd(1);
+            fence();
+#pragma unroll
+            for (int i = 0; i < NT; ++i) {
+                if (i + 2 < NT) rd(i + 2);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    pp = mfma4(ur[e], dor[e], pp);  // (U dO^T)[4 g + v][r] = (dO U^T)[r][4 g + v]
-                    pa = mfma4(ur[e], wrw[e], pa);
+                    qa[e & 1] = mfma4(dor[i][e], St[i][e], qa[e & 1]);
+                    wa[e & 1] = mfma4(wrw[i][e], St[i][e], wa[e & 1]);
                 }
+                fence();
             }
         }
         unsigned char* part = smem + G::OFF_PP + w * 2048;
         st4(part + 16 * (4 * r + g), pp);
         st4(part + 1024 + 16 * (4 * r + g), pa);
-        f32x4_t wj;  // W at this lane's columns 16 w + r of d_v
-#pragma unroll
-        for (int e = 0; e < 4; ++e) wj[e] = ix.colw(b + G::B_W, e, w, g);
-        const f32x4_t kk = own.k, qq = own.q, b4 = own.b4;
+        const f32x4_t kk = own.k, qq = own.q, b4 = own.b4, at = own.y;
         const float br = own.br;
         const Dec x = decays(own.lg);
         const f32x4_t khat = kk * x.F, kbar = kk * x.E;
-        // S^T = gC S^T + U^T K-
-#pragma unroll
-        for (int i = 0; i < NT; ++i) {
-            float uc[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) uc[e] = ix.col(b + G::B_U, e, i);
-            St[i] = St[i] * x.gc;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) St[i] = mfma4(uc[e], kbar[e], St[i]);
-        }
         const f32x4_t dQh = qa[0] + qa[1];          // dO S^T [4 g + v][16 w + r]
         const f32x4_t WS = wa[0] + wa[1];           // W S^T
         const f32x4_t kdk = -(b4 * WS);             // dL/dK^
+        lds_barrier();  // Y: the parts are in LDS
+        // the totals' operands, read here and summed behind the state update
+        constexpr int NZ = 512 / (NW * 64);  // entries of [dP, dA][t][s] per thread
+        float tv[NZ][NW];
+#pragma unroll
+        for (int n = 0; n < NZ; ++n)
+#pragma unroll
+            for (int u = 0; u < NW; ++u)
+                tv[n][u] = reinterpret_cast<const float*>(smem + G::OFF_PP + u * 2048)[tid + n * NW * 64];
+        f32x4_t wj;  // W at this lane's columns 16 w + r of d_v
+#pragma unroll
+        for (int e = 0; e < 4; ++e) wj[e] = ix.colw(b + G::B_W, e, w, g);
+        // S^T = gC S^T + U^T K-, tiles i and i + 4 together (their reads pair up)
+        {
+            constexpr int NP = NT > 4 ? 2 : 1;
+            float uc[2][NP][4];
+            auto rd = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int p = 0; p < NP; ++p) uc[i & 1][p][e] = ix.col(b + G::B_U, e, i + 4 * p);
+            };
+            rd(0);
+#pragma unroll
+            for (int i = 0; i < NT; ++i) St[i] = St[i] * x.gc;
+            fence();
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (i + 1 < 4) rd(i + 1);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int p = 0; p < NP; ++p) St[i + 4 * p] = mfma4(uc[i & 1][p][e], kbar[e], St[i + 4 * p]);
+                fence();
+            }
+        }
+#pragma unroll
+        for (int n = 0; n < NZ; ++n) {
+            float sum = tv[n][0];
+#pragma unroll
+            for (int u = 1; u < NW; ++u) sum += tv[n][u];
+            const int z = tid + n * NW * 64, mat = z >> 8, t = (z >> 4) & 15, s = z & 15;
+            const float val = mat == 0 ? (s <= t ? sum : 0.f) : (s < t ? -sum : 0.f);
+            reinterpret_cast<float*>(smem + G::OFF_TR + mat * 1024)[16 * t + s] = val;
+            reinterpret_cast<float*>(smem + G::OFF_TC + mat * 1280)[20 * s + t] = val;
+        }
         {
             // this wave's part of W.V - K^ . W S^T per token 4 g + v
             f32x4_t s = wj * own.x - khat * WS;
@@ -863,23 +968,10 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
             for (int e = 0; e < 4; ++e) s[e] = row16_sum(s[e]);
             if (r == 0) st4(smem + G::OFF_DB + ((m & 1) * NW + w) * 64 + 16 * g, s);
         }
-        lds_barrier();  // Y: the parts are in LDS; every wave is done reading chunk m's rows
+        // chunk m + 1's copies have landed (they are older than chunk m - 1's eight stores)
+        wait_vm_n<8>();
+        lds_barrier();  // Z: totals in LDS, chunk m + 1 in its buffer, every wave done with chunk m's
         if (m + 2 < nm) issue(m + 2);
-        for (int z = tid; z < 512; z += NW * 64) {
-            const int mat = z >> 8, t = (z >> 4) & 15, s = z & 15;
-            float sum = 0.f;
-#pragma unroll
-            for (int ww = 0; ww < NW; ++ww)
-                sum += reinterpret_cast<const float*>(smem + G::OFF_PP + ww * 2048 + mat * 1024)[16 * t + s];
-            const float val = mat == 0 ? (s <= t ? sum : 0.f) : (s < t ? -sum : 0.f);
-            reinterpret_cast<float*>(smem + G::OFF_TR + mat * 1024)[16 * t + s] = val;
-            reinterpret_cast<float*>(smem + G::OFF_TC + mat * 1280)[20 * s + t] = val;
-        }
-        // chunk m + 1's copies have landed; chunk m + 2's may be in flight
-        if (m + 2 < nm) wait_vm_n<kMine>();
-        else wait_vm_n<0>();
-        lds_barrier();  // Z: totals in LDS, chunk m + 1 in its buffer
-        if (m + 1 < nm) own = load_own(m + 1, true);
         const f32x4_t dpr = ld4(smem + G::OFF_TR + 16 * (4 * r + g));            // dP[r][4 g ..]
         const f32x4_t dar = ld4(smem + G::OFF_TR + 1024 + 16 * (4 * r + g));     // dA[r][4 g ..]
         const f32x4_t dpc = ld4(smem + G::OFF_TC + 4 * (20 * r + 4 * g));        // dP[4 g ..][r]
@@ -958,7 +1050,6 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
         }
         if (w == 0) {
             // dbeta_t = W_t . V_t - K^_t . (W S^T)_t + sum_s dA_ts A'_ts, t = r
-            const f32x4_t at = *reinterpret_cast<const f32x4_t*>(rec + (item0 + m) * R::FLOATS + R::AT + 4 * lane);
             float s = dar[0] * at[0] + dar[1] * at[1] + dar[2] * at[2] + dar[3] * at[3];
             s += __shfl_xor(s, 16);
             s += __shfl_xor(s, 32);
@@ -968,6 +1059,7 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
                 wx += reinterpret_cast<const float*>(smem + G::OFF_DB + ((m & 1) * NW + ww) * 64)[r];
             if (g == 0 && r < clen_of(m)) gbeta[(tok0 + m * kC16 + r) * H + h] = wx + s;
         }
+        own = next;
     }
 
     // ================ backwards ================
@@ -987,9 +1079,11 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
     float hs = 0.f;  // <S, G> of row 16 w + r at the end of the chunk
     for (int m = nm - 1; m >= 0; --m) {
         const unsigned char* b = buf(m);
-        if (m == nm - 1 || m == kSpan / 2 - 1) {
+        Own next = own;
+        if (m > 0) next = load_own(m - 1, false);
+        if (m == nm - 1 || m == span_len / 2 - 1) {
             // from the states themselves at two places of a span, so that the sums carried
-            // along the chunks span 64 tokens at most
+            // along the chunks cover 64 tokens at most
             f32x4_t s = kZero4;
             if (m == nm - 1) {
 #pragma unroll
@@ -1002,28 +1096,50 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
         }
         // U G^T
         f32x4_t ka[2] = {kZero4, kZero4};
+        {
+            f32x4_t ur[NT];
+            ur[0] = ix.row(b + G::B_U, 0);
+            ur[1] = ix.row(b + G::B_U, 1);
+            fence();
 #pragma unroll
-        for (int i = 0; i < NT; ++i) {
-            const f32x4_t ur = ix.row(b + G::B_U, i);
+            for (int i = 0; i < NT; ++i) {
+                if (i + 2 < NT) ur[i + 2] = ix.row(b + G::B_U, i + 2);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) ka[e & 1] = mfma4(ur[e], Gt[i][e], ka[e & 1]);
+                for (int e = 0; e < 4; ++e) ka[e & 1] = mfma4(ur[i][e], Gt[i][e], ka[e & 1]);
+                fence();
+            }
         }
         const Dec x = decays(own.lg);
         const f32x4_t khat = own.k * x.F, qhat = own.q * x.F;
-        // G^T = gC G^T + dO^T Q^ - (diag(beta) W)^T K^
+        // G^T = gC G^T + dO^T Q^ - W^T diag(beta) K^
+        {
+            constexpr int NP = NT > 4 ? 2 : 1;
+            const f32x4_t nk = -(own.b4 * khat);
+            float dc[2][NP][4], wc[2][NP][4];
+            auto rd = [&](int i) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < NT; ++i) {
-            float dc[4], wc[4];
+                for (int e = 0; e < 4; ++e)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                dc[e] = ix.col(b + G::B_O, e, i);
-                wc[e] = -own.b4[e] * ix.col(b + G::B_W, e, i);
-            }
-            Gt[i] = Gt[i] * x.gc;
+                    for (int p = 0; p < NP; ++p) {
+                        dc[i & 1][p][e] = ix.col(b + G::B_O, e, i + 4 * p);
+                        wc[i & 1][p][e] = ix.col(b + G::B_W, e, i + 4 * p);
+                    }
+            };
+            rd(0);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                Gt[i] = mfma4(dc[e], qhat[e], Gt[i]);
-                Gt[i] = mfma4(wc[e], khat[e], Gt[i]);
+            for (int i = 0; i < NT; ++i) Gt[i] = Gt[i] * x.gc;
+            fence();
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (i + 1 < 4) rd(i + 1);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int p = 0; p < NP; ++p) {
+                        Gt[i + 4 * p] = mfma4(dc[i & 1][p][e], qhat[e], Gt[i + 4 * p]);
+                        Gt[i + 4 * p] = mfma4(wc[i & 1][p][e], nk[e], Gt[i + 4 * p]);
+                    }
+                fence();
             }
         }
         const f32x4_t dKb = x.E * (ka[0] + ka[1]);  // dL/dK- scaled: dK's part
@@ -1067,7 +1183,7 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
             wait_vm_n<4>();
             lds_barrier();
             if (m >= 2) issue(m - 2);
-            own = load_own(m - 1, false);
+            own = next;
         }
     }
     if constexpr (!CHAN) {
@@ -1096,11 +1212,22 @@ hipError_t set_lds(int bytes) {
     return e;
 }
 
+// Chunks per span: a power of two up to kSpan, halved while the span kernel would leave CUs
+// without a workgroup (a span is one workgroup's sequence of 2 x span_len chunk steps; the
+// histories it reads grow as it shrinks, a quarter of the other traffic at 2).
+int span_len_for(long n_pairs, int T) {
+    const long n_ch = (T + kC16 - 1) / kC16;
+    int s = kSpan;
+    while (s > 2 && n_pairs * ((n_ch + s - 1) / s) < 256) s /= 2;
+    return s;
+}
+
 struct DecBwdWs {
     size_t kh, kb, qh, rec, s_hist, g_hist, w, u, bytes;
 };
 DecBwdWs dec_bwd_ws(long n_pairs, int T, int D) {
-    const size_t n_ch = static_cast<size_t>((T + kC16 - 1) / kC16), n_span = (n_ch + kSpan - 1) / kSpan;
+    const size_t n_ch = static_cast<size_t>((T + kC16 - 1) / kC16), sl = span_len_for(n_pairs, T);
+    const size_t n_span = (n_ch + sl - 1) / sl;
     const size_t np = static_cast<size_t>(n_pairs), tile = np * n_ch * kC16 * D * 4;
     const size_t rec = np * n_ch * (D == 128 ? DecRec<128>::FLOATS : DecRec<64>::FLOATS) * 4;
     auto al = [](size_t x) { return (x + 255) & ~static_cast<size_t>(255); };
@@ -1119,7 +1246,7 @@ DecBwdWs dec_bwd_ws(long n_pairs, int T, int D) {
 
 template <int D, typename InT, bool CHAN>
 hipError_t launch_t(const BwdArgs& a, hipStream_t st) {
-    const int n_ch = (a.T + kC16 - 1) / kC16, n_span = (n_ch + kSpan - 1) / kSpan;
+    const int n_ch = (a.T + kC16 - 1) / kC16, sl = span_len_for(a.n_pairs, a.T), n_span = (n_ch + sl - 1) / sl;
     const DecBwdWs o = dec_bwd_ws(a.n_pairs, a.T, D);
     unsigned char* base = reinterpret_cast<unsigned char*>(a.workspace);
     auto at = [&](size_t off) { return reinterpret_cast<float*>(base + off); };
@@ -1134,11 +1261,11 @@ hipError_t launch_t(const BwdArgs& a, hipStream_t st) {
     const int slots = (a.n_pairs + 7) / 8;
     hipLaunchKernelGGL((dec_sweep_kernel<D, InT>), dim3(static_cast<unsigned>(slots * (D / 32) * 8)), dim3(512),
                        DsGeo<D>::BYTES, st, v, a.s0, a.go, a.gs, a.gv, a.gs0, at(o.kh), at(o.kb), at(o.qh), at(o.rec),
-                       at(o.w), at(o.u), at(o.s_hist), at(o.g_hist), a.n_pairs, a.T, a.H, n_ch, n_span);
+                       at(o.w), at(o.u), at(o.s_hist), at(o.g_hist), a.n_pairs, a.T, a.H, n_ch, n_span, sl);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     hipLaunchKernelGGL((dec_span_kernel<D, InT, CHAN>), dim3(static_cast<unsigned>(a.n_pairs * n_span)), dim3(D * 4),
                        DcGeo<D>::BYTES, st, q, k, v, a.g, a.go, at(o.rec), at(o.s_hist), at(o.g_hist), at(o.w), at(o.u),
-                       a.gq, a.gk, a.gbeta, a.gg, a.T, a.H, n_ch, n_span);
+                       a.gq, a.gk, a.gbeta, a.gg, a.T, a.H, n_ch, n_span, sl);
     return hipGetLastError();
 }
 
