@@ -46,7 +46,7 @@
 extern "C" {
 #endif
 
-#define PM_DELTA_ABI_VERSION 13
+#define PM_DELTA_ABI_VERSION 14
 
 /* element types */
 #define PM_DTYPE_F32 0
@@ -359,6 +359,40 @@ int pm_kda_delta_bwd(const void* q, const void* k, const void* v, const float* b
  * pm_delta_bwd's per-token workspace plus, for D > 32, the partial sums of gg per
  * column tile. */
 size_t pm_kda_delta_bwd_workspace_bytes(int B, int T, int H, int D, int in_dtype);
+
+/*
+ * pm_delta_bwd (g NULL), pm_gated_delta_bwd (g given, per_channel 0) or
+ * pm_kda_delta_bwd (per_channel 1) for bf16 q/k/v with gq, gk and gv written
+ * as bf16 (each the fp32 gradient rounded to nearest even, once): what a
+ * training step that keeps bf16 gradients casts them to anyway (the
+ * reference's VJP returns its inputs' dtypes' cotangents after
+ * kernels/__init__.py:638-658).  gbeta, gg and gs0 stay fp32.  Workspace and
+ * alignment as those entry points'.  Only where they would run a chunked
+ * kernel; PM_E_UNSUPPORTED otherwise, with nothing launched.
+ */
+int pm_delta_bwd_bf16(const void* q, const void* k, const void* v, const float* beta,
+                      const float* g, const float* s0, const float* go, const float* gs, void* gq,
+                      void* gk, void* gv, float* gbeta, float* gg, float* gs0, int B, int T, int H,
+                      int D, int per_channel, void* workspace, size_t ws_bytes, void* stream);
+
+/*
+ * Reverse mode of pm_linear_attention: the gradients of q, k, v (in in_dtype,
+ * (B, T, H, D)) and of s0 (fp32) given go = dL/dO and gs = dL/dS_T (fp32, either
+ * may be NULL).  The counterpart of JAX differentiating
+ * model/__init__.py:393-432.  One pass normalises q and k into the workspace
+ * (x / max(||x||, 1e-6), rounded to in_dtype), pm_delta_bwd's kernels run on the
+ * normalised rows with beta = 1, and one pass takes the fp32 gradients of the
+ * normalised rows back through the normalisation.  Alignment as pm_delta_bwd's
+ * (v, go, gv); workspace: pm_linear_attention_bwd_workspace_bytes, 16-byte aligned.
+ */
+int pm_linear_attention_bwd(const void* q, const void* k, const void* v, const float* s0,
+                            const float* go, const float* gs, void* gq, void* gk, void* gv,
+                            float* gs0, int B, int T, int H, int D, int in_dtype, void* workspace,
+                            size_t ws_bytes, void* stream);
+/* Workspace bytes pm_linear_attention_bwd needs under the current path setting (0 for
+ * invalid shapes or dtypes): pm_delta_bwd's, the normalised rows, ones and their fp32
+ * gradients. */
+size_t pm_linear_attention_bwd_workspace_bytes(int B, int T, int H, int D, int in_dtype);
 
 /*
  * pm_delta_bwd without a caller workspace and without any allocation.

@@ -18,7 +18,7 @@ import torch  # noqa: F401  (see module docstring: must precede CDLL)
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libpmdelta.so")
 
-ABI_VERSION = 13
+ABI_VERSION = 14
 DTYPE_F32 = 0
 DTYPE_BF16 = 1
 MAX_D = 256
@@ -43,6 +43,9 @@ EXPORTS = (
     "pm_delta_bwd",
     "pm_delta_bwd_workspace_bytes",
     "pm_delta_bwd_noalloc",
+    "pm_delta_bwd_bf16",
+    "pm_linear_attention_bwd",
+    "pm_linear_attention_bwd_workspace_bytes",
     "pm_last_error",
     "pm_abi_version",
     "pm_delta_set_path",
@@ -119,6 +122,12 @@ def lib() -> ctypes.CDLL:
         L.pm_delta_bwd_workspace_bytes.restype = sz
         L.pm_delta_bwd_noalloc.argtypes = [vp] * 12 + [i] * 5 + [vp]
         L.pm_delta_bwd_noalloc.restype = i
+        L.pm_delta_bwd_bf16.argtypes = [vp] * 14 + [i] * 5 + [vp, sz, vp]
+        L.pm_delta_bwd_bf16.restype = i
+        L.pm_linear_attention_bwd.argtypes = [vp] * 10 + [i] * 5 + [vp, sz, vp]
+        L.pm_linear_attention_bwd.restype = i
+        L.pm_linear_attention_bwd_workspace_bytes.argtypes = [i] * 5
+        L.pm_linear_attention_bwd_workspace_bytes.restype = sz
         L.pm_last_error.argtypes = []
         L.pm_last_error.restype = ctypes.c_char_p
         L.pm_abi_version.argtypes = []

@@ -45,6 +45,17 @@
 //     its end gradient (the rest).  S cannot be walked back as the ungated backward does
 //     (that divides by gC), hence the two walks.
 
+// Why chunks: the per-token kernels walk T tokens in sequence at about 500 (forward) and
+// 1,270 cycles (reverse) a token, bound by VALU issue; here a chunk of 16 tokens takes
+// about 4,300 cycles of the one sequential launch, and the rest is parallel over chunks.
+// Measured, B4 T4096 H16 D128, bf16 q/k/v, per-head gate: 6.0 -> 1.45 ms (K10p 126, K10s
+// 530, K10c 800 us); B2, per-channel gate: 5.9 -> 1.06 ms; B3 T1000 H6 D64 fp32: 1.11 -> 0.13
+// ms.  Against 64 bits the gradients stay at 2e-7 to 5e-7 (the per-token kernels: 1.3e-7 to
+// 2e-7).  What bounds it: K10s the chain of its four recurrence waves (72 MFMAs of 32 cycles a
+// chunk, in sequence; without the helpers' Q^^T dO 460 us, without copies, stores and helpers
+// 405), K10c the fp32 MFMA pipe at half its rate (232 products per wave and chunk; two waves
+// per SIMD, which wait for the pipe half of the time and at its barriers a third).
+
 #include <type_traits>
 
 #include "pm_cdna4.h"
@@ -60,6 +71,10 @@ __device__ __forceinline__ f32x4_t ld4(const unsigned char* p) { return *reinter
 __device__ __forceinline__ void st4(unsigned char* p, f32x4_t x) { *reinterpret_cast<f32x4_t*>(p) = x; }
 __device__ __forceinline__ void fence() { __builtin_amdgcn_sched_barrier(0); }
 constexpr f32x4_t kZero4 = {0.f, 0.f, 0.f, 0.f};
+__device__ __forceinline__ f32x4_t fma4(f32x4_t a, f32x4_t b, f32x4_t c) {
+    const f32x4_t r = {fmaf(a[0], b[0], c[0]), fmaf(a[1], b[1], c[1]), fmaf(a[2], b[2], c[2]), fmaf(a[3], b[3], c[3])};
+    return r;
+}
 
 // One chunk's record (floats): T''^T, T, P, A'^T as accumulator registers, then gC (D) and
 // beta (16), padded to a multiple of 64 (copied 256 bytes an instruction).
@@ -114,6 +129,14 @@ __device__ __forceinline__ f32x4_t buf_el4(__amdgpu_buffer_rsrc_t rs, unsigned e
         return widen4(__builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(rs, elem * 2, 0, 0)));
     else
         return __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rs, elem * 4, 0, 0));
+}
+// One gradient element of GE bytes (rows past the range dropped)
+template <int GE>
+__device__ __forceinline__ void put(float x, __amdgpu_buffer_rsrc_t rs, unsigned elem) {
+    if constexpr (GE == 2)
+        __builtin_amdgcn_raw_buffer_store_b16(f32_to_bf16(x), rs, elem * 2, 0, 0);
+    else
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x), rs, elem * 4, 0, 0);
 }
 template <int CTRL>
 __device__ __forceinline__ float dpp_mov(float x) {
@@ -352,10 +375,11 @@ struct DsGeo {
     static_assert(HBUF % 16 == 0 && SBUF % 16 == 0, "alignment");
 };
 
-template <int D, typename InT>
+// GE: bytes per element of dQ, dK and dV (4: fp32; 2: bf16, rounded to nearest even)
+template <int D, typename InT, int GE>
 __global__ __launch_bounds__(512) void dec_sweep_kernel(
     const InT* __restrict__ v, const float* __restrict__ s0, const float* __restrict__ go,
-    const float* __restrict__ gs, float* __restrict__ gv, float* __restrict__ gs0, const float* __restrict__ kh,
+    const float* __restrict__ gs, void* __restrict__ gv, float* __restrict__ gs0, const float* __restrict__ kh,
     const float* __restrict__ kb, const float* __restrict__ qh, const float* __restrict__ rec,
     float* __restrict__ w_out, float* __restrict__ u_out, float* __restrict__ s_hist, float* __restrict__ g_hist,
     int n_pairs, int T, int H, int n_ch, int n_span, int span_len) {
@@ -591,10 +615,13 @@ __global__ __launch_bounds__(512) void dec_sweep_kernel(
                     for (int e = 0; e < 4; ++e) x[e] = ws[4 * (16 * (t >> 2) + 4 * p + e) + (t & 3)];
                     *reinterpret_cast<f32x4_t*>(w_out + (item0 + cs) * kC16 * D +
                                                 4 * f32_chunk<D>(t, (col0 + 16 * j) / 4 + p)) = x;
-                    __builtin_amdgcn_raw_buffer_store_b128(
-                        __builtin_bit_cast(u32x4_t, x * bt),
-                        make_rsrc(gv + row0_of(cs, col0 + 16 * j), els_of(cs, 16) * 4),
-                        static_cast<unsigned>((t * tstride + 4 * p) * 4), 0, 0);
+                    const __amdgpu_buffer_rsrc_t rv = make_rsrc(
+                        static_cast<unsigned char*>(gv) + row0_of(cs, col0 + 16 * j) * GE, els_of(cs, 16) * GE);
+                    const unsigned off = static_cast<unsigned>((t * tstride + 4 * p) * GE);
+                    if constexpr (GE == 2)
+                        __builtin_amdgcn_raw_buffer_store_b64(cvt4(x * bt), rv, off, 0, 0);
+                    else
+                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, x * bt), rv, off, 0, 0);
                 }
             }
             if (i <= n_ch) {
@@ -732,13 +759,16 @@ struct DcGeo {
     static_assert(BYTES <= 160 * 1024, "LDS");
 };
 
-template <int D, typename InT, bool CHAN>
+template <int D, typename InT, bool CHAN, int GE>
 __global__ __launch_bounds__(D * 4) void dec_span_kernel(
     const InT* __restrict__ q, const InT* __restrict__ k, const InT* __restrict__ v, const float* __restrict__ gate,
     const float* __restrict__ go, const float* __restrict__ rec, const float* __restrict__ s_hist,
     const float* __restrict__ g_hist, const float* __restrict__ w_in, const float* __restrict__ u_in,
-    float* __restrict__ gq, float* __restrict__ gk, float* __restrict__ gbeta, float* __restrict__ gg, int T, int H,
-    int n_ch, int n_span, int span_len) {
+    void* __restrict__ gq, void* __restrict__ gk, float* __restrict__ gbeta, float* __restrict__ gg,
+    float* __restrict__ pk_ws, float* __restrict__ pg_ws, int T, int H, int n_ch, int n_span, int span_len) {
+    // multiply-adds are fused only where written so (fmaf): every build of this kernel gives the
+    // same bits, and bf16 gradients are the fp32 ones rounded
+#pragma clang fp contract(off)
     using G = DcGeo<D>;
     using R = DecRec<D>;
     constexpr int NW = G::NW, NT = G::NT;
@@ -781,6 +811,9 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
     constexpr int kMine = G::NC / NW;  // copies each wave issues per chunk
     static_assert(G::NC % NW == 0, "copies divide over the waves");
 
+    // this lane's four values of a chunk in the scratch that the way forwards leaves the
+    // gradients of k and of a per-channel gate in for the way back (fp32, one 16-byte store)
+    auto part_of = [=](int m) { return (item0 + m) * kC16 * D + 256 * w + 4 * lane; };
     // this lane's tokens of a chunk, as loaded (tokens past the end read zeros)
     struct Own {
         f32x4_t k, q, x, lg, b4;  // x: v (forwards) or the gradient so far of k (backwards)
@@ -793,19 +826,21 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
         const unsigned nel = static_cast<unsigned>((clen - 1) * tstride + 16);
         const size_t r0 = row0_of(m, 16 * w);
         const __amdgpu_buffer_rsrc_t rk = make_rsrc(k + r0, nel * sizeof(InT)), rq = make_rsrc(q + r0, nel * sizeof(InT));
-        const __amdgpu_buffer_rsrc_t rv = make_rsrc(v + r0, nel * sizeof(InT)), rgk = make_rsrc(gk + r0, nel * 4);
+        const __amdgpu_buffer_rsrc_t rv = make_rsrc(v + r0, nel * sizeof(InT));
         const __amdgpu_buffer_rsrc_t rg = CHAN ? make_rsrc(gate + r0, nel * 4)
                                                : make_rsrc(gate + (tok0 + m * kC16) * H + h,
                                                            static_cast<unsigned>(((clen - 1) * H + 1) * 4));
-        const __amdgpu_buffer_rsrc_t rgg = make_rsrc(CHAN ? gg + r0 : gg, CHAN ? nel * 4 : 0u);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const unsigned el = static_cast<unsigned>((4 * g + e) * tstride + r);
             o.k[e] = buf_el<InT>(rk, el);
             o.q[e] = buf_el<InT>(rq, el);
             o.lg[e] = buf_el<float>(rg, CHAN ? el : static_cast<unsigned>((4 * g + e) * H));
-            o.x[e] = fwd ? buf_el<InT>(rv, el) : buf_el<float>(rgk, el);
-            if (!fwd) o.y[e] = CHAN ? buf_el<float>(rgg, el) : 0.f;
+            if (fwd) o.x[e] = buf_el<InT>(rv, el);
+        }
+        if (!fwd) {
+            o.x = *reinterpret_cast<const f32x4_t*>(pk_ws + part_of(m));
+            o.y = CHAN ? *reinterpret_cast<const f32x4_t*>(pg_ws + part_of(m)) : kZero4;
         }
         const float* rc = rec + (item0 + m) * R::FLOATS;
         if (fwd) o.y = *reinterpret_cast<const f32x4_t*>(rc + R::AT + 4 * lane);
@@ -963,13 +998,13 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
         }
         {
             // this wave's part of W.V - K^ . W S^T per token 4 g + v
-            f32x4_t s = wj * own.x - khat * WS;
+            f32x4_t s = fma4(wj, own.x, -(khat * WS));
 #pragma unroll
             for (int e = 0; e < 4; ++e) s[e] = row16_sum(s[e]);
             if (r == 0) st4(smem + G::OFF_DB + ((m & 1) * NW + w) * 64 + 16 * g, s);
         }
-        // chunk m + 1's copies have landed (they are older than chunk m - 1's eight stores)
-        wait_vm_n<8>();
+        // chunk m + 1's copies have landed (they are older than chunk m - 1's five stores)
+        wait_vm_n<4>();
         lds_barrier();  // Z: totals in LDS, chunk m + 1 in its buffer, every wave done with chunk m's
         if (m + 2 < nm) issue(m + 2);
         const f32x4_t dpr = ld4(smem + G::OFF_TR + 16 * (4 * r + g));            // dP[r][4 g ..]
@@ -996,7 +1031,7 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
             zc8 = mfma4(c8 ? dd : 0.f, kf8[e], zc8);
             zc4 = mfma4(c4 ? dd : 0.f, kf4[e], zc4);
         }
-        f32x4_t pq = x.F8 * zq8 + x.F4 * zq4, pk = x.F8 * zk8 + x.F4 * zk4, pc = x.E8 * zc8 + x.E4 * zc4;
+        f32x4_t pq = fma4(x.F8, zq8, x.F4 * zq4), pk = fma4(x.F8, zk8, x.F4 * zk4), pc = fma4(x.E8, zc8, x.E4 * zc4);
         // pairs inside this lane's four tokens
         f32x4_t dg;
 #pragma unroll
@@ -1015,8 +1050,8 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
             }
         }
         // the gate: own terms and pair terms, summed over the tokens at and after each
-        const f32x4_t own_t = qq * (x.F * dQh) + khat * kdk;
-        const f32x4_t pair_t = qq * pq + kk * (pk - pc);
+        const f32x4_t own_t = fma4(qq, x.F * dQh, khat * kdk);
+        const f32x4_t pair_t = fma4(qq, pq, kk * (pk - pc));
         const float ec = col_total(own_t);
         if (g == 0) reinterpret_cast<float*>(smem + G::OFF_EC)[m * D + 16 * w + r] = ec;
         f32x4_t suf = own_t + pair_t;
@@ -1028,20 +1063,16 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
             const float t8 = t4 + s4, s8 = __shfl_xor(t8, 32);
             suf += ((g & 1) ? 0.f : s4) + ((g & 2) ? 0.f : s8);
         }
-        const f32x4_t dQ = x.F * dQh + pq + dg * kk;
-        const f32x4_t dK = x.F * kdk + (pk + pc) + dg * qq;
+        const f32x4_t dQ = fma4(x.F, dQh, fma4(dg, kk, pq));
+        const f32x4_t dK = fma4(x.F, kdk, fma4(dg, qq, pk + pc));
         {
-            const unsigned nb = static_cast<unsigned>(((clen_of(m) - 1) * tstride + 16) * 4);
+            const unsigned nb = static_cast<unsigned>(((clen_of(m) - 1) * tstride + 16) * GE);
             const size_t r0 = row0_of(m, 16 * w);
-            const __amdgpu_buffer_rsrc_t rq = make_rsrc(gq + r0, nb), rk = make_rsrc(gk + r0, nb);
-            const __amdgpu_buffer_rsrc_t rgg = make_rsrc(CHAN ? gg + r0 : gg, CHAN ? nb : 0u);
+            const __amdgpu_buffer_rsrc_t rq = make_rsrc(static_cast<unsigned char*>(gq) + r0 * GE, nb);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const unsigned off = static_cast<unsigned>(((4 * g + e) * tstride + r) * 4);
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dQ[e]), rq, off, 0, 0);
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dK[e]), rk, off, 0, 0);
-                if constexpr (CHAN) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(suf[e]), rgg, off, 0, 0);
-            }
+            for (int e = 0; e < 4; ++e) put<GE>(dQ[e], rq, static_cast<unsigned>((4 * g + e) * tstride + r));
+            *reinterpret_cast<f32x4_t*>(pk_ws + part_of(m)) = dK;
+            if constexpr (CHAN) *reinterpret_cast<f32x4_t*>(pg_ws + part_of(m)) = suf;
         }
         if constexpr (!CHAN) {
 #pragma unroll
@@ -1050,7 +1081,7 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
         }
         if (w == 0) {
             // dbeta_t = W_t . V_t - K^_t . (W S^T)_t + sum_s dA_ts A'_ts, t = r
-            float s = dar[0] * at[0] + dar[1] * at[1] + dar[2] * at[2] + dar[3] * at[3];
+            float s = fmaf(dar[0], at[0], fmaf(dar[1], at[1], fmaf(dar[2], at[2], dar[3] * at[3])));
             s += __shfl_xor(s, 16);
             s += __shfl_xor(s, 32);
             float wx = 0.f;
@@ -1063,8 +1094,8 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
     }
 
     // ================ backwards ================
-    // (the last two chunks are still in their buffers; this wave's own stores of gk and gg are
-    // read back below, after the wait)
+    // (the last two chunks are still in their buffers; this wave's own stores of the scratch
+    // are read back below, after the wait)
     f32x4_t Gt[NT];
     {
         const float* gp = g_hist + (static_cast<size_t>(pair) * n_span + span) * D * D;
@@ -1087,10 +1118,10 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
             f32x4_t s = kZero4;
             if (m == nm - 1) {
 #pragma unroll
-                for (int i = 0; i < NT; ++i) s += St[i] * Gt[i];
+                for (int i = 0; i < NT; ++i) s = fma4(St[i], Gt[i], s);
             } else {
 #pragma unroll
-                for (int i = 0; i < NT; ++i) s += ld4(mid + 1024 * i) * Gt[i];
+                for (int i = 0; i < NT; ++i) s = fma4(ld4(mid + 1024 * i), Gt[i], s);
             }
             hs = col_total(s);
         }
@@ -1160,16 +1191,15 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
             pre += sg + (((g & 1) ? s4 : 0.f) + ((g & 2) ? s8 : 0.f));
         }
         {
-            const unsigned nb = static_cast<unsigned>(((clen_of(m) - 1) * tstride + 16) * 4);
+            const unsigned nel = static_cast<unsigned>((clen_of(m) - 1) * tstride + 16);
             const size_t r0 = row0_of(m, 16 * w);
-            const __amdgpu_buffer_rsrc_t rk = make_rsrc(gk + r0, nb);
-            const __amdgpu_buffer_rsrc_t rgg = make_rsrc(CHAN ? gg + r0 : gg, CHAN ? nb : 0u);
+            const __amdgpu_buffer_rsrc_t rk = make_rsrc(static_cast<unsigned char*>(gk) + r0 * GE, nel * GE);
+            const __amdgpu_buffer_rsrc_t rgg = make_rsrc(CHAN ? gg + r0 : gg, CHAN ? nel * 4 : 0u);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const unsigned off = static_cast<unsigned>(((4 * g + e) * tstride + r) * 4);
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dK[e]), rk, off, 0, 0);
-                if constexpr (CHAN)
-                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(own.y[e] + pre[e]), rgg, off, 0, 0);
+                const unsigned el = static_cast<unsigned>((4 * g + e) * tstride + r);
+                put<GE>(dK[e], rk, el);
+                if constexpr (CHAN) put<4>(own.y[e] + pre[e], rgg, el);
             }
         }
         if constexpr (!CHAN) {
@@ -1244,28 +1274,28 @@ DecBwdWs dec_bwd_ws(long n_pairs, int T, int D) {
     return w;
 }
 
-template <int D, typename InT, bool CHAN>
+template <int D, typename InT, bool CHAN, int GE>
 hipError_t launch_t(const BwdArgs& a, hipStream_t st) {
     const int n_ch = (a.T + kC16 - 1) / kC16, sl = span_len_for(a.n_pairs, a.T), n_span = (n_ch + sl - 1) / sl;
     const DecBwdWs o = dec_bwd_ws(a.n_pairs, a.T, D);
     unsigned char* base = reinterpret_cast<unsigned char*>(a.workspace);
     auto at = [&](size_t off) { return reinterpret_cast<float*>(base + off); };
     const InT *q = static_cast<const InT*>(a.q), *k = static_cast<const InT*>(a.k), *v = static_cast<const InT*>(a.v);
-    hipError_t e = set_lds<dec_sweep_kernel<D, InT>>(DsGeo<D>::BYTES);
+    hipError_t e = set_lds<dec_sweep_kernel<D, InT, GE>>(DsGeo<D>::BYTES);
     if (e != hipSuccess) return e;
-    if ((e = set_lds<dec_span_kernel<D, InT, CHAN>>(DcGeo<D>::BYTES)) != hipSuccess) return e;
+    if ((e = set_lds<dec_span_kernel<D, InT, CHAN, GE>>(DcGeo<D>::BYTES)) != hipSuccess) return e;
     const long n_items = static_cast<long>(a.n_pairs) * n_ch;
     hipLaunchKernelGGL((dec_prep_kernel<D, InT, CHAN>), dim3(static_cast<unsigned>((n_items + 3) / 4)), dim3(256), 0, st,
                        q, k, a.beta, a.g, a.T, a.H, n_ch, n_items, at(o.kh), at(o.kb), at(o.qh), at(o.rec));
     if ((e = hipGetLastError()) != hipSuccess) return e;
     const int slots = (a.n_pairs + 7) / 8;
-    hipLaunchKernelGGL((dec_sweep_kernel<D, InT>), dim3(static_cast<unsigned>(slots * (D / 32) * 8)), dim3(512),
+    hipLaunchKernelGGL((dec_sweep_kernel<D, InT, GE>), dim3(static_cast<unsigned>(slots * (D / 32) * 8)), dim3(512),
                        DsGeo<D>::BYTES, st, v, a.s0, a.go, a.gs, a.gv, a.gs0, at(o.kh), at(o.kb), at(o.qh), at(o.rec),
                        at(o.w), at(o.u), at(o.s_hist), at(o.g_hist), a.n_pairs, a.T, a.H, n_ch, n_span, sl);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL((dec_span_kernel<D, InT, CHAN>), dim3(static_cast<unsigned>(a.n_pairs * n_span)), dim3(D * 4),
+    hipLaunchKernelGGL((dec_span_kernel<D, InT, CHAN, GE>), dim3(static_cast<unsigned>(a.n_pairs * n_span)), dim3(D * 4),
                        DcGeo<D>::BYTES, st, q, k, v, a.g, a.go, at(o.rec), at(o.s_hist), at(o.g_hist), at(o.w), at(o.u),
-                       a.gq, a.gk, a.gbeta, a.gg, a.T, a.H, n_ch, n_span, sl);
+                       a.gq, a.gk, a.gbeta, a.gg, at(o.kh), at(o.kb), a.T, a.H, n_ch, n_span, sl);
     return hipGetLastError();
 }
 
@@ -1276,11 +1306,14 @@ size_t decay_bwd_ws_bytes(long n_pairs, int T, int D) { return dec_bwd_ws(n_pair
 hipError_t launch_decay_bwd(const BwdArgs& a, hipStream_t st) {
     if (a.n_pairs == 0 || a.T == 0) return hipSuccess;
     if (!f32_bwd_supported(a.D, a.H)) return hipErrorInvalidValue;
+    if (a.gqk_bf16 != a.gv_bf16 || (a.gv_bf16 && !a.in_bf16)) return hipErrorInvalidValue;
     auto go = [&](auto DD) {
         constexpr int D = decltype(DD)::value;
+        if (a.gv_bf16)
+            return a.per_channel ? launch_t<D, uint16_t, true, 2>(a, st) : launch_t<D, uint16_t, false, 2>(a, st);
         if (a.per_channel)
-            return a.in_bf16 ? launch_t<D, uint16_t, true>(a, st) : launch_t<D, float, true>(a, st);
-        return a.in_bf16 ? launch_t<D, uint16_t, false>(a, st) : launch_t<D, float, false>(a, st);
+            return a.in_bf16 ? launch_t<D, uint16_t, true, 4>(a, st) : launch_t<D, float, true, 4>(a, st);
+        return a.in_bf16 ? launch_t<D, uint16_t, false, 4>(a, st) : launch_t<D, float, false, 4>(a, st);
     };
     return a.D == 128 ? go(std::integral_constant<int, 128>{}) : go(std::integral_constant<int, 64>{});
 }

@@ -29,8 +29,10 @@
 //   3. bwd_grad_kernel, all chunks in parallel (one persistent workgroup
 //      per CU, the next chunk's inputs fetched during the last two phases):
 //      dQ, dK and dbeta from S_c, G_c, W and the chunk's q/k/v/beta.
-// Numerics as in the forward: bf16 operands, fp32 accumulation; G and the
-// outputs stay fp32.
+// Numerics as in the forward: bf16 operands, fp32 accumulation; G stays fp32, and the
+// outputs too unless the caller asks for dQ, dK, dV in bf16 (rounded once, at the store: a
+// training step that keeps bf16 gradients then saves a cast pass over each, 100 us of 638 at
+// B4 T4096 H16 D128).
 //
 // Operand orders.  An MFMA A (B) operand gives lane (g, l16) 8 values of row
 // (column) l16 along the contraction.  Operands read from LDS use the
@@ -169,11 +171,12 @@ struct RevGeo {
 // bank halves (2-way, the least two 128-byte rows of one parity allow).
 __device__ __forceinline__ int fdo(int t) { return 4 * ((t >> 2) & 1); }
 
-template <int D>
+// GV: bytes per element of dV (4: fp32; 2: bf16, rounded to nearest even at the store)
+template <int D, int GV>
 __global__ __launch_bounds__(320) __attribute__((amdgpu_waves_per_eu(2, 2))) void bwd_rev_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const float* __restrict__ beta,
     const float* __restrict__ go, const float* __restrict__ gs, uint16_t* __restrict__ t_ws,
-    uint16_t* __restrict__ g_hist, uint16_t* __restrict__ w_hist, float* __restrict__ gv,
+    uint16_t* __restrict__ g_hist, uint16_t* __restrict__ w_hist, void* __restrict__ gv,
     float* __restrict__ gs0, int n_pairs, int T, int H, int n_ch, int n_tiles) {
     using G = RevGeo<D>;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -368,12 +371,16 @@ __global__ __launch_bounds__(320) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     auto write_dv = [&](int cc, const u32x4_t (&x)[G::N_DO]) {
         const int cb = cc * kC, cl = min(kC, T - cb);
         const __amdgpu_buffer_rsrc_t rv =
-            make_rsrc(gv + (tok0 + cb) * tstride + static_cast<size_t>(h) * D + col0,
-                      static_cast<unsigned>(((cl - 1) * tstride + G::NC) * 4));
+            make_rsrc(static_cast<unsigned char*>(gv) + ((tok0 + cb) * tstride + static_cast<size_t>(h) * D + col0) * GV,
+                      static_cast<unsigned>(((cl - 1) * tstride + G::NC) * GV));
 #pragma unroll
         for (int ii = 0; ii < G::N_DO; ++ii) {
             const int r = 8 * ii + (lane >> 3), p = lane & 7;
-            __builtin_amdgcn_raw_buffer_store_b128(x[ii], rv, static_cast<unsigned>((r * tstride + 4 * p) * 4), 0, 0);
+            const unsigned off = static_cast<unsigned>((r * tstride + 4 * p) * GV);
+            if constexpr (GV == 2)
+                __builtin_amdgcn_raw_buffer_store_b64(cvt4(__builtin_bit_cast(f32x4_t, x[ii])), rv, off, 0, 0);
+            else
+                __builtin_amdgcn_raw_buffer_store_b128(x[ii], rv, off, 0, 0);
         }
     };
     // One LDS-only barrier per chunk: by then the chunk the chain takes next is in LDS with
@@ -636,12 +643,13 @@ struct GradGeo {
     static_assert(BYTES <= 160 * 1024, "LDS budget");
 };
 
-template <int D>
+// GQK: bytes per element of dQ and dK (4: fp32; 2: bf16)
+template <int D, int GQK>
 __global__ __launch_bounds__(256) void bwd_grad_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     const float* __restrict__ beta, const float* __restrict__ go, const uint16_t* __restrict__ s_hist,
     const uint16_t* __restrict__ g_hist, const uint16_t* __restrict__ w_hist,
-    const uint16_t* __restrict__ tp_ws, float* __restrict__ gq, float* __restrict__ gk,
+    const uint16_t* __restrict__ tp_ws, void* __restrict__ gq, void* __restrict__ gk,
     float* __restrict__ gbeta, int T, int H, int n_ch, int n_total) {
     using G = GradGeo<D>;
     constexpr int JW = G::JW;
@@ -1055,8 +1063,9 @@ __global__ __launch_bounds__(256) void bwd_grad_kernel(
         // every wave issues exactly kStores of them whatever the chunk's length.
         constexpr int kStores = 2 * 4 * JW;
         {
-            const unsigned nb = static_cast<unsigned>(((clen - 1) * tstride + D) * 4);
-            const __amdgpu_buffer_rsrc_t rq = make_rsrc(gq + row0, nb), rk = make_rsrc(gk + row0, nb);
+            const unsigned nb = static_cast<unsigned>(((clen - 1) * tstride + D) * GQK);
+            const __amdgpu_buffer_rsrc_t rq = make_rsrc(static_cast<unsigned char*>(gq) + row0 * GQK, nb);
+            const __amdgpu_buffer_rsrc_t rk = make_rsrc(static_cast<unsigned char*>(gk) + row0 * GQK, nb);
 #pragma unroll
             for (int m = 0; m < 4; ++m) {
                 const int t = 16 * m + l16;
@@ -1065,9 +1074,14 @@ __global__ __launch_bounds__(256) void bwd_grad_kernel(
                 for (int dd = 0; dd < JW; ++dd) {
                     const int d0 = 16 * (JW * w + dd) + 4 * lg;
                     const f32x4_t kk = dKa[m][dd] - bt * dKb[m][dd] + dKc[m][dd];
-                    const unsigned off = static_cast<unsigned>((t * tstride + d0) * 4);
-                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, dQ[m][dd]), rq, off, 0, 0);
-                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, kk), rk, off, 0, 0);
+                    const unsigned off = static_cast<unsigned>((t * tstride + d0) * GQK);
+                    if constexpr (GQK == 2) {
+                        __builtin_amdgcn_raw_buffer_store_b64(cvt4(dQ[m][dd]), rq, off, 0, 0);
+                        __builtin_amdgcn_raw_buffer_store_b64(cvt4(kk), rk, off, 0, 0);
+                    } else {
+                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, dQ[m][dd]), rq, off, 0, 0);
+                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, kk), rk, off, 0, 0);
+                    }
                 }
             }
         }
@@ -1126,12 +1140,14 @@ hipError_t launch_d(const BwdArgs& a, hipStream_t st) {
     }
     const int n_tiles = D / RevGeo<D>::NC;
     const int slots = (a.n_pairs + 7) / 8;
-    if ((e = set_lds(bwd_rev_kernel<D>, RevGeo<D>::BYTES)) != hipSuccess) return e;
-    hipLaunchKernelGGL(bwd_rev_kernel<D>, dim3(static_cast<unsigned>(slots * 8 * n_tiles)), dim3(RevGeo<D>::THREADS),
+    auto rev = a.gv_bf16 ? bwd_rev_kernel<D, 2> : bwd_rev_kernel<D, 4>;
+    if ((e = set_lds(rev, RevGeo<D>::BYTES)) != hipSuccess) return e;
+    hipLaunchKernelGGL(rev, dim3(static_cast<unsigned>(slots * 8 * n_tiles)), dim3(RevGeo<D>::THREADS),
                        RevGeo<D>::BYTES, st, q, k, a.beta, a.go, a.gs, tp, g_hist, w_hist, a.gv, a.gs0,
                        a.n_pairs, a.T, a.H, n_ch, n_tiles);
     if ((e = hipGetLastError()) != hipSuccess || n_ch == 0) return e;
-    if ((e = set_lds(bwd_grad_kernel<D>, GradGeo<D>::BYTES)) != hipSuccess) return e;
+    auto grad = a.gqk_bf16 ? bwd_grad_kernel<D, 2> : bwd_grad_kernel<D, 4>;
+    if ((e = set_lds(grad, GradGeo<D>::BYTES)) != hipSuccess) return e;
     // persistent: one workgroup per CU (its LDS allows no more), each taking every
     // gridDim.x-th chunk
     int dev = 0, n_cu = 0;
@@ -1140,7 +1156,7 @@ hipError_t launch_d(const BwdArgs& a, hipStream_t st) {
     const long n_total = static_cast<long>(a.n_pairs) * n_ch;
     if (n_total > (1L << 30)) return hipErrorInvalidValue;  // chunk indices stay in int
     const long grid = n_total < n_cu ? n_total : (n_cu > 0 ? n_cu : 1);
-    hipLaunchKernelGGL(bwd_grad_kernel<D>, dim3(static_cast<unsigned>(grid)), dim3(256), GradGeo<D>::BYTES, st, q,
+    hipLaunchKernelGGL(grad, dim3(static_cast<unsigned>(grid)), dim3(256), GradGeo<D>::BYTES, st, q,
                        k, v, a.beta, a.go, s_hist, g_hist, w_hist, tp, a.gq, a.gk, a.gbeta, a.T, a.H, n_ch,
                        static_cast<int>(n_total));
     return hipGetLastError();

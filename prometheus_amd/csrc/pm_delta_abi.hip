@@ -361,12 +361,17 @@ size_t bwd_ws_bytes(int B, int T, int H, int D, int in_dtype, int gm = 0) {
     return sizeof(float) * pm::bwd_workspace_floats(n_pairs, T, D, gm);
 }
 
+// Type of gq, gk and gv: fp32, all bf16, or gv alone bf16 (bf16 needs bf16 q/k/v on a chunked
+// path; PM_E_UNSUPPORTED otherwise, nothing launched).
+enum GradType { kGradF32, kGradBf16, kGradBf16V };
+
 // Common backward dispatch; g != NULL: a gated variant (K10 or the per-token kernels, gg
 // out, the per-token kernels' workspace either way: it holds K10's), with per_channel its KDA form (g and gg (B, T, H, D)).
 int backward(const void* q, const void* k, const void* v, const float* beta, const float* g,
-             const float* s0, const float* go, const float* gs, float* gq, float* gk, float* gv,
+             const float* s0, const float* go, const float* gs, void* gq, void* gk, void* gv,
              float* gbeta, float* gg, float* gs0, int B, int T, int H, int D, int in_dtype,
-             void* workspace, size_t ws_bytes, void* stream, bool per_channel = false) {
+             void* workspace, size_t ws_bytes, void* stream, bool per_channel = false,
+             GradType gt = kGradF32) {
     if (B < 0 || T < 0 || H < 0)
         return fail(PM_E_SHAPE, "B, T, H must be >= 0 (got %d, %d, %d)", B, T, H);
     if (D < 1 || D > pm::kBwdMaxD)
@@ -382,9 +387,9 @@ int backward(const void* q, const void* k, const void* v, const float* beta, con
         return fail(PM_E_NULL, "q, k, v, beta, gq, gk, gv and gbeta must be non-NULL");
     const bool gated = g != nullptr || gg != nullptr;
     if (gated && n_tok > 0 && (!g || !gg)) return fail(PM_E_NULL, "g and gg must be non-NULL");
-    const void* f32s[] = {beta, g, s0, go, gs, gq, gk, gv, gbeta, gg, gs0, workspace};
-    for (const void* p : f32s)
-        if (p && !aligned(p, 4)) return fail(PM_E_ALIGN, "fp32 buffers must be 4-byte aligned");
+    const void* f32s[] = {beta, g, s0, go, gs, gbeta, gg, gs0, workspace, gq, gk, gv};
+    for (int i = 0; i < (gt == kGradF32 ? 12 : 9); ++i)
+        if (f32s[i] && !aligned(f32s[i], 4)) return fail(PM_E_ALIGN, "fp32 buffers must be 4-byte aligned");
     const bool chunked16 = !gated && bwd_chunked(H, D, in_dtype);
     const bool chunked32 = !gated && bwd_chunked_f32(H, D, in_dtype);
     const bool chunked = chunked16 || chunked32;
@@ -404,15 +409,22 @@ int backward(const void* q, const void* k, const void* v, const float* beta, con
     if (need > 0 && (!workspace || ws_bytes < need))
         return fail(PM_E_WORKSPACE, "workspace of %zu bytes needed (got %zu)", need,
                     workspace ? ws_bytes : static_cast<size_t>(0));
-    pm::BwdArgs a{q, k, v, beta, s0, go, gs, gq, gk, gv, gbeta, gs0,
+    pm::BwdArgs a{q, k, v, beta, s0, go, gs, static_cast<float*>(gq), static_cast<float*>(gk),
+                  static_cast<float*>(gv), gbeta, gs0,
                   static_cast<float*>(workspace), static_cast<int>(n_pairs), T, H, D,
                   in_dtype == PM_DTYPE_BF16};
     a.g = g;
     a.gg = gg;
     a.per_channel = per_channel;
-    if (gated && n_tok > 0 && bwd_decay_chunked(T, H, D) && aligned(q, 16) && aligned(k, 16) && aligned(v, 16) &&
-        (!go || aligned(go, 16)) && aligned(gv, 16) && (!per_channel || aligned(g, 16)) && aligned(workspace, 16) &&
-        pm::decay_bwd_ws_bytes(n_pairs, T, D) <= need) {
+    a.gqk_bf16 = gt == kGradBf16;
+    a.gv_bf16 = gt != kGradF32;
+    const bool decay = gated && n_tok > 0 && bwd_decay_chunked(T, H, D) && aligned(q, 16) && aligned(k, 16) &&
+                       aligned(v, 16) && (!go || aligned(go, 16)) && aligned(gv, 16) &&
+                       (!per_channel || aligned(g, 16)) && aligned(workspace, 16) &&
+                       pm::decay_bwd_ws_bytes(n_pairs, T, D) <= need;
+    if (gt != kGradF32 && n_tok > 0 && !(in_dtype == PM_DTYPE_BF16 && (chunked16 || decay)))
+        return fail(PM_E_UNSUPPORTED, "bf16 gradients need bf16 q/k/v on a chunked path (D in {64, 128})");
+    if (decay) {
         hipError_t e = pm::launch_decay_bwd(a, static_cast<hipStream_t>(stream));
         return e == hipSuccess ? 0 : hip_fail(e, "chunked decay backward launch");
     }
@@ -420,6 +432,29 @@ int backward(const void* q, const void* k, const void* v, const float* beta, con
                    : chunked32 ? pm::launch_bwd_chunked_f32(a, static_cast<hipStream_t>(stream))
                                : pm::launch_bwd(a, static_cast<hipStream_t>(stream));
     return e == hipSuccess ? 0 : hip_fail(e, "backward launch");
+}
+
+// The model's backward: the normalised q and k in their type, ones for beta, the fp32
+// gradients of the normalised rows, of beta (unused) and, where dV is not written in its type
+// directly, of v; then the ungated backward's workspace.
+struct LinBwdWs {
+    size_t qn, kn, ones, gqn, gkn, gb, gvn, inner, bytes;
+};
+LinBwdWs lin_bwd_ws(int B, int T, int H, int D, int in_dtype) {
+    const size_t rows = static_cast<size_t>(B) * T * H, el = rows * D;
+    const size_t es = in_dtype == PM_DTYPE_BF16 ? 2 : 4;
+    auto al = [](size_t x) { return (x + 255) & ~static_cast<size_t>(255); };
+    LinBwdWs w;
+    w.qn = 0;
+    w.kn = al(el * es);
+    w.ones = w.kn + al(el * es);
+    w.gqn = w.ones + al(rows * 4);
+    w.gkn = w.gqn + al(el * 4);
+    w.gb = w.gkn + al(el * 4);
+    w.gvn = w.gb + al(rows * 4);
+    w.inner = w.gvn + (es == 2 && !bwd_chunked(H, D, in_dtype) ? al(el * 4) : 0);
+    w.bytes = w.inner + bwd_ws_bytes(B, T, H, D, in_dtype) + 256;
+    return w;
 }
 
 // The forward's workspace: the split form's T blocks (bf16 inputs, where split_chosen), the
@@ -467,6 +502,15 @@ int pm_delta_bwd(const void* q, const void* k, const void* v, const float* beta,
     g_err[0] = '\0';
     return backward(q, k, v, beta, nullptr, s0, go, gs, gq, gk, gv, gbeta, nullptr, gs0, B, T, H, D,
                     in_dtype, workspace, ws_bytes, stream);
+}
+
+int pm_delta_bwd_bf16(const void* q, const void* k, const void* v, const float* beta, const float* g,
+                      const float* s0, const float* go, const float* gs, void* gq, void* gk, void* gv,
+                      float* gbeta, float* gg, float* gs0, int B, int T, int H, int D, int per_channel,
+                      void* workspace, size_t ws_bytes, void* stream) {
+    g_err[0] = '\0';
+    return backward(q, k, v, beta, g, s0, go, gs, gq, gk, gv, gbeta, gg, gs0, B, T, H, D, PM_DTYPE_BF16, workspace,
+                    ws_bytes, stream, per_channel != 0, kGradBf16);
 }
 
 size_t pm_gated_delta_bwd_workspace_bytes(int B, int T, int H, int D, int in_dtype) {
@@ -685,6 +729,51 @@ int pm_linear_attention_ws(const void* q, const void* k, const void* v, const fl
                         in_dtype == PM_DTYPE_BF16, out_dtype == PM_DTYPE_BF16, true};
     hipError_t e = pm::launch_recurrent(a, st);
     return e == hipSuccess ? 0 : hip_fail(e, "linear attention launch");
+}
+
+size_t pm_linear_attention_bwd_workspace_bytes(int B, int T, int H, int D, int in_dtype) {
+    if (B < 0 || T < 0 || H < 0 || D < 1 || D > pm::kBwdMaxD) return 0;
+    if (in_dtype != PM_DTYPE_F32 && in_dtype != PM_DTYPE_BF16) return 0;
+    return lin_bwd_ws(B, T, H, D, in_dtype).bytes;
+}
+
+int pm_linear_attention_bwd(const void* q, const void* k, const void* v, const float* s0, const float* go,
+                            const float* gs, void* gq, void* gk, void* gv, float* gs0, int B, int T, int H,
+                            int D, int in_dtype, void* workspace, size_t ws_bytes, void* stream) {
+    g_err[0] = '\0';
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (B < 0 || T < 0 || H < 0)
+        return fail(PM_E_SHAPE, "B, T, H must be >= 0 (got %d, %d, %d)", B, T, H);
+    if (D < 1 || D > pm::kBwdMaxD)
+        return fail(PM_E_SHAPE, "backward D must be in [1, %d] (got %d)", pm::kBwdMaxD, D);
+    if (int rc = check_dtypes(in_dtype, PM_DTYPE_F32)) return rc;
+    const long n_tok = static_cast<long>(B) * T, rows = n_tok * H;
+    if (static_cast<long>(B) * H == 0) return 0;
+    if (static_cast<long>(B) * H > (1L << 30) || n_tok > (1L << 40)) return fail(PM_E_SHAPE, "problem too large");
+    if (n_tok > 0 && (!q || !k || !v || !gq || !gk || !gv))
+        return fail(PM_E_NULL, "q, k, v, gq, gk and gv must be non-NULL");
+    const LinBwdWs w = lin_bwd_ws(B, T, H, D, in_dtype);
+    if (!workspace || ws_bytes < w.bytes || !aligned(workspace, 16))
+        return fail(PM_E_WORKSPACE, "a 16-byte aligned workspace of %zu bytes needed (got %zu)", w.bytes,
+                    workspace ? ws_bytes : static_cast<size_t>(0));
+    unsigned char* base = static_cast<unsigned char*>(workspace);
+    auto f = [&](size_t off) { return reinterpret_cast<float*>(base + off); };
+    const bool bf16 = in_dtype == PM_DTYPE_BF16;
+    hipError_t e = pm::launch_norm_rows(q, k, base + w.qn, base + w.kn, f(w.ones), static_cast<size_t>(rows), rows, D,
+                                        bf16, st);
+    if (e != hipSuccess) return hip_fail(e, "row normalisation launch");
+    // bf16 inputs: dV in bf16 straight from the chunked kernels, through fp32 otherwise
+    const bool direct = !bf16 || bwd_chunked(H, D, in_dtype);
+    int rc = backward(base + w.qn, base + w.kn, v, f(w.ones), nullptr, s0, go, gs, f(w.gqn), f(w.gkn),
+                      direct ? gv : static_cast<void*>(f(w.gvn)), f(w.gb), nullptr, gs0, B, T, H, D, in_dtype,
+                      base + w.inner, ws_bytes - w.inner, stream, false,
+                      bf16 && direct && n_tok > 0 ? kGradBf16V : kGradF32);
+    if (rc != 0) return rc;
+    if (!direct && (e = pm::launch_cast_bf16(f(w.gvn), static_cast<uint16_t*>(gv), static_cast<size_t>(rows) * D, st)) !=
+                       hipSuccess)
+        return hip_fail(e, "cast launch");
+    e = pm::launch_norm_rows_bwd(q, k, f(w.gqn), f(w.gkn), gq, gk, rows, D, bf16, st);
+    return e == hipSuccess ? 0 : hip_fail(e, "normalisation gradient launch");
 }
 
 int pm_delta_step(float* s_inout, const void* q, const void* k, const void* v,

@@ -186,6 +186,8 @@ struct BwdArgs {
     float* gg = nullptr;
     // with g: one log-gate per (token, head, key channel) (KDA), g and gg (B, T, H, D)
     bool per_channel = false;
+    // gq and gk, and gv, written as bf16 (K6 and K10 only)
+    bool gqk_bf16 = false, gv_bf16 = false;
 };
 constexpr int kBwdMaxD = 256;
 // gm: 0 ungated, 1 gated, 2 per-channel gated
@@ -216,6 +218,15 @@ hipError_t launch_bwd_chunked_f32(const BwdArgs& a, hipStream_t st);
 // workspace 16-byte aligned.
 size_t decay_bwd_ws_bytes(long n_pairs, int T, int D);
 hipError_t launch_decay_bwd(const BwdArgs& a, hipStream_t st);
+
+// Row normalisation of the model's linear attention (norm_rows.hip): x / max(||x||, 1e-6)
+// for every row of q and k, in their own type, and n_ones ones; and its reverse, from the
+// fp32 gradients of the normalised rows to the raw rows' in their type.
+hipError_t launch_norm_rows(const void* q, const void* k, void* qn, void* kn, float* ones, size_t n_ones, long rows,
+                            int D, bool bf16, hipStream_t st);
+hipError_t launch_norm_rows_bwd(const void* q, const void* k, const float* gqn, const float* gkn, void* gq, void* gk,
+                                long rows, int D, bool bf16, hipStream_t st);
+hipError_t launch_cast_bf16(const float* src, uint16_t* dst, size_t n, hipStream_t st);
 
 // Zero fill (used instead of hipMemsetAsync so callers may graph-capture).
 hipError_t launch_fill_zero(float* p, size_t n, hipStream_t st);

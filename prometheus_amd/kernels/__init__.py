@@ -257,7 +257,7 @@ class _ChunkedDeltaRule(torch.autograd.Function):
         qd, kd, vd, bd, sd = ctx.saved_tensors
         res = _DeltaResidual(q=qd, k=kd, v=vd, beta=bd, state0=sd, chunk=ctx.chunk)
         with _native.use_knobs(*ctx.knobs):
-            grads = chunked_delta_rule_bwd(res, (go, gs))
+            grads = _delta_bwd(res, (go, gs), _grads_bf16(ctx.like))
         out = []
         for g, like, need in zip(grads, ctx.like, ctx.needs_input_grad[:5]):
             out.append(g.to(device=like[1], dtype=like[0]) if (like is not None and need) else None)
@@ -319,6 +319,29 @@ def chunked_delta_rule_bwd(residual: _DeltaResidual, grads):
     reverse-mode kernel with state checkpoints (fp32 parity). None keeps the
     reference's per-token state history.
     """
+    return _delta_bwd(residual, grads)
+
+
+def _grads_bf16(like) -> bool:
+    """Whether autograd asks for q's, k's and v's gradients as bf16 on the GPU."""
+    return all(x is not None and x[0] == torch.bfloat16 and x[1].type == "cuda" for x in like[:3])
+
+
+def _run_bwd(run, bf16):
+    """``run(dtype)`` with bf16 gradients where asked for and served, else with fp32 ones."""
+    if bf16:
+        rc, *out = run(torch.bfloat16)
+        if rc != _native.E_UNSUPPORTED:
+            _native.check(rc)
+            return out
+    rc, *out = run(torch.float32)
+    _native.check(rc)
+    return out
+
+
+def _delta_bwd(residual, grads, bf16=False):
+    """``chunked_delta_rule_bwd``; with ``bf16`` (autograd's bf16 leaves) gq, gk and gv come back
+    as bf16 where the kernels write them so, sparing a cast pass over each."""
     go, gs = grads
     q, k, v, beta, s0 = residual.q, residual.k, residual.v, residual.beta, residual.state0
     batch, seq, heads, dim = _validate(q, k, v, beta, s0)
@@ -338,19 +361,27 @@ def chunked_delta_rule_bwd(residual: _DeltaResidual, grads):
         # the chunked backward reads q, k, v and dO with 16-byte vector loads: a view at an
         # odd offset is copied to a fresh (aligned) buffer rather than refused
         qd, kd, vd, god = (_aligned16(x) for x in (qd, kd, vd, god))
-        gq = torch.empty((batch, seq, heads, dim), dtype=f32, device=call.device)
-        gk, gv = torch.empty_like(gq), torch.empty_like(gq)
         gb = torch.empty((batch, seq, heads), dtype=f32, device=call.device)
         gs0 = torch.empty((batch, heads, dim, dim), dtype=f32, device=call.device)
         L = _native.lib()
         nbytes = L.pm_delta_bwd_workspace_bytes(batch, seq, heads, dim, _code(cdt))
         ws = torch.empty(((nbytes + 3) // 4,), dtype=f32, device=call.device) if nbytes else None
-        rc = L.pm_delta_bwd(
-            _ptr(qd), _ptr(kd), _ptr(vd), _ptr(bd), _ptr(sd), _ptr(god), _ptr(gsd),
-            _ptr(gq), _ptr(gk), _ptr(gv), _ptr(gb), _ptr(gs0),
-            batch, seq, heads, dim, _code(cdt), _ptr(ws), nbytes, _stream(call.device),
-        )
-        _native.check(rc)
+
+        def run(dt):
+            gq = torch.empty((batch, seq, heads, dim), dtype=dt, device=call.device)
+            gk, gv = torch.empty_like(gq), torch.empty_like(gq)
+            ins = (_ptr(qd), _ptr(kd), _ptr(vd), _ptr(bd))
+            outs = (_ptr(gq), _ptr(gk), _ptr(gv), _ptr(gb))
+            tail = (_ptr(ws), nbytes, _stream(call.device))
+            if dt == f32:
+                rc = L.pm_delta_bwd(*ins, _ptr(sd), _ptr(god), _ptr(gsd), *outs, _ptr(gs0),
+                                    batch, seq, heads, dim, _code(cdt), *tail)
+            else:
+                rc = L.pm_delta_bwd_bf16(*ins, None, _ptr(sd), _ptr(god), _ptr(gsd), *outs, None, _ptr(gs0),
+                                         batch, seq, heads, dim, 0, *tail)
+            return rc, gq, gk, gv
+
+        gq, gk, gv = _run_bwd(run, bf16 and cdt == torch.bfloat16)
     return tuple(call.out(x) for x in (gq, gk, gv, gb, gs0))
 
 
@@ -623,7 +654,7 @@ def chunked_kda_rule_bwd(residual: _GatedDeltaResidual, grads):
     return _gated_bwd(residual, grads, per_channel=True)
 
 
-def _gated_bwd(residual, grads, per_channel):
+def _gated_bwd(residual, grads, per_channel, bf16=False):
     go, gs = grads
     q, k, v, beta, g, s0 = residual.q, residual.k, residual.v, residual.beta, residual.g, residual.state0
     batch, seq, heads, dim = _validate(q, k, v, beta, s0)
@@ -643,8 +674,6 @@ def _gated_bwd(residual, grads, per_channel):
         qd, kd, vd = call.dev(q, cdt), call.dev(k, cdt), call.dev(v, cdt)
         bd, gd, sd = call.dev(beta, f32), call.dev(g, f32), call.dev(s0, f32)
         god, gsd = call.dev(go, f32), call.dev(gs, f32)
-        gq = torch.empty((batch, seq, heads, dim), dtype=f32, device=call.device)
-        gk, gv = torch.empty_like(gq), torch.empty_like(gq)
         gb = torch.empty((batch, seq, heads), dtype=f32, device=call.device)
         gg = torch.empty(gshape, dtype=f32, device=call.device)
         gs0 = torch.empty((batch, heads, dim, dim), dtype=f32, device=call.device)
@@ -652,12 +681,17 @@ def _gated_bwd(residual, grads, per_channel):
         wsf = L.pm_kda_delta_bwd_workspace_bytes if per_channel else L.pm_gated_delta_bwd_workspace_bytes
         nbytes = wsf(batch, seq, heads, dim, _code(cdt))
         ws = torch.empty(((nbytes + 3) // 4,), dtype=f32, device=call.device) if nbytes else None
-        rc = (L.pm_kda_delta_bwd if per_channel else L.pm_gated_delta_bwd)(
-            _ptr(qd), _ptr(kd), _ptr(vd), _ptr(bd), _ptr(gd), _ptr(sd), _ptr(god), _ptr(gsd),
-            _ptr(gq), _ptr(gk), _ptr(gv), _ptr(gb), _ptr(gg), _ptr(gs0),
-            batch, seq, heads, dim, _code(cdt), _ptr(ws), nbytes, _stream(call.device),
-        )
-        _native.check(rc)
+
+        def run(dt):
+            gq = torch.empty((batch, seq, heads, dim), dtype=dt, device=call.device)
+            gk, gv = torch.empty_like(gq), torch.empty_like(gq)
+            f = (L.pm_delta_bwd_bf16 if dt != f32 else L.pm_kda_delta_bwd if per_channel else L.pm_gated_delta_bwd)
+            rc = f(_ptr(qd), _ptr(kd), _ptr(vd), _ptr(bd), _ptr(gd), _ptr(sd), _ptr(god), _ptr(gsd),
+                   _ptr(gq), _ptr(gk), _ptr(gv), _ptr(gb), _ptr(gg), _ptr(gs0), batch, seq, heads, dim,
+                   int(per_channel) if dt != f32 else _code(cdt), _ptr(ws), nbytes, _stream(call.device))
+            return rc, gq, gk, gv
+
+        gq, gk, gv = _run_bwd(run, bf16 and cdt == torch.bfloat16)
     return tuple(call.out(x) for x in (gq, gk, gv, gb, gg, gs0))
 
 
@@ -683,7 +717,7 @@ class _ChunkedGatedDeltaRule(torch.autograd.Function):
         qd, kd, vd, bd, gd, sd = ctx.saved_tensors
         res = _GatedDeltaResidual(q=qd, k=kd, v=vd, beta=bd, g=gd, state0=sd, chunk=ctx.chunk)
         with _native.use_knobs(*ctx.knobs):
-            grads = _gated_bwd(res, (go, gs), ctx.per_channel)
+            grads = _gated_bwd(res, (go, gs), ctx.per_channel, _grads_bf16(ctx.like))
         out = []
         for gr, like, need in zip(grads, ctx.like, ctx.needs_input_grad[:6]):
             out.append(gr.to(device=like[1], dtype=like[0]) if (like is not None and need) else None)

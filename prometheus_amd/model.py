@@ -26,7 +26,7 @@ import numpy as np
 import torch
 
 from prometheus_amd import _native
-from prometheus_amd.kernels import _Call, _code, _DeltaResidual, _ptr, _stream, chunked_delta_rule_bwd
+from prometheus_amd.kernels import _aligned16, _Call, _code, _ptr, _stream
 
 __all__ = ["linear_attention", "_linear_attn"]
 
@@ -51,11 +51,6 @@ def _dtype(q, k, v) -> torch.dtype:
     return torch.float32
 
 
-def _l2n(x):
-    """``x / max(||x||, 1e-6)`` over the last axis (model/__init__.py:203-205)."""
-    return x / torch.clamp_min(torch.linalg.vector_norm(x, dim=-1, keepdim=True), 1e-6)
-
-
 def _run_linear_attention(qd, kd, vd, sd, cdt, device):
     batch, seq, heads, dim = qd.shape
     o = torch.empty(qd.shape, dtype=torch.float32, device=device)
@@ -72,10 +67,10 @@ def _run_linear_attention(qd, kd, vd, sd, cdt, device):
 
 
 class _LinearAttention(torch.autograd.Function):
-    """The fused kernel forward; the backward runs ``chunked_delta_rule_bwd`` (the
-    reverse kernels) on the normalised rows with beta = 1, then differentiates the
-    normalisation ``x / max(||x||, 1e-6)`` with torch.  bf16 q/k run the chunked
-    bf16 backward on bf16-rounded normalised rows; fp32 q/k the fp32 backward."""
+    """The fused kernel forward; the backward (``pm_linear_attention_bwd``) normalises the
+    rows, runs the reverse kernels on them with beta = 1 (bf16 q/k: the chunked bf16 backward
+    on bf16-rounded normalised rows; fp32 q/k the fp32 backward) and takes the gradients back
+    through ``x / max(||x||, 1e-6)``; q's, k's and v's come in their type."""
 
     @staticmethod
     def forward(ctx, qd, kd, vd, sd, cdt):
@@ -90,21 +85,22 @@ class _LinearAttention(torch.autograd.Function):
     @staticmethod
     def backward(ctx, go, gs):
         qd, kd, vd, sd = ctx.saved_tensors
-        with torch.enable_grad():
-            qf = qd.detach().float().requires_grad_(True)
-            kf = kd.detach().float().requires_grad_(True)
-            qn, kn = _l2n(qf), _l2n(kf)
-        ones = torch.ones(qd.shape[:3], dtype=torch.float32, device=qd.device)
-        s0 = sd if sd is not None else torch.zeros(
-            (qd.shape[0], qd.shape[2], qd.shape[3], qd.shape[3]), dtype=torch.float32, device=qd.device)
-        res = _DeltaResidual(q=qn.detach().to(ctx.cdt), k=kn.detach().to(ctx.cdt), v=vd, beta=ones,
-                             state0=s0, chunk=64)
-        with _native.use_knobs(*ctx.knobs):
-            gqn, gkn, gv, _, gs0 = chunked_delta_rule_bwd(res, (go, gs))
-        gq, gk = torch.autograd.grad((qn, kn), (qf, kf), (gqn, gkn))
+        batch, seq, heads, dim = qd.shape
+        f32 = torch.float32
+        with torch.cuda.device(qd.device), _native.use_knobs(*ctx.knobs):
+            god, gsd = (None if x is None else x.to(f32).contiguous() for x in (go, gs))
+            vd, god = _aligned16(vd), _aligned16(god)
+            gq, gk, gv = (torch.empty_like(x) for x in (qd, kd, vd))
+            gs0 = torch.empty((batch, heads, dim, dim), dtype=f32, device=qd.device)
+            lib = _native.lib()
+            nbytes = lib.pm_linear_attention_bwd_workspace_bytes(batch, seq, heads, dim, _code(ctx.cdt))
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=qd.device)
+            _native.check(lib.pm_linear_attention_bwd(
+                _ptr(qd), _ptr(kd), _ptr(vd), _ptr(sd), _ptr(god), _ptr(gsd), _ptr(gq), _ptr(gk), _ptr(gv),
+                _ptr(gs0), batch, seq, heads, dim, _code(ctx.cdt), _ptr(ws), nbytes, _stream(qd.device)))
         need = ctx.needs_input_grad
-        return (gq.to(qd.dtype) if need[0] else None, gk.to(kd.dtype) if need[1] else None,
-                gv.to(vd.dtype) if need[2] else None, gs0 if (sd is not None and need[3]) else None, None)
+        return (gq if need[0] else None, gk if need[1] else None, gv if need[2] else None,
+                gs0 if (sd is not None and need[3]) else None, None)
 
 
 def linear_attention(q, k, v, state=None):
