@@ -156,6 +156,22 @@ int pm_gated_delta_fwd(const void* q, const void* k, const void* v, const float*
                        int D, int in_dtype, int out_dtype, void* stream);
 
 /*
+ * pm_gated_delta_fwd with a workspace: fp32 q/k/v with D in {64, 128}, H * D <=
+ * 2^24, T >= 160 (and B * H < 256 at D = 64) and 16-byte aligned q, k, v run in
+ * chunks of 16 tokens on fp32 MFMA (fp32 arithmetic, fp32 parity) when workspace
+ * holds pm_decay_fwd_workspace_bytes bytes (16-byte aligned); without it, under path 1 and
+ * for other inputs as pm_gated_delta_fwd.  pm_kda_delta_fwd takes the same
+ * workspace for fp32 q/k/v (with g 16-byte aligned too).  No reference counterpart.
+ */
+int pm_gated_delta_fwd_ws(const void* q, const void* k, const void* v, const float* beta,
+                          const float* g, const float* s0, void* o, float* s_out, int B, int T,
+                          int H, int D, int in_dtype, int out_dtype, void* workspace,
+                          size_t ws_bytes, void* stream);
+/* Workspace bytes of the chunked fp32 forward of the rules with a decay (0 where they run
+ * another kernel): per (b, h) and 16-token chunk three 16 x D fp32 tiles and 512 + D floats. */
+size_t pm_decay_fwd_workspace_bytes(int B, int T, int H, int D, int in_dtype);
+
+/*
  * One gated step: S' = alpha (S - beta k (k^T S)) + beta k v^T, o = q S',
  * alpha = exp(g), g (B, H) fp32; otherwise as pm_delta_step.
  */
@@ -177,6 +193,8 @@ int pm_gated_delta_step(float* s_inout, const void* q, const void* k, const void
  *     MFMA (a parallel pass writes every chunk's decayed operands, T and P into the
  *     workspace, then the chunk recurrence).  It clamps each log-gate into [-10, 1]
  *     (alpha >= 4.5e-5: a difference below bf16 resolution).
+ *   * fp32 q/k/v and a workspace of pm_decay_fwd_workspace_bytes (where that is not 0):
+ *     the chunked form on fp32 MFMA (see pm_gated_delta_fwd_ws), g as given.
  *   * otherwise, without a large enough workspace, and under path 1: the fp32
  *     per-token kernel, every in_dtype and D <= 256, g as given.
  * Path 2 or 3 (chunked kernel required) returns PM_E_UNSUPPORTED for inputs the

@@ -34,6 +34,8 @@ EXPORTS = (
     "pm_delta_step",
     "pm_delta_step_slots",
     "pm_gated_delta_fwd",
+    "pm_gated_delta_fwd_ws",
+    "pm_decay_fwd_workspace_bytes",
     "pm_gated_delta_step",
     "pm_linear_attention",
     "pm_linear_attention_ws",
@@ -96,6 +98,10 @@ def lib() -> ctypes.CDLL:
         L.pm_delta_step.restype = i
         L.pm_gated_delta_fwd.argtypes = [vp] * 8 + [i] * 6 + [vp]
         L.pm_gated_delta_fwd.restype = i
+        L.pm_gated_delta_fwd_ws.argtypes = [vp] * 8 + [i] * 6 + [vp, sz, vp]
+        L.pm_gated_delta_fwd_ws.restype = i
+        L.pm_decay_fwd_workspace_bytes.argtypes = [i] * 5
+        L.pm_decay_fwd_workspace_bytes.restype = sz
         L.pm_gated_delta_step.argtypes = [vp] * 7 + [i] * 4 + [vp]
         L.pm_gated_delta_step.restype = i
         L.pm_kda_delta_fwd.argtypes = [vp] * 8 + [i] * 6 + [vp, sz, vp]

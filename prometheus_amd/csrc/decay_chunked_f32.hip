@@ -1,6 +1,6 @@
 // decay_chunked_f32.hip — K10: the rules with a decay (a log-gate per token and head, or
-// one per key channel) in chunked form on fp32 MFMA (v_mfma_f32_16x16x4f32), reverse mode,
-// D in {64, 128}, fixed-length batches, fp32 or bf16 q/k/v.  Every product is fp32 x fp32
+// one per key channel) in chunked form on fp32 MFMA (v_mfma_f32_16x16x4f32), D in {64, 128},
+// fixed-length batches: the reverse mode for fp32 or bf16 q/k/v, the forward for fp32.  Every product is fp32 x fp32
 // with fp32 accumulation, as in the per-token kernels (delta_bwd.hip).
 //
 // Per token, alpha_t = exp(g_t) (a d_k-vector; constant over d_k for the per-head gate):
@@ -82,6 +82,8 @@ template <int D>
 struct DecRec {
     static constexpr int T2 = 0, TA = 256, PA = 512, AT = 768, GB = 1024, GBN = D + 64;
     static constexpr int FLOATS = GB + GBN;
+    // the forward's: T''^T, P^T, gC
+    static constexpr int FPT = 256, FGB = 512, FFLOATS = FGB + D;
 };
 
 // Lane (g, r)'s operand reads of a swizzled tile of 16 fp32 rows (f32_chunk): row(b, i) =
@@ -156,7 +158,8 @@ __device__ __forceinline__ void wave_lds_fence() { __asm__ volatile("" ::: "memo
 // operand of products contracting over d.  MFMA-bound: 4 levels x 2 products of 16 x 16 x D
 // (256 MFMAs at D = 128; a per-head gate needs the two Gram products only once, since its
 // D_ts does not depend on d).
-template <int D, typename InT, bool CHAN>
+// FWD: what the forward needs alone: Q^ as rows, T''^T, P^T and gC.
+template <int D, typename InT, bool CHAN, bool FWD>
 __global__ __launch_bounds__(256) void dec_prep_kernel(
     const InT* __restrict__ q, const InT* __restrict__ k, const float* __restrict__ beta,
     const float* __restrict__ gate, int T, int H, int n_ch, long n_items, float* __restrict__ kh_ws,
@@ -184,7 +187,8 @@ __global__ __launch_bounds__(256) void dec_prep_kernel(
     float* const kh = kh_ws + static_cast<size_t>(item) * kC16 * D;
     float* const kb = kb_ws + static_cast<size_t>(item) * kC16 * D;
     float* const qh = qh_ws + static_cast<size_t>(item) * kC16 * D;
-    float* const rec = rec_ws + static_cast<size_t>(item) * R::FLOATS;
+    constexpr int kGB = FWD ? R::FGB : R::GB;
+    float* const rec = rec_ws + static_cast<size_t>(item) * (FWD ? R::FFLOATS : R::FLOATS);
 
     const __amdgpu_buffer_rsrc_t rb = make_rsrc(beta + tok0 * H + h, n_hd * 4);
     const float bc = buf_el<float>(rb, static_cast<unsigned>(r * H));
@@ -296,30 +300,41 @@ __global__ __launch_bounds__(256) void dec_prep_kernel(
             const int o = 4 * f32_chunk<D>(r, 4 * (hf * NJ + j) + g);
             *reinterpret_cast<f32x4_t*>(kh + o) = x;
             *reinterpret_cast<f32x4_t*>(kb + o) = y;
-            st4(tile + 4 * o, z);
-            if (r == 0) *reinterpret_cast<f32x4_t*>(rec + R::GB + 16 * (hf * NJ + j) + 4 * g) = gc;
+            if constexpr (FWD) *reinterpret_cast<f32x4_t*>(qh + o) = z;
+            else st4(tile + 4 * o, z);
+            if (r == 0) *reinterpret_cast<f32x4_t*>(rec + kGB + 16 * (hf * NJ + j) + 4 * g) = gc;
         }
     }
     qk += __shfl_xor(qk, 16);
     qk += __shfl_xor(qk, 32);
 #pragma unroll
     for (int v = 0; v < 4; ++v) P[v] = (4 * g + v == r) ? qk : P[v];
-    if (g == 0) rec[R::GB + D + r] = bc;
-    // A'^T through LDS
+    if (!FWD && g == 0) rec[R::GB + D + r] = bc;
+    // A'^T (FWD: and P^T) through LDS
 #pragma unroll
     for (int v = 0; v < 4; ++v) tr[(4 * g + v) * 17 + r] = A[v];
     wave_lds_fence();
     f32x4_t At;  // A'[r][4 g + v]
 #pragma unroll
     for (int v = 0; v < 4; ++v) At[v] = tr[r * 17 + 4 * g + v];
-    const TileIdx<D> ix(r, g);
+    f32x4_t Pt = kZero4;  // P[r][4 g + v]
+    if constexpr (FWD) {
+        wave_lds_fence();
+#pragma unroll
+        for (int v = 0; v < 4; ++v) tr[(4 * g + v) * 17 + r] = P[v];
+        wave_lds_fence();
+#pragma unroll
+        for (int v = 0; v < 4; ++v) Pt[v] = tr[r * 17 + 4 * g + v];
+    } else {
     // Q^ as the A operand of Q^^T dO: [m][lane][e] = Q^[4 g + e][16 m + r]
+    const TileIdx<D> ix(r, g);
 #pragma unroll
     for (int m = 0; m < D / 16; ++m) {
         f32x4_t x;
 #pragma unroll
         for (int e = 0; e < 4; ++e) x[e] = ix.col(tile, e, m);
         *reinterpret_cast<f32x4_t*>(qh + 4 * (64 * m + lane)) = x;
+    }
     }
 
     // T = (I + diag(beta) A')^-1 = (I+N)(I+N^2)(I+N^4)(I+N^8), N = -diag(beta) A' (N^16 = 0)
@@ -341,9 +356,208 @@ __global__ __launch_bounds__(256) void dec_prep_kernel(
 #pragma unroll
     for (int v = 0; v < 4; ++v) tw[v] = -bt[v] * Tt[v];
     *reinterpret_cast<f32x4_t*>(rec + R::T2 + 4 * lane) = tw;
-    *reinterpret_cast<f32x4_t*>(rec + R::TA + 4 * lane) = Ta;
-    *reinterpret_cast<f32x4_t*>(rec + R::PA + 4 * lane) = P;
-    *reinterpret_cast<f32x4_t*>(rec + R::AT + 4 * lane) = At;
+    if constexpr (FWD) {
+        *reinterpret_cast<f32x4_t*>(rec + R::FPT + 4 * lane) = Pt;
+    } else {
+        *reinterpret_cast<f32x4_t*>(rec + R::TA + 4 * lane) = Ta;
+        *reinterpret_cast<f32x4_t*>(rec + R::PA + 4 * lane) = P;
+        *reinterpret_cast<f32x4_t*>(rec + R::AT + 4 * lane) = At;
+    }
+}
+
+// ---------------------------------------------------------------- K10f
+// The forward (fp32 q/k/v): one workgroup per (b, h, DV columns of d_v), DV/16 chain waves as
+// K10s's state chain and as many output waves one chunk behind (Y = Q^ S, O = Y + P U, stores),
+// which the chain hands S and U through LDS.  The last output wave copies every chunk two
+// ahead through four buffers; one barrier per chunk.
+template <int D, int DV>
+struct DfGeo {
+    static constexpr int NCW = DV / 16, NT = D / 16, NI = kC16 * D * 4 / 1024, TILE = kC16 * D * 4, NB = 4;
+    static constexpr int B_KH = 0, B_KB = TILE, B_QH = 2 * TILE, B_T = 3 * TILE, B_P = B_T + 1024, B_V = B_P + 1024;
+    static constexpr int B_G = B_V + NCW * 1024, BUF = B_G + D * 4;
+    static constexpr int OFF_S = NB * BUF;                    // 2 slots x NCW: S of a chunk's start
+    static constexpr int OFF_U = OFF_S + 2 * NCW * NT * 1024; // 2 slots x NCW: U
+    static constexpr int BYTES = OFF_U + 2 * NCW * 1024;
+    static constexpr int NCP = 3 * NI + 2 + NCW + D / 64;     // copies per chunk
+    static constexpr int NST = 4;                             // O stores per output wave per chunk
+    static_assert(BYTES <= 160 * 1024 && NCP + NST <= 63, "LDS / vmcnt");
+};
+
+template <int D, int DV, bool OUT_BF16>
+__global__ __launch_bounds__(DV == 32 ? 256 : 128) void dec_fwd_kernel(
+    const float* __restrict__ v, const float* __restrict__ s0, void* __restrict__ o_out, float* __restrict__ s_out,
+    const float* __restrict__ kh, const float* __restrict__ kb, const float* __restrict__ qh,
+    const float* __restrict__ rec, int n_pairs, int T, int H, int n_ch) {
+    using G = DfGeo<D, DV>;
+    using R = DecRec<D>;
+    constexpr int NCW = G::NCW, NT = G::NT, n_tiles = D / DV;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    // XCD-aware placement: the n_tiles workgroups of a pair share bid % 8
+    const int bid = blockIdx.x, xcd = bid & 7, bslot = bid >> 3;
+    const int tile = bslot % n_tiles, pair = (bslot / n_tiles) * 8 + xcd;
+    if (pair >= n_pairs || n_ch <= 0) return;
+    const int seq = pair / H, h = pair % H;
+    const size_t tok0 = static_cast<size_t>(seq) * T;
+    const int col0 = tile * DV;
+    const int w = static_cast<int>(uniform(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int r = lane & 15, g = lane >> 4;
+    const size_t tstride = static_cast<size_t>(H) * D;
+    const size_t sbase = static_cast<size_t>(pair) * D * D;
+    const size_t item0 = static_cast<size_t>(pair) * n_ch;
+    const TileIdx<D> ix(r, g);
+    auto buf = [=](int c) { return smem + (c % G::NB) * G::BUF; };
+    auto sslot = [=](int c, int which) { return smem + G::OFF_S + ((c & 1) * NCW + which) * NT * 1024; };
+    auto uslot = [=](int c, int which) { return smem + G::OFF_U + ((c & 1) * NCW + which) * 1024; };
+    auto row0_of = [=](int c, int col) { return (tok0 + c * kC16) * tstride + static_cast<size_t>(h) * D + col; };
+    auto els_of = [=](int c, int cols) {
+        return static_cast<unsigned>((min(kC16, T - c * kC16) - 1) * tstride + cols);
+    };
+
+    if (w < NCW) {
+        // ============ chain: S columns col0 + 16 w + [0, 16) ============
+        const int ecol = col0 + 16 * w + r;
+        f32x4_t S[NT];
+#pragma unroll
+        for (int m = 0; m < NT; ++m)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                S[m][e] = s0 ? s0[sbase + static_cast<size_t>(16 * m + 4 * g + e) * D + ecol] : 0.f;
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), seen by the compiler
+        __builtin_amdgcn_s_setprio(3);
+        lds_barrier();  // B0
+        f32x4_t Up = kZero4;
+        float kt[4][NT] = {};  // K-^T operand of the last chunk: K-[4 g + e][16 m + r]
+        auto rd_kt = [&](const unsigned char* b, int e, int m) __attribute__((always_inline)) {
+            kt[e][m] = ix.col(b + G::B_KB, e, m);
+            kt[e][m + NT / 2] = ix.col(b + G::B_KB, e, m + NT / 2);
+        };
+        for (int i = 0; i < n_ch; ++i) {
+            const unsigned char* b = buf(i);
+            const float* Vf = reinterpret_cast<const float*>(b + G::B_V + 1024 * w);
+            f32x4_t kf[NT], gc[NT], vr, tt;
+            // S += K-^T U of the last chunk; every LDS access behind one product (see K10s)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int m = 0; m < NT; ++m) {
+                    S[m] = mfma4(kt[e][m], Up[e], S[m]);
+                    if (e == 0) kf[m] = ix.row(b + G::B_KH, m);
+                    if (e > 0 && m < NT / 2) rd_kt(b, e - 1, m);
+                    if (e == 1 && m >= NT / 2 && m < NT / 2 + 2) {
+                        vr[2 * (m - NT / 2)] = Vf[(4 * g + 2 * (m - NT / 2)) * 16 + r];
+                        vr[2 * (m - NT / 2) + 1] = Vf[(4 * g + 2 * (m - NT / 2) + 1) * 16 + r];
+                    }
+                    if (e == 2 && m == NT - 1) tt = ld4(b + G::B_T + 16 * lane);
+                    fence();
+                }
+            unsigned char* ss = sslot(i, w) + 16 * lane;
+            // X = K^ S - V, U = T'' X; S handed to the output wave
+            f32x4_t xa[4] = {-vr, kZero4, kZero4, kZero4};
+#pragma unroll
+            for (int m = 0; m < NT; ++m)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    xa[e] = mfma4(kf[m][e], S[m][e], xa[e]);
+                    const int n = 4 * m + e;
+                    if (e == 0) st4(ss + 1024 * m, S[m]);
+                    if (n < NT / 2) rd_kt(b, 3, n);
+                    if (n >= NT / 2 && n < NT / 2 + NT) gc[n - NT / 2] = ld4(b + G::B_G + 4 * (16 * (n - NT / 2) + 4 * g));
+                    fence();
+                }
+            const f32x4_t X = (xa[0] + xa[1]) + (xa[2] + xa[3]);
+            Up = mm16(tt, X);
+            st4(uslot(i, w) + 16 * lane, Up);
+#pragma unroll
+            for (int m = 0; m < NT; ++m) S[m] = gc[m] * S[m];
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), seen by the compiler
+            lds_barrier();
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int m = 0; m < NT; ++m) S[m] = mfma4(kt[e][m], Up[e], S[m]);
+#pragma unroll
+        for (int m = 0; m < NT; ++m)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s_out[sbase + static_cast<size_t>(16 * m + 4 * g + e) * D + ecol] = S[m][e];
+    } else {
+        // ============ output waves: O of chunk i - 1, the chain's columns; the last copies ============
+        const int cw = w - NCW;
+        const bool copy_wave = w == 2 * NCW - 1;
+        constexpr int ES = OUT_BF16 ? 2 : 4;
+        auto copies = [=](int c) __attribute__((always_inline)) {
+            unsigned char* b = buf(c);
+            const float* rc = rec + (item0 + c) * R::FFLOATS;
+            const float* src[3] = {kh, kb, qh};
+#pragma unroll
+            for (int x = 0; x < 3; ++x) {
+                const __amdgpu_buffer_rsrc_t rs = make_rsrc(src[x] + (item0 + c) * kC16 * D, G::TILE);
+                unsigned char* d0 = uniform_ptr(b + x * G::TILE);
+#pragma unroll
+                for (int i = 0; i < G::NI; ++i) dma16_asm(rs, d0 + 1024 * i, static_cast<unsigned>(1024 * i + 16 * lane));
+            }
+            dma16_asm(make_rsrc(rc + R::T2, 1024), uniform_ptr(b + G::B_T), static_cast<unsigned>(16 * lane));
+            dma16_asm(make_rsrc(rc + R::FPT, 1024), uniform_ptr(b + G::B_P), static_cast<unsigned>(16 * lane));
+#pragma unroll
+            for (int j = 0; j < NCW; ++j)
+                dma16_asm(make_rsrc(v + row0_of(c, col0 + 16 * j), els_of(c, 16) * 4), uniform_ptr(b + G::B_V + 1024 * j),
+                          static_cast<unsigned>((lane >> 2) * tstride * 4 + 16 * (lane & 3)));
+            const __amdgpu_buffer_rsrc_t rg = make_rsrc(rc + R::FGB, D * 4);
+#pragma unroll
+            for (int j = 0; j < D / 64; ++j)
+                dma4_asm(rg, uniform_ptr(b + G::B_G + 256 * j), static_cast<unsigned>(256 * j + 4 * lane));
+        };
+        if (copy_wave) {
+            copies(0);
+            if (n_ch > 1) {
+                copies(1);
+                wait_vm_n<G::NCP>();
+            } else {
+                wait_vm_n<0>();
+            }
+        }
+        lds_barrier();  // B0
+        for (int i = 0; i <= n_ch; ++i) {
+            const bool cp = copy_wave && i + 2 < n_ch, st = i >= 1;
+            if (cp) copies(i + 2);
+            if (st) {
+                const int c = i - 1;
+                const unsigned char* b = buf(c);
+                const unsigned char* ss = sslot(c, cw) + 16 * lane;
+                f32x4_t ya[4] = {kZero4, kZero4, kZero4, kZero4}, qy[NT], sc[NT];
+                auto rd = [&](int m) __attribute__((always_inline)) {
+                    qy[m] = ix.row(b + G::B_QH, m);
+                    sc[m] = ld4(ss + 1024 * m);
+                };
+                rd(0);
+                rd(1);
+                fence();
+#pragma unroll
+                for (int m = 0; m < NT; ++m) {
+                    if (m + 2 < NT) rd(m + 2);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) ya[e] = mfma4(qy[m][e], sc[m][e], ya[e]);
+                    fence();
+                }
+                const f32x4_t pt = ld4(b + G::B_P + 16 * lane), u = ld4(uslot(c, cw) + 16 * lane);
+                const f32x4_t O = mm16(pt, u, (ya[0] + ya[1]) + (ya[2] + ya[3]));
+                // lane (g, r) holds O[4 g + e][16 cw + r]; rows past the end are dropped
+                const __amdgpu_buffer_rsrc_t ro = make_rsrc(
+                    static_cast<unsigned char*>(o_out) + row0_of(c, col0 + 16 * cw) * ES, els_of(c, 16) * ES);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) put<ES>(O[e], ro, static_cast<unsigned>((4 * g + e) * tstride + r));
+            }
+            if (i < n_ch) {
+                // chunk i + 1 has landed; the newest copies and this iteration's stores may be in flight
+                if (copy_wave && i + 1 < n_ch) {
+                    if (cp && st) wait_vm_n<G::NCP + G::NST>();
+                    else if (cp) wait_vm_n<G::NCP>();
+                    else wait_vm_n<0>();
+                }
+                lds_barrier();
+            }
+        }
+    }
 }
 
 // ---------------------------------------------------------------- K10s
@@ -1274,6 +1488,46 @@ DecBwdWs dec_bwd_ws(long n_pairs, int T, int D) {
     return w;
 }
 
+// forward workspace: K^, K-, Q^ tiles and the records
+struct DecFwdWs {
+    size_t kh, kb, qh, rec, bytes;
+};
+DecFwdWs dec_fwd_ws(long n_pairs, int T, int D) {
+    const size_t n = static_cast<size_t>(n_pairs) * ((T + kC16 - 1) / kC16), tile = n * kC16 * D * 4;
+    DecFwdWs w;
+    w.kh = 0;
+    w.kb = w.kh + tile;
+    w.qh = w.kb + tile;
+    w.rec = w.qh + tile;
+    w.bytes = w.rec + n * (D == 128 ? DecRec<128>::FFLOATS : DecRec<64>::FFLOATS) * 4;
+    return w;
+}
+
+template <int D, int DV, bool OB>
+hipError_t launch_fwd_t(const DecayFwdArgs& a, hipStream_t st) {
+    const int n_ch = (a.T + kC16 - 1) / kC16, n_pairs = a.B * a.H;
+    const DecFwdWs o = dec_fwd_ws(n_pairs, a.T, D);
+    unsigned char* base = static_cast<unsigned char*>(a.workspace);
+    auto at = [&](size_t off) { return reinterpret_cast<float*>(base + off); };
+    const long n_items = static_cast<long>(n_pairs) * n_ch;
+    const dim3 pg(static_cast<unsigned>((n_items + 3) / 4));
+    if (a.per_channel)
+        hipLaunchKernelGGL((dec_prep_kernel<D, float, true, true>), pg, dim3(256), 0, st, a.q, a.k, a.beta, a.g, a.T, a.H,
+                           n_ch, n_items, at(o.kh), at(o.kb), at(o.qh), at(o.rec));
+    else
+        hipLaunchKernelGGL((dec_prep_kernel<D, float, false, true>), pg, dim3(256), 0, st, a.q, a.k, a.beta, a.g, a.T, a.H,
+                           n_ch, n_items, at(o.kh), at(o.kb), at(o.qh), at(o.rec));
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    using G = DfGeo<D, DV>;
+    if ((e = set_lds<dec_fwd_kernel<D, DV, OB>>(G::BYTES)) != hipSuccess) return e;
+    const int slots = (n_pairs + 7) / 8;
+    hipLaunchKernelGGL((dec_fwd_kernel<D, DV, OB>), dim3(static_cast<unsigned>(slots * (D / DV) * 8)), dim3(128 * G::NCW),
+                       G::BYTES, st, a.v, a.s0, a.o, a.s_out, at(o.kh), at(o.kb), at(o.qh), at(o.rec), n_pairs, a.T, a.H,
+                       n_ch);
+    return hipGetLastError();
+}
+
 template <int D, typename InT, bool CHAN, int GE>
 hipError_t launch_t(const BwdArgs& a, hipStream_t st) {
     const int n_ch = (a.T + kC16 - 1) / kC16, sl = span_len_for(a.n_pairs, a.T), n_span = (n_ch + sl - 1) / sl;
@@ -1285,7 +1539,7 @@ hipError_t launch_t(const BwdArgs& a, hipStream_t st) {
     if (e != hipSuccess) return e;
     if ((e = set_lds<dec_span_kernel<D, InT, CHAN, GE>>(DcGeo<D>::BYTES)) != hipSuccess) return e;
     const long n_items = static_cast<long>(a.n_pairs) * n_ch;
-    hipLaunchKernelGGL((dec_prep_kernel<D, InT, CHAN>), dim3(static_cast<unsigned>((n_items + 3) / 4)), dim3(256), 0, st,
+    hipLaunchKernelGGL((dec_prep_kernel<D, InT, CHAN, false>), dim3(static_cast<unsigned>((n_items + 3) / 4)), dim3(256), 0, st,
                        q, k, a.beta, a.g, a.T, a.H, n_ch, n_items, at(o.kh), at(o.kb), at(o.qh), at(o.rec));
     if ((e = hipGetLastError()) != hipSuccess) return e;
     const int slots = (a.n_pairs + 7) / 8;
@@ -1302,6 +1556,24 @@ hipError_t launch_t(const BwdArgs& a, hipStream_t st) {
 }  // namespace
 
 size_t decay_bwd_ws_bytes(long n_pairs, int T, int D) { return dec_bwd_ws(n_pairs, T, D).bytes; }
+size_t decay_fwd_ws_bytes(long n_pairs, int T, int D) { return dec_fwd_ws(n_pairs, T, D).bytes; }
+
+hipError_t launch_decay_fwd(const DecayFwdArgs& a, hipStream_t st) {
+    const long n_pairs = static_cast<long>(a.B) * a.H;
+    if (n_pairs == 0 || a.T == 0) return hipSuccess;
+    if (!f32_bwd_supported(a.D, a.H)) return hipErrorInvalidValue;
+    const int dv = chunked_f32_pick_tile(a.D, n_pairs, a.dv_tile);
+    auto go = [&](auto DD, auto VV) {
+        constexpr int D = decltype(DD)::value, DV = decltype(VV)::value;
+        return a.out_bf16 ? launch_fwd_t<D, DV, true>(a, st) : launch_fwd_t<D, DV, false>(a, st);
+    };
+    using I = std::integral_constant<int, 128>;
+    using J = std::integral_constant<int, 64>;
+    using W = std::integral_constant<int, 32>;
+    using N = std::integral_constant<int, 16>;
+    if (a.D == 128) return dv == 16 ? go(I{}, N{}) : go(I{}, W{});
+    return dv == 16 ? go(J{}, N{}) : go(J{}, W{});
+}
 
 hipError_t launch_decay_bwd(const BwdArgs& a, hipStream_t st) {
     if (a.n_pairs == 0 || a.T == 0) return hipSuccess;

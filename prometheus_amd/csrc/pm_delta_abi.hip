@@ -199,6 +199,21 @@ int check_dtypes(int in_dtype, int out_dtype) {
     return 0;
 }
 
+// Workspace of the chunked fp32 forward of the rules with a decay (K10f: fp32 q/k/v, D in {64,
+// 128}, the default path), 0 where it does not serve the call.  It walks 16 tokens a step
+// where the per-token kernel walks one, behind a parallel pass over all chunks: level to about
+// 130 tokens (both at the cost of their launches: 26 against 22 us), then ahead (T = 1000:
+// 97 against 184 us at 2 pairs, 124 against 224 at 64, 504 against 727 at 256, D = 128; at D =
+// 64 62 against 168, 75 against 170, but 200 against 208 at 256 pairs, where the per-token
+// kernel fills the chip and the extra pass over memory eats the gain).
+constexpr int kDecayFwdMinT = 160;
+size_t decay_fwd_need(int B, int T, int H, int D) {
+    if (B < 0 || H < 0 || g_path != 0 || T < kDecayFwdMinT || !pm::f32_bwd_supported(D, H)) return 0;
+    const long n_pairs = static_cast<long>(B) * H;
+    if (n_pairs > (1L << 30) || (D == 64 && n_pairs >= 256)) return 0;
+    return pm::decay_fwd_ws_bytes(n_pairs, T, D);
+}
+
 // Common forward dispatch. cu == nullptr: fixed length (n_seq = B, T).
 int forward(const void* q, const void* k, const void* v, const float* beta, const float* s0,
             void* o, float* s_out, const int32_t* cu, int n_seq, int T, int total_T, int H,
@@ -228,10 +243,7 @@ int forward(const void* q, const void* k, const void* v, const float* beta, cons
     const int path = g_path;
     const bool in_bf16 = in_dtype == PM_DTYPE_BF16;
     const bool want_chunked = path != 1;
-    // per-channel gates (gk): the per-token kernel only
-    if (gk && path >= 2)
-        return fail(PM_E_UNSUPPORTED, "the per-channel gated forward runs on the per-token kernel only "
-                    "(path %d asks for the chunked one)", path);
+    // (per-channel gates gk never come here under path 2 or 3: pm_kda_delta_fwd answers those)
     const bool can_chunked = !gk && in_bf16 && pm::chunked_supported(D, H) && aligned(q, 16) &&
                              aligned(k, 16) && aligned(v, 16) &&
                              (out_dtype == PM_DTYPE_F32 ? aligned(o, 16) : aligned(o, 8));
@@ -285,6 +297,19 @@ int forward(const void* q, const void* k, const void* v, const float* beta, cons
         }
         hipError_t e = pm::launch_chunked(a, st);
         return e == hipSuccess ? 0 : hip_fail(e, "chunked forward launch");
+    }
+    // fp32 q/k/v with a decay: the chunked forward with the caller's workspace
+    const float* gate = gk ? gk : g;
+    if (gate && !varlen && !in_bf16) {
+        const size_t need = decay_fwd_need(n_seq, T, H, D);
+        if (need && workspace && ws_bytes >= need && aligned(workspace, 16) && aligned(q, 16) && aligned(k, 16) &&
+            aligned(v, 16) && aligned(o, out_dtype == PM_DTYPE_F32 ? 4 : 2) && (!gk || aligned(gk, 16))) {
+            pm::DecayFwdArgs a{static_cast<const float*>(q), static_cast<const float*>(k), static_cast<const float*>(v),
+                               beta, gate, s0, o, s_out, n_seq, T, H, D, gk != nullptr,
+                               out_dtype == PM_DTYPE_BF16, g_tile, workspace};
+            hipError_t e = pm::launch_decay_fwd(a, st);
+            return e == hipSuccess ? 0 : hip_fail(e, "chunked decay forward launch");
+        }
     }
     (void)chunk;
     pm::RecurrentArgs a{q, k, v, beta, s0, o, s_out, cu, static_cast<int>(n_pairs),
@@ -793,6 +818,16 @@ int pm_gated_delta_step(float* s_inout, const void* q, const void* k, const void
 int pm_gated_delta_fwd(const void* q, const void* k, const void* v, const float* beta,
                        const float* g, const float* s0, void* o, float* s_out, int B, int T, int H,
                        int D, int in_dtype, int out_dtype, void* stream) {
+    return pm_gated_delta_fwd_ws(q, k, v, beta, g, s0, o, s_out, B, T, H, D, in_dtype, out_dtype, nullptr, 0, stream);
+}
+
+size_t pm_decay_fwd_workspace_bytes(int B, int T, int H, int D, int in_dtype) {
+    return in_dtype == PM_DTYPE_F32 && T >= 0 ? decay_fwd_need(B, T, H, D) : 0;
+}
+
+int pm_gated_delta_fwd_ws(const void* q, const void* k, const void* v, const float* beta,
+                          const float* g, const float* s0, void* o, float* s_out, int B, int T, int H,
+                          int D, int in_dtype, int out_dtype, void* workspace, size_t ws_bytes, void* stream) {
     g_err[0] = '\0';
     if (B < 0 || T < 0 || H < 0)
         return fail(PM_E_SHAPE, "B, T, H must be >= 0 (got %d, %d, %d)", B, T, H);
@@ -802,7 +837,7 @@ int pm_gated_delta_fwd(const void* q, const void* k, const void* v, const float*
     if (static_cast<long>(B) * T * H > 0 && !g) return fail(PM_E_NULL, "g is NULL");
     if (g && !aligned(g, 4)) return fail(PM_E_ALIGN, "g must be 4-byte aligned");
     return forward(q, k, v, beta, s0, o, s_out, nullptr, B, T, 0, H, D, in_dtype, out_dtype, 64,
-                   static_cast<hipStream_t>(stream), g);
+                   static_cast<hipStream_t>(stream), g, workspace, ws_bytes);
 }
 
 size_t pm_kda_delta_workspace_bytes(int B, int T, int H, int D, int in_dtype) {
@@ -850,13 +885,10 @@ int pm_kda_delta_fwd(const void* q, const void* k, const void* v, const float* b
                     "the KDA chunked forward needs bf16 q/k/v, D in {64, 128} and 16-byte aligned q/k/v/o "
                     "(got in_dtype %d, D %d)", in_dtype, D);
     }
-    // per-token kernel: forward() with the per-channel gates, as path 1
-    const int old = g_path;
-    g_path = 1;
-    const int rc = forward(q, k, v, beta, s0, o, s_out, nullptr, B, T, 0, H, D, in_dtype, out_dtype, 64, st,
-                           nullptr, nullptr, 0, g);
-    g_path = old;
-    return rc;
+    // fp32 q/k/v: the chunked fp32 forward with its workspace, else the per-token kernel (bf16
+    // q/k/v without a workspace among them)
+    return forward(q, k, v, beta, s0, o, s_out, nullptr, B, T, 0, H, D, in_dtype, out_dtype, 64, st,
+                   nullptr, workspace, ws_bytes, g);
 }
 
 int pm_kda_delta_step(float* s_inout, const void* q, const void* k, const void* v,

@@ -217,6 +217,24 @@ hipError_t launch_bwd_chunked_f32(const BwdArgs& a, hipStream_t st);
 // a.workspace holds decay_bwd_ws_bytes bytes; q, k, v, go, gv, g (per channel) and
 // workspace 16-byte aligned.
 size_t decay_bwd_ws_bytes(long n_pairs, int T, int D);
+// ... and the forward for fp32 q/k/v; workspace decay_fwd_ws_bytes bytes; q, k, v, g (per
+// channel), o and workspace 16-byte aligned.
+struct DecayFwdArgs {
+    const float* q;
+    const float* k;
+    const float* v;
+    const float* beta;
+    const float* g;
+    const float* s0;  // nullable
+    void* o;
+    float* s_out;
+    int B, T, H, D;
+    bool per_channel, out_bf16;
+    int dv_tile;  // 0 = automatic
+    void* workspace;
+};
+size_t decay_fwd_ws_bytes(long n_pairs, int T, int D);
+hipError_t launch_decay_fwd(const DecayFwdArgs& a, hipStream_t st);
 hipError_t launch_decay_bwd(const BwdArgs& a, hipStream_t st);
 
 // Row normalisation of the model's linear attention (norm_rows.hip): x / max(||x||, 1e-6)

@@ -617,18 +617,13 @@ def _gated_forward(q, k, v, beta, g, state, out_dtype, per_channel=False):
         o = torch.empty((batch, seq, heads, dim), dtype=odt, device=call.device)
         s_out = torch.empty((batch, heads, dim, dim), dtype=torch.float32, device=call.device)
         L = _native.lib()
-        if per_channel:
-            nbytes = L.pm_kda_delta_workspace_bytes(batch, seq, heads, dim, _code(cdt))
-            ws = torch.empty((nbytes,), dtype=torch.uint8, device=call.device) if nbytes else None
-            rc = L.pm_kda_delta_fwd(
-                _ptr(qd), _ptr(kd), _ptr(vd), _ptr(bd), _ptr(gd), _ptr(sd), _ptr(o), _ptr(s_out),
-                batch, seq, heads, dim, _code(cdt), _code(odt), _ptr(ws), nbytes, _stream(call.device),
-            )
-        else:
-            rc = L.pm_gated_delta_fwd(
-                _ptr(qd), _ptr(kd), _ptr(vd), _ptr(bd), _ptr(gd), _ptr(sd), _ptr(o), _ptr(s_out),
-                batch, seq, heads, dim, _code(cdt), _code(odt), _stream(call.device),
-            )
+        dims = (batch, seq, heads, dim, _code(cdt))
+        nbytes = L.pm_decay_fwd_workspace_bytes(*dims) or (L.pm_kda_delta_workspace_bytes(*dims) if per_channel else 0)
+        ws = torch.empty((nbytes,), dtype=torch.uint8, device=call.device) if nbytes else None
+        rc = (L.pm_kda_delta_fwd if per_channel else L.pm_gated_delta_fwd_ws)(
+            _ptr(qd), _ptr(kd), _ptr(vd), _ptr(bd), _ptr(gd), _ptr(sd), _ptr(o), _ptr(s_out),
+            *dims, _code(odt), _ptr(ws), nbytes, _stream(call.device),
+        )
         _native.check(rc)
         if sd is None:
             sd = torch.zeros((batch, heads, dim, dim), dtype=torch.float32, device=call.device)
@@ -731,8 +726,8 @@ def chunked_gated_delta_rule(q, k, v, beta, g, state=None, config=None, *, out_d
     ``o_t = q_t S_t``. q, k, v, beta, state and the return value as
     ``chunked_delta_rule``; g: (batch, seq, heads) fp32 log-gates (g = 0 gives
     ``chunked_delta_rule``). bf16 q/k/v with dim 64 or 128 run the chunked
-    MFMA kernel with the in-chunk decays folded into its tiles; other inputs
-    run the fp32 per-token kernel. Differentiable: when autograd records and a
+    MFMA kernel with the in-chunk decays folded into its tiles, fp32 q/k/v the chunked
+    form on fp32 MFMA; other inputs run the fp32 per-token kernel. Differentiable: when autograd records and a
     torch input (the gates included) requires grad, the backward runs
     ``chunked_gated_delta_rule_bwd``.
     """
@@ -772,8 +767,9 @@ def chunked_kda_rule(q, k, v, beta, g, state=None, config=None, *, out_dtype=Non
     ``chunked_delta_rule``; g: (batch, seq, heads, dim) fp32 log-gates, one per
     key channel (g constant along dim gives ``chunked_gated_delta_rule``). bf16 q/k/v
     with dim 64 or 128 run the chunked WY form on bf16 MFMA (``pm_kda_delta_fwd`` with
-    a workspace; log-gates clamped into [-10, 1] there); other inputs run the fp32
-    per-token kernel for every dim up to 256.
+    a workspace; log-gates clamped into [-10, 1] there), fp32 q/k/v the chunked form on
+    fp32 MFMA (g as given); other inputs run the fp32 per-token kernel for every dim up
+    to 256.
     Differentiable: when autograd records and a torch input (the gates included)
     requires grad, the backward runs ``chunked_kda_rule_bwd``.
     """

@@ -1,7 +1,7 @@
-"""GPU tests of the chunked fp32 backward of the rules with a decay (gated and KDA, D in
-{64, 128}, from 16 tokens) against the fp64 oracles at the fp32 bounds, at the edges of its
-16-token chunks and its spans of chunks, and against the per-token kernels that every other
-call runs."""
+"""GPU tests of the chunked fp32 kernels of the rules with a decay (gated and KDA, D in {64,
+128}: the backward from 16 tokens, the forward of fp32 q/k/v from 160) against the fp64
+oracles at the fp32 bounds, at the edges of their 16-token chunks and of the spans of chunks,
+and against the per-token kernels that every other call runs."""
 
 from __future__ import annotations
 
@@ -95,3 +95,48 @@ def test_against_the_per_token_kernels(chan):
             np.testing.assert_array_equal(a, b, err_msg=name)
             assert_f32_parity(a, e, name, scaled=True)
             assert_f32_parity(c, e, f"shifted gate {name}", scaled=True)
+
+
+def _fwd(x, g, chan, **kw):
+    f = kernels.chunked_kda_rule if chan else kernels.chunked_gated_delta_rule
+    gd = g if isinstance(g, torch.Tensor) else _dev(g)
+    return [t.float().cpu().numpy() for t in f(_dev(x.q), _dev(x.k), _dev(x.v), _dev(x.beta), gd, _dev(x.s0), **kw)]
+
+
+@pytest.mark.parametrize("chan", [False, True])
+@pytest.mark.parametrize("t,d,h", [(160, 128, 3), (161, 64, 9), (175, 128, 1), (333, 64, 4), (200, 128, 66)])
+def test_forward_edges(t, d, h, chan):
+    """Whole and partial chunks, both tile widths (66 pairs of D 128 take 32 columns), with and
+    without a state; bf16 O is the fp32 one rounded."""
+    x, g, _, _ = _case((1, t, h, d), t + d + chan, chan, state=t % 2 == 0)
+    got = _fwd(x, g, chan)
+    exp = (gref.kda_delta_rule if chan else gref.gated_delta_rule)(x.q, x.k, x.v, x.beta, g, x.s0)
+    for name, a, e in zip(("o", "state"), got, exp):
+        assert_f32_parity(a, e, f"T{t} D{d} {name}")
+    with _native.use_knobs(0, 16):
+        narrow = _fwd(x, g, chan)
+    half = _fwd(x, g, chan, out_dtype=torch.bfloat16)
+    np.testing.assert_array_equal(narrow[0], got[0])
+    np.testing.assert_array_equal(half[0], torch.from_numpy(got[0]).bfloat16().float().numpy())
+    np.testing.assert_array_equal(half[1], got[1])
+
+
+def test_forward_decays_of_every_strength_and_routes():
+    """Channels at alpha 0, 1e-9, 1 and above 1 with a strong decay inside a chunk; a gate that is
+    not 16-byte aligned and other paths keep the per-token kernel; T = 0 passes the state."""
+    x, g, _, _ = _case((1, 170, 2, 64), 17, True, scale=0.05)
+    g[..., 0], g[..., 1], g[..., 2], g[..., 3] = -np.inf, -20.0, 0.0, 0.02
+    g[:, 37, :, 8:24] = -60.0
+    exp = gref.kda_delta_rule(x.q, x.k, x.v, x.beta, g, x.s0)
+    off = torch.empty(g.size + 1, device="cuda")[1:].copy_(_dev(g).flatten()).view(g.shape)
+    got, shifted = _fwd(x, g, True), _fwd(x, off, True)
+    with _native.use_knobs(1, 0):
+        per_token = _fwd(x, g, True)
+    for name, a, b, c, e in zip(("o", "state"), got, shifted, per_token, exp):
+        assert_f32_parity(a, e, name)
+        np.testing.assert_array_equal(b, c)
+    lib = _native.lib()
+    f32, bf16 = _native.DTYPE_F32, _native.DTYPE_BF16
+    assert lib.pm_decay_fwd_workspace_bytes(1, 170, 2, 64, f32) == 2 * 11 * (3 * 16 * 64 + 512 + 64) * 4
+    for args in ((1, 159, 2, 64, f32), (1, 170, 2, 48, f32), (1, 170, 2, 64, bf16), (1, 170, 256, 64, f32)):
+        assert lib.pm_decay_fwd_workspace_bytes(*args) == 0
