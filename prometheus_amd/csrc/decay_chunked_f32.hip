@@ -37,7 +37,7 @@
 //
 // Launches:
 //   K10p (prep, one wave per (b, h, chunk)): K^, K-, Q^, T'', T, P, A', gC, beta.
-//   K10s (one workgroup of eight waves per (b, h, 32 columns of d_v)): the state recurrence
+//   K10s (one workgroup per (b, h, 16 or 32 columns of d_v)): the state recurrence
 //     forwards (U per token, S at every span start) beside the G recurrence backwards (W
 //     and dV per token, G at every span end, dS0).
 //   K10c (one workgroup of D/16 waves per (b, h, span of 2 to 8 chunks)): the span forwards from
@@ -46,15 +46,16 @@
 //     (that divides by gC), hence the two walks.
 
 // Why chunks: the per-token kernels walk T tokens in sequence at about 500 (forward) and
-// 1,270 cycles (reverse) a token, bound by VALU issue; here a chunk of 16 tokens takes
-// about 4,300 cycles of the one sequential launch, and the rest is parallel over chunks.
-// Measured, B4 T4096 H16 D128, bf16 q/k/v, per-head gate: 6.0 -> 1.45 ms (K10p 126, K10s
-// 530, K10c 800 us); B2, per-channel gate: 5.9 -> 1.06 ms; B3 T1000 H6 D64 fp32: 1.11 -> 0.13
-// ms.  Against 64 bits the gradients stay at 2e-7 to 5e-7 (the per-token kernels: 1.3e-7 to
-// 2e-7).  What bounds it: K10s the chain of its four recurrence waves (72 MFMAs of 32 cycles a
-// chunk, in sequence; without the helpers' Q^^T dO 460 us, without copies, stores and helpers
-// 405), K10c the fp32 MFMA pipe at half its rate (232 products per wave and chunk; two waves
-// per SIMD, which wait for the pipe half of the time and at its barriers a third).
+// 1,270 cycles (reverse) a token, bound by VALU issue; here a chunk of 16 tokens takes about
+// 2,800 to 4,100 cycles of the one sequential launch, and the rest is parallel over chunks.
+// Measured, B4 T4096 H16 D128, bf16 q/k/v, per-head gate: 6.0 -> 1.45 ms (K10p 125, K10s
+// 505, K10c 825 us); B2, per-channel gate: 5.9 -> 0.87 ms (97, 340, 432); B3 T1000 H6 D64
+// fp32: 1.11 -> 0.10 ms.  Against 64 bits the gradients stay at 2e-7 to 5e-7 (the per-token
+// kernels: 1.3e-7 to 2e-7).  What bounds it: K10s the products of its recurrence waves (32
+// pairs: 54 of 32 cycles in a chunk of 2,800 cycles, the two barriers and exchanges most of
+// the rest, the copies 10%; 64 pairs: 94 on each SIMD), K10c the fp32 MFMA pipe at half its
+// rate (232 products per wave and chunk; two waves per SIMD, which wait for the pipe half of
+// the time and at its barriers a third).
 
 #include <type_traits>
 
@@ -107,6 +108,18 @@ struct TileIdx {
     }
     __device__ __forceinline__ float col(const unsigned char* b, int e, int i) const {
         return *reinterpret_cast<const float*>(b + cb[e] + cx[i & 3] + 256 * (i >> 2));
+    }
+    // Tiles i = hh + 2 j of a wave that holds every other one (TileIdx(r, g, hh)): the same, over j
+    int hx[2], hc[2];
+    __device__ __forceinline__ TileIdx(int r, int g, int hh) : TileIdx(r, g) {
+        hx[0] = hh ? rx[1] : rx[0], hx[1] = hh ? rx[3] : rx[2];
+        hc[0] = hh ? cx[1] : cx[0], hc[1] = hh ? cx[3] : cx[2];
+    }
+    __device__ __forceinline__ f32x4_t row2(const unsigned char* b, int j) const {
+        return ld4(b + rb + hx[j & 1] + 256 * (j >> 1));
+    }
+    __device__ __forceinline__ float col2(const unsigned char* b, int e, int j) const {
+        return *reinterpret_cast<const float*>(b + cb[e] + hc[j & 1] + 256 * (j >> 1));
     }
     // row and col for an i known only at run time
     __device__ __forceinline__ f32x4_t roww(const unsigned char* b, int i, int r) const {
@@ -561,45 +574,56 @@ __global__ __launch_bounds__(DV == 32 ? 256 : 128) void dec_fwd_kernel(
 }
 
 // ---------------------------------------------------------------- K10s
-// Eight waves: 0, 1 the state recurrence (16 columns of S each), 3 its copies; 6, 7 the
-// gradient recurrence (16 columns of G each), 5 its copies and the stores of W and dV; 2, 3
-// and 4 form Q^^T dO for waves 6 and 7 one chunk ahead.  Waves w and w + 4 share a SIMD, so
-// the four chains take one each, and the 64 products of Q^^T dO a chunk spread over three of
-// them (a chain's 72 products are dense: a helper's delay it one for one).  The two recurrences walk the chunks in opposite directions and share the workgroup's barriers
-// (one per chunk); each keeps three chunk buffers, one in use, one landed, one landing.
-template <int D>
+// The two recurrences, over S forwards and over G backwards, in one workgroup per (b, h, DV
+// columns of d_v).  They bound the launch: their chunks run in sequence, and a chain of one
+// wave per 16 columns needs 72 products of 32 cycles a chunk.  So two waves share 16 columns,
+// each holding every other tile of 16 rows of d (and half of every product over or onto d):
+// the products that contract over d (X = K^ S, Y = K- G) come in two halves, exchanged through
+// LDS at a barrier in mid-chunk and added by both, and each wave updates its own rows.  Per
+// chunk and wave 40 products (S) and 54 (G, its Q^^T dO among them) instead of 72 and 104;
+// one wave per 16 columns, with Q^^T dO in helper waves, took 510 us at 32 pairs of T 4096
+// (now 340) and 535 at 64 (now 505).
+// Waves: 2 DV/16 for S, as many for G (a SIMD holds one of each at DV = 32, one of either at
+// 16), one that copies for S (and Q^), one that copies for G and stores W and dV.  Each
+// recurrence keeps three chunk buffers: a chain holds its chunk's operands in registers and
+// reads the next chunk's, each behind a product (fenced: a product holds the MFMA pipe for 32
+// cycles, in which its wave issues a read for free, while a group of reads between products
+// holds the products up), so the copies run three chunks ahead into the buffer of the chunk
+// in registers.  (With the end-of-chunk barrier left out and the exchange slots doubled the
+// chains alone gain 4%, but the copies then come in one burst and the whole is 8% slower.)
+template <int D, int DV>
 struct DsGeo {
-    static constexpr int NT = D / 16, NI = kC16 * D * 4 / 1024, TILE = kC16 * D * 4;
-    static constexpr int NB = 3;
-    // state half: K^, K- rows, T''^T, V columns of each chain wave, gC
-    static constexpr int H_KH = 0, H_KB = TILE, H_T = 2 * TILE, H_V = H_T + 1024, H_G = H_V + 2048;
+    static constexpr int NC = DV / 16, NT = D / 16, NH = NT / 2, NI = kC16 * D * 4 / 1024, TILE = kC16 * D * 4;
+    static constexpr int NB = 3, WAVES = 4 * NC + 2;
+    // state half: K^, K- rows, T''^T, V columns, gC
+    static constexpr int H_KH = 0, H_KB = TILE, H_T = 2 * TILE, H_V = H_T + 1024, H_G = H_V + NC * 1024;
     static constexpr int HBUF = H_G + D * 4;
-    static constexpr int H_NCP = 2 * NI + 3 + D / 64;
-    // gradient half: K^, K- rows, dO columns, T, P, gC and beta
-    static constexpr int S_KH = 0, S_KB = TILE, S_O = 2 * TILE, S_T = S_O + 2048, S_P = S_T + 1024, S_G = S_P + 1024;
+    static constexpr int H_NCP = 3 * NI + 1 + NC + D / 64;
+    // gradient half: K^, K- rows, Q^ in operand order, dO columns, T, P, gC and beta
+    static constexpr int S_KH = 0, S_KB = TILE, S_QH = 2 * TILE, S_O = 3 * TILE, S_T = S_O + NC * 1024, S_P = S_T + 1024, S_G = S_P + 1024;
     static constexpr int SBUF = S_G + DecRec<D>::GBN * 4;
-    static constexpr int S_NCP = 2 * NI + 4 + DecRec<D>::GBN / 64;
-    static constexpr int S_NST = 4;  // W and dV stores per chunk
+    static constexpr int S_NCP = 2 * NI + 2 + NC + DecRec<D>::GBN / 64;
+    static constexpr int S_NST = 2 * NC;  // W and dV stores per chunk
     static constexpr int OFF_S = NB * HBUF;
-    static constexpr int OFF_H = OFF_S + NB * SBUF;           // 2 slots x 2 chains: Q^^T dO
-    static constexpr int OFF_W = OFF_H + 4 * NT * 1024;       // 2 slots x 2 chains: W, beta
+    static constexpr int OFF_X = OFF_S + NB * SBUF;     // half products: S, G x NC x 2 halves
+    static constexpr int OFF_W = OFF_X + 4 * NC * 1024; // 2 slots x NC: W, beta
     static constexpr int WSLOT = 1024 + 64;
-    static constexpr int BYTES = OFF_W + 4 * WSLOT;
+    static constexpr int BYTES = OFF_W + 2 * NC * WSLOT;
     static_assert(BYTES <= 160 * 1024 && S_NCP + S_NST <= 63 && H_NCP <= 63, "LDS / vmcnt");
     static_assert(HBUF % 16 == 0 && SBUF % 16 == 0, "alignment");
 };
 
 // GE: bytes per element of dQ, dK and dV (4: fp32; 2: bf16, rounded to nearest even)
-template <int D, typename InT, int GE>
-__global__ __launch_bounds__(512) void dec_sweep_kernel(
+template <int D, int DV, typename InT, int GE>
+__global__ __launch_bounds__((DsGeo<D, DV>::WAVES * 64)) void dec_sweep_kernel(
     const InT* __restrict__ v, const float* __restrict__ s0, const float* __restrict__ go,
     const float* __restrict__ gs, void* __restrict__ gv, float* __restrict__ gs0, const float* __restrict__ kh,
     const float* __restrict__ kb, const float* __restrict__ qh, const float* __restrict__ rec,
     float* __restrict__ w_out, float* __restrict__ u_out, float* __restrict__ s_hist, float* __restrict__ g_hist,
     int n_pairs, int T, int H, int n_ch, int n_span, int span_len) {
-    using G = DsGeo<D>;
+    using G = DsGeo<D, DV>;
     using R = DecRec<D>;
-    constexpr int NT = G::NT, NI = G::NI, NB = G::NB, n_tiles = D / 32;
+    constexpr int NC = G::NC, NT = G::NT, NH = G::NH, NI = G::NI, NB = G::NB, n_tiles = D / DV;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     // XCD-aware placement: the n_tiles workgroups of a pair share bid % 8
     const int bid = blockIdx.x, xcd = bid & 7, bslot = bid >> 3;
@@ -607,18 +631,16 @@ __global__ __launch_bounds__(512) void dec_sweep_kernel(
     if (pair >= n_pairs || n_ch <= 0) return;
     const int seq = pair / H, h = pair % H;
     const size_t tok0 = static_cast<size_t>(seq) * T;
-    const int col0 = tile * 32;
+    const int col0 = tile * DV;
     const int w = static_cast<int>(uniform(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     const int r = lane & 15, g = lane >> 4;
     const size_t tstride = static_cast<size_t>(H) * D;
     const size_t sbase = static_cast<size_t>(pair) * D * D;
     const size_t item0 = static_cast<size_t>(pair) * n_ch;
-    const TileIdx<D> ix(r, g);
 
     auto hbuf = [=](int c) { return smem + (c % NB) * G::HBUF; };
     auto sbuf = [=](int c) { return smem + G::OFF_S + (c % NB) * G::SBUF; };
-    auto hslot = [=](int c, int which) { return smem + G::OFF_H + ((c & 1) * 2 + which) * NT * 1024; };
-    auto wslot = [=](int c, int which) { return smem + G::OFF_W + ((c & 1) * 2 + which) * G::WSLOT; };
+    auto wslot = [=](int c, int which) { return smem + G::OFF_W + ((c & 1) * NC + which) * G::WSLOT; };
     auto row0_of = [=](int c, int col) { return (tok0 + c * kC16) * tstride + static_cast<size_t>(h) * D + col; };
     auto els_of = [=](int c, int cols) {  // elements from a column block's first row to its last row's end
         return static_cast<unsigned>((min(kC16, T - c * kC16) - 1) * tstride + cols);
@@ -630,113 +652,252 @@ __global__ __launch_bounds__(512) void dec_sweep_kernel(
         for (int i = 0; i < NI; ++i) dma16_asm(rs, d0 + 1024 * i, static_cast<unsigned>(1024 * i + 16 * lane));
     };
 
-    // Q^^T dO, tiles m0 .. m0 + N - 1 (rows 16 m .. of d): Q^ in operand order straight into
-    // registers, dO of the chain's columns from the gradient half's buffer, into its slot
-    constexpr int NA = NT * 5 / 8, NC = NT - NA;
-    auto fetch_q = [=](int c, int m0, auto& x) __attribute__((always_inline)) {
-        const float* qp = qh + (item0 + c) * kC16 * D + 256 * m0 + 4 * lane;
+    if (w < 4 * NC) {
+        // ============ chain waves: columns col0 + 16 cw + [0, 16), tiles m = hh + 2 j of 16 rows ============
+        const bool state = w < 2 * NC;
+        const int cw = (w >> 1) % NC, hh = w & 1;
+        const int ecol = col0 + 16 * cw + r;
+        const TileIdx<D> ix(r, g, hh);
+        unsigned char* const xs = smem + G::OFF_X + ((state ? 0 : NC) + cw) * 2048 + 16 * lane;
+        f32x4_t M[NH];  // this wave's rows of S or G
+        {
+            const float* m0 = state ? s0 : gs;
 #pragma unroll
-        for (unsigned m = 0; m < sizeof(x) / 16; ++m) x[m] = *reinterpret_cast<const f32x4_t*>(qp + 256 * m);
-    };
-    auto qtdo = [=](int c, int cw, int m0, auto& x) __attribute__((always_inline)) {
-        constexpr unsigned N = sizeof(x) / 16;
-        const float* Of = reinterpret_cast<const float*>(sbuf(c) + G::S_O + 1024 * cw);
-        f32x4_t dOc, hq[N];
+            for (int j = 0; j < NH; ++j)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) dOc[e] = Of[(4 * g + e) * 16 + r];
-#pragma unroll
-        for (unsigned m = 0; m < N; ++m) hq[m] = kZero4;
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-            for (unsigned m = 0; m < N; ++m) hq[m] = mfma4(x[m][e], dOc[e], hq[m]);
-        unsigned char* slot = hslot(c, cw) + 1024 * m0 + 16 * lane;
-#pragma unroll
-        for (unsigned m = 0; m < N; ++m) st4(slot + 1024 * m, hq[m]);
-    };
-
-    if (w < 2) {
-        // ============ the state recurrence: S columns col0 + 16 w + [0, 16) ============
-        const int ecol = col0 + 16 * w + r;
-        f32x4_t S[NT];
-#pragma unroll
-        for (int m = 0; m < NT; ++m)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                S[m][e] = s0 ? s0[sbase + static_cast<size_t>(16 * m + 4 * g + e) * D + ecol] : 0.f;
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), seen by the compiler: no wait for S0 in the loop
-        __builtin_amdgcn_s_setprio(3);       // the chains bound the chunk: first on their SIMD's MFMA pipe
-        lds_barrier();                       // B0
-        // One iteration: S += K-^T U of the last chunk (its K-^T operand kt was read an iteration
-        // ago), then X and U of this one.  Every LDS read sits right behind one product (fenced:
-        // a 16x16x4 product holds the MFMA pipe for 32 cycles, in which the wave issues its
-        // reads for free, while a group of reads between products holds the products up); the
-        // decay Diag(gC) S falls into the latency of U's short products.
-        f32x4_t Up = kZero4;
-        float kt[4][NT] = {};  // K-^T operand: K-[4 g + e][16 m + r]
-        auto rd_kt = [&](const unsigned char* b, int e, int m) __attribute__((always_inline)) {
-            kt[e][m] = ix.col(b + G::H_KB, e, m);  // (tiles m and m + 4: one paired read)
-            kt[e][m + NT / 2] = ix.col(b + G::H_KB, e, m + NT / 2);
+                for (int e = 0; e < 4; ++e)
+                    M[j][e] = m0 ? m0[sbase + static_cast<size_t>(16 * (hh + 2 * j) + 4 * g + e) * D + ecol] : 0.f;
+        }
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), seen by the compiler: no wait for these in the loop
+        __builtin_amdgcn_s_setprio(3);
+        lds_barrier();  // B0
+        // this wave's operand over d (rows) and onto d (columns), and the decay of its rows
+        f32x4_t kf[NH], gc[NH];
+        float kt[4][NH];
+        auto rd_kt = [&](const unsigned char* b, int e, int j) __attribute__((always_inline)) { kt[e][j] = ix.col2(b, e, j); };
+        // a product over d from this wave's half and, after the barrier, the other's
+        auto total = [&](f32x4_t p) __attribute__((always_inline)) {
+            return p + ld4(xs + 1024 * (hh ^ 1));
         };
-        for (int i = 0; i < n_ch; ++i) {
-            const unsigned char* b = hbuf(i);
-            const InT* Vf = reinterpret_cast<const InT*>(b + G::H_V + 1024 * w);
-            f32x4_t kf[NT], gc[NT], vr, tt;
-            // (kt starts as zeros; kt[e] is read anew behind its products)
+        if (state) {
+            f32x4_t vr, tt;
+            auto rd_v = [&](const unsigned char* b, int e) __attribute__((always_inline)) {
+                vr[e] = to_f32<InT>(reinterpret_cast<const InT*>(b + G::H_V + 1024 * cw)[(4 * g + e) * 16 + r]);
+            };
+            auto rd_gc = [&](const unsigned char* b, int j) __attribute__((always_inline)) {
+                gc[j] = ld4(b + G::H_G + 4 * (16 * (hh + 2 * j) + 4 * g));
+            };
+            {
+                const unsigned char* b = hbuf(0);
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int m = 0; m < NT; ++m) {
-                    S[m] = mfma4(kt[e][m], Up[e], S[m]);
-                    if (e == 0) kf[m] = ix.row(b + G::H_KH, m);
-                    if (e > 0 && m < NT / 2) rd_kt(b, e - 1, m);
-                    if (e == 1 && m >= NT / 2 && m < NT / 2 + 2) {
-                        vr[2 * (m - NT / 2)] = to_f32<InT>(Vf[(4 * g + 2 * (m - NT / 2)) * 16 + r]);
-                        vr[2 * (m - NT / 2) + 1] = to_f32<InT>(Vf[(4 * g + 2 * (m - NT / 2) + 1) * 16 + r]);
-                    }
-                    if (e == 2 && m == NT - 1) tt = ld4(b + G::H_T + 16 * lane);
-                    fence();
+                for (int j = 0; j < NH; ++j) {
+                    kf[j] = ix.row2(b + G::H_KH, j);
+                    rd_gc(b, j);
                 }
-            if ((i & (span_len - 1)) == 0) {
-                float* hp = s_hist + ((static_cast<size_t>(pair) * n_span + i / span_len) * NT + col0 / 16 + w) * NT * 256;
-#pragma unroll
-                for (int m = 0; m < NT; ++m) *reinterpret_cast<f32x4_t*>(hp + m * 256 + 4 * lane) = S[m];
-            }
-            // X = K^ S - V, U = T'' X
-            f32x4_t xa[4] = {-vr, kZero4, kZero4, kZero4};
-#pragma unroll
-            for (int m = 0; m < NT; ++m)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    xa[e] = mfma4(kf[m][e], S[m][e], xa[e]);
-                    const int n = 4 * m + e;
-                    if (n < NT / 2) rd_kt(b, 3, n);
-                    if (n >= NT / 2 && n < NT / 2 + NT) gc[n - NT / 2] = ld4(b + G::H_G + 4 * (16 * (n - NT / 2) + 4 * g));
+                    rd_v(b, e);
+#pragma unroll
+                    for (int j = 0; j < NH; ++j) rd_kt(b + G::H_KB, e, j);
+                }
+                tt = ld4(b + G::H_T + 16 * lane);
+                __builtin_amdgcn_s_waitcnt(0xC07F);
+                lds_barrier();  // B1: chunk 0's buffer may be refilled
+            }
+            for (int i = 0; i < n_ch; ++i) {
+                const unsigned char* bn = hbuf(min(i + 1, n_ch - 1));  // (the last chunk reads itself again, unused)
+                // X = K^ S - V, this wave's half
+                f32x4_t xa[4] = {kZero4, kZero4, kZero4, kZero4};
+                if (hh == 0) xa[0] = -vr;
+                fence();
+#pragma unroll
+                for (int j = 0; j < NH; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        xa[e] = mfma4(kf[j][e], M[j][e], xa[e]);
+                        if (e == 1 && j > 0) kf[j - 1] = ix.row2(bn + G::H_KH, j - 1);
+                        if (j < 2 && (e == 2 || e == 3)) rd_v(bn, 2 * j + e - 2);
+                        fence();
+                    }
+                kf[NH - 1] = ix.row2(bn + G::H_KH, NH - 1);
+                const f32x4_t p = (xa[0] + xa[1]) + (xa[2] + xa[3]);
+                st4(xs + 1024 * hh, p);
+                if ((i & (span_len - 1)) == 0) {
+                    float* hp = s_hist + ((static_cast<size_t>(pair) * n_span + i / span_len) * NT + col0 / 16 + cw) * NT * 256;
+#pragma unroll
+                    for (int j = 0; j < NH; ++j) *reinterpret_cast<f32x4_t*>(hp + (hh + 2 * j) * 256 + 4 * lane) = M[j];
+                }
+#pragma unroll
+                for (int j = 0; j < NH; ++j) M[j] = gc[j] * M[j];
+                lds_barrier();  // mid-chunk: the halves are in LDS
+                const f32x4_t X = total(p);
+#pragma unroll
+                for (int j = 0; j < NH; ++j) rd_gc(bn, j);
+                const f32x4_t tn = ld4(bn + G::H_T + 16 * lane);
+                const f32x4_t U = mm16(tt, X);
+                // S = Diag(gC) S + K-^T U
+                fence();
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int j = 0; j < NH; ++j) {
+                        M[j] = mfma4(kt[e][j], U[e], M[j]);
+                        if (e > 0) rd_kt(bn + G::H_KB, e - 1, j);
+                        if (e == 3) rd_kt(bn + G::H_KB, 3, j);
+                        fence();
+                    }
+                // U's rows (U^T = X^T T''^T): lane (g, r) holds U[r][col0 + 16 cw + 4 g ..]
+                if (hh == 0)
+                    *reinterpret_cast<f32x4_t*>(u_out + (item0 + i) * kC16 * D +
+                                                4 * f32_chunk<D>(r, (col0 + 16 * cw) / 4 + g)) = mm16(X, tt);
+                tt = tn;
+                __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), seen by the compiler
+                lds_barrier();                       // end of the chunk
+            }
+        } else {
+            f32x4_t dOc, ta, b4, qc[NH];
+            f32x2_t pp;  // P^T's operand for tokens e = 2 hh, 2 hh + 1: each half adds its part of P^T dO
+            auto rd_do = [&](const unsigned char* b, int e) __attribute__((always_inline)) {
+                return reinterpret_cast<const float*>(b + G::S_O + 1024 * cw)[(4 * g + e) * 16 + r];
+            };
+            auto rd_gc = [&](const unsigned char* b, int j) __attribute__((always_inline)) {
+                gc[j] = ld4(b + G::S_G + 4 * (16 * (hh + 2 * j) + 4 * g));
+            };
+            auto rd_q = [&](const unsigned char* b, int j) __attribute__((always_inline)) {
+                qc[j] = ld4(b + G::S_QH + 1024 * (hh + 2 * j) + 16 * lane);
+            };
+            {
+                const unsigned char* b = sbuf(n_ch - 1);
+#pragma unroll
+                for (int j = 0; j < NH; ++j) {
+                    kf[j] = ix.row2(b + G::S_KB, j);
+                    rd_q(b, j);
+                    rd_gc(b, j);
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    dOc[e] = rd_do(b, e);
+#pragma unroll
+                    for (int j = 0; j < NH; ++j) rd_kt(b + G::S_KH, e, j);
+                }
+                ta = ld4(b + G::S_T + 16 * lane);
+                pp = *reinterpret_cast<const f32x2_t*>(b + G::S_P + 16 * lane + 8 * hh);
+                b4 = ld4(b + G::S_G + 4 * D + 16 * g);
+                __builtin_amdgcn_s_waitcnt(0xC07F);
+                lds_barrier();  // B1
+            }
+            for (int c = n_ch - 1; c >= 0; --c) {
+                const unsigned char* bn = sbuf(max(c - 1, 0));
+                f32x4_t dOn, tn, bn4;
+                f32x2_t pn;
+                if (c == n_ch - 1 || ((c + 1) & (span_len - 1)) == 0) {
+                    float* hp = g_hist + ((static_cast<size_t>(pair) * n_span + c / span_len) * NT + col0 / 16 + cw) * NT * 256;
+#pragma unroll
+                    for (int j = 0; j < NH; ++j) *reinterpret_cast<f32x4_t*>(hp + (hh + 2 * j) * 256 + 4 * lane) = M[j];
+                }
+                // dU = K- G + P^T dO, this wave's half; a tile's decay behind its last product
+                f32x4_t ya[4] = {kZero4, kZero4, kZero4, kZero4};
+                ya[0] = mfma4(pp[0], hh ? dOc[2] : dOc[0], kZero4);
+                ya[1] = mfma4(pp[1], hh ? dOc[3] : dOc[1], kZero4);
+                fence();
+#pragma unroll
+                for (int j = 0; j < NH; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        ya[e] = mfma4(kf[j][e], M[j][e], ya[e]);
+                        if (e == 1 && j > 0) kf[j - 1] = ix.row2(bn + G::S_KB, j - 1);
+                        if (j < 2 && (e == 2 || e == 3)) dOn[2 * j + e - 2] = rd_do(bn, 2 * j + e - 2);
+                        if (e == 0 && j > 0) M[j - 1] = gc[j - 1] * M[j - 1];
+                        fence();
+                    }
+                kf[NH - 1] = ix.row2(bn + G::S_KB, NH - 1);
+                M[NH - 1] = gc[NH - 1] * M[NH - 1];
+                fence();
+                // G = Diag(gC) G + Q^^T dO: half of it ahead of the exchange, the rest in its latency
+                auto q_prod = [&](int e, int j) __attribute__((always_inline)) { M[j] = mfma4(qc[j][e], dOc[e], M[j]); };
+#pragma unroll
+                for (int j = 0; j < NH; ++j) {
+                    q_prod(0, j);
+                    rd_gc(bn, j);
                     fence();
                 }
-            const f32x4_t X = (xa[0] + xa[1]) + (xa[2] + xa[3]);
-            Up = mm16(tt, X);
-            // U's rows (U^T = X^T T''^T): lane (g, r) holds U[r][col0 + 16 w + 4 g ..]
-            const f32x4_t Ut = mm16(X, tt);
+                const f32x4_t p = (ya[0] + ya[1]) + (ya[2] + ya[3]);
+                st4(xs + 1024 * hh, p);
+                fence();
 #pragma unroll
-            for (int m = 0; m < NT; ++m) S[m] = gc[m] * S[m];
-            *reinterpret_cast<f32x4_t*>(u_out + (item0 + i) * kC16 * D +
-                                        4 * f32_chunk<D>(r, (col0 + 16 * w) / 4 + g)) = Ut;
-            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), seen by the compiler
-            lds_barrier();
+                for (int j = 0; j < NH; ++j) {
+                    q_prod(1, j);
+                    if (j == 0) tn = ld4(bn + G::S_T + 16 * lane);
+                    if (j == 1) pn = *reinterpret_cast<const f32x2_t*>(bn + G::S_P + 16 * lane + 8 * hh);
+                    fence();
+                }
+                lds_barrier();  // mid-chunk
+                const f32x4_t po = ld4(xs + 1024 * (hh ^ 1));
+                fence();
+#pragma unroll
+                for (int j = 0; j < NH; ++j) {
+                    q_prod(2, j);
+                    fence();
+                }
+                // W = T^T dU
+                const f32x4_t dU = p + po;
+                f32x4_t w0 = mfma4(ta[0], dU[0], kZero4), w1 = mfma4(ta[1], dU[1], kZero4);
+                __asm__ volatile("" : "+v"(w0), "+v"(w1));  // (issued here, not where the sum needs them)
+                fence();
+                q_prod(3, 0);
+                rd_q(bn, 0);
+                fence();
+                w0 = mfma4(ta[2], dU[2], w0), w1 = mfma4(ta[3], dU[3], w1);
+                __asm__ volatile("" : "+v"(w0), "+v"(w1));
+                fence();
+#pragma unroll
+                for (int j = 1; j < NH; ++j) {
+                    q_prod(3, j);
+                    rd_q(bn, j);
+                    if (j == 1) bn4 = ld4(bn + G::S_G + 4 * D + 16 * g);
+                    fence();
+                }
+                const f32x4_t W = w0 + w1;
+                const f32x4_t nbW = -(W * b4);
+                // G -= K^^T diag(beta) W
+                fence();
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int j = 0; j < NH; ++j) {
+                        M[j] = mfma4(kt[e][j], nbW[e], M[j]);
+                        if (e > 0) rd_kt(bn + G::S_KH, e - 1, j);
+                        if (e == 3) rd_kt(bn + G::S_KH, 3, j);
+                        if (e == 0 && j == 0 && hh == 0) st4(wslot(c, cw) + 16 * lane, W);
+                        if (e == 0 && j == 1 && hh == 0 && r == 0) st4(wslot(c, cw) + 1024 + 16 * g, b4);
+                        fence();
+                    }
+                dOc = dOn, ta = tn, pp = pn, b4 = bn4;
+                __builtin_amdgcn_s_waitcnt(0xC07F);
+                lds_barrier();  // end of the chunk
+            }
+#pragma unroll
+            for (int j = 0; j < NH; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    gs0[sbase + static_cast<size_t>(16 * (hh + 2 * j) + 4 * g + e) * D + ecol] = M[j][e];
         }
-        lds_barrier();
-    } else if (w == 3) {
-        // ============ the state half's copies, two chunks ahead ============
-        auto copies = [=](int c) __attribute__((always_inline)) {
+    } else if (w == 4 * NC) {
+        // ============ the state half's copies, three chunks ahead ============
+        // (each half of a chunk issues half of the copies: 28 in one go hold the barrier up)
+        auto copies_a = [=](int c) __attribute__((always_inline)) {
             unsigned char* b = hbuf(c);
-            const float* rc = rec + (item0 + c) * R::FLOATS;
             copy_tile(kh, c, b + G::H_KH);
             copy_tile(kb, c, b + G::H_KB);
+        };
+        auto copies_b = [=](int c) __attribute__((always_inline)) {
+            unsigned char* b = hbuf(c);
+            const float* rc = rec + (item0 + c) * R::FLOATS;
+            copy_tile(qh, n_ch - 1 - c, sbuf(n_ch - 1 - c) + G::S_QH);  // (a share of the gradient half's)
             dma16_asm(make_rsrc(rc + R::T2, 1024), uniform_ptr(b + G::H_T), static_cast<unsigned>(16 * lane));
             constexpr int LPR = 16 * sizeof(InT) / 16;  // lanes per row of 16 columns
 #pragma unroll
-            for (int j = 0; j < 2; ++j)  // (bf16: lanes 32 .. 63 address rows past the chunk and read zeros)
+            for (int j = 0; j < NC; ++j)  // (bf16: lanes 32 .. 63 address rows past the chunk and read zeros)
                 dma16_asm(make_rsrc(v + row0_of(c, col0 + 16 * j), els_of(c, 16) * sizeof(InT)),
                           uniform_ptr(b + G::H_V + 1024 * j),
                           static_cast<unsigned>((lane / LPR) * tstride * sizeof(InT) + 16 * (lane % LPR)));
@@ -745,57 +906,45 @@ __global__ __launch_bounds__(512) void dec_sweep_kernel(
             for (int j = 0; j < D / 64; ++j)
                 dma4_asm(rg, uniform_ptr(b + G::H_G + 256 * j), static_cast<unsigned>(256 * j + 4 * lane));
         };
+        auto copies = [=](int c) __attribute__((always_inline)) {
+            copies_a(c);
+            copies_b(c);
+        };
         copies(0);
-        if (n_ch > 1) {
-            copies(1);
+        if (n_ch > 1) copies(1);
+        if (n_ch > 2) {
+            copies(2);
             wait_vm_n<G::H_NCP>();
         } else {
             wait_vm_n<0>();
         }
-        // ... and the remaining tiles of both chains' Q^^T dO, ahead of the copies (the compiler,
-        // which does not see the copies, waits for all of them where it waits for Q^)
-        f32x4_t qc[NC];
-        fetch_q(n_ch - 1, NA, qc);
-        lds_barrier();  // B0
+        lds_barrier();  // B0: chunks 0 and 1 landed
+        lds_barrier();  // B1
         for (int i = 0; i < n_ch; ++i) {
-            const int ch = n_ch - 1 - i;
-            qtdo(ch, 0, NA, qc);
-            qtdo(ch, 1, NA, qc);
-            if (i + 2 < n_ch) {
-                copies(i + 2);
+            // chunk i's buffer is free (its operands were read before this iteration); chunk i + 2
+            // has landed at the end
+            if (i + 3 < n_ch) copies_a(i + 3);
+            lds_barrier();  // mid-chunk
+            if (i + 3 < n_ch) {
+                copies_b(i + 3);
                 wait_vm_n<G::H_NCP>();
             } else {
                 wait_vm_n<0>();
             }
-            if (ch > 0) fetch_q(ch - 1, NA, qc);
             lds_barrier();
         }
-        lds_barrier();
-    } else if (w == 2 || w == 4) {
-        // ============ Q^^T dO of chunk n_ch - 1 - i, tiles [0, NA) of the gradient chain cw ============
-        const int cw = w == 4 ? 0 : 1;
-        f32x4_t qn[NA];
-        fetch_q(n_ch - 1, 0, qn);
-        lds_barrier();  // B0
-        for (int i = 0; i < n_ch; ++i) {
-            const int ch = n_ch - 1 - i;
-            f32x4_t qc[NA];
-#pragma unroll
-            for (int m = 0; m < NA; ++m) qc[m] = qn[m];
-            if (ch > 0) fetch_q(ch - 1, 0, qn);
-            qtdo(ch, cw, 0, qc);
-            lds_barrier();
-        }
-        lds_barrier();
-    } else if (w == 5) {
+    } else {
         // ============ the gradient half's copies, and its stores one chunk behind ============
-        auto copies = [=](int c) __attribute__((always_inline)) {
+        auto copies_a = [=](int c) __attribute__((always_inline)) {
             unsigned char* b = sbuf(c);
-            const float* rc = rec + (item0 + c) * R::FLOATS;
             copy_tile(kh, c, b + G::S_KH);
             copy_tile(kb, c, b + G::S_KB);
+        };
+        auto copies_b = [=](int c) __attribute__((always_inline)) {
+            unsigned char* b = sbuf(c);
+            const float* rc = rec + (item0 + c) * R::FLOATS;
 #pragma unroll
-            for (int j = 0; j < 2; ++j)  // a null dO reads zeros (a zero-length range)
+            for (int j = 0; j < NC; ++j)  // a null dO reads zeros (a zero-length range)
                 dma16_asm(make_rsrc(go ? go + row0_of(c, col0 + 16 * j) : go, go ? els_of(c, 16) * 4 : 0u),
                           uniform_ptr(b + G::S_O + 1024 * j),
                           static_cast<unsigned>((lane >> 2) * tstride * 4 + 16 * (lane & 3)));
@@ -806,147 +955,55 @@ __global__ __launch_bounds__(512) void dec_sweep_kernel(
             for (int j = 0; j < R::GBN / 64; ++j)
                 dma4_asm(rg, uniform_ptr(b + G::S_G + 256 * j), static_cast<unsigned>(256 * j + 4 * lane));
         };
-        copies(n_ch - 1);
-        if (n_ch > 1) {
-            copies(n_ch - 2);
+        auto store = [=](int cs) __attribute__((always_inline)) {
+            const int t = lane >> 2, p = lane & 3;
+#pragma unroll
+            for (int j = 0; j < NC; ++j) {
+                const float* ws = reinterpret_cast<const float*>(wslot(cs, j));
+                const float bt = ws[256 + t];
+                f32x4_t x;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[e] = ws[4 * (16 * (t >> 2) + 4 * p + e) + (t & 3)];
+                *reinterpret_cast<f32x4_t*>(w_out + (item0 + cs) * kC16 * D +
+                                            4 * f32_chunk<D>(t, (col0 + 16 * j) / 4 + p)) = x;
+                const __amdgpu_buffer_rsrc_t rv = make_rsrc(
+                    static_cast<unsigned char*>(gv) + row0_of(cs, col0 + 16 * j) * GE, els_of(cs, 16) * GE);
+                const unsigned off = static_cast<unsigned>((t * tstride + 4 * p) * GE);
+                if constexpr (GE == 2)
+                    __builtin_amdgcn_raw_buffer_store_b64(cvt4(x * bt), rv, off, 0, 0);
+                else
+                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, x * bt), rv, off, 0, 0);
+            }
+        };
+        auto copies = [=](int c) __attribute__((always_inline)) {
+            copies_a(c);
+            copies_b(c);
+        };
+        const int last = n_ch - 1;
+        copies(last);
+        if (n_ch > 1) copies(last - 1);
+        if (n_ch > 2) {
+            copies(last - 2);
             wait_vm_n<G::S_NCP>();
         } else {
             wait_vm_n<0>();
         }
         lds_barrier();  // B0
-        for (int i = 0; i <= n_ch + 1; ++i) {
-            const bool cp = n_ch - 3 - i >= 0, st = i >= 2;
-            if (cp) copies(n_ch - 3 - i);
-            if (st) {
-                const int cs = n_ch - i + 1;  // the chunk the chains ran in iteration i - 1
-                const int t = lane >> 2, p = lane & 3;
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const float* ws = reinterpret_cast<const float*>(wslot(cs, j));
-                    const float bt = ws[256 + t];
-                    f32x4_t x;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) x[e] = ws[4 * (16 * (t >> 2) + 4 * p + e) + (t & 3)];
-                    *reinterpret_cast<f32x4_t*>(w_out + (item0 + cs) * kC16 * D +
-                                                4 * f32_chunk<D>(t, (col0 + 16 * j) / 4 + p)) = x;
-                    const __amdgpu_buffer_rsrc_t rv = make_rsrc(
-                        static_cast<unsigned char*>(gv) + row0_of(cs, col0 + 16 * j) * GE, els_of(cs, 16) * GE);
-                    const unsigned off = static_cast<unsigned>((t * tstride + 4 * p) * GE);
-                    if constexpr (GE == 2)
-                        __builtin_amdgcn_raw_buffer_store_b64(cvt4(x * bt), rv, off, 0, 0);
-                    else
-                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, x * bt), rv, off, 0, 0);
-                }
-            }
-            if (i <= n_ch) {
-                // chunk n_ch - 2 - i has landed (the next iteration's); the newest copies and
-                // this iteration's stores may be in flight
-                if (n_ch - 2 - i >= 0) {
-                    if (cp && st) wait_vm_n<G::S_NCP + G::S_NST>();
-                    else if (cp) wait_vm_n<G::S_NCP>();
-                    else wait_vm_n<0>();
-                }
-                lds_barrier();
-            }
-        }
-    } else {
-        // ============ the gradient recurrence: G columns col0 + 16 cw + [0, 16) ============
-        const int cw = w - 6;
-        const int ecol = col0 + 16 * cw + r;
-        f32x4_t Gm[NT];
-#pragma unroll
-        for (int m = 0; m < NT; ++m)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                Gm[m][e] = gs ? gs[sbase + static_cast<size_t>(16 * m + 4 * g + e) * D + ecol] : 0.f;
-        __builtin_amdgcn_s_waitcnt(0x0F70);
-        __builtin_amdgcn_s_setprio(3);
-        lds_barrier();  // B0
-        // One iteration runs chunk c from operands read an iteration ago (its buffer had landed
-        // by then; only Q^^T dO is read here) and reads chunk c - 1's behind its products, as
-        // the state chain does; the decay and Q^^T dO enter G in the latency of dU and W.
-        f32x4_t kf[NT], gc[NT], dOc, ta, b4, pp;
-        float kt[4][NT];  // K^^T operand: K^[4 g + e][16 m + r]
-        auto rd_kt = [&](const unsigned char* b, int e, int m) __attribute__((always_inline)) {
-            kt[e][m] = ix.col(b + G::S_KH, e, m);
-            kt[e][m + NT / 2] = ix.col(b + G::S_KH, e, m + NT / 2);
-        };
-        auto rd_gc = [&](const unsigned char* b, int m) __attribute__((always_inline)) {
-            gc[m] = ld4(b + G::S_G + 4 * (16 * m + 4 * g));
-        };
-        auto rd_do = [&](const unsigned char* b, int e) __attribute__((always_inline)) {
-            return reinterpret_cast<const float*>(b + G::S_O + 1024 * cw)[(4 * g + e) * 16 + r];
-        };
-        {
-            const unsigned char* b = sbuf(n_ch - 1);
-#pragma unroll
-            for (int m = 0; m < NT; ++m) {
-                kf[m] = ix.row(b + G::S_KB, m);
-                rd_gc(b, m);
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                dOc[e] = rd_do(b, e);
-#pragma unroll
-                for (int m = 0; m < NT / 2; ++m) rd_kt(b, e, m);
-            }
-            ta = ld4(b + G::S_T + 16 * lane);
-            pp = ld4(b + G::S_P + 16 * lane);
-            b4 = ld4(b + G::S_G + 4 * D + 16 * g);
-            lds_barrier();  // iteration 0: Q^^T dO of chunk n_ch - 1
-        }
-        for (int c = n_ch - 1; c >= 0; --c) {
-            if (c == n_ch - 1 || ((c + 1) & (span_len - 1)) == 0) {
-                float* hp = g_hist + ((static_cast<size_t>(pair) * n_span + c / span_len) * NT + col0 / 16 + cw) * NT * 256;
-#pragma unroll
-                for (int m = 0; m < NT; ++m) *reinterpret_cast<f32x4_t*>(hp + m * 256 + 4 * lane) = Gm[m];
-            }
-            const unsigned char* bn = sbuf(max(c - 1, 0));  // (chunk 0 reads its own buffer again, unused)
-            const unsigned char* hs = hslot(c, cw) + 16 * lane;
-            f32x4_t hq[NT], dOn, tn, pn, bn4;
-            // Y = K- G, dU = Y + P^T dO, W = T^T dU
-            f32x4_t ya[4] = {kZero4, kZero4, kZero4, kZero4};
-#pragma unroll
-            for (int m = 0; m < NT; ++m)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    ya[e] = mfma4(kf[m][e], Gm[m][e], ya[e]);
-                    if (e == 0) hq[m] = ld4(hs + 1024 * m);
-                    if (e == 1 && m > 0) kf[m - 1] = ix.row(bn + G::S_KB, m - 1);
-                    if (e == 2 && m < 4) dOn[m] = rd_do(bn, m);
-                    if (e == 3 && m == 0) tn = ld4(bn + G::S_T + 16 * lane);
-                    if (e == 3 && m == 1) pn = ld4(bn + G::S_P + 16 * lane);
-                    if (e == 3 && m == 2) bn4 = ld4(bn + G::S_G + 4 * D + 16 * g);
-                    fence();
-                }
-            kf[NT - 1] = ix.row(bn + G::S_KB, NT - 1);
-            const f32x4_t dU = mm16(pp, dOc, (ya[0] + ya[1]) + (ya[2] + ya[3]));
-#pragma unroll
-            for (int m = 0; m < NT; ++m) Gm[m] = gc[m] * Gm[m] + hq[m];
-            const f32x4_t W = mm16(ta, dU);
-            const f32x4_t nbW = -(W * b4);
-            st4(wslot(c, cw) + 16 * lane, W);
-            if (r == 0) st4(wslot(c, cw) + 1024 + 16 * g, b4);
-            // G = Diag(gC) G + Q^^T dO - K^^T diag(beta) W
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int m = 0; m < NT; ++m) {
-                    Gm[m] = mfma4(kt[e][m], nbW[e], Gm[m]);
-                    if (e == 0) rd_gc(bn, m);
-                    if (e > 0 && m < NT / 2) rd_kt(bn, e - 1, m);
-                    fence();
-                }
-#pragma unroll
-            for (int m = 0; m < NT / 2; ++m) rd_kt(bn, 3, m);
-            dOc = dOn, ta = tn, pp = pn, b4 = bn4;
-            __builtin_amdgcn_s_waitcnt(0xC07F);
+        lds_barrier();  // B1
+        for (int c = last; c >= 0; --c) {
+            const bool cp = c >= 3, st = c < last;
+            // chunk c's buffer is free; chunk c - 2 has landed at the end (the newest copies and
+            // this iteration's stores may be in flight)
+            if (cp) copies_a(c - 3);
+            lds_barrier();  // mid-chunk
+            if (cp) copies_b(c - 3);
+            if (st) store(c + 1);  // what the chains handed over in the last chunk
+            if (cp && st) wait_vm_n<G::S_NCP + G::S_NST>();
+            else if (cp) wait_vm_n<G::S_NCP>();
+            else wait_vm_n<0>();
             lds_barrier();
         }
-#pragma unroll
-        for (int m = 0; m < NT; ++m)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) gs0[sbase + static_cast<size_t>(16 * m + 4 * g + e) * D + ecol] = Gm[m][e];
+        store(0);
     }
 }
 
@@ -1535,18 +1592,28 @@ hipError_t launch_t(const BwdArgs& a, hipStream_t st) {
     unsigned char* base = reinterpret_cast<unsigned char*>(a.workspace);
     auto at = [&](size_t off) { return reinterpret_cast<float*>(base + off); };
     const InT *q = static_cast<const InT*>(a.q), *k = static_cast<const InT*>(a.k), *v = static_cast<const InT*>(a.v);
-    hipError_t e = set_lds<dec_sweep_kernel<D, InT, GE>>(DsGeo<D>::BYTES);
-    if (e != hipSuccess) return e;
+    hipError_t e;
     if ((e = set_lds<dec_span_kernel<D, InT, CHAN, GE>>(DcGeo<D>::BYTES)) != hipSuccess) return e;
     const long n_items = static_cast<long>(a.n_pairs) * n_ch;
     hipLaunchKernelGGL((dec_prep_kernel<D, InT, CHAN, false>), dim3(static_cast<unsigned>((n_items + 3) / 4)), dim3(256), 0, st,
                        q, k, a.beta, a.g, a.T, a.H, n_ch, n_items, at(o.kh), at(o.kb), at(o.qh), at(o.rec));
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    const int slots = (a.n_pairs + 7) / 8;
-    hipLaunchKernelGGL((dec_sweep_kernel<D, InT, GE>), dim3(static_cast<unsigned>(slots * (D / 32) * 8)), dim3(512),
-                       DsGeo<D>::BYTES, st, v, a.s0, a.go, a.gs, a.gv, a.gs0, at(o.kh), at(o.kb), at(o.qh), at(o.rec),
-                       at(o.w), at(o.u), at(o.s_hist), at(o.g_hist), a.n_pairs, a.T, a.H, n_ch, n_span, sl);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    // 16 columns a workgroup while that leaves at most one per CU: a chain wave then has its
+    // SIMD to itself (T 4096, D 128: 367 us against 489 at 32 pairs, 668 against 512 at 48)
+    const long slots = (a.n_pairs + 7) / 8;
+    auto sweep = [&](auto VV) {
+        constexpr int DV = decltype(VV)::value;
+        using G = DsGeo<D, DV>;
+        const hipError_t err = set_lds<dec_sweep_kernel<D, DV, InT, GE>>(G::BYTES);
+        if (err != hipSuccess) return err;
+        hipLaunchKernelGGL((dec_sweep_kernel<D, DV, InT, GE>), dim3(static_cast<unsigned>(slots * (D / DV) * 8)),
+                           dim3(G::WAVES * 64), G::BYTES, st, v, a.s0, a.go, a.gs, a.gv, a.gs0, at(o.kh), at(o.kb),
+                           at(o.qh), at(o.rec), at(o.w), at(o.u), at(o.s_hist), at(o.g_hist), a.n_pairs, a.T, a.H, n_ch,
+                           n_span, sl);
+        return hipGetLastError();
+    };
+    e = a.n_pairs * (D / 16) <= 256 ? sweep(std::integral_constant<int, 16>{}) : sweep(std::integral_constant<int, 32>{});
+    if (e != hipSuccess) return e;
     hipLaunchKernelGGL((dec_span_kernel<D, InT, CHAN, GE>), dim3(static_cast<unsigned>(a.n_pairs * n_span)), dim3(D * 4),
                        DcGeo<D>::BYTES, st, q, k, v, a.g, a.go, at(o.rec), at(o.s_hist), at(o.g_hist), at(o.w), at(o.u),
                        a.gq, a.gk, a.gbeta, a.gg, at(o.kh), at(o.kb), a.T, a.H, n_ch, n_span, sl);
