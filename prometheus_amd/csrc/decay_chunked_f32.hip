@@ -87,48 +87,6 @@ struct DecRec {
     static constexpr int FPT = 256, FGB = 512, FFLOATS = FGB + D;
 };
 
-// Lane (g, r)'s operand reads of a swizzled tile of 16 fp32 rows (f32_chunk): row(b, i) =
-// X[r][16 i + 4 g ..] and col(b, e, i) = X[4 g + e][16 i + r].  The swizzle splits into a
-// part that depends on i mod 4 and a constant one: (4 i + x) ^ (4 y + z) = 4 (i ^ y) + (x ^ z)
-// for x, z < 4, and y < 4 leaves i's upper bit alone, so 13 registers address every read.
-template <int D>
-struct TileIdx {
-    int rb, rx[4], cb[4], cx[4];  // byte offsets
-    __device__ __forceinline__ TileIdx(int r, int g) {
-        rb = 16 * (r * (D / 4) + (g ^ (r & 3)));
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            rx[k] = 64 * (k ^ (r >> 2));
-            cb[k] = 16 * ((4 * g + k) * (D / 4) + ((r >> 2) ^ k)) + 4 * (r & 3);
-            cx[k] = 64 * (k ^ g);
-        }
-    }
-    __device__ __forceinline__ f32x4_t row(const unsigned char* b, int i) const {
-        return ld4(b + rb + rx[i & 3] + 256 * (i >> 2));
-    }
-    __device__ __forceinline__ float col(const unsigned char* b, int e, int i) const {
-        return *reinterpret_cast<const float*>(b + cb[e] + cx[i & 3] + 256 * (i >> 2));
-    }
-    // Tiles i = hh + 2 j of a wave that holds every other one (TileIdx(r, g, hh)): the same, over j
-    int hx[2], hc[2];
-    __device__ __forceinline__ TileIdx(int r, int g, int hh) : TileIdx(r, g) {
-        hx[0] = hh ? rx[1] : rx[0], hx[1] = hh ? rx[3] : rx[2];
-        hc[0] = hh ? cx[1] : cx[0], hc[1] = hh ? cx[3] : cx[2];
-    }
-    __device__ __forceinline__ f32x4_t row2(const unsigned char* b, int j) const {
-        return ld4(b + rb + hx[j & 1] + 256 * (j >> 1));
-    }
-    __device__ __forceinline__ float col2(const unsigned char* b, int e, int j) const {
-        return *reinterpret_cast<const float*>(b + cb[e] + hc[j & 1] + 256 * (j >> 1));
-    }
-    // row and col for an i known only at run time
-    __device__ __forceinline__ f32x4_t roww(const unsigned char* b, int i, int r) const {
-        return ld4(b + rb + 64 * (i ^ (r >> 2)));
-    }
-    __device__ __forceinline__ float colw(const unsigned char* b, int e, int i, int g) const {
-        return *reinterpret_cast<const float*>(b + cb[e] + 64 * (i ^ g));
-    }
-};
 // One element, and four consecutive ones, of a row through a range-checked buffer (byte
 // offsets off; zeros past the range)
 template <typename InT>

@@ -206,10 +206,6 @@ ChunkedBwdWs chunked_bwd_ws(long n_pairs, int T, int D);
 bool chunked_bwd_supported(int D, int H);  // chunked_supported and H*D <= 2^23 (fp32 dO rows)
 hipError_t launch_bwd_chunked(const BwdArgs& a, hipStream_t st);
 // K9 (the fp32 chunked backward): a.workspace holds f32_bwd_ws(...).bytes bytes.
-// K9a + K9b in one launch: the state history (s_hist, U into u_out) and the gradient sweep
-// (gv, gs0, W into w_out, g_hist), from K9p's records.
-hipError_t launch_f32_hist_sweep(const BwdArgs& a, const float* t2, const float* rec, float* w_out, float* s_hist,
-                                 float* g_hist, float* u_out, hipStream_t st);
 hipError_t launch_bwd_chunked_f32(const BwdArgs& a, hipStream_t st);
 
 // K10 (decay_chunked_f32.hip): the reverse mode of the rules with a decay (a.g, a.gg,
