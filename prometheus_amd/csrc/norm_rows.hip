@@ -17,6 +17,7 @@ namespace pm {
 namespace {
 
 constexpr float kEps = 1e-6f;
+__device__ __forceinline__ float floored(float n) { return n < kEps ? kEps : n; }  // (NaN stays)
 
 template <typename T>
 __device__ __forceinline__ void load8(const T* p, float (&x)[8]);
@@ -53,13 +54,14 @@ __device__ __forceinline__ void store8<uint16_t>(uint16_t* p, const float (&x)[8
 
 // Gradient of x / max(||x||, eps) given g = dL/d(normalised row), ss = ||x||^2, dot = g . x:
 // (g - x^ (x^ . g)) / ||x|| where the norm counts (torch's clamp_min passes its gradient at
-// and above the bound), g / eps below.
+// and above the bound), g / eps below.  A NaN norm counts (the comparisons are written so), so
+// that a row with a NaN gives NaNs as elementwise tensor operations do.
 struct NormBwd {
     float inv, coef;  // gx = inv * (g - coef * x)
     __device__ __forceinline__ NormBwd(float ss, float dot) {
         const float n = sqrtf(ss);
-        const bool live = n >= kEps;
-        inv = 1.f / (live ? n : kEps);
+        const bool live = !(n < kEps);
+        inv = 1.f / floored(n);
         coef = live ? (dot * inv) * inv : 0.f;
     }
 };
@@ -79,7 +81,7 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(const T* __restrict__ q,
 #pragma unroll
         for (int e = 0; e < 8; ++e) ss = fmaf(x[e], x[e], ss);
         ss = lane_sum<LPR>(ss);  // (a row's lanes are adjacent and all in range together)
-        const float m = fmaxf(sqrtf(ss), kEps);
+        const float m = floored(sqrtf(ss));
 #pragma unroll
         for (int e = 0; e < 8; ++e) x[e] = x[e] / m;
         store8<T>((second ? kn : qn) + o, x);
@@ -134,7 +136,7 @@ __global__ __launch_bounds__(256) void norm_rows_any_kernel(const T* __restrict_
         ss = lane_sum<64>(ss);
         if constexpr (BWD) dot = lane_sum<64>(dot);
         const NormBwd nb(ss, dot);
-        const float m = fmaxf(sqrtf(ss), kEps);
+        const float m = floored(sqrtf(ss));
         T* y = (second ? ok : oq) + o;
         for (int d = lane; d < D; d += 64) {
             const float a = to_f32<T>(x[d]);

@@ -84,7 +84,8 @@ class _LinearAttention(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, go, gs):
-        qd, kd, vd, sd = ctx.saved_tensors
+        # (contiguous again: saved-tensor hooks may hand back another layout)
+        qd, kd, vd, sd = (None if x is None else x.contiguous() for x in ctx.saved_tensors)
         batch, seq, heads, dim = qd.shape
         f32 = torch.float32
         with torch.cuda.device(qd.device), _native.use_knobs(*ctx.knobs):

@@ -120,3 +120,31 @@ def test_linear_attention_backward_of_zero_and_tiny_rows():
         a = a.cpu().numpy()
         assert_f32_parity(a[:, rows], e[:, rows], name, scaled=True)
         assert_f32_parity(a[:, ~rows], e[:, ~rows], name + " small rows", scaled=True)
+
+
+@pytest.mark.parametrize("dim", [16, 64, 128])
+def test_linear_attention_backward_of_a_nan_row(dim):
+    """A query row with one NaN: its whole gradient row is NaN, as the elementwise normalisation's
+    reverse gives it, and only the rows of that head can be affected."""
+    shape = (1, 20, 2, dim)
+    x = synth.fwd_inputs(shape, seed=dim, dtype="fp32", normalize=False)
+    q = x.q.copy()
+    q[0, 19, 1, 3] = np.nan
+    leaves = [_f(a).requires_grad_(True) for a in (q, x.k, x.v)]
+    o, _ = model.linear_attention(*leaves)
+    gq, gk, gv = torch.autograd.grad(o, leaves, torch.ones_like(o))
+    assert gq[0, 19, 1].isnan().all()
+    assert all(t[:, :, 0].isfinite().all() for t in (gq, gk, gv))
+
+
+def test_linear_attention_backward_under_saved_tensor_hooks():
+    """Saved tensors that come back in another memory layout give the same gradients."""
+    shape = (2, 37, 3, 64)
+    x = synth.fwd_inputs(shape, seed=4, dtype="fp32", normalize=False)
+    leaves = [_f(a).requires_grad_(True) for a in (x.q, x.k, x.v)]
+    go = torch.randn(shape, device="cuda")
+    exp = torch.autograd.grad(model.linear_attention(*leaves)[0], leaves, go)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.transpose(1, 2).contiguous(), lambda t: t.transpose(1, 2)):
+        o = model.linear_attention(*leaves)[0]
+    for a, e in zip(torch.autograd.grad(o, leaves, go), exp):
+        assert torch.equal(a, e)
