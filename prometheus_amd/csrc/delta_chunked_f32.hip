@@ -24,17 +24,15 @@
 // as products of accumulators with transposed accumulators.  It writes (T'')^T as
 // accumulator registers, 1 KiB per chunk: the A operand of U = T'' X, lane-linear.
 //
-// K7 (recurrence): one workgroup per (sequence, head, d_v tile of DV columns) with DV/16
-// chain waves and as many output waves.  Chain wave w owns the S columns col0 + 16 w +
-// [0, 16) as D/16 accumulator tiles and runs chunk i (X, U, S: 68 MFMAs at D = 128),
-// handing S_i (before its update) and U_i to output wave w through LDS; output wave w
-// runs chunk i - 1 (Y = Q S, P^T = K Q^T, O = Y + P U: 68 MFMAs at D = 128, as many as
-// the chain's) and stores O.  Products of one accumulator are spread over several
-// accumulators (a dependent MFMA waits for its predecessor's result), summed at the end.
-// HBM -> LDS copies (buffer_load ... lds) run two chunks ahead: the output waves copy K
-// and Q rows, the chain waves their V columns and (wave 0) T''^T.  One LDS-only barrier
-// per chunk.
-
+// K7 (recurrence): one workgroup per (sequence, head, d_v tile of DV columns).  Per 16 columns,
+// two chain waves hold every other 16-row tile of S each (and half of every product over or
+// onto d: X = K S in two halves, exchanged through LDS and added by both, S += K^T U on the
+// own rows), 36 products a chunk at D = 128; an output wave forms Y = Q S one chunk behind and
+// O = Y + P U two behind.  One wave builds P^T = K Q^T for all and issues every HBM -> LDS
+// copy (buffer_load ... lds) two chunks ahead.  One LDS-only barrier per chunk.
+// The chain bounds it: with one wave per 16 columns (68 products, the output wave as many with
+// P^T) 32 pairs of T 1024 took 113 us at D = 128 and 76 at D = 64, now 72 and 51; 128 pairs of
+// D = 128, where the MFMA pipes of every CU are shared, 208, now 195.
 #include <type_traits>
 
 #include "pm_cdna4.h"
@@ -194,8 +192,9 @@ __global__ __launch_bounds__(256) void delta_f32_prep_kernel(const float* __rest
 // ---------------------------------------------------------------- K7
 template <int D, int DV, bool NORM>
 struct F32Geo {
-    static constexpr int NCW = DV / 16;            // chain waves 0 .. NCW-1, output waves NCW ..
-    static constexpr int NT = D / 16;              // S accumulator tiles per chain wave
+    static constexpr int NCW = DV / 16;            // 16-column blocks: two chain waves and an output wave each
+    static constexpr int WAVES = 3 * NCW + 1;      // chain 0 .., output 2 NCW .., the last P^T and copies
+    static constexpr int NT = D / 16;              // S accumulator tiles per block
     static constexpr int NI = kC16 * D * 4 / 1024; // 1 KiB copies per K or Q tile
     static constexpr int NB = 4;        // rotating chunk buffers
     // one chunk buffer: K rows, Q rows, (T'')^T, V columns of each chain wave
@@ -208,18 +207,18 @@ struct F32Geo {
     static constexpr int OFF_U = OFF_S + 2 * NCW * NT * 1024;  // 2 slots x NCW KiB: U_i
     static constexpr int PSLOT = NORM ? 1024 + 64 : 1024;                   // P^T, then the queries' scales
     static constexpr int OFF_P = OFF_U + 2 * NCW * 1024;       // 2 slots: P^T of a chunk
-    static constexpr int BYTES = OFF_P + 2 * PSLOT;
-    // the last output wave (the copy wave) issues every copy of a chunk: K and Q rows,
+    static constexpr int OFF_X = OFF_P + 2 * PSLOT;            // 2 slots x NCW x 2 halves of X
+    static constexpr int BYTES = OFF_X + 4096 * NCW;
+    // the last wave issues every copy of a chunk: K and Q rows,
     // (T'')^T and the V columns of each chain wave
     static constexpr int NCP = 2 * NI + 1 + NCW + (NORM ? 1 : 0);
-    static constexpr int NST = 4;  // O stores per output wave per chunk
     static_assert(D == 64 || D == 128, "D");
     static_assert(DV == 16 || DV == 32, "DV");
-    static_assert(BYTES <= 160 * 1024 && NCP + NST <= 63, "LDS / vmcnt");
+    static_assert(BYTES <= 160 * 1024 && NCP <= 63, "LDS / vmcnt");
 };
 
 template <int D, int DV, bool OUT_BF16, bool NORM>
-__global__ __launch_bounds__(DV == 32 ? 256 : 128) void delta_f32_kernel(
+__global__ __launch_bounds__((F32Geo<D, DV, NORM>::WAVES * 64)) void delta_f32_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
     const float* __restrict__ s0, void* __restrict__ o_out, float* __restrict__ s_out,
     const int32_t* __restrict__ cu_seqlens, const float* __restrict__ ws, int n_pairs, int T, int H,
@@ -228,7 +227,6 @@ __global__ __launch_bounds__(DV == 32 ? 256 : 128) void delta_f32_kernel(
     using G = F32Geo<D, DV, NORM>;
     constexpr int NCW = G::NCW, NT = G::NT;
     constexpr int NCP = G::NCP;  // copies per chunk
-    constexpr int NST = G::NST;  // O stores per output wave per chunk
     constexpr int WSF = ws_floats<NORM>();
     const int w = static_cast<int>(uniform(static_cast<unsigned>(threadIdx.x >> 6)));
 
@@ -257,10 +255,8 @@ __global__ __launch_bounds__(DV == 32 ? 256 : 128) void delta_f32_kernel(
 
     const int lane = threadIdx.x & 63;
     const int r = lane & 15, g = lane >> 4;
-    const bool chain = w < NCW;
-    const int cw = chain ? w : w - NCW;  // the 16 columns this wave works on
-    const bool p_wave = w == NCW;         // builds P^T for every output wave
-    const bool copy_wave = w == 2 * NCW - 1;
+    const bool chain = w < 2 * NCW, copy_wave = w == 3 * NCW;
+    const int cw = chain ? w >> 1 : w - 2 * NCW;  // the 16 columns this wave works on
     const size_t tstride = static_cast<size_t>(H) * D;
     const size_t sbase = static_cast<size_t>(pair) * D * D;
     const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
@@ -309,136 +305,139 @@ __global__ __launch_bounds__(DV == 32 ? 256 : 128) void delta_f32_kernel(
 #pragma unroll
         for (int j = 0; j < NCW; ++j) copy_v(c, j, b + G::B_V + 1024 * j);
     };
-    // the copy wave: wait until the next chunk's copies have landed, with the operations
-    // issued after them (this and the last iteration's O stores, the copies of the chunk
-    // after next) possibly in flight
-    auto wait_next = [&](bool extra_stores, bool extra_copies) __attribute__((always_inline)) {
-        if (extra_copies && extra_stores) wait_vm_n<NCP + NST>();
-        else if (extra_copies) wait_vm_n<NCP>();
-        else if (extra_stores) wait_vm_n<NST>();
-        else wait_vm_n<0>();
+    // P^T of chunk c (registers: q_r . k_{4 g + e}) into its slot, kept for i <= j (lower_incl P);
+    // normalised mode: the queries' scales 1 / max(||q||, 1e-6) beside it (qss: this lane's
+    // part of ||q_r||^2; a row's four slices are lanes r, r + 16, r + 32, r + 48)
+    auto store_p = [&](int c, f32x4_t pq, float qss) __attribute__((always_inline)) {
+        f32x4_t pt;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) pt[e] = (4 * g + e <= r) ? pq[e] : 0.f;
+        st4(pslot(c) + 16 * lane, pt);
+        if constexpr (NORM) {
+            float ss = qss;
+            ss += __shfl_xor(ss, 16);
+            ss += __shfl_xor(ss, 32);
+            if (g == 0) reinterpret_cast<float*>(pslot(c) + 1024)[r] = 1.f / fmaxf(sqrtf(ss), 1e-6f);
+        }
+    };
+    // O = Y + P U of chunk c, stored: lane (g, r) holds O[4 g + e][16 cw + r]; rows past the end
+    // are dropped by the range-checked stores
+    auto store_o = [&](int c, f32x4_t y) __attribute__((always_inline)) {
+        constexpr int ES = OUT_BF16 ? 2 : 4;
+        const f32x4_t pt = ld4(pslot(c) + 16 * lane);
+        const f32x4_t u = ld4(uslot(c, cw) + 16 * lane);
+        f32x4_t O = mm16(pt, u, y);
+        if constexpr (NORM) O = O * ld4(pslot(c) + 1024 + 16 * g);  // rows scaled by the queries' scales
+        const int clen = min(kC16, len - c * kC16);
+        const size_t rowe = static_cast<size_t>(tok0 + c * kC16) * tstride + static_cast<size_t>(h) * D + col0 + 16 * cw;
+        const __amdgpu_buffer_rsrc_t ro = make_rsrc(static_cast<unsigned char*>(o_out) + rowe * ES,
+                                                    static_cast<unsigned>(((clen - 1) * tstride + 16) * ES));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const unsigned off = static_cast<unsigned>(((4 * g + e) * tstride + r) * ES);
+            if constexpr (OUT_BF16)
+                __builtin_amdgcn_raw_buffer_store_b16(f32_to_bf16(O[e]), ro, off, 0, 0);
+            else
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(O[e]), ro, off, 0, 0);
+        }
     };
 
     if (n_chunks > 0) {
         if (copy_wave) {
             copies(0);
             if (n_chunks > 1) copies(1);
-            wait_next(false, n_chunks > 1);
+            if (n_chunks > 1) wait_vm_n<NCP>();
+            else wait_vm_n<0>();
         }
         lds_barrier();  // B0
     }
 
     if (chain) {
-        // ============ chain wave: S columns col0 + 16 cw + [0, 16) ============
-        const int ecol = col0 + 16 * cw + r;
-        f32x4_t S[NT];
+        // ============ chain wave hh of two: S columns col0 + 16 cw + [0, 16), tiles m = hh + 2 j ============
+        // Phase p (up to barrier M_p) finishes chunk p - 1 (the other wave's half of X, U, S +=
+        // K^T U) and forms this wave's half of X of chunk p: one barrier a chunk.  Every LDS
+        // read is issued ahead of the products or behind one of them.
+        constexpr int NH = NT / 2;
+        const int hh = w & 1, ecol = col0 + 16 * cw + r;
+        const TileIdx<D> ix(r, g, hh);
+        f32x4_t S[NH];
 #pragma unroll
-        for (int m = 0; m < NT; ++m)
+        for (int j = 0; j < NH; ++j)
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                S[m][e] = s0 ? s0[sbase + static_cast<size_t>(16 * m + 4 * g + e) * D + ecol] : 0.f;
-        // s_waitcnt vmcnt(0) as the intrinsic, which the compiler's wait insertion sees: with
-        // the S0 loads settled here it puts no wait for them inside the loop, where a
-        // vmcnt(0) would also wait for the copies of two chunks ahead
-        __builtin_amdgcn_s_waitcnt(0x0F70);
-        // Iteration i (after barrier B_i) finishes chunk i - 1 (S += K^T U, its K^T operands
-        // read before the barrier) and runs chunk i up to U, so the state update of one chunk
-        // and X of the next run back to back on the MFMA pipe; the LDS reads of each phase
-        // are issued ahead of it, in groups fenced by sched_barrier (left to itself the
-        // compiler reads each operand right before its MFMA and waits out the LDS latency).
-        float kt[4][NT];  // K^T operand of chunk i - 1: K[4 g + e][16 m + r]
-        f32x4_t Up = zero;
-        for (int i = 0; i <= n_chunks; ++i) {
-            const bool run = i < n_chunks;
-            const unsigned char* b = buf(run ? i : 0);
-            const float* Vf = reinterpret_cast<const float*>(b + G::B_V + 1024 * cw);
-            f32x4_t kf[NT], xa[4] = {zero, zero, zero, zero}, tt = zero, vr = zero;
-            if (run) {
+                S[j][e] = s0 ? s0[sbase + static_cast<size_t>(16 * (hh + 2 * j) + 4 * g + e) * D + ecol] : 0.f;
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), seen by the compiler: no wait for these in the loop
+        __builtin_amdgcn_s_setprio(3);
+        unsigned char* const xs = smem + G::OFF_X + 2048 * cw + 16 * lane;
+        float kt[4][NH] = {};
+        f32x4_t kf[NH], half = zero, tt = zero, vr = zero, skc = zero;
+        if (n_chunks > 0) {
+            for (int p = 0; p <= n_chunks; ++p) {
+                const bool run = p < n_chunks;
+                const unsigned char* b = buf(run ? p : n_chunks - 1);  // (past the end: read, unused)
+                const f32x4_t other = ld4(xs + ((p & 1) ^ 1) * 2048 * NCW + (hh ^ 1) * 1024);
+                f32x4_t tn, vn, sn = zero;
 #pragma unroll
-                for (int m = 0; m < NT; ++m) kf[m] = ld4(b + G::B_K + 16 * f32_chunk<D>(r, 4 * m + g));
-#pragma unroll
-                for (int e = 0; e < 4; ++e) vr[e] = Vf[(4 * g + e) * 16 + r];
-                tt = ld4(b + G::B_T + 16 * lane);
-            }
-            fence();
-            // S += K^T U of chunk i - 1 (consecutive MFMAs go to different tiles)
-            if (i > 0) {
+                for (int j = 0; j < NH; ++j) kf[j] = ix.row2(b + G::B_K, j);
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
+                    vn[e] = reinterpret_cast<const float*>(b + G::B_V + 1024 * cw)[(4 * g + e) * 16 + r];
+                tn = ld4(b + G::B_T + 16 * lane);
+                if constexpr (NORM) sn = ld4(b + G::B_T + 1024 + 16 * g);
+                fence();
+                if (p > 0) {
+                    f32x4_t X = half + other;
+                    if constexpr (NORM) X = X * skc - vr;
+                    f32x4_t U = mm16(tt, X);
+                    if constexpr (NORM) U = U * skc;
+                    if (hh == 0) st4(uslot(p - 1, cw) + 16 * lane, U);
 #pragma unroll
-                    for (int m = 0; m < NT; ++m) S[m] = mfma4(kt[e][m], Up[e], S[m]);
-            }
-            if (!run) break;
-            fence();
-            if constexpr (!NORM) xa[0] = -vr;  // (negated only here: a use right after the read would wait for it)
-            // X = K S - V (accumulator e takes the steps (m, e))
+                    for (int e = 0; e < 4; ++e)
 #pragma unroll
-            for (int m = 0; m < NT; ++m)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) xa[e] = mfma4(kf[m][e], S[m][e], xa[e]);
-            f32x4_t X = (xa[0] + xa[1]) + (xa[2] + xa[3]);
-            // normalised mode: X = diag(s) K S - V with s the keys' scales (rows 4 g + e)
-            f32x4_t skc = {1.f, 1.f, 1.f, 1.f};
-            if constexpr (NORM) {
-                skc = ld4(b + G::B_T + 1024 + 16 * g);
-                X = X * skc - vr;
-            }
-            // U = T'' X (normalised mode: the state update and P U take diag(s) U)
-            Up = mm16(tt, X);
-            if constexpr (NORM) Up = Up * skc;
-            // hand S_i and U_i to the output wave
-            unsigned char* ss = sslot(i, cw);
-#pragma unroll
-            for (int m = 0; m < NT; ++m) st4(ss + 1024 * m + 16 * lane, S[m]);
-            st4(uslot(i, cw) + 16 * lane, Up);
-            // K^T operand of chunk i, for the next iteration's state update
-            const float* Kf = reinterpret_cast<const float*>(b + G::B_K);
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int m = 0; m < NT; ++m) {
-                    const int t = 4 * g + e, d = 16 * m + r;
-                    kt[e][m] = Kf[4 * f32_chunk<D>(t, d >> 2) + (d & 3)];
+                        for (int j = 0; j < NH; ++j) S[j] = mfma4(kt[e][j], U[e], S[j]);
                 }
-            // lgkmcnt(0) as the intrinsic, so that the compiler knows kt has landed and puts
-            // no wait for it after the barrier (where it would also wait for the new reads)
-            __builtin_amdgcn_s_waitcnt(0xC07F);
-            lds_barrier();
+                fence();
+                if (run) {
+                    tt = tn, vr = vn, skc = sn;
+                    f32x4_t xa[4] = {zero, zero, zero, zero};
+                    if constexpr (!NORM) {
+                        if (hh == 0) xa[0] = -vr;
+                    }
+                    unsigned char* ss = sslot(p, cw) + 16 * lane;
+#pragma unroll
+                    for (int j = 0; j < NH; ++j)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            xa[e] = mfma4(kf[j][e], S[j][e], xa[e]);
+                            kt[e][j] = ix.col2(b + G::B_K, e, j);
+                            if (e == 3) st4(ss + 1024 * (hh + 2 * j), S[j]);
+                            fence();
+                        }
+                    half = (xa[0] + xa[1]) + (xa[2] + xa[3]);
+                    st4(xs + (p & 1) * 2048 * NCW + hh * 1024, half);
+                }
+                __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), seen by the compiler
+                lds_barrier();                       // M_p
+            }
         }
 #pragma unroll
-        for (int m = 0; m < NT; ++m)
+        for (int j = 0; j < NH; ++j)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) s_out[sbase + static_cast<size_t>(16 * m + 4 * g + e) * D + ecol] = S[m][e];
-    } else if (n_chunks > 0) {
-        // ============ output waves: O of chunk i - 1 for the columns of chain wave cw ============
-        // Iteration i: the P wave builds P^T of chunk i (for the next iteration, into LDS);
-        // every output wave forms Y = Q S and O = Y + P U of chunk i - 1 and stores O; the
-        // copy wave issues chunk i + 2's copies.
-        constexpr int ES = OUT_BF16 ? 2 : 4;
-        for (int i = 0; i <= n_chunks; ++i) {
-            const bool cp = copy_wave && i + 2 < n_chunks;
-            if (cp) copies(i + 2);
-            const bool st = i >= 1;
-            const bool pp = p_wave && i < n_chunks;
-            // accumulator e takes the steps (m, e); each tile's operand reads are issued two
-            // tiles ahead.  One straight-line body per combination of the two products.
-            f32x4_t ya[4] = {zero, zero, zero, zero}, pa[4] = {zero, zero, zero, zero};
-            float qss = 0.f;  // normalised mode: this lane's part of ||q_r||^2 of chunk i
-            const unsigned char* by = buf(st ? i - 1 : 0);
-            const unsigned char* bp = buf(i);
-            const unsigned char* ss = sslot(st ? i - 1 : 0, cw);
-            auto products = [&](auto ST, auto PP) __attribute__((always_inline)) {
-                constexpr bool DO_Y = decltype(ST)::value, DO_P = decltype(PP)::value;
-                f32x4_t qy[NT], sc[NT], qp[NT], kp[NT];
+            for (int e = 0; e < 4; ++e)
+                s_out[sbase + static_cast<size_t>(16 * (hh + 2 * j) + 4 * g + e) * D + ecol] = S[j][e];
+    } else if (n_chunks > 0 && copy_wave) {
+        // ============ P and copy wave: phase p builds P^T of chunk p - 1, copies chunk p + 2 ============
+        for (int p = 0; p <= n_chunks; ++p) {
+            const bool cp = p + 2 < n_chunks;
+            if (cp) copies(p + 2);
+            if (p >= 1) {
+                const int c = p - 1;
+                const unsigned char* b = buf(c);
+                f32x4_t pa[4] = {zero, zero, zero, zero}, qp[NT], kp[NT];
+                float qss = 0.f;  // normalised mode: this lane's part of ||q_r||^2
                 auto rd = [&](int m) __attribute__((always_inline)) {
-                    if constexpr (DO_Y) {
-                        qy[m] = ld4(by + G::B_Q + 16 * f32_chunk<D>(r, 4 * m + g));
-                        sc[m] = ld4(ss + 1024 * m + 16 * lane);
-                    }
-                    if constexpr (DO_P) {
-                        qp[m] = ld4(bp + G::B_Q + 16 * f32_chunk<D>(r, 4 * m + g));
-                        kp[m] = ld4(bp + G::B_K + 16 * f32_chunk<D>(r, 4 * m + g));
-                    }
+                    qp[m] = ld4(b + G::B_Q + 16 * f32_chunk<D>(r, 4 * m + g));
+                    kp[m] = ld4(b + G::B_K + 16 * f32_chunk<D>(r, 4 * m + g));
                 };
                 rd(0);
                 rd(1);
@@ -448,60 +447,45 @@ __global__ __launch_bounds__(DV == 32 ? 256 : 128) void delta_f32_kernel(
                     if (m + 2 < NT) rd(m + 2);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        if constexpr (DO_Y) ya[e] = mfma4(qy[m][e], sc[m][e], ya[e]);
-                        if constexpr (DO_P) pa[e] = mfma4(kp[m][e], qp[m][e], pa[e]);
-                        if constexpr (DO_P && NORM) qss = fmaf(qp[m][e], qp[m][e], qss);
+                        pa[e] = mfma4(kp[m][e], qp[m][e], pa[e]);
+                        if constexpr (NORM) qss = fmaf(qp[m][e], qp[m][e], qss);
                     }
                     fence();
                 }
-            };
-            using T_ = std::true_type;
-            using F_ = std::false_type;
-            if (st && pp) products(T_{}, T_{});
-            else if (st) products(T_{}, F_{});
-            else if (pp) products(F_{}, T_{});
-            if (pp) {
-                // P^T[i][j] = P[j][i] = q_j . k_i, kept for i <= j (lower_incl P)
-                const f32x4_t pq = (pa[0] + pa[1]) + (pa[2] + pa[3]);
-                f32x4_t pt;
+                store_p(c, (pa[0] + pa[1]) + (pa[2] + pa[3]), qss);
+            }
+            // chunk p + 1 has landed; the copies of the one after may be in flight
+            if (cp) wait_vm_n<NCP>();
+            else wait_vm_n<0>();
+            lds_barrier();
+        }
+    } else if (n_chunks > 0) {
+        // ============ output wave: phase p finishes O of chunk p - 2 and forms Y = Q S of chunk p - 1 ============
+        f32x4_t y = zero;
+        for (int p = 0; p <= n_chunks + 1; ++p) {
+            if (p >= 2) store_o(p - 2, y);
+            if (p > n_chunks) break;
+            if (p >= 1) {
+                const unsigned char* b = buf(p - 1);
+                const unsigned char* ss = sslot(p - 1, cw);
+                f32x4_t ya[4] = {zero, zero, zero, zero}, qy[NT], sc[NT];
+                auto rd = [&](int m) __attribute__((always_inline)) {
+                    qy[m] = ld4(b + G::B_Q + 16 * f32_chunk<D>(r, 4 * m + g));
+                    sc[m] = ld4(ss + 1024 * m + 16 * lane);
+                };
+                rd(0);
+                rd(1);
+                fence();
 #pragma unroll
-                for (int e = 0; e < 4; ++e) pt[e] = (4 * g + e <= r) ? pq[e] : 0.f;
-                st4(pslot(i) + 16 * lane, pt);
-                if constexpr (NORM) {
-                    // the queries' scales 1 / max(||q||, 1e-6) of chunk i, from the Q operands
-                    // just used (a row's four slices are lanes r, r + 16, r + 32, r + 48)
-                    float ss = qss;
-                    ss += __shfl_xor(ss, 16);
-                    ss += __shfl_xor(ss, 32);
-                    if (g == 0) reinterpret_cast<float*>(pslot(i) + 1024)[r] = 1.f / fmaxf(sqrtf(ss), 1e-6f);
-                }
-            }
-            if (st) {
-                const int c = i - 1;
-                const f32x4_t pt = ld4(pslot(c) + 16 * lane);
-                const f32x4_t u = ld4(uslot(c, cw) + 16 * lane);
-                f32x4_t O = mm16(pt, u, (ya[0] + ya[1]) + (ya[2] + ya[3]));
-                if constexpr (NORM) O = O * ld4(pslot(c) + 1024 + 16 * g);  // rows scaled by the queries' scales
-                // lane (g, r) holds O[4 g + e][16 cw + r]; rows past the end are dropped by
-                // the range-checked stores
-                const int clen = min(kC16, len - c * kC16);
-                const size_t rowe = static_cast<size_t>(tok0 + c * kC16) * tstride + static_cast<size_t>(h) * D +
-                                    col0 + 16 * cw;
-                const __amdgpu_buffer_rsrc_t ro = make_rsrc(static_cast<unsigned char*>(o_out) + rowe * ES,
-                                                            static_cast<unsigned>(((clen - 1) * tstride + 16) * ES));
+                for (int m = 0; m < NT; ++m) {
+                    if (m + 2 < NT) rd(m + 2);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const unsigned off = static_cast<unsigned>(((4 * g + e) * tstride + r) * ES);
-                    if constexpr (OUT_BF16)
-                        __builtin_amdgcn_raw_buffer_store_b16(f32_to_bf16(O[e]), ro, off, 0, 0);
-                    else
-                        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(O[e]), ro, off, 0, 0);
+                    for (int e = 0; e < 4; ++e) ya[e] = mfma4(qy[m][e], sc[m][e], ya[e]);
+                    fence();
                 }
+                y = (ya[0] + ya[1]) + (ya[2] + ya[3]);
             }
-            if (i < n_chunks) {
-                if (copy_wave && i + 1 < n_chunks) wait_next(st, cp);
-                lds_barrier();
-            }
+            lds_barrier();
         }
     }
 }
@@ -539,7 +523,7 @@ hipError_t launch_f32_t(const ChunkedF32Args& a, float* ws, hipStream_t st) {
     if (e != hipSuccess) return e;
     const int n_tiles = D / DV;
     const int slots = (n_pairs + 7) / 8;
-    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(slots * n_tiles * 8)), dim3(128 * G::NCW), G::BYTES, st, q, k,
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(slots * n_tiles * 8)), dim3(G::WAVES * 64), G::BYTES, st, q, k,
                        v, a.s0, a.o, a.s_out, a.cu_seqlens, ws, n_pairs, a.T, a.H, n_tiles, n_slot);
     return hipGetLastError();
 }
@@ -560,10 +544,15 @@ size_t chunked_f32_ws_bytes(bool varlen, int n_seq, int T, int H, bool norm) {
     return static_cast<size_t>(rows) * f32_n_slot(varlen, T, n_seq) * (norm ? ws_floats<true>() : ws_floats<false>()) * 4;
 }
 
+// D = 128: 16 columns a workgroup while that leaves at most one per CU (LDS holds one), so that
+// a chain wave has its SIMD to itself; a second round costs more than the wider form (T 1024:
+// 32 pairs 72 against 95 us, 33 pairs 126 against 97, 63 pairs 128 against 100).  D = 64: two
+// fit a CU, and the two forms are level from 65 to 128 pairs (72 against 73 us at 96) before
+// the narrow one needs a second round (200 pairs 135 against 115).
 int chunked_f32_pick_tile(int D, long n_pairs, int requested) {
     if (requested == 16 || requested == 32) return requested;
     if (requested == 64) return 32;
-    return n_pairs * (D / 32) >= 256 ? 32 : 16;
+    return n_pairs > (D == 128 ? 32 : 127) ? 32 : 16;
 }
 
 hipError_t launch_f32_bwd_prep(const float* q, const float* k, const float* beta, int n_pairs, int T, int H, int D,
