@@ -337,25 +337,30 @@ __global__ __launch_bounds__(256) void dec_prep_kernel(
 }
 
 // ---------------------------------------------------------------- K10f
-// The forward (fp32 q/k/v): one workgroup per (b, h, DV columns of d_v), DV/16 chain waves as
-// K10s's state chain and as many output waves one chunk behind (Y = Q^ S, O = Y + P U, stores),
-// which the chain hands S and U through LDS.  The last output wave copies every chunk two
-// ahead through four buffers; one barrier per chunk.
+// The forward (fp32 q/k/v): one workgroup per (b, h, DV columns of d_v).  Per 16 columns two
+// chain waves as K10s's state chain and an output wave (Y = Q^ S one chunk behind, O = Y + P U
+// two behind, stores), which the chains hand S and U through LDS.  The last wave copies every
+// chunk two ahead through four buffers; one barrier per chunk, at which the halves of X are
+// exchanged.
+// The chain bounds it: one wave per 16 columns (68 products in sequence at D = 128) took 108 us
+// at 32 pairs of T 1024, D = 128, per-head gate, and 63 at 2 pairs of D = 64; now 78 and 51.  At
+// many pairs of D = 64 the shared pipes cost a little (128 pairs 104, now 108).
 template <int D, int DV>
 struct DfGeo {
     static constexpr int NCW = DV / 16, NT = D / 16, NI = kC16 * D * 4 / 1024, TILE = kC16 * D * 4, NB = 4;
+    static constexpr int WAVES = 3 * NCW + 1;
     static constexpr int B_KH = 0, B_KB = TILE, B_QH = 2 * TILE, B_T = 3 * TILE, B_P = B_T + 1024, B_V = B_P + 1024;
     static constexpr int B_G = B_V + NCW * 1024, BUF = B_G + D * 4;
     static constexpr int OFF_S = NB * BUF;                    // 2 slots x NCW: S of a chunk's start
     static constexpr int OFF_U = OFF_S + 2 * NCW * NT * 1024; // 2 slots x NCW: U
-    static constexpr int BYTES = OFF_U + 2 * NCW * 1024;
+    static constexpr int OFF_X = OFF_U + 2 * NCW * 1024;      // 2 slots x NCW x 2 halves of X
+    static constexpr int BYTES = OFF_X + 4096 * NCW;
     static constexpr int NCP = 3 * NI + 2 + NCW + D / 64;     // copies per chunk
-    static constexpr int NST = 4;                             // O stores per output wave per chunk
-    static_assert(BYTES <= 160 * 1024 && NCP + NST <= 63, "LDS / vmcnt");
+    static_assert(BYTES <= 160 * 1024 && NCP <= 63, "LDS / vmcnt");
 };
 
 template <int D, int DV, bool OUT_BF16>
-__global__ __launch_bounds__(DV == 32 ? 256 : 128) void dec_fwd_kernel(
+__global__ __launch_bounds__((DfGeo<D, DV>::WAVES * 64)) void dec_fwd_kernel(
     const float* __restrict__ v, const float* __restrict__ s0, void* __restrict__ o_out, float* __restrict__ s_out,
     const float* __restrict__ kh, const float* __restrict__ kb, const float* __restrict__ qh,
     const float* __restrict__ rec, int n_pairs, int T, int H, int n_ch) {
@@ -375,7 +380,6 @@ __global__ __launch_bounds__(DV == 32 ? 256 : 128) void dec_fwd_kernel(
     const size_t tstride = static_cast<size_t>(H) * D;
     const size_t sbase = static_cast<size_t>(pair) * D * D;
     const size_t item0 = static_cast<size_t>(pair) * n_ch;
-    const TileIdx<D> ix(r, g);
     auto buf = [=](int c) { return smem + (c % G::NB) * G::BUF; };
     auto sslot = [=](int c, int which) { return smem + G::OFF_S + ((c & 1) * NCW + which) * NT * 1024; };
     auto uslot = [=](int c, int which) { return smem + G::OFF_U + ((c & 1) * NCW + which) * 1024; };
@@ -384,78 +388,117 @@ __global__ __launch_bounds__(DV == 32 ? 256 : 128) void dec_fwd_kernel(
         return static_cast<unsigned>((min(kC16, T - c * kC16) - 1) * tstride + cols);
     };
 
-    if (w < NCW) {
-        // ============ chain: S columns col0 + 16 w + [0, 16) ============
-        const int ecol = col0 + 16 * w + r;
-        f32x4_t S[NT];
+    if (w < 2 * NCW) {
+        // ============ chain wave hh of two: S columns col0 + 16 cw + [0, 16), tiles m = hh + 2 j ============
+        // Phase p (up to barrier M_p) finishes chunk p - 1 (the other wave's half of X, U, S's own
+        // rows) and forms this wave's half of X of chunk p.
+        constexpr int NH = NT / 2;
+        const int cw = w >> 1, hh = w & 1, ecol = col0 + 16 * cw + r;
+        const TileIdx<D> ix(r, g, hh);
+        f32x4_t S[NH];
 #pragma unroll
-        for (int m = 0; m < NT; ++m)
+        for (int j = 0; j < NH; ++j)
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                S[m][e] = s0 ? s0[sbase + static_cast<size_t>(16 * m + 4 * g + e) * D + ecol] : 0.f;
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), seen by the compiler
+                S[j][e] = s0 ? s0[sbase + static_cast<size_t>(16 * (hh + 2 * j) + 4 * g + e) * D + ecol] : 0.f;
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), seen by the compiler: no wait for these in the loop
         __builtin_amdgcn_s_setprio(3);
         lds_barrier();  // B0
-        f32x4_t Up = kZero4;
-        float kt[4][NT] = {};  // K-^T operand of the last chunk: K-[4 g + e][16 m + r]
-        auto rd_kt = [&](const unsigned char* b, int e, int m) __attribute__((always_inline)) {
-            kt[e][m] = ix.col(b + G::B_KB, e, m);
-            kt[e][m + NT / 2] = ix.col(b + G::B_KB, e, m + NT / 2);
-        };
-        for (int i = 0; i < n_ch; ++i) {
-            const unsigned char* b = buf(i);
-            const float* Vf = reinterpret_cast<const float*>(b + G::B_V + 1024 * w);
-            f32x4_t kf[NT], gc[NT], vr, tt;
-            // S += K-^T U of the last chunk; every LDS access behind one product (see K10s)
+        unsigned char* const xs = smem + G::OFF_X + 2048 * cw + 16 * lane;
+        float kt[4][NH] = {};  // K-^T operand of the last chunk
+        f32x4_t kf[NH], half = kZero4, tt = kZero4;
+        for (int p = 0; p <= n_ch; ++p) {
+            const bool run = p < n_ch;
+            const unsigned char* b = buf(run ? p : n_ch - 1);  // (past the end: read, unused)
+            const f32x4_t other = ld4(xs + ((p & 1) ^ 1) * 2048 * NCW + (hh ^ 1) * 1024);
+            f32x4_t tn, vr;
+#pragma unroll
+            for (int j = 0; j < NH; ++j) kf[j] = ix.row2(b + G::B_KH, j);
 #pragma unroll
             for (int e = 0; e < 4; ++e)
+                vr[e] = reinterpret_cast<const float*>(b + G::B_V + 1024 * cw)[(4 * g + e) * 16 + r];
+            tn = ld4(b + G::B_T + 16 * lane);
+            fence();
+            if (p > 0) {
+                const f32x4_t U = mm16(tt, half + other);
+                if (hh == 0) st4(uslot(p - 1, cw) + 16 * lane, U);
 #pragma unroll
-                for (int m = 0; m < NT; ++m) {
-                    S[m] = mfma4(kt[e][m], Up[e], S[m]);
-                    if (e == 0) kf[m] = ix.row(b + G::B_KH, m);
-                    if (e > 0 && m < NT / 2) rd_kt(b, e - 1, m);
-                    if (e == 1 && m >= NT / 2 && m < NT / 2 + 2) {
-                        vr[2 * (m - NT / 2)] = Vf[(4 * g + 2 * (m - NT / 2)) * 16 + r];
-                        vr[2 * (m - NT / 2) + 1] = Vf[(4 * g + 2 * (m - NT / 2) + 1) * 16 + r];
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int j = 0; j < NH; ++j) S[j] = mfma4(kt[e][j], U[e], S[j]);
+            }
+            fence();
+            if (run) {
+                tt = tn;
+                f32x4_t xa[4] = {kZero4, kZero4, kZero4, kZero4}, gc[NH];
+                if (hh == 0) xa[0] = -vr;
+                unsigned char* ss = sslot(p, cw) + 16 * lane;
+#pragma unroll
+                for (int j = 0; j < NH; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        xa[e] = mfma4(kf[j][e], S[j][e], xa[e]);
+                        kt[e][j] = ix.col2(b + G::B_KB, e, j);
+                        if (e == 1) gc[j] = ld4(b + G::B_G + 4 * (16 * (hh + 2 * j) + 4 * g));
+                        if (e == 3) st4(ss + 1024 * (hh + 2 * j), S[j]);
+                        fence();
                     }
-                    if (e == 2 && m == NT - 1) tt = ld4(b + G::B_T + 16 * lane);
-                    fence();
-                }
-            unsigned char* ss = sslot(i, w) + 16 * lane;
-            // X = K^ S - V, U = T'' X; S handed to the output wave
-            f32x4_t xa[4] = {-vr, kZero4, kZero4, kZero4};
+                half = (xa[0] + xa[1]) + (xa[2] + xa[3]);
+                st4(xs + (p & 1) * 2048 * NCW + hh * 1024, half);
 #pragma unroll
-            for (int m = 0; m < NT; ++m)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    xa[e] = mfma4(kf[m][e], S[m][e], xa[e]);
-                    const int n = 4 * m + e;
-                    if (e == 0) st4(ss + 1024 * m, S[m]);
-                    if (n < NT / 2) rd_kt(b, 3, n);
-                    if (n >= NT / 2 && n < NT / 2 + NT) gc[n - NT / 2] = ld4(b + G::B_G + 4 * (16 * (n - NT / 2) + 4 * g));
-                    fence();
-                }
-            const f32x4_t X = (xa[0] + xa[1]) + (xa[2] + xa[3]);
-            Up = mm16(tt, X);
-            st4(uslot(i, w) + 16 * lane, Up);
-#pragma unroll
-            for (int m = 0; m < NT; ++m) S[m] = gc[m] * S[m];
+                for (int j = 0; j < NH; ++j) S[j] = gc[j] * S[j];
+            }
             __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), seen by the compiler
-            lds_barrier();
+            lds_barrier();                       // M_p
         }
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
+        for (int j = 0; j < NH; ++j)
 #pragma unroll
-            for (int m = 0; m < NT; ++m) S[m] = mfma4(kt[e][m], Up[e], S[m]);
-#pragma unroll
-        for (int m = 0; m < NT; ++m)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) s_out[sbase + static_cast<size_t>(16 * m + 4 * g + e) * D + ecol] = S[m][e];
-    } else {
-        // ============ output waves: O of chunk i - 1, the chain's columns; the last copies ============
-        const int cw = w - NCW;
-        const bool copy_wave = w == 2 * NCW - 1;
+            for (int e = 0; e < 4; ++e)
+                s_out[sbase + static_cast<size_t>(16 * (hh + 2 * j) + 4 * g + e) * D + ecol] = S[j][e];
+    } else if (w < 3 * NCW) {
+        // ============ output wave: phase p finishes O of chunk p - 2 and forms Y of chunk p - 1 ============
+        const int cw = w - 2 * NCW;
         constexpr int ES = OUT_BF16 ? 2 : 4;
+        const TileIdx<D> ix(r, g);
+        f32x4_t y = kZero4, pt = kZero4;
+        lds_barrier();  // B0
+        for (int p = 0; p <= n_ch + 1; ++p) {
+            if (p >= 2) {
+                const int c = p - 2;
+                const f32x4_t O = mm16(pt, ld4(uslot(c, cw) + 16 * lane), y);
+                // lane (g, r) holds O[4 g + e][16 cw + r]; rows past the end are dropped
+                const __amdgpu_buffer_rsrc_t ro = make_rsrc(
+                    static_cast<unsigned char*>(o_out) + row0_of(c, col0 + 16 * cw) * ES, els_of(c, 16) * ES);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) put<ES>(O[e], ro, static_cast<unsigned>((4 * g + e) * tstride + r));
+            }
+            if (p > n_ch) break;
+            if (p >= 1) {
+                const unsigned char* b = buf(p - 1);
+                const unsigned char* ss = sslot(p - 1, cw) + 16 * lane;
+                f32x4_t ya[4] = {kZero4, kZero4, kZero4, kZero4}, qy[NT], sc[NT];
+                auto rd = [&](int m) __attribute__((always_inline)) {
+                    qy[m] = ix.row(b + G::B_QH, m);
+                    sc[m] = ld4(ss + 1024 * m);
+                };
+                rd(0);
+                rd(1);
+                pt = ld4(b + G::B_P + 16 * lane);
+                fence();
+#pragma unroll
+                for (int m = 0; m < NT; ++m) {
+                    if (m + 2 < NT) rd(m + 2);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) ya[e] = mfma4(qy[m][e], sc[m][e], ya[e]);
+                    fence();
+                }
+                y = (ya[0] + ya[1]) + (ya[2] + ya[3]);
+            }
+            lds_barrier();
+        }
+    } else {
+        // ============ copy wave: phase p issues chunk p + 2's copies ============
         auto copies = [=](int c) __attribute__((always_inline)) {
             unsigned char* b = buf(c);
             const float* rc = rec + (item0 + c) * R::FFLOATS;
@@ -478,55 +521,23 @@ __global__ __launch_bounds__(DV == 32 ? 256 : 128) void dec_fwd_kernel(
             for (int j = 0; j < D / 64; ++j)
                 dma4_asm(rg, uniform_ptr(b + G::B_G + 256 * j), static_cast<unsigned>(256 * j + 4 * lane));
         };
-        if (copy_wave) {
-            copies(0);
-            if (n_ch > 1) {
-                copies(1);
+        copies(0);
+        if (n_ch > 1) {
+            copies(1);
+            wait_vm_n<G::NCP>();
+        } else {
+            wait_vm_n<0>();
+        }
+        lds_barrier();  // B0
+        for (int p = 0; p <= n_ch; ++p) {
+            // chunk p + 1 has landed; the copies of the one after may be in flight
+            if (p + 2 < n_ch) {
+                copies(p + 2);
                 wait_vm_n<G::NCP>();
             } else {
                 wait_vm_n<0>();
             }
-        }
-        lds_barrier();  // B0
-        for (int i = 0; i <= n_ch; ++i) {
-            const bool cp = copy_wave && i + 2 < n_ch, st = i >= 1;
-            if (cp) copies(i + 2);
-            if (st) {
-                const int c = i - 1;
-                const unsigned char* b = buf(c);
-                const unsigned char* ss = sslot(c, cw) + 16 * lane;
-                f32x4_t ya[4] = {kZero4, kZero4, kZero4, kZero4}, qy[NT], sc[NT];
-                auto rd = [&](int m) __attribute__((always_inline)) {
-                    qy[m] = ix.row(b + G::B_QH, m);
-                    sc[m] = ld4(ss + 1024 * m);
-                };
-                rd(0);
-                rd(1);
-                fence();
-#pragma unroll
-                for (int m = 0; m < NT; ++m) {
-                    if (m + 2 < NT) rd(m + 2);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) ya[e] = mfma4(qy[m][e], sc[m][e], ya[e]);
-                    fence();
-                }
-                const f32x4_t pt = ld4(b + G::B_P + 16 * lane), u = ld4(uslot(c, cw) + 16 * lane);
-                const f32x4_t O = mm16(pt, u, (ya[0] + ya[1]) + (ya[2] + ya[3]));
-                // lane (g, r) holds O[4 g + e][16 cw + r]; rows past the end are dropped
-                const __amdgpu_buffer_rsrc_t ro = make_rsrc(
-                    static_cast<unsigned char*>(o_out) + row0_of(c, col0 + 16 * cw) * ES, els_of(c, 16) * ES);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) put<ES>(O[e], ro, static_cast<unsigned>((4 * g + e) * tstride + r));
-            }
-            if (i < n_ch) {
-                // chunk i + 1 has landed; the newest copies and this iteration's stores may be in flight
-                if (copy_wave && i + 1 < n_ch) {
-                    if (cp && st) wait_vm_n<G::NCP + G::NST>();
-                    else if (cp) wait_vm_n<G::NCP>();
-                    else wait_vm_n<0>();
-                }
-                lds_barrier();
-            }
+            lds_barrier();
         }
     }
 }
@@ -1537,7 +1548,7 @@ hipError_t launch_fwd_t(const DecayFwdArgs& a, hipStream_t st) {
     using G = DfGeo<D, DV>;
     if ((e = set_lds<dec_fwd_kernel<D, DV, OB>>(G::BYTES)) != hipSuccess) return e;
     const int slots = (n_pairs + 7) / 8;
-    hipLaunchKernelGGL((dec_fwd_kernel<D, DV, OB>), dim3(static_cast<unsigned>(slots * (D / DV) * 8)), dim3(128 * G::NCW),
+    hipLaunchKernelGGL((dec_fwd_kernel<D, DV, OB>), dim3(static_cast<unsigned>(slots * (D / DV) * 8)), dim3(G::WAVES * 64),
                        G::BYTES, st, a.v, a.s0, a.o, a.s_out, at(o.kh), at(o.kb), at(o.qh), at(o.rec), n_pairs, a.T, a.H,
                        n_ch);
     return hipGetLastError();

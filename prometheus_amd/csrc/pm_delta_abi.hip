@@ -202,10 +202,10 @@ int check_dtypes(int in_dtype, int out_dtype) {
 // Workspace of the chunked fp32 forward of the rules with a decay (K10f: fp32 q/k/v, D in {64,
 // 128}, the default path), 0 where it does not serve the call.  It walks 16 tokens a step
 // where the per-token kernel walks one, behind a parallel pass over all chunks: level to about
-// 130 tokens (both at the cost of their launches: 26 against 22 us), then ahead (T = 1000:
-// 97 against 184 us at 2 pairs, 124 against 224 at 64, 504 against 727 at 256, D = 128; at D =
-// 64 62 against 168, 75 against 170, but 200 against 208 at 256 pairs, where the per-token
-// kernel fills the chip and the extra pass over memory eats the gain).
+// 130 tokens (both at the cost of their launches: 26 against 22 us), then ahead (T = 1024,
+// D = 128: 70 against 190 us at 2 pairs, 128 against 228 at 64, 264 against 421 at 128; at D =
+// 64 51 against 171, 64 against 175, and 189 against 206 at 200 pairs; from 256 pairs of D = 64
+// the per-token kernel fills the chip and the extra pass over memory eats the gain).
 constexpr int kDecayFwdMinT = 160;
 size_t decay_fwd_need(int B, int T, int H, int D) {
     if (B < 0 || H < 0 || g_path != 0 || T < kDecayFwdMinT || !pm::f32_bwd_supported(D, H)) return 0;
