@@ -22,16 +22,14 @@
 //     recurrence forwards, storing U per token and S at the start of every span of kF32Span
 //     chunks and at the end of the sequence; beside it the G recurrence backwards over all
 //     chunks, storing W and dV per token, G at the end of every span, dS0.
-//   K9c (span, one workgroup per (b, h, span)): from the span's start state, the forward
-//     again (X', U, with U kept in LDS for the whole span), then backwards from the
-//     span's end state and end gradient: S reconstructed as S - K^T U (no growth: U is
-//     the stored forward value), G as in K9b, and dQ, dK, dbeta.
+//   K9c (span, one workgroup per (b, h, span)): backwards from the span's end state and end
+//     gradient: S reconstructed as S - K^T U (no growth: U is the stored forward value),
+//     G as in K9b, and dQ, dK, dbeta.
 // Column ownership differs by phase: the recurrences over S and G keep their columns
 // independent (a wave owns 16 columns of d_v), while the products contracting over d_v
-// (dO S^T, U G^T, ...) need all of them: K9c's forward keeps S by columns (j), its
-// reverse keeps S^T and G^T by rows of d (a wave owns 16 of them), and the two small
-// products that contract over d_v inside a chunk (dO U^T, W U^T) are summed over the
-// waves in LDS, in a fixed order.
+// (dO S^T, U G^T, ...) need all of them: K9c keeps S^T and G^T by rows of d (a wave owns 16
+// of them), and the two small products that contract over d_v inside a chunk (dO U^T,
+// W U^T) are summed over the waves in LDS, in a fixed order.
 
 #include <type_traits>
 
