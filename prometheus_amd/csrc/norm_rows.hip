@@ -13,6 +13,9 @@
 #include "pm_internal.h"
 #include "pm_rec.h"
 
+// (multiply-adds are fused only where written so)
+#pragma clang fp contract(off)
+
 namespace pm {
 namespace {
 
@@ -52,19 +55,47 @@ __device__ __forceinline__ void store8<uint16_t>(uint16_t* p, const float (&x)[8
     *reinterpret_cast<uint4*>(p) = make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-// Gradient of x / max(||x||, eps) given g = dL/d(normalised row), ss = ||x||^2, dot = g . x:
-// (g - x^ (x^ . g)) / ||x|| where the norm counts (torch's clamp_min passes its gradient at
-// and above the bound), g / eps below.  A NaN norm counts (the comparisons are written so), so
-// that a row with a NaN gives NaNs as elementwise tensor operations do.
-struct NormBwd {
-    float inv, coef;  // gx = inv * (g - coef * x)
-    __device__ __forceinline__ NormBwd(float ss, float dot) {
-        const float n = sqrtf(ss);
-        const bool live = !(n < kEps);
-        inv = 1.f / floored(n);
-        coef = live ? (dot * inv) * inv : 0.f;
+// Sum over a row of the eight values of each of its LPR = D / 8 lanes, in the order of the
+// elementwise tensor operations that these kernels stand for: pairs of neighbours throughout at
+// D = 64, four consecutive values in sequence and then pairs of neighbours from D = 128 on.  The
+// bf16 gradients follow the rounding of the normalised rows to bf16, which another order of
+// their norm's sum moves by one unit here and there (1e-3 of the gradients).
+template <int LPR>
+__device__ __forceinline__ float row_sum8(const float (&y)[8]) {
+    float s;
+    if constexpr (LPR == 8) s = ((y[0] + y[1]) + (y[2] + y[3])) + ((y[4] + y[5]) + (y[6] + y[7]));
+    else s = (((y[0] + y[1]) + y[2]) + y[3]) + (((y[4] + y[5]) + y[6]) + y[7]);
+    return lane_sum<LPR>(s);
+}
+// ... and over a row of any D <= 256 by one wave: f(acc, d) adds element d's value to acc.
+// Below 128 elements lane l takes elements l and l + n in two sums, n the power of two at most D
+// (and 64); from there on it takes the four elements from 4 l on and from 4 (l + n) on in four,
+// n the power of two at most D / 4.
+template <typename F>
+__device__ __forceinline__ float row_sum_any(int D, int lane, F f) {
+    const int n = 1 << min(6, 31 - __clz(D < 128 ? D : D / 4));
+    float a[4] = {0.f, 0.f, 0.f, 0.f};
+    if (lane < n) {
+        if (D < 128) {
+            a[0] = f(0.f, lane);
+            if (lane + n < D) a[1] = f(0.f, lane + n);
+        } else {
+            for (int v = lane; v < D / 4; v += n)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) a[e] = f(a[e], 4 * v + e);
+            if (lane < D % 4) a[0] = f(a[0], D - D % 4 + lane);
+        }
     }
-};
+    return lane_sum<64>(((a[0] + a[1]) + a[2]) + a[3]);
+}
+
+// One element of the gradient of y = x / m, m = max(n, eps), n = ||x||, given g = dL/dy and dot
+// = sum -g (x / m) / m = dL/dm: the norm's part only where the norm counts (live: at and above
+// the bound; a row with a NaN gives NaNs through m).  norm_dot is one element of dot.
+__device__ __forceinline__ float norm_dot(float g, float x, float m) { return -g * ((x / m) / m); }
+__device__ __forceinline__ float norm_grad(float g, float x, float m, float dot, bool live) {
+    return g / m + (live ? dot : 0.f) * (x / m);
+}
 
 // LPR = D / 8 lanes per row; 2 * rows rows in all, q's then k's
 template <typename T, int LPR>
@@ -76,12 +107,11 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(const T* __restrict__ q,
     for (long i = t; i < n; i += step) {
         const bool second = i >= rows * LPR;
         const long o = (second ? i - rows * LPR : i) * 8;
-        float x[8], ss = 0.f;
+        float x[8], y[8];
         load8<T>((second ? k : q) + o, x);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) ss = fmaf(x[e], x[e], ss);
-        ss = lane_sum<LPR>(ss);  // (a row's lanes are adjacent and all in range together)
-        const float m = floored(sqrtf(ss));
+        for (int e = 0; e < 8; ++e) y[e] = x[e] * x[e];
+        const float m = floored(sqrtf(row_sum8<LPR>(y)));  // (a row's lanes are adjacent and all in range together)
 #pragma unroll
         for (int e = 0; e < 8; ++e) x[e] = x[e] / m;
         store8<T>((second ? kn : qn) + o, x);
@@ -98,17 +128,17 @@ __global__ __launch_bounds__(256) void norm_rows_bwd_kernel(const T* __restrict_
     for (long i = static_cast<long>(blockIdx.x) * 256 + threadIdx.x; i < n; i += step) {
         const bool second = i >= rows * LPR;
         const long o = (second ? i - rows * LPR : i) * 8;
-        float x[8], g[8], ss = 0.f, dot = 0.f;
+        float x[8], g[8], y[8];
         load8<T>((second ? k : q) + o, x);
         load8<float>((second ? gkn : gqn) + o, g);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            ss = fmaf(x[e], x[e], ss);
-            dot = fmaf(g[e], x[e], dot);
-        }
-        const NormBwd nb(lane_sum<LPR>(ss), lane_sum<LPR>(dot));
+        for (int e = 0; e < 8; ++e) y[e] = x[e] * x[e];
+        const float nrm = sqrtf(row_sum8<LPR>(y)), m = floored(nrm);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) g[e] = nb.inv * (g[e] - nb.coef * x[e]);
+        for (int e = 0; e < 8; ++e) y[e] = norm_dot(g[e], x[e], m);
+        const float dot = row_sum8<LPR>(y);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) g[e] = norm_grad(g[e], x[e], m, dot, nrm >= kEps);
         store8<T>((second ? gk : gq) + o, g);
     }
 }
@@ -127,20 +157,18 @@ __global__ __launch_bounds__(256) void norm_rows_any_kernel(const T* __restrict_
         const long o = (second ? i - rows : i) * D;
         const T* x = (second ? k : q) + o;
         const float* g = BWD ? (second ? gkn : gqn) + o : nullptr;
-        float ss = 0.f, dot = 0.f;
-        for (int d = lane; d < D; d += 64) {
+        const float nrm = sqrtf(row_sum_any(D, lane, [=](float acc, int d) {
             const float a = to_f32<T>(x[d]);
-            ss = fmaf(a, a, ss);
-            if constexpr (BWD) dot = fmaf(g[d], a, dot);
-        }
-        ss = lane_sum<64>(ss);
-        if constexpr (BWD) dot = lane_sum<64>(dot);
-        const NormBwd nb(ss, dot);
-        const float m = floored(sqrtf(ss));
+            return fmaf(a, a, acc);
+        }));
+        const float m = floored(nrm);
+        float dot = 0.f;
+        if constexpr (BWD)
+            dot = row_sum_any(D, lane, [=](float acc, int d) { return acc + norm_dot(g[d], to_f32<T>(x[d]), m); });
         T* y = (second ? ok : oq) + o;
         for (int d = lane; d < D; d += 64) {
             const float a = to_f32<T>(x[d]);
-            y[d] = from_f32<T>(BWD ? nb.inv * (g[d] - nb.coef * a) : a / m);
+            y[d] = from_f32<T>(BWD ? norm_grad(g[d], a, m, dot, nrm >= kEps) : a / m);
         }
     }
     if (!BWD)

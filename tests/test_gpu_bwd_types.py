@@ -148,3 +148,33 @@ def test_linear_attention_backward_under_saved_tensor_hooks():
         o = model.linear_attention(*leaves)[0]
     for a, e in zip(torch.autograd.grad(o, leaves, go), exp):
         assert torch.equal(a, e)
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+@pytest.mark.parametrize("dim", [5, 16, 48, 64, 96, 128, 160, 256])
+def test_linear_attention_backward_normalises_as_tensor_operations_do(dtype, dim):
+    """Bit for bit the reverse kernels on rows normalised by elementwise tensor operations and
+    those operations' own reverse, rows at and below the norm's bound among them: a sum of
+    squares in another order moves the rounding of the normalised rows to bf16, and with it the
+    gradients by 1e-3."""
+    shape = (2, 67, 3, dim)
+    x = synth.fwd_inputs(shape, seed=dim, dtype=dtype, s0_std=0.05, normalize=False)
+    qkv = [_bf(b) for b in (x.q_bits, x.k_bits, x.v_bits)] if dtype == "bf16" else [_f(a) for a in (x.q, x.k, x.v)]
+    qkv[0][0, 3], qkv[1][1, 5], qkv[0][1, 9] = 0.0, qkv[1][1, 5] * 1e-9, 0.0
+    qkv[0][1, 9, :, 0] = 1e-6
+    s0 = _f(x.s0)
+    go, gs = torch.randn(shape, device="cuda"), 0.05 * torch.randn(s0.shape, device="cuda")
+    leaves = [t.requires_grad_(True) for t in (*qkv, s0)]
+    got = torch.autograd.grad(model.linear_attention(*leaves), leaves, (go, gs))
+
+    def norm(t):
+        return t / torch.clamp_min(torch.linalg.vector_norm(t, dim=-1, keepdim=True), 1e-6)
+
+    raw = [t.detach().float().requires_grad_(True) for t in qkv[:2]]
+    rows = [norm(t) for t in raw]
+    res = kernels._DeltaResidual(q=rows[0].detach().to(qkv[0].dtype), k=rows[1].detach().to(qkv[0].dtype),
+                                 v=qkv[2].detach(), beta=torch.ones(shape[:3], device="cuda"), state0=s0.detach(), chunk=64)
+    gqn, gkn, gv, _, gs0 = kernels.chunked_delta_rule_bwd(res, (go, gs))
+    exp = (*torch.autograd.grad(rows, raw, (gqn, gkn)), gv, gs0)
+    for name, a, e in zip(("gq", "gk", "gv", "gs0"), got, exp):
+        assert torch.equal(a, e.to(a.dtype)), (name, (a != e.to(a.dtype)).sum().item())
