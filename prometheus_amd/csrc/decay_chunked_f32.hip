@@ -234,7 +234,7 @@ __global__ __launch_bounds__(256) void dec_prep_kernel(
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const int t = 4 * g + v;
-                const bool in = ((t ^ r) >> hb) == 1 && t > r;
+                const bool in = in_level<hb>(t, r);
                 float d = 1.f;
                 if constexpr (!CHAN) d = __shfl(F[0][0], t) * E[0][0];
                 A[v] += in ? d * a4[v] : 0.f;
@@ -308,21 +308,14 @@ __global__ __launch_bounds__(256) void dec_prep_kernel(
     }
     }
 
-    // T = (I + diag(beta) A')^-1 = (I+N)(I+N^2)(I+N^4)(I+N^8), N = -diag(beta) A' (N^16 = 0)
-    f32x4_t N, Nt, eye;
+    // T = (I + diag(beta) A')^-1 = (I - N)^-1, N = -diag(beta) A'
+    f32x4_t N, Nt, Ta, Tt;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
         N[v] = -bt[v] * A[v];
         Nt[v] = -bc * At[v];
-        eye[v] = 4 * g + v == r ? 1.f : 0.f;
     }
-    const f32x4_t N2 = mm16(Nt, N), N2t = mm16(N, Nt);
-    const f32x4_t N4 = mm16(N2t, N2), N4t = mm16(N2, N2t);
-    const f32x4_t N8 = mm16(N4t, N4);
-    const f32x4_t F1t = mm16(eye + N2, eye + Nt);
-    const f32x4_t F2t = mm16(eye + N4, F1t);
-    const f32x4_t Tt = mm16(eye + N8, F2t);   // T^T
-    const f32x4_t Ta = mm16(F2t, eye + N8);   // T
+    inv_lower16<!FWD>(N, Nt, r, g, Ta, Tt);
     f32x4_t tw;
 #pragma unroll
     for (int v = 0; v < 4; ++v) tw[v] = -bt[v] * Tt[v];

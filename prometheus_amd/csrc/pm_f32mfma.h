@@ -10,6 +10,8 @@
 // and a product contracting over M's columns needs the registers of M^T instead.
 #pragma once
 
+#include <type_traits>
+
 namespace pm {
 namespace {
 
@@ -26,6 +28,43 @@ __device__ __forceinline__ f32x4_t mm16(f32x4_t lt, f32x4_t r, f32x4_t c = f32x4
     a0 = mfma4(lt[2], r[2], a0);
     a1 = mfma4(lt[3], r[3], a1);
     return a0 + a1;
+}
+
+// Entry (i, j) of a 16x16 matrix is strictly lower and the highest bit in which i and j differ
+// is HB: the lower left block of a 2h x 2h diagonal block, h = 2^HB.
+template <int HB>
+__device__ __forceinline__ bool in_level(int i, int j) {
+    return ((i ^ j) >> HB) == 1 && i > j;
+}
+// T = (I - N)^-1 of a strictly lower N and T^T, from the accumulators of N and N^T: T starts as
+// the inverse of I - N's diagonal 2x2 blocks, and T + T N_h T, N_h the lower left blocks at h,
+// is that of its 2h x 2h blocks.  Only true inverses of blocks are multiplied: where the keys of
+// a chunk are alike T's entries stay of the size of N's, while the powers of N, of which (I + N)
+// (I + N^2)(I + N^4)(I + N^8) is made in as many products, grow as binomials (3,432 at N = -1)
+// and cancel (O of a gated rule with keys of mutual cosine 0.9 was 2e-5 off at beta 1 and 8e-3
+// at 1.95, now 3e-7 and 9e-7).  TOO false: T^T alone.
+template <bool TOO>
+__device__ __forceinline__ void inv_lower16(f32x4_t N, f32x4_t Nt, int r, int g, f32x4_t& T, f32x4_t& Tt) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const int i = 4 * g + v;
+        const float eye = i == r ? 1.f : 0.f;
+        T[v] = in_level<0>(i, r) ? N[v] : eye;
+        Tt[v] = in_level<0>(r, i) ? Nt[v] : eye;
+    }
+    auto level = [&](auto HB, auto BOTH) __attribute__((always_inline)) {
+        f32x4_t nt;  // N_h^T
+#pragma unroll
+        for (int v = 0; v < 4; ++v) nt[v] = in_level<decltype(HB)::value>(r, 4 * g + v) ? Nt[v] : 0.f;
+        const f32x4_t y = mm16(nt, T);  // N_h T
+        const f32x4_t t = Tt;
+        Tt = mm16(y, t, t);  // (N_h T)^T T^T + T^T
+        if constexpr (decltype(BOTH)::value) T = mm16(t, y, T);
+    };
+    using B = std::true_type;
+    level(std::integral_constant<int, 1>{}, B{});
+    level(std::integral_constant<int, 2>{}, B{});
+    level(std::integral_constant<int, 3>{}, std::integral_constant<bool, TOO>{});
 }
 
 // LDS tile of 16 fp32 token rows of D values: the 16-byte chunk p of row t is stored at

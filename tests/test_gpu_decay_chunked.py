@@ -140,3 +140,44 @@ def test_forward_decays_of_every_strength_and_routes():
     assert lib.pm_decay_fwd_workspace_bytes(1, 170, 2, 64, f32) == 2 * 11 * (3 * 16 * 64 + 512 + 64) * 4
     for args in ((1, 159, 2, 64, f32), (1, 170, 2, 48, f32), (1, 170, 2, 64, bf16), (1, 170, 256, 64, f32)):
         assert lib.pm_decay_fwd_workspace_bytes(*args) == 0
+
+
+def _alike(shape, seed, chan, rho, beta, dtype="fp32"):
+    """Unit keys of mutual cosine rho^2 (rho 1: one repeated key a head), constant beta."""
+    x, g, go, gs = _case(shape, seed, chan, dtype, scale=0.1)
+    rng = np.random.default_rng(seed)
+
+    def unit(z):
+        return z / np.linalg.norm(z, axis=-1, keepdims=True)
+
+    common = unit(rng.standard_normal((shape[0], 1, *shape[2:])))
+    k = unit(rho * common + np.sqrt(1 - rho * rho) * unit(rng.standard_normal(shape)))
+    x.k, x.k_bits = synth._cast(k.astype(np.float32), dtype)
+    x.beta = np.full(shape[:3], beta, np.float32)
+    return x, g, go, gs
+
+
+@pytest.mark.parametrize("chan", [False, True])
+@pytest.mark.parametrize("rho,beta", [(0.8, 0.9), (0.95, 1.0), (1.0, 0.9), (1.0, 1.0), (1.0, 1.9), (0.95, 1.95)])
+@pytest.mark.parametrize("shape,dtype", [((1, 256, 2, 64), "fp32"), ((1, 170, 2, 128), "fp32"), ((1, 100, 2, 128), "bf16")])
+def test_alike_keys(shape, dtype, rho, beta, chan):
+    """Repeated and near-repeated keys, up to betas where the powers of diag(beta) A' are large
+    and the inverse of I + diag(beta) A' is not: forward (fp32) and all gradients."""
+    x, g, go, gs = _alike(shape, 3, chan, rho, beta, dtype)
+    if dtype == "fp32":
+        exp = (gref.kda_delta_rule if chan else gref.gated_delta_rule)(x.q, x.k, x.v, x.beta, g, x.s0)
+        for name, a, e in zip(("o", "state"), _fwd(x, g, chan), exp):
+            assert_f32_parity(a, e, name)
+    what = f"rho {rho} beta {beta}"
+    if chan:
+        _check(x, g, go, gs, chan, what)
+        return
+    got = _bwd(x, g, go, gs, chan)
+    exp = gref.gated_vjp(x.q, x.k, x.v, x.beta, g, go, gs, x.s0)
+    for name, a, e in zip(NAMES, got, exp):
+        if name != "gg":
+            assert_f32_parity(a, e, f"{what} {name}", scaled=True)
+    # a head's gg sums its channels', which cancel where one key is repeated at beta 1 (the
+    # per-token kernels' error there is 3e-6 of the sum): each channel's to 1e-5
+    channels = gref.kda_vjp(x.q, x.k, x.v, x.beta, np.repeat(g[..., None], shape[3], -1), go, gs, x.s0)[4]
+    assert np.linalg.norm(got[4] - exp[4]) <= 1e-5 * np.linalg.norm(channels), what
