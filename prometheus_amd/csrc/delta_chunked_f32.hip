@@ -20,8 +20,8 @@
 //
 // K7p (prep, one wave per (sequence, head, chunk), all chunks at once): G = K K^T from K
 // rows read straight into operand registers, N = -A and N^T from G (which is symmetric),
-// and T^T = ((I+N)(I+N^2)(I+N^4)(I+N^8))^T (N is strictly lower triangular, so N^16 = 0)
-// as products of accumulators with transposed accumulators.  It writes (T'')^T as
+// and T = (I - N)^-1 from the inverses of its diagonal blocks of 2, 4 and 8 (inv_lower16), as
+// products of accumulators with transposed accumulators.  It writes (T'')^T as
 // accumulator registers, 1 KiB per chunk: the A operand of U = T'' X, lane-linear.
 //
 // K7 (recurrence): one workgroup per (sequence, head, d_v tile of DV columns).  Per 16 columns,
@@ -142,20 +142,14 @@ __global__ __launch_bounds__(256) void delta_f32_prep_kernel(const float* __rest
     f32x4_t G = (ga[0] + ga[1]) + (ga[2] + ga[3]);
     if constexpr (NORM) G = G * s4 * sk;  // Gram matrix of the normalised keys
     // N[i][j] = -beta_i G[i][j] (i > j), N^T[i][j] = -beta_j G[i][j] (j > i); i = 4 g + v, j = r
-    f32x4_t N, Nt, eye;
+    f32x4_t N, Nt, Tacc, Tt;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
         const int i = 4 * g + v;
         N[v] = i > r ? -bt[v] * G[v] : 0.f;
         Nt[v] = r > i ? -bc * G[v] : 0.f;
-        eye[v] = i == r ? 1.f : 0.f;
     }
-    const f32x4_t N2 = mm16(Nt, N), N2t = mm16(N, Nt);
-    const f32x4_t N4 = mm16(N2t, N2), N4t = mm16(N2, N2t);
-    const f32x4_t N8 = mm16(N4t, N4);
-    const f32x4_t F1t = mm16(eye + N2, eye + Nt);   // ((I+N)(I+N^2))^T
-    const f32x4_t F2t = mm16(eye + N4, F1t);        // (... (I+N^4))^T
-    const f32x4_t Tt = mm16(eye + N8, F2t);         // T^T
+    inv_lower16<BWD>(N, Nt, r, g, Tacc, Tt);
     f32x4_t tw;
 #pragma unroll
     for (int v = 0; v < 4; ++v) tw[v] = -bt[v] * Tt[v];  // (T'')^T[i][j] = -beta_i T[j][i]
@@ -164,7 +158,6 @@ __global__ __launch_bounds__(256) void delta_f32_prep_kernel(const float* __rest
     if constexpr (BWD) {
         // the backward's record: T (accumulator registers: T[4 g + v][r]), the Gram matrix
         // K K^T (symmetric, so its registers are also those of its transpose), beta and P
-        const f32x4_t Tacc = mm16(F2t, eye + N8);  // (I+N)(I+N^2)(I+N^4) (I+N^8)
         float* ob = ws_b + (static_cast<size_t>(row) * n_slot + slot) * kBwdRec;
         *reinterpret_cast<f32x4_t*>(ob + lane * 4) = Tacc;
         *reinterpret_cast<f32x4_t*>(ob + 256 + lane * 4) = G;

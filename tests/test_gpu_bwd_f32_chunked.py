@@ -149,3 +149,24 @@ def test_graph_capture_replays():
         torch.cuda.synchronize()
         for name, o, e in zip(NAMES, outs, eager):
             assert torch.equal(o, e), name
+
+
+@pytest.mark.parametrize("rho,beta", [(0.8, 0.9), (0.95, 1.0), (1.0, 1.0), (1.0, 1.9), (0.95, 1.95)])
+@pytest.mark.parametrize("shape", [(1, 256, 2, 64), (1, 170, 2, 128)])
+def test_alike_keys(shape, rho, beta):
+    """Unit keys of mutual cosine rho^2 (1: one repeated key a head), forward and gradients, up to
+    betas where the powers of diag(beta) K K^T are large and the inverse of I + them is not."""
+    x, go, gs = _case(shape, 3)
+    rng = np.random.default_rng(3)
+
+    def unit(z):
+        return z / np.linalg.norm(z, axis=-1, keepdims=True)
+
+    common = unit(rng.standard_normal((shape[0], 1, *shape[2:])))
+    x.k = unit(rho * common + np.sqrt(1 - rho * rho) * unit(rng.standard_normal(shape))).astype(np.float32)
+    x.beta = np.full(shape[:3], beta, np.float32)
+    exp = ref.gated_delta_rule(x.q, x.k, x.v, x.beta, x.s0, dtype=np.float64)
+    got = kernels.chunked_delta_rule(*(_dev(a) for a in (x.q, x.k, x.v, x.beta, x.s0)))
+    for name, a, e in zip(("o", "state"), got, exp):
+        assert_f32_parity(_np(a), e, name)
+    _check(_bwd(x, go, gs), ref.delta_vjp(x.q, x.k, x.v, x.beta, go, gs, x.s0), f"rho {rho} beta {beta}")
