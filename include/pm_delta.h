@@ -354,7 +354,9 @@ int pm_gated_delta_bwd(const void* q, const void* k, const void* v, const float*
                        int H, int D, int in_dtype, void* workspace, size_t ws_bytes, void* stream);
 
 /* Workspace bytes pm_gated_delta_bwd needs (0 for invalid shapes, dtypes or D > 256):
- * pm_delta_bwd's per-token workspace plus, for D > 32, the partial sums of gg. */
+ * pm_delta_bwd's per-token workspace plus, for D > 32, the partial sums of gg, or what the
+ * chunked path takes under the current path setting where that is more (a workspace of the
+ * former size alone runs the per-token kernels). */
 size_t pm_gated_delta_bwd_workspace_bytes(int B, int T, int H, int D, int in_dtype);
 
 /*
@@ -375,7 +377,7 @@ int pm_kda_delta_bwd(const void* q, const void* k, const void* v, const float* b
 
 /* Workspace bytes pm_kda_delta_bwd needs (0 for invalid shapes, dtypes or D > 256):
  * pm_delta_bwd's per-token workspace plus, for D > 32, the partial sums of gg per
- * column tile. */
+ * column tile, or the chunked path's as pm_gated_delta_bwd_workspace_bytes. */
 size_t pm_kda_delta_bwd_workspace_bytes(int B, int T, int H, int D, int in_dtype);
 
 /*

@@ -19,6 +19,7 @@
 #include <stdarg.h>
 #include <stdio.h>
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -386,12 +387,21 @@ size_t bwd_ws_bytes(int B, int T, int H, int D, int in_dtype, int gm = 0) {
     return sizeof(float) * pm::bwd_workspace_floats(n_pairs, T, D, gm);
 }
 
+// ... and what the size functions of the rules with a decay give: enough for K10 and for the
+// per-token kernels, which take its misaligned calls and those with a workspace that holds only
+// theirs (K10's is the larger one at D = 64 for T 16 to 24 and 33 to 40)
+size_t decay_bwd_need(int B, int T, int H, int D, int in_dtype, int gm) {
+    const size_t per_token = bwd_ws_bytes(B, T, H, D, in_dtype, gm);
+    if (!bwd_decay_chunked(T, H, D)) return per_token;
+    return std::max(per_token, pm::decay_bwd_ws_bytes(static_cast<long>(B) * H, T, D));
+}
+
 // Type of gq, gk and gv: fp32, all bf16, or gv alone bf16 (bf16 needs bf16 q/k/v on a chunked
 // path; PM_E_UNSUPPORTED otherwise, nothing launched).
 enum GradType { kGradF32, kGradBf16, kGradBf16V };
 
-// Common backward dispatch; g != NULL: a gated variant (K10 or the per-token kernels, gg
-// out, the per-token kernels' workspace either way: it holds K10's), with per_channel its KDA form (g and gg (B, T, H, D)).
+// Common backward dispatch; g != NULL: a gated variant (K10 or the per-token kernels, gg out),
+// with per_channel its KDA form (g and gg (B, T, H, D)).
 int backward(const void* q, const void* k, const void* v, const float* beta, const float* g,
              const float* s0, const float* go, const float* gs, void* gq, void* gk, void* gv,
              float* gbeta, float* gg, float* gs0, int B, int T, int H, int D, int in_dtype,
@@ -446,7 +456,7 @@ int backward(const void* q, const void* k, const void* v, const float* beta, con
     const bool decay = gated && n_tok > 0 && bwd_decay_chunked(T, H, D) && aligned(q, 16) && aligned(k, 16) &&
                        aligned(v, 16) && (!go || aligned(go, 16)) && aligned(gv, 16) &&
                        (!per_channel || aligned(g, 16)) && aligned(workspace, 16) &&
-                       pm::decay_bwd_ws_bytes(n_pairs, T, D) <= need;
+                       ws_bytes >= pm::decay_bwd_ws_bytes(n_pairs, T, D);
     if (gt != kGradF32 && n_tok > 0 && !(in_dtype == PM_DTYPE_BF16 && (chunked16 || decay)))
         return fail(PM_E_UNSUPPORTED, "bf16 gradients need bf16 q/k/v on a chunked path (D in {64, 128})");
     if (decay) {
@@ -541,13 +551,13 @@ int pm_delta_bwd_bf16(const void* q, const void* k, const void* v, const float* 
 size_t pm_gated_delta_bwd_workspace_bytes(int B, int T, int H, int D, int in_dtype) {
     if (B < 0 || T < 0 || H < 0 || D < 1 || D > pm::kBwdMaxD) return 0;
     if (in_dtype != PM_DTYPE_F32 && in_dtype != PM_DTYPE_BF16) return 0;
-    return bwd_ws_bytes(B, T, H, D, in_dtype, 1);
+    return decay_bwd_need(B, T, H, D, in_dtype, 1);
 }
 
 size_t pm_kda_delta_bwd_workspace_bytes(int B, int T, int H, int D, int in_dtype) {
     if (B < 0 || T < 0 || H < 0 || D < 1 || D > pm::kBwdMaxD) return 0;
     if (in_dtype != PM_DTYPE_F32 && in_dtype != PM_DTYPE_BF16) return 0;
-    return bwd_ws_bytes(B, T, H, D, in_dtype, 2);
+    return decay_bwd_need(B, T, H, D, in_dtype, 2);
 }
 
 int pm_kda_delta_bwd(const void* q, const void* k, const void* v, const float* beta,

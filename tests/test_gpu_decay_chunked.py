@@ -62,6 +62,23 @@ def test_edges_of_chunks_and_spans(t, d, chan):
     _check(x, g, go, gs, chan, f"T{t} D{d}")
 
 
+@pytest.mark.parametrize("chan", [0, 1])
+@pytest.mark.parametrize("d", [64, 128])
+def test_every_length_from_a_chunk_on_is_served(d, chan):
+    """The bf16 entry point, which the chunked kernels alone serve, takes the workspace that the
+    size function gives for every length from 16 tokens on, and refuses shorter ones."""
+    lib = _native.lib()
+    size = lib.pm_kda_delta_bwd_workspace_bytes if chan else lib.pm_gated_delta_bwd_workspace_bytes
+    p = torch.zeros(1 << 20, device="cuda").data_ptr()
+    for t in (*range(15, 49), 64, 129):
+        n = size(1, t, 3, d, _native.DTYPE_BF16)
+        ws = torch.empty(n, dtype=torch.uint8, device="cuda")
+        rc = lib.pm_delta_bwd_bf16(p, p, p, p, p, None, None, None, p, p, p, p, p, p, 1, t, 3, d, chan,
+                                   ws.data_ptr(), n, torch.cuda.current_stream().cuda_stream)
+        assert rc == (0 if t >= 16 else _native.E_UNSUPPORTED), t
+    torch.cuda.synchronize()
+
+
 @pytest.mark.parametrize("chan", [False, True])
 def test_bf16_inputs_in_fp32_arithmetic(chan):
     x, g, go, gs = _case((2, 145, 2, 128), 7, chan, dtype="bf16")
