@@ -22,7 +22,10 @@
 //   dbeta_t = W_t . V_t - K^_t . (W S^T)_t + sum_s dA_ts A'_ts
 //   dg_j = sum_{t>=j} (Q^ dO S^T - K^ beta W S^T)_t + sum_{s<j} (K- U G^T)_s
 //          + gC <S, G>_rows + sum_{t>=j, s<j} x_ts,
-// x_ts the pair term dP_ts q_t k_s D_ts + beta_t dA_ts k_t k_s D_ts.
+// x_ts the pair term dP_ts q_t k_s D_ts + beta_t dA_ts k_t k_s D_ts.  Every term of dg_j holds
+// alpha_j: none is a difference of larger ones, which a strong decay would leave without a digit
+// (as <S', G'> less the chunk's own terms, gC <S, G> was 4e-5 of dg off at g = -8 throughout
+// and noise at -20; now 1e-7 to 3e-7 at every strength).
 //
 // Decays without exponents of differences.  D_ts is never formed as exp(G_t - G_s) (whose
 // difference of prefix sums loses what a strong decay elsewhere in the chunk adds to both)
@@ -43,15 +46,17 @@
 //   K10c (one workgroup of D/16 waves per (b, h, span of 2 to 8 chunks)): the span forwards from
 //     its start state (dQ, dbeta, dK and dg but for what depends on G), then backwards from
 //     its end gradient (the rest).  S cannot be walked back as the ungated backward does
-//     (that divides by gC), hence the two walks.
+//     (that divides by gC), hence the two walks; <S, G> needs S at every chunk's start again, which
+//     the way forwards keeps (in LDS at mid-span, else in the workspace: 64 KiB a chunk at D = 128,
+//     5% of the training pass).
 
 // Why chunks: the per-token kernels walk T tokens in sequence at about 500 (forward) and
 // 1,270 cycles (reverse) a token, bound by VALU issue; here a chunk of 16 tokens takes about
 // 2,800 to 4,100 cycles of the one sequential launch, and the rest is parallel over chunks.
 // Measured, B4 T4096 H16 D128, bf16 q/k/v, per-head gate: 6.0 -> 1.45 ms (K10p 125, K10s
 // 505, K10c 825 us); B2, per-channel gate: 5.9 -> 0.87 ms (97, 340, 432); B3 T1000 H6 D64
-// fp32: 1.11 -> 0.10 ms.  Against 64 bits the gradients stay at 2e-7 to 5e-7 (the per-token
-// kernels: 1.3e-7 to 2e-7).  What bounds it: K10s the products of its recurrence waves (32
+// fp32: 1.11 -> 0.10 ms.  Against 64 bits the gradients of training inputs are at 1.6e-7 to
+// 2.5e-7 (the per-token kernels: 1.3e-7 to 1.9e-7).  What bounds it: K10s the products of its recurrence waves (32
 // pairs: 54 of 32 cycles in a chunk of 2,800 cycles, the two barriers and exchanges most of
 // the rest, the copies 10%; 64 pairs: 94 on each SIMD), K10c the fp32 MFMA pipe at half its
 // rate (232 products per wave and chunk; two waves per SIMD, which wait for the pipe half of
@@ -985,8 +990,7 @@ struct DcGeo {
     static constexpr int OFF_TR = OFF_PP + NW * 2048;        // totals dP, diag(beta) dA as rows [t][s]
     static constexpr int OFF_TC = OFF_TR + 2048;             // ... as columns [s][t], stride 20
     static constexpr int OFF_DB = OFF_TC + 2 * 16 * 20 * 4;  // dbeta parts: 2 slots x NW x 16
-    static constexpr int OFF_EC = OFF_DB + 2 * NW * 64;      // per chunk of the span: sum_t of dg's own terms, D
-    static constexpr int OFF_GG = OFF_EC + kSpan * D * 4;    // per-head gate: dg parts, chunk x wave x 16
+    static constexpr int OFF_GG = OFF_DB + 2 * NW * 64;      // per-head gate: dg parts, chunk x wave x 16
     static constexpr int OFF_MID = OFF_GG + kSpan * NW * 64;  // S^T in mid-span
     static constexpr int BYTES = OFF_MID + NW * NT * 1024;
     static_assert(BYTES <= 160 * 1024, "LDS");
@@ -998,7 +1002,7 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
     const float* __restrict__ go, const float* __restrict__ rec, const float* __restrict__ s_hist,
     const float* __restrict__ g_hist, const float* __restrict__ w_in, const float* __restrict__ u_in,
     void* __restrict__ gq, void* __restrict__ gk, float* __restrict__ gbeta, float* __restrict__ gg,
-    float* __restrict__ pk_ws, float* __restrict__ pg_ws, int T, int H, int n_ch, int n_span, int span_len) {
+    float* __restrict__ pk_ws, float* __restrict__ pg_ws, float* __restrict__ s_ch, int T, int H, int n_ch, int n_span, int span_len) {
     // multiply-adds are fused only where written so (fmaf): every build of this kernel gives the
     // same bits, and bf16 gradients are the fp32 ones rounded
 #pragma clang fp contract(off)
@@ -1114,17 +1118,27 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
         return s;
     };
 
-    // S^T at the span's start, by rows of d, gathered from the column-block layout: S[16 w +
-    // r][16 i + 4 g + e] is in column block i, tile w, lane 16 (r >> 2) + 4 g + e, register r & 3
+    // tile i of S^T or G^T at the span's start or end, by rows of d, gathered from the column-block
+    // layout: S[16 w + r][16 i + 4 g + e] is in column block i, tile w, lane 16 (r >> 2) + 4 g + e,
+    // register r & 3
+    auto gather = [=](const float* hist, int i) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc(hist + (static_cast<size_t>(pair) * n_span + span) * D * D, D * D * 4);
+        const unsigned off = static_cast<unsigned>(4 * (4 * (16 * (r >> 2) + 4 * g) + (r & 3)));
+        f32x4_t x;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            x[e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, off + 16 * e, (i * NT + w) * 1024, 0));
+        return x;
+    };
+    // this wave's S^T at the start of chunk m, left for the way back; m = 0 is in s_hist and m =
+    // span_len / 2 in LDS
+    auto start_of = [=](int m) __attribute__((always_inline)) {
+        const size_t slot = (static_cast<size_t>(pair) * n_span + span) * (span_len - 2) + m - (m < span_len / 2 ? 1 : 2);
+        return make_rsrc(s_ch + slot * D * D + w * NT * 256, NT * 1024);
+    };
     f32x4_t St[NT];
-    {
-        const float* sp = s_hist + (static_cast<size_t>(pair) * n_span + span) * D * D;
 #pragma unroll
-        for (int i = 0; i < NT; ++i)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                St[i][e] = sp[(static_cast<size_t>(i) * NT + w) * 256 + 4 * (16 * (r >> 2) + 4 * g + e) + (r & 3)];
-    }
+    for (int i = 0; i < NT; ++i) St[i] = gather(s_hist, i);
     issue(0);
     if (nm > 1) issue(1);
     Own own = load_own(0, true);
@@ -1132,16 +1146,12 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
     lds_barrier();
 
     // ================ forwards ================
-    // S^T at the end of the span's first half, kept for the way back (this wave's own)
+    // S^T in mid-span, kept for the way back (this wave's own)
     unsigned char* const mid = smem + G::OFF_MID + w * NT * 1024 + 16 * lane;
     for (int m = 0; m < nm; ++m) {
         const unsigned char* b = buf(m);
         Own next = own;  // the next chunk's values, loaded a whole chunk ahead
         if (m + 1 < nm) next = load_own(m + 1, true);
-        if (m == span_len / 2) {
-#pragma unroll
-            for (int i = 0; i < NT; ++i) st4(mid + 1024 * i, St[i]);
-        }
         // dO S^T, W S^T, and this wave's parts of dO U^T and W U^T.  (Operand reads go two
         // tiles ahead of their products, fenced: left to itself the compiler reads each right
         // before its use and waits out the LDS latency.)
@@ -1183,6 +1193,15 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
         const f32x4_t dQh = qa[0] + qa[1];          // dO S^T [4 g + v][16 w + r]
         const f32x4_t WS = wa[0] + wa[1];           // W S^T
         const f32x4_t kdk = -(b4 * WS);             // dL/dK^
+        if (m == span_len / 2) {
+#pragma unroll
+            for (int i = 0; i < NT; ++i) st4(mid + 1024 * i, St[i]);
+        } else if (m != 0) {
+            const __amdgpu_buffer_rsrc_t rs = start_of(m);
+#pragma unroll
+            for (int i = 0; i < NT; ++i)
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, St[i]), rs, 16 * lane, 1024 * i, 0);
+        }
         lds_barrier();  // Y: the parts are in LDS
         // the totals' operands, read here and summed behind the state update
         constexpr int NZ = 512 / (NW * 64);  // entries of [dP, dA][t][s] per thread
@@ -1236,8 +1255,10 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
             for (int e = 0; e < 4; ++e) s[e] = row16_sum(s[e]);
             if (r == 0) st4(smem + G::OFF_DB + ((m & 1) * NW + w) * 64 + 16 * g, s);
         }
-        // chunk m + 1's copies have landed (they are older than chunk m - 1's five stores)
-        wait_vm_n<4>();
+        // chunk m + 1's copies have landed (they are older than chunk m - 1's five stores, and those
+        // of S^T above are the newest)
+        if (m != 0 && m != span_len / 2) wait_vm_n<4 + NT>();
+        else wait_vm_n<4>();
         lds_barrier();  // Z: totals in LDS, chunk m + 1 in its buffer, every wave done with chunk m's
         if (m + 2 < nm) issue(m + 2);
         const f32x4_t dpr = ld4(smem + G::OFF_TR + 16 * (4 * r + g));            // dP[r][4 g ..]
@@ -1265,6 +1286,21 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
             zc4 = mfma4(c4 ? dd : 0.f, kf4[e], zc4);
         }
         f32x4_t pq = fma4(x.F8, zq8, x.F4 * zq4), pk = fma4(x.F8, zk8, x.F4 * zk4), pc = fma4(x.E8, zc8, x.E4 * zc4);
+        // the gate's pair terms, t >= j > s: of a level, for j in the upper half of a block the rows
+        // t from j on, for j in the lower half the columns s before j
+        const bool up8 = g >= 2, up4 = g & 1;
+        const f32x4_t x8 = (up8 ? x.F8 : x.E8) * (up8 ? fma4(qq, zq8, kk * zk8) : kk * zc8);
+        const f32x4_t x4 = (up4 ? x.F4 : x.E4) * (up4 ? fma4(qq, zq4, kk * zk4) : kk * zc4);
+        f32x4_t pg;
+        {
+            const float t8 = __shfl_xor((x8[0] + x8[1]) + (x8[2] + x8[3]), 16);  // the half's other four tokens
+            const f32x4_t a = up8 ? x8 : f32x4_t{x8[2], x8[1], x8[0], 0.f};
+            const f32x4_t b = up4 ? x4 : f32x4_t{x4[2], x4[1], x4[0], 0.f};
+            const float a2 = a[3] + a[2], a1 = a2 + a[1], b2 = b[3] + b[2], b1 = b2 + b[1];
+            const f32x4_t sa = {a1 + a[0], a1, a2, a[3]}, sb = {b1 + b[0], b1, b2, b[3]};  // from each on
+            pg = (up8 ? sa : f32x4_t{0.f, sa[2], sa[1], sa[0]}) + (up4 ? sb : f32x4_t{0.f, sb[2], sb[1], sb[0]}) +
+                 ((g == 1 || g == 2) ? t8 : 0.f);
+        }
         // pairs inside this lane's four tokens
         f32x4_t dg;
 #pragma unroll
@@ -1276,18 +1312,19 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
 #pragma unroll
             for (int s = a - 1; s >= 0; --s) {
                 f *= x.al[s + 1];
-                const float ws = kk[s] * f, ab = b4[a] * da[s];
+                const float ws = kk[s] * f, ab = b4[a] * da[s], both = fmaf(dp[s], qq[a], ab * kk[a]);
                 pq[a] = fmaf(dp[s], ws, pq[a]);
                 pk[a] = fmaf(ab, ws, pk[a]);
-                pc[s] = fmaf(fmaf(dp[s], qq[a], ab * kk[a]), f, pc[s]);
+                pc[s] = fmaf(both, f, pc[s]);
+#pragma unroll
+                for (int j = s + 1; j <= a; ++j) pg[j] = fmaf(both, ws, pg[j]);
             }
         }
-        // the gate: own terms and pair terms, summed over the tokens at and after each
+        // the gate: own terms, summed over the tokens at and after each, and the pair terms.  (Rows
+        // less columns of all pairs, summed over the tokens at and after, is the same sum but
+        // leaves a strongly decaying token's to the rounding of its neighbours'.)
         const f32x4_t own_t = fma4(qq, x.F * dQh, khat * kdk);
-        const f32x4_t pair_t = fma4(qq, pq, kk * (pk - pc));
-        const float ec = col_total(own_t);
-        if (g == 0) reinterpret_cast<float*>(smem + G::OFF_EC)[m * D + 16 * w + r] = ec;
-        f32x4_t suf = own_t + pair_t;
+        f32x4_t suf = own_t;
         suf[2] += suf[3];
         suf[1] += suf[2];
         suf[0] += suf[1];
@@ -1296,6 +1333,7 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
             const float t8 = t4 + s4, s8 = __shfl_xor(t8, 32);
             suf += ((g & 1) ? 0.f : s4) + ((g & 2) ? 0.f : s8);
         }
+        suf += pg;
         const f32x4_t dQ = fma4(x.F, dQh, fma4(dg, kk, pq));
         const f32x4_t dK = fma4(x.F, kdk, fma4(dg, qq, pk + pc));
         {
@@ -1330,33 +1368,26 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
     // (the last two chunks are still in their buffers; this wave's own stores of the scratch
     // are read back below, after the wait)
     f32x4_t Gt[NT];
-    {
-        const float* gp = g_hist + (static_cast<size_t>(pair) * n_span + span) * D * D;
 #pragma unroll
-        for (int i = 0; i < NT; ++i)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                Gt[i][e] = gp[(static_cast<size_t>(i) * NT + w) * 256 + 4 * (16 * (r >> 2) + 4 * g + e) + (r & 3)];
-    }
+    for (int i = 0; i < NT; ++i) Gt[i] = gather(g_hist, i);
     wait_vm_n<0>();
     own = load_own(nm - 1, false);
-    float hs = 0.f;  // <S, G> of row 16 w + r at the end of the chunk
     for (int m = nm - 1; m >= 0; --m) {
         const unsigned char* b = buf(m);
         Own next = own;
         if (m > 0) next = load_own(m - 1, false);
-        if (m == nm - 1 || m == span_len / 2 - 1) {
-            // from the states themselves at two places of a span, so that the sums carried
-            // along the chunks cover 64 tokens at most
-            f32x4_t s = kZero4;
-            if (m == nm - 1) {
+        f32x4_t Sm[NT];  // S^T at the chunk's start
+        if (m == 0) {
 #pragma unroll
-                for (int i = 0; i < NT; ++i) s = fma4(St[i], Gt[i], s);
-            } else {
+            for (int i = 0; i < NT; ++i) Sm[i] = gather(s_hist, i);
+        } else if (m == span_len / 2) {
 #pragma unroll
-                for (int i = 0; i < NT; ++i) s = fma4(ld4(mid + 1024 * i), Gt[i], s);
-            }
-            hs = col_total(s);
+            for (int i = 0; i < NT; ++i) Sm[i] = ld4(mid + 1024 * i);
+        } else {
+            const __amdgpu_buffer_rsrc_t rs = start_of(m);
+#pragma unroll
+            for (int i = 0; i < NT; ++i)
+                Sm[i] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rs, 16 * lane, 1024 * i, 0));
         }
         // U G^T
         f32x4_t ka[2] = {kZero4, kZero4};
@@ -1375,6 +1406,7 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
         }
         const Dec x = decays(own.lg);
         const f32x4_t khat = own.k * x.F, qhat = own.q * x.F;
+        f32x4_t sg = kZero4;  // <S, G> of row 16 w + r, S from the chunk's start and G from its end
         // G^T = gC G^T + dO^T Q^ - W^T diag(beta) K^
         {
             constexpr int NP = NT > 4 ? 2 : 1;
@@ -1391,7 +1423,10 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
             };
             rd(0);
 #pragma unroll
-            for (int i = 0; i < NT; ++i) Gt[i] = Gt[i] * x.gc;
+            for (int i = 0; i < NT; ++i) {
+                sg = fma4(Sm[i], Gt[i], sg);
+                Gt[i] = Gt[i] * x.gc;
+            }
             fence();
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -1409,9 +1444,6 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
         const f32x4_t dKb = x.E * (ka[0] + ka[1]);  // dL/dK- scaled: dK's part
         const f32x4_t ct = own.k * dKb;             // K- . dL/dK- per token
         const f32x4_t dK = own.x + dKb;
-        const float tot = col_total(ct);
-        const float sg = hs - tot;                  // gC <S, G> of the chunk
-        hs = sg + reinterpret_cast<const float*>(smem + G::OFF_EC)[m * D + 16 * w + r];
         // dg: gC <S, G> plus the sums over the tokens before each
         f32x4_t pre;
         pre[0] = 0.f;
@@ -1421,7 +1453,7 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
         {
             const float t4 = pre[3] + ct[3], s4 = __shfl_xor(t4, 16);
             const float t8 = t4 + s4, s8 = __shfl_xor(t8, 32);
-            pre += sg + (((g & 1) ? s4 : 0.f) + ((g & 2) ? s8 : 0.f));
+            pre += x.gc * col_total(sg) + (((g & 1) ? s4 : 0.f) + ((g & 2) ? s8 : 0.f));
         }
         {
             const unsigned nel = static_cast<unsigned>((clen_of(m) - 1) * tstride + 16);
@@ -1486,7 +1518,7 @@ int span_len_for(long n_pairs, int T) {
 }
 
 struct DecBwdWs {
-    size_t kh, kb, qh, rec, s_hist, g_hist, w, u, bytes;
+    size_t kh, kb, qh, rec, s_hist, g_hist, w, u, s_ch, bytes;
 };
 DecBwdWs dec_bwd_ws(long n_pairs, int T, int D) {
     const size_t n_ch = static_cast<size_t>((T + kC16 - 1) / kC16), sl = span_len_for(n_pairs, T);
@@ -1503,7 +1535,8 @@ DecBwdWs dec_bwd_ws(long n_pairs, int T, int D) {
     w.g_hist = al(w.s_hist + np * n_span * D * D * 4);
     w.w = al(w.g_hist + np * n_span * D * D * 4);
     w.u = al(w.w + tile);
-    w.bytes = al(w.u + tile);
+    w.s_ch = al(w.u + tile);
+    w.bytes = w.s_ch + np * n_span * (sl - 2) * D * D * 4;  // (span starts and middles are kept elsewhere)
     return w;
 }
 
@@ -1578,7 +1611,7 @@ hipError_t launch_t(const BwdArgs& a, hipStream_t st) {
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL((dec_span_kernel<D, InT, CHAN, GE>), dim3(static_cast<unsigned>(a.n_pairs * n_span)), dim3(D * 4),
                        DcGeo<D>::BYTES, st, q, k, v, a.g, a.go, at(o.rec), at(o.s_hist), at(o.g_hist), at(o.w), at(o.u),
-                       a.gq, a.gk, a.gbeta, a.gg, at(o.kh), at(o.kb), a.T, a.H, n_ch, n_span, sl);
+                       a.gq, a.gk, a.gbeta, a.gg, at(o.kh), at(o.kb), at(o.s_ch), a.T, a.H, n_ch, n_span, sl);
     return hipGetLastError();
 }
 

@@ -198,3 +198,46 @@ def test_alike_keys(shape, dtype, rho, beta, chan):
     # per-token kernels' error there is 3e-6 of the sum): each channel's to 1e-5
     channels = gref.kda_vjp(x.q, x.k, x.v, x.beta, np.repeat(g[..., None], shape[3], -1), go, gs, x.s0)[4]
     assert np.linalg.norm(got[4] - exp[4]) <= 1e-5 * np.linalg.norm(channels), what
+
+
+@pytest.mark.parametrize("chan", [False, True])
+@pytest.mark.parametrize("gate", [-1.0, -3.0, -5.0, -8.0, -12.0, -20.0])
+@pytest.mark.parametrize("d", [64, 128])
+def test_gate_gradient_of_strong_decays(d, gate, chan):
+    """dL/dg alone, where every gate is equally strong and where single tokens are, among weak
+    ones: it is about alpha times the sums that it must not be a difference of."""
+    vjp = gref.kda_vjp if chan else gref.gated_vjp
+    x, g, go, gs = _case((1, 150, 2, d), 11, chan)
+    g = np.full_like(g, gate)
+    exp = vjp(x.q, x.k, x.v, x.beta, g, go, gs, x.s0)[4]
+    assert_f32_parity(_bwd(x, g, go, gs, chan)[4], exp, "all gates")
+    g = (-0.1 * np.abs(np.random.default_rng(1).standard_normal(g.shape))).astype(np.float32)
+    rows = [5, 20, 37, 64, 127, 149]
+    g[:, rows] = gate
+    got, exp = _bwd(x, g, go, gs, chan), vjp(x.q, x.k, x.v, x.beta, g, go, gs, x.s0)
+    for name, a, e in zip(NAMES, got, exp):
+        assert_f32_parity(a, e, name, scaled=True)
+    assert_f32_parity(got[4][:, rows], exp[4][:, rows], "the strong tokens' gates")
+
+
+@pytest.mark.parametrize("chan", [False, True])
+@pytest.mark.parametrize("shape", [(2, 520, 16, 64), (4, 505, 16, 64)])
+def test_gate_gradient_of_strong_decays_in_long_spans(shape, chan):
+    """Spans of four chunks (the first shape) and eight, whose strong chunks find their start state
+    in the span's, in its middle's and in those kept per chunk: strong gates in every chunk of
+    one head, in every other chunk of the next, in single tokens of the rest; against the
+    per-token kernels, the strong tokens' gates apart."""
+    x, g, go, gs = _case(shape, 3, chan, scale=0.1)
+    strong = np.zeros(shape[:3], bool)
+    strong[:, :, 0] = True
+    strong[:, :, 1] = (np.arange(shape[1]) // 16 % 2 == 1)[None]
+    strong[:, ::29, 2:] = True
+    g[strong] = -6.0
+    got = _bwd(x, g, go, gs, chan)
+    with _native.use_knobs(1, 0):
+        exp = _bwd(x, g, go, gs, chan)
+    for name, a, e in zip(NAMES, got, exp):
+        assert_f32_parity(a, e, name, scaled=True)
+    for h in range(4):
+        sel = strong[:, :, h]
+        assert_f32_parity(got[4][:, :, h][sel], exp[4][:, :, h][sel], f"head {h}")
