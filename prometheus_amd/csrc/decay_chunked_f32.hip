@@ -82,6 +82,38 @@ __device__ __forceinline__ f32x4_t fma4(f32x4_t a, f32x4_t b, f32x4_t c) {
     return r;
 }
 
+// Infinities and NaN keep to the tokens that they reach in the recurrence.  A product over the
+// chunk's tokens would carry one to all of them, through the exact zeros of T'', T^T and P: where
+// an operand of such a product holds one (looked for once a chunk, behind the product) the rows
+// that it does not reach are formed again without it.
+__device__ __forceinline__ bool any_bad(f32x4_t x) {
+    const float z = fmaf(x[0], 0.f, fmaf(x[1], 0.f, fmaf(x[2], 0.f, x[3] * 0.f)));  // 0, or NaN
+    return __any(z != 0.f);
+}
+__device__ __forceinline__ bool bad(float x) { return !__builtin_isfinite(x); }
+// First (16: none) and last (-1: none) row of this lane's column that holds one
+__device__ __forceinline__ int first_bad(f32x4_t x, int g) {
+    int b = 16;
+#pragma unroll
+    for (int e = 3; e >= 0; --e) b = bad(x[e]) ? 4 * g + e : b;
+    b = min(b, __shfl_xor(b, 16));
+    return min(b, __shfl_xor(b, 32));
+}
+__device__ __forceinline__ int last_bad(f32x4_t x, int g) {
+    int b = -1;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) b = bad(x[e]) ? 4 * g + e : b;
+    b = max(b, __shfl_xor(b, 16));
+    return max(b, __shfl_xor(b, 32));
+}
+// x where this lane's rows 4 g + e are before row b, else y
+__device__ __forceinline__ f32x4_t before(int b, int g, f32x4_t x, f32x4_t y) {
+    f32x4_t z;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) z[e] = 4 * g + e < b ? x[e] : y[e];
+    return z;
+}
+
 // One chunk's record (floats): T''^T, T, P, A'^T as accumulator registers, then gC (D) and
 // beta (16), padded to a multiple of 64 (copied 256 bytes an instruction).
 template <int D>
@@ -317,13 +349,25 @@ __global__ __launch_bounds__(256) void dec_prep_kernel(
     f32x4_t N, Nt, Ta, Tt;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-        N[v] = -bt[v] * A[v];
-        Nt[v] = -bc * At[v];
+        N[v] = 4 * g + v > r ? -bt[v] * A[v] : 0.f;
+        Nt[v] = r > 4 * g + v ? -bc * At[v] : 0.f;
     }
-    inv_lower16<!FWD>(N, Nt, r, g, Ta, Tt);
+    // (an infinity or NaN counts where it stands: its row of U and the columns of W before it)
+    f32x4_t Nf, Ntf;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        Nf[v] = bad(N[v]) ? 0.f : N[v];
+        Ntf[v] = bad(Nt[v]) ? 0.f : Nt[v];
+    }
+    inv_lower16<!FWD>(Nf, Ntf, r, g, Ta, Tt);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        Ta[v] = bad(N[v]) ? N[v] : Ta[v];
+        Tt[v] = bad(Nt[v]) ? Nt[v] : Tt[v];
+    }
     f32x4_t tw;
 #pragma unroll
-    for (int v = 0; v < 4; ++v) tw[v] = -bt[v] * Tt[v];
+    for (int v = 0; v < 4; ++v) tw[v] = 4 * g + v <= r ? -bt[v] * Tt[v] : 0.f;
     *reinterpret_cast<f32x4_t*>(rec + R::T2 + 4 * lane) = tw;
     if constexpr (FWD) {
         *reinterpret_cast<f32x4_t*>(rec + R::FPT + 4 * lane) = Pt;
@@ -404,7 +448,7 @@ __global__ __launch_bounds__((DfGeo<D, DV>::WAVES * 64)) void dec_fwd_kernel(
         lds_barrier();  // B0
         unsigned char* const xs = smem + G::OFF_X + 2048 * cw + 16 * lane;
         float kt[4][NH] = {};  // K-^T operand of the last chunk
-        f32x4_t kf[NH], half = kZero4, tt = kZero4;
+        f32x4_t kf[NH], gc[NH] = {}, half = kZero4, tt = kZero4;
         for (int p = 0; p <= n_ch; ++p) {
             const bool run = p < n_ch;
             const unsigned char* b = buf(run ? p : n_ch - 1);  // (past the end: read, unused)
@@ -418,7 +462,21 @@ __global__ __launch_bounds__((DfGeo<D, DV>::WAVES * 64)) void dec_fwd_kernel(
             tn = ld4(b + G::B_T + 16 * lane);
             fence();
             if (p > 0) {
-                const f32x4_t U = mm16(tt, half + other);
+                const f32x4_t X = half + other;
+                f32x4_t u0 = mfma4(tt[0], X[0], kZero4), u1 = mfma4(tt[1], X[1], kZero4);
+                __asm__ volatile("" : "+v"(u0), "+v"(u1));  // (issued here, with what follows in their shadow)
+#pragma unroll
+                for (int j = 0; j < NH; ++j) {
+                    S[j] = gc[j] * S[j];
+                    __asm__ volatile("" : "+v"(S[j]));
+                }
+                const bool xbad = any_bad(X);
+                u0 = mfma4(tt[2], X[2], u0), u1 = mfma4(tt[3], X[3], u1);
+                f32x4_t U = u0 + u1;
+                if (__builtin_expect(xbad, 0)) {
+                    const int b = first_bad(X, g);
+                    U = before(b, g, mm16(tt, before(b, g, X, kZero4)), U);
+                }
                 if (hh == 0) st4(uslot(p - 1, cw) + 16 * lane, U);
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
@@ -428,7 +486,7 @@ __global__ __launch_bounds__((DfGeo<D, DV>::WAVES * 64)) void dec_fwd_kernel(
             fence();
             if (run) {
                 tt = tn;
-                f32x4_t xa[4] = {kZero4, kZero4, kZero4, kZero4}, gc[NH];
+                f32x4_t xa[4] = {kZero4, kZero4, kZero4, kZero4};
                 if (hh == 0) xa[0] = -vr;
                 unsigned char* ss = sslot(p, cw) + 16 * lane;
 #pragma unroll
@@ -443,8 +501,6 @@ __global__ __launch_bounds__((DfGeo<D, DV>::WAVES * 64)) void dec_fwd_kernel(
                     }
                 half = (xa[0] + xa[1]) + (xa[2] + xa[3]);
                 st4(xs + (p & 1) * 2048 * NCW + hh * 1024, half);
-#pragma unroll
-                for (int j = 0; j < NH; ++j) S[j] = gc[j] * S[j];
             }
             __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), seen by the compiler
             lds_barrier();                       // M_p
@@ -464,7 +520,12 @@ __global__ __launch_bounds__((DfGeo<D, DV>::WAVES * 64)) void dec_fwd_kernel(
         for (int p = 0; p <= n_ch + 1; ++p) {
             if (p >= 2) {
                 const int c = p - 2;
-                const f32x4_t O = mm16(pt, ld4(uslot(c, cw) + 16 * lane), y);
+                const f32x4_t U = ld4(uslot(c, cw) + 16 * lane);
+                f32x4_t O = mm16(pt, U, y);
+                if (__builtin_expect(any_bad(U), 0)) {
+                    const int b = first_bad(U, g);
+                    O = before(b, g, mm16(pt, before(b, g, U, kZero4), y), O);
+                }
                 // lane (g, r) holds O[4 g + e][16 cw + r]; rows past the end are dropped
                 const __amdgpu_buffer_rsrc_t ro = make_rsrc(
                     static_cast<unsigned char*>(o_out) + row0_of(c, col0 + 16 * cw) * ES, els_of(c, 16) * ES);
@@ -694,14 +755,24 @@ __global__ __launch_bounds__((DsGeo<D, DV>::WAVES * 64)) void dec_sweep_kernel(
 #pragma unroll
                     for (int j = 0; j < NH; ++j) *reinterpret_cast<f32x4_t*>(hp + (hh + 2 * j) * 256 + 4 * lane) = M[j];
                 }
-#pragma unroll
-                for (int j = 0; j < NH; ++j) M[j] = gc[j] * M[j];
                 lds_barrier();  // mid-chunk: the halves are in LDS
                 const f32x4_t X = total(p);
-#pragma unroll
-                for (int j = 0; j < NH; ++j) rd_gc(bn, j);
                 const f32x4_t tn = ld4(bn + G::H_T + 16 * lane);
-                const f32x4_t U = mm16(tt, X);
+                f32x4_t u0 = mfma4(tt[0], X[0], kZero4), u1 = mfma4(tt[1], X[1], kZero4);
+                __asm__ volatile("" : "+v"(u0), "+v"(u1));  // (issued here, with what follows in their shadow)
+#pragma unroll
+                for (int j = 0; j < NH; ++j) {
+                    M[j] = gc[j] * M[j];
+                    __asm__ volatile("" : "+v"(M[j]));
+                    rd_gc(bn, j);
+                }
+                const bool xbad = any_bad(X);
+                u0 = mfma4(tt[2], X[2], u0), u1 = mfma4(tt[3], X[3], u1);
+                f32x4_t U = u0 + u1;
+                if (__builtin_expect(xbad, 0)) {
+                    const int b = first_bad(X, g);
+                    U = before(b, g, mm16(tt, before(b, g, X, kZero4)), U);
+                }
                 // S = Diag(gC) S + K-^T U
                 fence();
 #pragma unroll
@@ -714,15 +785,24 @@ __global__ __launch_bounds__((DsGeo<D, DV>::WAVES * 64)) void dec_sweep_kernel(
                         fence();
                     }
                 // U's rows (U^T = X^T T''^T): lane (g, r) holds U[r][col0 + 16 cw + 4 g ..]
-                if (hh == 0)
+                if (hh == 0) {
+                    f32x4_t Ur = mm16(X, tt);
+                    if (__builtin_expect(xbad, 0)) {
+                        const int b = first_bad(X, g);
+                        const f32x4_t clean = mm16(before(b, g, X, kZero4), tt);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) Ur[e] = r < __shfl(b, 4 * g + e) ? clean[e] : Ur[e];
+                    }
                     *reinterpret_cast<f32x4_t*>(u_out + (item0 + i) * kC16 * D +
-                                                4 * f32_chunk<D>(r, (col0 + 16 * cw) / 4 + g)) = mm16(X, tt);
+                                                4 * f32_chunk<D>(r, (col0 + 16 * cw) / 4 + g)) = Ur;
+                }
                 tt = tn;
                 __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), seen by the compiler
                 lds_barrier();                       // end of the chunk
             }
         } else {
             f32x4_t dOc, ta, b4, qc[NH];
+            bool obad;  // any_bad(dOc)
             f32x2_t pp;  // P^T's operand for tokens e = 2 hh, 2 hh + 1: each half adds its part of P^T dO
             auto rd_do = [&](const unsigned char* b, int e) __attribute__((always_inline)) {
                 return reinterpret_cast<const float*>(b + G::S_O + 1024 * cw)[(4 * g + e) * 16 + r];
@@ -751,6 +831,7 @@ __global__ __launch_bounds__((DsGeo<D, DV>::WAVES * 64)) void dec_sweep_kernel(
                 pp = *reinterpret_cast<const f32x2_t*>(b + G::S_P + 16 * lane + 8 * hh);
                 b4 = ld4(b + G::S_G + 4 * D + 16 * g);
                 __builtin_amdgcn_s_waitcnt(0xC07F);
+                obad = any_bad(dOc);
                 lds_barrier();  // B1
             }
             for (int c = n_ch - 1; c >= 0; --c) {
@@ -764,8 +845,13 @@ __global__ __launch_bounds__((DsGeo<D, DV>::WAVES * 64)) void dec_sweep_kernel(
                 }
                 // dU = K- G + P^T dO, this wave's half; a tile's decay behind its last product
                 f32x4_t ya[4] = {kZero4, kZero4, kZero4, kZero4};
-                ya[0] = mfma4(pp[0], hh ? dOc[2] : dOc[0], kZero4);
-                ya[1] = mfma4(pp[1], hh ? dOc[3] : dOc[1], kZero4);
+                float do0 = hh ? dOc[2] : dOc[0], do1 = hh ? dOc[3] : dOc[1];
+                if (__builtin_expect(obad, 0)) {
+                    do0 = bad(do0) ? 0.f : do0;
+                    do1 = bad(do1) ? 0.f : do1;
+                }
+                ya[0] = mfma4(pp[0], do0, kZero4);
+                ya[1] = mfma4(pp[1], do1, kZero4);
                 fence();
 #pragma unroll
                 for (int j = 0; j < NH; ++j)
@@ -816,6 +902,7 @@ __global__ __launch_bounds__((DsGeo<D, DV>::WAVES * 64)) void dec_sweep_kernel(
                 fence();
                 w0 = mfma4(ta[2], dU[2], w0), w1 = mfma4(ta[3], dU[3], w1);
                 __asm__ volatile("" : "+v"(w0), "+v"(w1));
+                const bool wbad = static_cast<int>(obad) | static_cast<int>(any_bad(dU));
                 fence();
 #pragma unroll
                 for (int j = 1; j < NH; ++j) {
@@ -824,7 +911,11 @@ __global__ __launch_bounds__((DsGeo<D, DV>::WAVES * 64)) void dec_sweep_kernel(
                     if (j == 1) bn4 = ld4(bn + G::S_G + 4 * D + 16 * g);
                     fence();
                 }
-                const f32x4_t W = w0 + w1;
+                f32x4_t W = w0 + w1;
+                if (__builtin_expect(wbad, 0)) {
+                    const int b = max(last_bad(dOc, g), last_bad(dU, g)) + 1;
+                    W = before(b, g, kZero4 + __builtin_nanf(""), mm16(ta, before(b, g, kZero4, dU)));
+                }
                 const f32x4_t nbW = -(W * b4);
                 // G -= K^^T diag(beta) W
                 fence();
@@ -837,6 +928,7 @@ __global__ __launch_bounds__((DsGeo<D, DV>::WAVES * 64)) void dec_sweep_kernel(
                         if (e == 3) rd_kt(bn + G::S_KH, 3, j);
                         if (e == 0 && j == 0 && hh == 0) st4(wslot(c, cw) + 16 * lane, W);
                         if (e == 0 && j == 1 && hh == 0 && r == 0) st4(wslot(c, cw) + 1024 + 16 * g, b4);
+                        if (e == 2 && j == 0) obad = any_bad(dOn);
                         fence();
                     }
                 dOc = dOn, ta = tn, pp = pn, b4 = bn4;
@@ -1270,8 +1362,18 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
         const int rb = r >> 2;
         const bool r8 = r >= 8 && g < 2, c8 = r < 8 && g >= 2;
         const bool r4 = (rb & 1) && g == rb - 1, c4 = !(rb & 1) && g == rb + 1;
-        const f32x4_t ke8 = kk * x.E8, kf8 = kk * x.F8, qf8 = qq * x.F8;
-        const f32x4_t ke4 = kk * x.E4, kf4 = kk * x.F4, qf4 = qq * x.F4;
+        f32x4_t ke8 = kk * x.E8, kf8 = kk * x.F8, qf8 = qq * x.F8;
+        f32x4_t ke4 = kk * x.E4, kf4 = kk * x.F4, qf4 = qq * x.F4;
+        {
+            // (as above: a token's infinity or NaN in k, q or the decays stays with its own pairs, in
+            // which dP, dA or the decay by which a sum is scaled carries it too)
+            const f32x4_t z = kk * kZero4 + qq * kZero4;
+            if (__builtin_expect(any_bad(f32x4_t{z[0] + z[1], z[2] + z[3], x.gc, 0.f}), 0)) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    for (f32x4_t* y : {&ke8, &kf8, &qf8, &ke4, &kf4, &qf4}) (*y)[e] = bad((*y)[e]) ? 0.f : (*y)[e];
+            }
+        }
         f32x4_t zq8 = kZero4, zk8 = kZero4, zc8 = kZero4, zq4 = kZero4, zk4 = kZero4, zc4 = kZero4;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
