@@ -32,7 +32,10 @@
 // copy (buffer_load ... lds) two chunks ahead.  One LDS-only barrier per chunk.
 // The chain bounds it: with one wave per 16 columns (68 products, the output wave as many with
 // P^T) 32 pairs of T 1024 took 113 us at D = 128 and 76 at D = 64, now 72 and 51; 128 pairs of
-// D = 128, where the MFMA pipes of every CU are shared, 208, now 195.
+// D = 128, where the MFMA pipes of every CU are shared, 208, now 195.  At D = 64 and 32 columns
+// (128 pairs on) one wave holds 16 columns alone: its 36 products are few enough, and the
+// exchange and two waves more cost what the halves save (128 pairs 73 us, with two chain waves
+// 75; 200 pairs 113 and 116).  There the output waves share P^T and the copies.
 #include <type_traits>
 
 #include "pm_cdna4.h"
@@ -185,8 +188,11 @@ __global__ __launch_bounds__(256) void delta_f32_prep_kernel(const float* __rest
 // ---------------------------------------------------------------- K7
 template <int D, int DV, bool NORM>
 struct F32Geo {
-    static constexpr int NCW = DV / 16;            // 16-column blocks: two chain waves and an output wave each
-    static constexpr int WAVES = 3 * NCW + 1;      // chain 0 .., output 2 NCW .., the last P^T and copies
+    static constexpr int NCW = DV / 16;            // 16-column blocks: CW chain waves and an output wave each
+    static constexpr int CW = D == 64 && DV == 32 ? 1 : 2;
+    // chain 0 .., output CW NCW .., and at CW 2 a last one for P^T and the copies, which the two
+    // output waves share at CW 1
+    static constexpr int WAVES = (CW + 1) * NCW + CW - 1;
     static constexpr int NT = D / 16;              // S accumulator tiles per block
     static constexpr int NI = kC16 * D * 4 / 1024; // 1 KiB copies per K or Q tile
     static constexpr int NB = 4;        // rotating chunk buffers
@@ -248,8 +254,9 @@ __global__ __launch_bounds__((F32Geo<D, DV, NORM>::WAVES * 64)) void delta_f32_k
 
     const int lane = threadIdx.x & 63;
     const int r = lane & 15, g = lane >> 4;
-    const bool chain = w < 2 * NCW, copy_wave = w == 3 * NCW;
-    const int cw = chain ? w >> 1 : w - 2 * NCW;  // the 16 columns this wave works on
+    constexpr int CW = G::CW;
+    const bool chain = w < CW * NCW, copy_wave = w == G::WAVES - 1;
+    const int cw = chain ? w / CW : w - CW * NCW;  // the 16 columns this wave works on
     const size_t tstride = static_cast<size_t>(H) * D;
     const size_t sbase = static_cast<size_t>(pair) * D * D;
     const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
@@ -335,6 +342,39 @@ __global__ __launch_bounds__((F32Geo<D, DV, NORM>::WAVES * 64)) void delta_f32_k
         }
     };
 
+    // Y = Q S of chunk c (returned) and P^T of it (stored), either or both: a tile's operands are
+    // read two tiles ahead of its products, accumulator e takes the steps (m, e)
+    auto products = [&](int c, auto DO_Y, auto DO_P) __attribute__((always_inline)) {
+        constexpr bool doy = decltype(DO_Y)::value, dop = decltype(DO_P)::value;
+        const unsigned char* b = buf(c);
+        const unsigned char* ss = sslot(c, doy ? cw : 0);
+        f32x4_t ya[4] = {zero, zero, zero, zero}, pa[4] = {zero, zero, zero, zero}, qv[NT], kp[NT], sc[NT];
+        float qss = 0.f;  // normalised mode: this lane's part of ||q_r||^2
+        auto rd = [&](int m) __attribute__((always_inline)) {
+            qv[m] = ld4(b + G::B_Q + 16 * f32_chunk<D>(r, 4 * m + g));
+            if constexpr (doy) sc[m] = ld4(ss + 1024 * m + 16 * lane);
+            if constexpr (dop) kp[m] = ld4(b + G::B_K + 16 * f32_chunk<D>(r, 4 * m + g));
+        };
+        rd(0);
+        rd(1);
+        fence();
+#pragma unroll
+        for (int m = 0; m < NT; ++m) {
+            if (m + 2 < NT) rd(m + 2);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if constexpr (doy) ya[e] = mfma4(qv[m][e], sc[m][e], ya[e]);
+                if constexpr (dop) pa[e] = mfma4(kp[m][e], qv[m][e], pa[e]);
+                if constexpr (dop && NORM) qss = fmaf(qv[m][e], qv[m][e], qss);
+            }
+            fence();
+        }
+        if constexpr (dop) store_p(c, (pa[0] + pa[1]) + (pa[2] + pa[3]), qss);
+        return (ya[0] + ya[1]) + (ya[2] + ya[3]);
+    };
+    using Yes = std::true_type;
+    using No = std::false_type;
+
     if (n_chunks > 0) {
         if (copy_wave) {
             copies(0);
@@ -346,32 +386,41 @@ __global__ __launch_bounds__((F32Geo<D, DV, NORM>::WAVES * 64)) void delta_f32_k
     }
 
     if (chain) {
-        // ============ chain wave hh of two: S columns col0 + 16 cw + [0, 16), tiles m = hh + 2 j ============
+        // ============ chain wave hh of CW: S columns col0 + 16 cw + [0, 16), tiles m = hh + CW j ============
         // Phase p (up to barrier M_p) finishes chunk p - 1 (the other wave's half of X, U, S +=
         // K^T U) and forms this wave's half of X of chunk p: one barrier a chunk.  Every LDS
-        // read is issued ahead of the products or behind one of them.
-        constexpr int NH = NT / 2;
-        const int hh = w & 1, ecol = col0 + 16 * cw + r;
+        // read is issued ahead of the products or behind one of them.  A wave alone forms U
+        // right behind X and leaves the LDS accesses to the end, in U's latency (spread over the
+        // products as the halves' they hold its one sequence up: 75 us for 73 at 128 pairs).
+        constexpr int NH = NT / CW;
+        const int hh = CW == 2 ? w & 1 : 0, ecol = col0 + 16 * cw + r;
         const TileIdx<D> ix(r, g, hh);
         f32x4_t S[NH];
 #pragma unroll
         for (int j = 0; j < NH; ++j)
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                S[j][e] = s0 ? s0[sbase + static_cast<size_t>(16 * (hh + 2 * j) + 4 * g + e) * D + ecol] : 0.f;
+                S[j][e] = s0 ? s0[sbase + static_cast<size_t>(16 * (hh + CW * j) + 4 * g + e) * D + ecol] : 0.f;
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), seen by the compiler: no wait for these in the loop
         __builtin_amdgcn_s_setprio(3);
         unsigned char* const xs = smem + G::OFF_X + 2048 * cw + 16 * lane;
         float kt[4][NH] = {};
-        f32x4_t kf[NH], half = zero, tt = zero, vr = zero, skc = zero;
+        f32x4_t kf[NH], half = zero, tt = zero, vr = zero, skc = zero, U = zero;
+        auto form_u = [&](f32x4_t X) __attribute__((always_inline)) {
+            if constexpr (NORM) X = X * skc - vr;
+            f32x4_t u = mm16(tt, X);
+            if constexpr (NORM) u = u * skc;
+            return u;
+        };
         if (n_chunks > 0) {
             for (int p = 0; p <= n_chunks; ++p) {
                 const bool run = p < n_chunks;
                 const unsigned char* b = buf(run ? p : n_chunks - 1);  // (past the end: read, unused)
-                const f32x4_t other = ld4(xs + ((p & 1) ^ 1) * 2048 * NCW + (hh ^ 1) * 1024);
+                f32x4_t other = zero;
+                if constexpr (CW == 2) other = ld4(xs + ((p & 1) ^ 1) * 2048 * NCW + (hh ^ 1) * 1024);
                 f32x4_t tn, vn, sn = zero;
 #pragma unroll
-                for (int j = 0; j < NH; ++j) kf[j] = ix.row2(b + G::B_K, j);
+                for (int j = 0; j < NH; ++j) kf[j] = CW == 2 ? ix.row2(b + G::B_K, j) : ix.row(b + G::B_K, j);
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
                     vn[e] = reinterpret_cast<const float*>(b + G::B_V + 1024 * cw)[(4 * g + e) * 16 + r];
@@ -379,10 +428,7 @@ __global__ __launch_bounds__((F32Geo<D, DV, NORM>::WAVES * 64)) void delta_f32_k
                 if constexpr (NORM) sn = ld4(b + G::B_T + 1024 + 16 * g);
                 fence();
                 if (p > 0) {
-                    f32x4_t X = half + other;
-                    if constexpr (NORM) X = X * skc - vr;
-                    f32x4_t U = mm16(tt, X);
-                    if constexpr (NORM) U = U * skc;
+                    if constexpr (CW == 2) U = form_u(half + other);
                     if (hh == 0) st4(uslot(p - 1, cw) + 16 * lane, U);
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
@@ -392,7 +438,8 @@ __global__ __launch_bounds__((F32Geo<D, DV, NORM>::WAVES * 64)) void delta_f32_k
                 fence();
                 if (run) {
                     tt = tn, vr = vn, skc = sn;
-                    f32x4_t xa[4] = {zero, zero, zero, zero};
+                    // (a wave alone sums its even and odd tiles apart: the bits of the two halves)
+                    f32x4_t xa[4] = {zero, zero, zero, zero}, xb[4] = {zero, zero, zero, zero};
                     if constexpr (!NORM) {
                         if (hh == 0) xa[0] = -vr;
                     }
@@ -401,13 +448,25 @@ __global__ __launch_bounds__((F32Geo<D, DV, NORM>::WAVES * 64)) void delta_f32_k
                     for (int j = 0; j < NH; ++j)
 #pragma unroll
                         for (int e = 0; e < 4; ++e) {
-                            xa[e] = mfma4(kf[j][e], S[j][e], xa[e]);
-                            kt[e][j] = ix.col2(b + G::B_K, e, j);
-                            if (e == 3) st4(ss + 1024 * (hh + 2 * j), S[j]);
-                            fence();
+                            f32x4_t& x = CW == 1 && (j & 1) ? xb[e] : xa[e];
+                            x = mfma4(kf[j][e], S[j][e], x);
+                            if constexpr (CW == 2) {
+                                kt[e][j] = ix.col2(b + G::B_K, e, j);
+                                if (e == 3) st4(ss + 1024 * (hh + CW * j), S[j]);
+                                fence();
+                            }
                         }
                     half = (xa[0] + xa[1]) + (xa[2] + xa[3]);
-                    st4(xs + (p & 1) * 2048 * NCW + hh * 1024, half);
+                    if constexpr (CW == 2) st4(xs + (p & 1) * 2048 * NCW + hh * 1024, half);
+                    else {
+                        U = form_u(half + ((xb[0] + xb[1]) + (xb[2] + xb[3])));
+#pragma unroll
+                        for (int j = 0; j < NH; ++j) st4(ss + 1024 * j, S[j]);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+#pragma unroll
+                            for (int j = 0; j < NH; ++j) kt[e][j] = ix.col(b + G::B_K, e, j);
+                    }
                 }
                 __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), seen by the compiler
                 lds_barrier();                       // M_p
@@ -417,36 +476,13 @@ __global__ __launch_bounds__((F32Geo<D, DV, NORM>::WAVES * 64)) void delta_f32_k
         for (int j = 0; j < NH; ++j)
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                s_out[sbase + static_cast<size_t>(16 * (hh + 2 * j) + 4 * g + e) * D + ecol] = S[j][e];
-    } else if (n_chunks > 0 && copy_wave) {
+                s_out[sbase + static_cast<size_t>(16 * (hh + CW * j) + 4 * g + e) * D + ecol] = S[j][e];
+    } else if (CW == 2 && n_chunks > 0 && copy_wave) {
         // ============ P and copy wave: phase p builds P^T of chunk p - 1, copies chunk p + 2 ============
         for (int p = 0; p <= n_chunks; ++p) {
             const bool cp = p + 2 < n_chunks;
             if (cp) copies(p + 2);
-            if (p >= 1) {
-                const int c = p - 1;
-                const unsigned char* b = buf(c);
-                f32x4_t pa[4] = {zero, zero, zero, zero}, qp[NT], kp[NT];
-                float qss = 0.f;  // normalised mode: this lane's part of ||q_r||^2
-                auto rd = [&](int m) __attribute__((always_inline)) {
-                    qp[m] = ld4(b + G::B_Q + 16 * f32_chunk<D>(r, 4 * m + g));
-                    kp[m] = ld4(b + G::B_K + 16 * f32_chunk<D>(r, 4 * m + g));
-                };
-                rd(0);
-                rd(1);
-                fence();
-#pragma unroll
-                for (int m = 0; m < NT; ++m) {
-                    if (m + 2 < NT) rd(m + 2);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        pa[e] = mfma4(kp[m][e], qp[m][e], pa[e]);
-                        if constexpr (NORM) qss = fmaf(qp[m][e], qp[m][e], qss);
-                    }
-                    fence();
-                }
-                store_p(c, (pa[0] + pa[1]) + (pa[2] + pa[3]), qss);
-            }
+            if (p >= 1) products(p - 1, No{}, Yes{});
             // chunk p + 1 has landed; the copies of the one after may be in flight
             if (cp) wait_vm_n<NCP>();
             else wait_vm_n<0>();
@@ -454,29 +490,19 @@ __global__ __launch_bounds__((F32Geo<D, DV, NORM>::WAVES * 64)) void delta_f32_k
         }
     } else if (n_chunks > 0) {
         // ============ output wave: phase p finishes O of chunk p - 2 and forms Y = Q S of chunk p - 1 ============
+        // (CW 1: the first one builds P^T of chunk p - 1 too, the last one issues the copies of p + 2)
         f32x4_t y = zero;
         for (int p = 0; p <= n_chunks + 1; ++p) {
+            const bool cp = CW == 1 && copy_wave && p + 2 < n_chunks;
+            if (cp) copies(p + 2);
             if (p >= 2) store_o(p - 2, y);
             if (p > n_chunks) break;
-            if (p >= 1) {
-                const unsigned char* b = buf(p - 1);
-                const unsigned char* ss = sslot(p - 1, cw);
-                f32x4_t ya[4] = {zero, zero, zero, zero}, qy[NT], sc[NT];
-                auto rd = [&](int m) __attribute__((always_inline)) {
-                    qy[m] = ld4(b + G::B_Q + 16 * f32_chunk<D>(r, 4 * m + g));
-                    sc[m] = ld4(ss + 1024 * m + 16 * lane);
-                };
-                rd(0);
-                rd(1);
-                fence();
-#pragma unroll
-                for (int m = 0; m < NT; ++m) {
-                    if (m + 2 < NT) rd(m + 2);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) ya[e] = mfma4(qy[m][e], sc[m][e], ya[e]);
-                    fence();
-                }
-                y = (ya[0] + ya[1]) + (ya[2] + ya[3]);
+            if (p >= 1) y = CW == 1 && cw == 0 ? products(p - 1, Yes{}, Yes{}) : products(p - 1, Yes{}, No{});
+            if (CW == 1 && copy_wave) {
+                // as above, with the four stores of this phase behind this phase's copies
+                if (cp && p >= 2) wait_vm_n<NCP + 4>();
+                else if (cp) wait_vm_n<NCP>();
+                else wait_vm_n<0>();
             }
             lds_barrier();
         }
@@ -540,8 +566,8 @@ size_t chunked_f32_ws_bytes(bool varlen, int n_seq, int T, int H, bool norm) {
 // D = 128: 16 columns a workgroup while that leaves at most one per CU (LDS holds one), so that
 // a chain wave has its SIMD to itself; a second round costs more than the wider form (T 1024:
 // 32 pairs 72 against 95 us, 33 pairs 126 against 97, 63 pairs 128 against 100).  D = 64: two
-// fit a CU, and the two forms are level from 65 to 128 pairs (72 against 73 us at 96) before
-// the narrow one needs a second round (200 pairs 135 against 115).
+// fit a CU, and the two forms are level from 65 to 128 pairs (71 us at 96, 74 against 73 at 128)
+// before the narrow one needs a second round (200 pairs 135 against 113).
 int chunked_f32_pick_tile(int D, long n_pairs, int requested) {
     if (requested == 16 || requested == 32) return requested;
     if (requested == 64) return 32;
