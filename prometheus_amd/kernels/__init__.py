@@ -669,6 +669,9 @@ def _gated_bwd(residual, grads, per_channel, bf16=False):
         qd, kd, vd = call.dev(q, cdt), call.dev(k, cdt), call.dev(v, cdt)
         bd, gd, sd = call.dev(beta, f32), call.dev(g, f32), call.dev(s0, f32)
         god, gsd = call.dev(go, f32), call.dev(gs, f32)
+        # as the ungated backward: views at odd offsets are copied, not run token by token
+        qd, kd, vd, god = (_aligned16(x) for x in (qd, kd, vd, god))
+        gd = _aligned16(gd) if per_channel else gd
         gb = torch.empty((batch, seq, heads), dtype=f32, device=call.device)
         gg = torch.empty(gshape, dtype=f32, device=call.device)
         gs0 = torch.empty((batch, heads, dim, dim), dtype=f32, device=call.device)

@@ -263,3 +263,27 @@ def test_infinities_and_nans_reach_what_they_reach_token_by_token(what, value, d
         np.testing.assert_array_equal(np.isfinite(a), np.isfinite(e), err_msg=name)
         ok = np.isfinite(e)
         assert_f32_parity(a[ok], e[ok], name, scaled=True)
+
+
+@pytest.mark.parametrize("chan", [False, True])
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+def test_views_at_odd_offsets_run_the_chunked_backward(dtype, chan):
+    """Slices of packed buffers give the aligned tensors' gradients bit for bit (the per-token
+    kernels' differ in rounding)."""
+    x, g, go, gs = _case((2, 70, 3, 64), 31, chan, dtype)
+
+    def shifted(t):
+        return torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")[1:].copy_(t.flatten()).view(t.shape)
+
+    def run(place):
+        def qkv(name):
+            bits = getattr(x, name + "_bits")
+            return _dev(getattr(x, name)) if bits is None else torch.from_numpy(bits.view(np.int16)).view(torch.bfloat16).cuda()
+
+        ins = [place(qkv(n)) for n in "qkv"] + [_dev(x.beta), place(_dev(g)), _dev(x.s0)]
+        res = kernels._GatedDeltaResidual(*ins, chunk=64)
+        f = kernels.chunked_kda_rule_bwd if chan else kernels.chunked_gated_delta_rule_bwd
+        return f(res, (place(_dev(go)), _dev(gs)))
+
+    for name, a, b in zip(NAMES, run(shifted), run(lambda t: t)):
+        assert torch.equal(a, b), name
