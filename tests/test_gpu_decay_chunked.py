@@ -1,7 +1,11 @@
 """GPU tests of the chunked fp32 kernels of the rules with a decay (gated and KDA, D in {64,
 128}: the backward from 16 tokens, the forward of fp32 q/k/v from 160) against the fp64
 oracles at the fp32 bounds, at the edges of their 16-token chunks and of the spans of chunks,
-and against the per-token kernels that every other call runs."""
+and against the per-token kernels that every other call runs.
+
+The backward's plan follows the pairs n (batch x heads) and the chunks of 16 tokens c: a
+workgroup of its sweep takes 16 columns up to n D/16 = 256 and 32 above, a span is 8 chunks
+where n ceil(c / 8) >= 256, else 4 where n ceil(c / 4) >= 256, else 2."""
 
 from __future__ import annotations
 
@@ -57,7 +61,8 @@ def _check(x, g, go, gs, chan, what):
 @pytest.mark.parametrize("chan", [False, True])
 @pytest.mark.parametrize("t,d", [(16, 128), (17, 64), (31, 64), (64, 128), (127, 64), (128, 128), (129, 64), (273, 128)])
 def test_edges_of_chunks_and_spans(t, d, chan):
-    """Whole and partial chunks, one chunk up to several spans, with and without a state."""
+    """Whole and partial chunks, one chunk up to several spans (of two chunks here; longer ones
+    below), with and without a state."""
     x, g, go, gs = _case((1, t, 3, d), t + d + chan, chan, state=t % 2 == 0)
     _check(x, g, go, gs, chan, f"T{t} D{d}")
 
@@ -263,6 +268,40 @@ def test_infinities_and_nans_reach_what_they_reach_token_by_token(what, value, d
         np.testing.assert_array_equal(np.isfinite(a), np.isfinite(e), err_msg=name)
         ok = np.isfinite(e)
         assert_f32_parity(a[ok], e[ok], name, scaled=True)
+
+
+@pytest.mark.parametrize("chan", [False, True])
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+@pytest.mark.parametrize("d,h,t", [
+    # 34 pairs of D = 128 and 66 of 64: 32 columns; spans of eight chunks, the last one of
+    # 1, 4, 5 and 8, the last chunk whole or partial
+    (128, 34, 912), (128, 34, 955), (128, 34, 971), (128, 34, 1024),
+    (64, 66, 400), (64, 66, 443), (64, 66, 459), (64, 66, 512),
+    # ... spans of four, the last one of 1, 2, 3 and 4
+    (128, 34, 464), (128, 34, 475), (64, 66, 235), (64, 66, 256),
+    # 16 columns, spans of eight
+    (64, 64, 505), (128, 32, 1010)])
+def test_plans_of_large_calls(d, h, t, dtype, chan):
+    """Each form of the sweep and each span length, against the per-token kernels."""
+    x, g, go, gs = _case((1, t, h, d), t + chan, chan, dtype, scale=0.1)
+    got = _bwd(x, g, go, gs, chan)
+    with _native.use_knobs(1, 0):
+        exp = _bwd(x, g, go, gs, chan)
+    for name, a, e in zip(NAMES, got, exp):
+        assert_f32_parity(a, e, name, scaled=True)
+
+
+@pytest.mark.parametrize("chan", [False, True])
+@pytest.mark.parametrize("d,h,t", [(64, 128, 165), (64, 255, 176), (64, 127, 161), (128, 40, 200)])
+def test_forward_plans_of_large_calls(d, h, t, chan):
+    """The forward's automatic 32 columns (128 pairs of D = 64 on, 33 of 128) and the last
+    call on 16, against the per-token kernel."""
+    x, g, _, _ = _case((1, t, h, d), t + chan, chan, scale=0.1)
+    got = _fwd(x, g, chan)
+    with _native.use_knobs(1, 0):
+        exp = _fwd(x, g, chan)
+    for name, a, e in zip(("o", "state"), got, exp):
+        assert_f32_parity(a, e, name)
 
 
 @pytest.mark.parametrize("chan", [False, True])

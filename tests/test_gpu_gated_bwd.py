@@ -64,14 +64,16 @@ def test_against_the_oracle(shape, state):
 
 @pytest.mark.parametrize("gate_scale", [0.02, 1.0, 4.0])
 def test_gate_strengths(gate_scale):
-    """Weak to strong decay (alpha down to ~1e-4 at scale 4): the blocks are recomputed
-    forward from their start states, never walked back through a division by alpha."""
+    """Weak to strong decay (alpha down to ~1e-4 at scale 4), on the chunked kernels and on the
+    per-token ones: neither walks the state back through a division by alpha."""
     shape = (2, 90, 2, 64)
     x, g, go, gs = _case(shape, 41, gate_scale, True)
-    got = _gpu_bwd(x.q, x.k, x.v, x.beta, g, x.s0, go, gs)
     exp = gref.gated_vjp(x.q, x.k, x.v, x.beta, g, go, gs, x.s0)
-    for name, a, e in zip(NAMES, got, exp):
-        assert_f32_parity(_np(a), e, f"scale {gate_scale} {name}", scaled=True)
+    for path in (0, 1):
+        with _native.use_knobs(path, 0):
+            got = _gpu_bwd(x.q, x.k, x.v, x.beta, g, x.s0, go, gs)
+        for name, a, e in zip(NAMES, got, exp):
+            assert_f32_parity(_np(a), e, f"path {path} scale {gate_scale} {name}", scaled=True)
 
 
 def test_zero_gate_matches_the_ungated_backward():
@@ -174,3 +176,14 @@ def test_chunked_path_is_refused_for_the_gated_backward():
         assert ei.value.code == _native.E_UNSUPPORTED
     finally:
         _native.set_path(old)
+
+
+@pytest.mark.parametrize("shape", [(2, 100, 2, 64), (1, 130, 2, 128)])
+def test_the_per_token_kernels_where_the_chunked_ones_run(shape):
+    """Path 1, which misaligned and short calls of these head dimensions take too."""
+    x, g, go, gs = _case(shape, sum(shape), 0.3, True)
+    with _native.use_knobs(1, 0):
+        got = _gpu_bwd(x.q, x.k, x.v, x.beta, g, x.s0, go, gs)
+    exp = gref.gated_vjp(x.q, x.k, x.v, x.beta, g, go, gs, x.s0)
+    for name, a, e in zip(NAMES, got, exp):
+        assert_f32_parity(_np(a), e, f"{shape} {name}", scaled=True)

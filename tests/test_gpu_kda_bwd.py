@@ -160,3 +160,14 @@ def test_chunked_path_is_refused():
     with _native.use_knobs(2, 0), pytest.raises(_native.NativeError) as ei:
         _gpu_bwd(x.q, x.k, x.v, x.beta, g, None, go, gs)
     assert ei.value.code == _native.E_UNSUPPORTED
+
+
+@pytest.mark.parametrize("shape", [(2, 100, 2, 64), (1, 130, 2, 128)])
+def test_the_per_token_kernels_where_the_chunked_ones_run(shape):
+    """Path 1, which misaligned and short calls of these head dimensions take too."""
+    x, g, go, gs = _case(shape, sum(shape), 0.3, True)
+    with _native.use_knobs(1, 0):
+        got = _gpu_bwd(x.q, x.k, x.v, x.beta, g, x.s0, go, gs)
+    exp = gref.kda_vjp(x.q, x.k, x.v, x.beta, g, go, gs, x.s0)
+    for name, a, e in zip(NAMES, got, exp):
+        assert_f32_parity(_np(a), e, f"{shape} {name}", scaled=True)
