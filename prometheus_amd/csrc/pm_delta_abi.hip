@@ -10,7 +10,9 @@
 //   K7    delta_chunked_f32.hip     chunked forward on fp32 MFMA, fp32 inputs
 //   K8    kda_chunked.hip           chunked forward with a decay per key channel
 //   K9    delta_chunked_f32_bwd.hip chunked reverse mode on fp32 MFMA, fp32 inputs
-//   K10   decay_chunked_f32.hip     chunked reverse mode of the gated rules on fp32 MFMA
+//   K10   decay_chunked_f32.hip     chunked reverse mode of the gated rules on fp32 MFMA, and
+//                                   their chunked forward for fp32 inputs (K10f)
+//   K11   norm_rows.hip             row normalisation of the model's backward and its reverse
 // Mirrors the checks of kernels/__init__.py:308-338 (shapes), :613-614 and
 // :676-677 (chunk >= 1); shapes arrive as integers, so the Python layer
 // (prometheus_amd/kernels) raises KernelError for the tensor-level checks
@@ -430,7 +432,7 @@ int backward(const void* q, const void* k, const void* v, const float* beta, con
     const bool chunked = chunked16 || chunked32;
     if (g_path >= 2 && !chunked)
         return fail(PM_E_UNSUPPORTED,
-                    gated ? "the gated backward runs on the per-token kernels only (path 2 asks for the chunked one)"
+                    gated ? "the gated backward has no bf16 chunked form, which path 2 asks for (path 0: chunked in fp32, or per-token)"
                           : "chunked backward needs D in {64, 128} (got in_dtype %d, D %d)",
                     in_dtype, D);
     if (chunked && n_tok > 0) {

@@ -180,7 +180,7 @@ struct BwdArgs {
     float* workspace;
     int n_pairs, T, H, D;
     bool in_bf16;
-    // gated variant (per-token fp32 kernels only): log-gates per (token, head), alpha =
+    // gated variant (K10 and the per-token fp32 kernels): log-gates per (token, head), alpha =
     // exp(g), and their gradient gg (B, T, H)
     const float* g = nullptr;
     float* gg = nullptr;
@@ -214,7 +214,7 @@ hipError_t launch_bwd_chunked_f32(const BwdArgs& a, hipStream_t st);
 // workspace 16-byte aligned.
 size_t decay_bwd_ws_bytes(long n_pairs, int T, int D);
 // ... and the forward for fp32 q/k/v; workspace decay_fwd_ws_bytes bytes; q, k, v, g (per
-// channel), o and workspace 16-byte aligned.
+// channel) and workspace 16-byte aligned, o to its elements.
 struct DecayFwdArgs {
     const float* q;
     const float* k;
