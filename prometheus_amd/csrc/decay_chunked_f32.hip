@@ -53,14 +53,15 @@
 // Why chunks: the per-token kernels walk T tokens in sequence at about 500 (forward) and
 // 1,270 cycles (reverse) a token, bound by VALU issue; here a chunk of 16 tokens takes about
 // 2,800 to 4,100 cycles of the one sequential launch, and the rest is parallel over chunks.
-// Measured, B4 T4096 H16 D128, bf16 q/k/v, per-head gate: 6.0 -> 1.45 ms (K10p 125, K10s
-// 505, K10c 825 us); B2, per-channel gate: 5.9 -> 0.87 ms (97, 340, 432); B3 T1000 H6 D64
-// fp32: 1.11 -> 0.10 ms.  Against 64 bits the gradients of training inputs are at 1.6e-7 to
-// 2.5e-7 (the per-token kernels: 1.3e-7 to 1.9e-7).  What bounds it: K10s the products of its recurrence waves (32
-// pairs: 54 of 32 cycles in a chunk of 2,800 cycles, the two barriers and exchanges most of
-// the rest, the copies 10%; 64 pairs: 94 on each SIMD), K10c the fp32 MFMA pipe at half its
-// rate (232 products per wave and chunk; two waves per SIMD, which wait for the pipe half of
-// the time and at its barriers a third).
+// Measured (backward alone), B4 T4096 H16 D128, bf16 q/k/v, per-head gate: 6.0 -> 1.55 ms (K10p
+// 122, K10s 515, K10c 910 us); B2, per-channel gate: 5.9 -> 0.93 ms (98, 345, 485); B3 T1000 H6
+// D64 fp32: 1.11 -> 0.11 ms (11, 57, 39).  Against 64 bits the gradients of training inputs are at
+// 1.6e-7 to 2.5e-7 (the per-token kernels: 1.3e-7 to 1.9e-7).  What bounds it, by counters: K10s
+// the products of its recurrence waves (MFMA pipes busy 58% of the time at 64 pairs and 47% at 32,
+// where each chain wave has a SIMD to itself; the rest is the two exchanges and barriers of a
+// chunk), K10c the two together of the fp32 MFMA pipe (busy 44%, 41% per channel; its two waves
+// per SIMD wait to issue half of their time and at barriers a quarter) and of its workspace (3.5
+// GB in 910 us, 3.8 TB/s, where a copy reaches 4.7; 1.6 GB of it the states of the chunks).
 
 #include <type_traits>
 
