@@ -74,10 +74,6 @@ namespace {
 
 constexpr int kSpan = 8;  // chunks per span (128 tokens) at most
 
-__device__ __forceinline__ f32x4_t ld4(const unsigned char* p) { return *reinterpret_cast<const f32x4_t*>(p); }
-__device__ __forceinline__ void st4(unsigned char* p, f32x4_t x) { *reinterpret_cast<f32x4_t*>(p) = x; }
-__device__ __forceinline__ void fence() { __builtin_amdgcn_sched_barrier(0); }
-constexpr f32x4_t kZero4 = {0.f, 0.f, 0.f, 0.f};
 __device__ __forceinline__ f32x4_t fma4(f32x4_t a, f32x4_t b, f32x4_t c) {
     const f32x4_t r = {fmaf(a[0], b[0], c[0]), fmaf(a[1], b[1], c[1]), fmaf(a[2], b[2], c[2]), fmaf(a[3], b[3], c[3])};
     return r;
@@ -1595,19 +1591,6 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
             if (t < clen_of(m)) gg[(tok0 + z) * H + h] = s;
         }
     }
-}
-
-// The dynamic-LDS limit is a per-device function attribute, set once per device and kernel.
-template <auto KERN>
-hipError_t set_lds(int bytes) {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    static bool done[64] = {};
-    if (dev >= 0 && dev < 64 && done[dev]) return hipSuccess;
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(KERN), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    if (e == hipSuccess && dev >= 0 && dev < 64) done[dev] = true;
-    return e;
 }
 
 // Chunks per span: a power of two up to kSpan, halved while the span kernel would leave CUs

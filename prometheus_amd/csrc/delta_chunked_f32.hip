@@ -136,8 +136,7 @@ __global__ __launch_bounds__(256) void delta_f32_prep_kernel(const float* __rest
     }
 
     // G = K K^T (one accumulator per step of a tile, summed at the end)
-    const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
-    f32x4_t ga[4] = {zero, zero, zero, zero};
+    f32x4_t ga[4] = {kZero4, kZero4, kZero4, kZero4};
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
 #pragma unroll
@@ -167,7 +166,7 @@ __global__ __launch_bounds__(256) void delta_f32_prep_kernel(const float* __rest
         if (g == 0) ob[512 + r] = bc;
         // P = lower_incl(Q K^T): P[4 g + v][r] = q_{4 g + v} . k_r, kept for r <= 4 g + v
         const __amdgpu_buffer_rsrc_t rq = make_rsrc(q + row0, nb);
-        f32x4_t pa[4] = {zero, zero, zero, zero};
+        f32x4_t pa[4] = {kZero4, kZero4, kZero4, kZero4};
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
             const unsigned vo = static_cast<unsigned>((r * tstride + 16 * j + 4 * g) * 4);
@@ -259,15 +258,11 @@ __global__ __launch_bounds__((F32Geo<D, DV, NORM>::WAVES * 64)) void delta_f32_k
     const int cw = chain ? w / CW : w - CW * NCW;  // the 16 columns this wave works on
     const size_t tstride = static_cast<size_t>(H) * D;
     const size_t sbase = static_cast<size_t>(pair) * D * D;
-    const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
-    auto fence = []() __attribute__((always_inline)) { __builtin_amdgcn_sched_barrier(0); };
 
     auto buf = [&](int c) { return smem + (c % G::NB) * G::BUF; };
     auto sslot = [&](int c, int which) { return smem + G::OFF_S + ((c & 1) * NCW + which) * NT * 1024; };
     auto uslot = [&](int c, int which) { return smem + G::OFF_U + ((c & 1) * NCW + which) * 1024; };
     auto pslot = [&](int c) { return smem + G::OFF_P + (c & 1) * G::PSLOT; };
-    auto ld4 = [&](const unsigned char* p) { return *reinterpret_cast<const f32x4_t*>(p); };
-    auto st4 = [&](unsigned char* p, f32x4_t x) { *reinterpret_cast<f32x4_t*>(p) = x; };
 
     // ---- HBM -> LDS copies of chunk c (c < n_chunks) ----
     auto chunk_rsrc = [&](const float* base, int c, int row_floats, int col) {
@@ -348,7 +343,7 @@ __global__ __launch_bounds__((F32Geo<D, DV, NORM>::WAVES * 64)) void delta_f32_k
         constexpr bool doy = decltype(DO_Y)::value, dop = decltype(DO_P)::value;
         const unsigned char* b = buf(c);
         const unsigned char* ss = sslot(c, doy ? cw : 0);
-        f32x4_t ya[4] = {zero, zero, zero, zero}, pa[4] = {zero, zero, zero, zero}, qv[NT], kp[NT], sc[NT];
+        f32x4_t ya[4] = {kZero4, kZero4, kZero4, kZero4}, pa[4] = {kZero4, kZero4, kZero4, kZero4}, qv[NT], kp[NT], sc[NT];
         float qss = 0.f;  // normalised mode: this lane's part of ||q_r||^2
         auto rd = [&](int m) __attribute__((always_inline)) {
             qv[m] = ld4(b + G::B_Q + 16 * f32_chunk<D>(r, 4 * m + g));
@@ -405,7 +400,7 @@ __global__ __launch_bounds__((F32Geo<D, DV, NORM>::WAVES * 64)) void delta_f32_k
         __builtin_amdgcn_s_setprio(3);
         unsigned char* const xs = smem + G::OFF_X + 2048 * cw + 16 * lane;
         float kt[4][NH] = {};
-        f32x4_t kf[NH], half = zero, tt = zero, vr = zero, skc = zero, U = zero;
+        f32x4_t kf[NH], half = kZero4, tt = kZero4, vr = kZero4, skc = kZero4, U = kZero4;
         auto form_u = [&](f32x4_t X) __attribute__((always_inline)) {
             if constexpr (NORM) X = X * skc - vr;
             f32x4_t u = mm16(tt, X);
@@ -416,9 +411,9 @@ __global__ __launch_bounds__((F32Geo<D, DV, NORM>::WAVES * 64)) void delta_f32_k
             for (int p = 0; p <= n_chunks; ++p) {
                 const bool run = p < n_chunks;
                 const unsigned char* b = buf(run ? p : n_chunks - 1);  // (past the end: read, unused)
-                f32x4_t other = zero;
+                f32x4_t other = kZero4;
                 if constexpr (CW == 2) other = ld4(xs + ((p & 1) ^ 1) * 2048 * NCW + (hh ^ 1) * 1024);
-                f32x4_t tn, vn, sn = zero;
+                f32x4_t tn, vn, sn = kZero4;
 #pragma unroll
                 for (int j = 0; j < NH; ++j) kf[j] = CW == 2 ? ix.row2(b + G::B_K, j) : ix.row(b + G::B_K, j);
 #pragma unroll
@@ -439,7 +434,7 @@ __global__ __launch_bounds__((F32Geo<D, DV, NORM>::WAVES * 64)) void delta_f32_k
                 if (run) {
                     tt = tn, vr = vn, skc = sn;
                     // (a wave alone sums its even and odd tiles apart: the bits of the two halves)
-                    f32x4_t xa[4] = {zero, zero, zero, zero}, xb[4] = {zero, zero, zero, zero};
+                    f32x4_t xa[4] = {kZero4, kZero4, kZero4, kZero4}, xb[4] = {kZero4, kZero4, kZero4, kZero4};
                     if constexpr (!NORM) {
                         if (hh == 0) xa[0] = -vr;
                     }
@@ -491,7 +486,7 @@ __global__ __launch_bounds__((F32Geo<D, DV, NORM>::WAVES * 64)) void delta_f32_k
     } else if (n_chunks > 0) {
         // ============ output wave: phase p finishes O of chunk p - 2 and forms Y = Q S of chunk p - 1 ============
         // (CW 1: the first one builds P^T of chunk p - 1 too, the last one issues the copies of p + 2)
-        f32x4_t y = zero;
+        f32x4_t y = kZero4;
         for (int p = 0; p <= n_chunks + 1; ++p) {
             const bool cp = CW == 1 && copy_wave && p + 2 < n_chunks;
             if (cp) copies(p + 2);
@@ -509,20 +504,6 @@ __global__ __launch_bounds__((F32Geo<D, DV, NORM>::WAVES * 64)) void delta_f32_k
     }
 }
 
-// The dynamic-LDS limit is a per-device function attribute, set once per device for each
-// kernel (KERN: one static flag array per kernel, not per signature).
-template <auto KERN>
-hipError_t set_lds_f32(int bytes) {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    static bool done[64] = {};
-    if (dev >= 0 && dev < 64 && done[dev]) return hipSuccess;
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(KERN), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    if (e == hipSuccess && dev >= 0 && dev < 64) done[dev] = true;
-    return e;
-}
-
 template <int D, int DV, bool OB, bool NORM>
 hipError_t launch_f32_t(const ChunkedF32Args& a, float* ws, hipStream_t st) {
     using G = F32Geo<D, DV, NORM>;
@@ -538,7 +519,7 @@ hipError_t launch_f32_t(const ChunkedF32Args& a, float* ws, hipStream_t st) {
         if (e != hipSuccess) return e;
     }
     auto kern = delta_f32_kernel<D, DV, OB, NORM>;
-    hipError_t e = set_lds_f32<delta_f32_kernel<D, DV, OB, NORM>>(G::BYTES);
+    hipError_t e = set_lds<delta_f32_kernel<D, DV, OB, NORM>>(G::BYTES);
     if (e != hipSuccess) return e;
     const int n_tiles = D / DV;
     const int slots = (n_pairs + 7) / 8;

@@ -40,12 +40,6 @@
 namespace pm {
 namespace {
 
-__device__ __forceinline__ f32x4_t ld4(const unsigned char* p) { return *reinterpret_cast<const f32x4_t*>(p); }
-__device__ __forceinline__ void st4(unsigned char* p, f32x4_t x) { *reinterpret_cast<f32x4_t*>(p) = x; }
-__device__ __forceinline__ void fence() { __builtin_amdgcn_sched_barrier(0); }
-
-constexpr f32x4_t kZero4 = {0.f, 0.f, 0.f, 0.f};
-
 // ---------------------------------------------------------------- K9a + K9b
 // The two recurrences, over S forwards and over G backwards, in one workgroup per (b, h, DV
 // columns of d_v).  They bound the launch: their chunks run in sequence.  Two waves share 16
@@ -745,11 +739,6 @@ __global__ __launch_bounds__(D * 4) void f32_bwd_span_kernel(
     }
 }
 
-template <typename Kern>
-hipError_t set_lds(Kern kern, int bytes) {
-    return hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-}
-
 template <int D>
 hipError_t launch_d(const BwdArgs& a, hipStream_t st) {
     const int n_ch = (a.T + kC16 - 1) / kC16;
@@ -766,7 +755,7 @@ hipError_t launch_d(const BwdArgs& a, hipStream_t st) {
     const float* k = static_cast<const float*>(a.k);
     const float* v = static_cast<const float*>(a.v);
     hipError_t e;
-    if ((e = set_lds(f32_bwd_span_kernel<D>, SpGeo<D>::BYTES)) != hipSuccess) return e;
+    if ((e = set_lds<f32_bwd_span_kernel<D>>(SpGeo<D>::BYTES)) != hipSuccess) return e;
     if (n_ch > 0 && (e = launch_f32_bwd_prep(q, k, a.beta, a.n_pairs, a.T, a.H, D, t2, rec, st)) != hipSuccess) return e;
     // 16 columns a workgroup while that leaves at most one per CU: a chain wave then has its SIMD
     // to itself (the decayed rules' same sweep: 367 us against 489 at 32 pairs, 668 against 512 at 48)
@@ -774,7 +763,7 @@ hipError_t launch_d(const BwdArgs& a, hipStream_t st) {
     auto sweep = [&](auto VV) {
         constexpr int DV = decltype(VV)::value;
         using G = SwGeo<D, DV>;
-        const hipError_t err = set_lds(f32_sweep_kernel<D, DV>, G::BYTES);
+        const hipError_t err = set_lds<f32_sweep_kernel<D, DV>>(G::BYTES);
         if (err != hipSuccess) return err;
         hipLaunchKernelGGL((f32_sweep_kernel<D, DV>), dim3(static_cast<unsigned>(slots * (D / DV) * 8)),
                            dim3(G::WAVES * 64), G::BYTES, st, q, k, v, a.s0, a.go, a.gs, a.gv, a.gs0, t2, rec, w_ws,

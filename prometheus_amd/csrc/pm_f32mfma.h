@@ -10,6 +10,7 @@
 // and a product contracting over M's columns needs the registers of M^T instead.
 #pragma once
 
+#include <atomic>
 #include <type_traits>
 
 namespace pm {
@@ -17,14 +18,32 @@ namespace {
 
 constexpr int kC16 = 16;  // tokens per chunk
 
+constexpr f32x4_t kZero4 = {0.f, 0.f, 0.f, 0.f};
+__device__ __forceinline__ f32x4_t ld4(const unsigned char* p) { return *reinterpret_cast<const f32x4_t*>(p); }
+__device__ __forceinline__ void st4(unsigned char* p, f32x4_t x) { *reinterpret_cast<f32x4_t*>(p) = x; }
+__device__ __forceinline__ void fence() { __builtin_amdgcn_sched_barrier(0); }
+
+// The dynamic-LDS limit is a per-device function attribute, set once per device for each
+// kernel (KERN: one static flag array per kernel, not per signature).
+template <auto KERN>
+hipError_t set_lds(int bytes) {
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    static std::atomic<bool> done[64] = {};
+    if (dev >= 0 && dev < 64 && done[dev].load(std::memory_order_relaxed)) return hipSuccess;
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(KERN), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (e == hipSuccess && dev >= 0 && dev < 64) done[dev].store(true, std::memory_order_relaxed);
+    return e;
+}
+
 __device__ __forceinline__ f32x4_t mfma4(float a, float b, f32x4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 // Left * Right over a 16-token contraction, given the accumulators of Left^T and Right
 // (plus c), in two accumulators.
-__device__ __forceinline__ f32x4_t mm16(f32x4_t lt, f32x4_t r, f32x4_t c = f32x4_t{0.f, 0.f, 0.f, 0.f}) {
-    const f32x4_t z = {0.f, 0.f, 0.f, 0.f};
-    f32x4_t a0 = mfma4(lt[0], r[0], c), a1 = mfma4(lt[1], r[1], z);
+__device__ __forceinline__ f32x4_t mm16(f32x4_t lt, f32x4_t r, f32x4_t c = kZero4) {
+    f32x4_t a0 = mfma4(lt[0], r[0], c), a1 = mfma4(lt[1], r[1], kZero4);
     a0 = mfma4(lt[2], r[2], a0);
     a1 = mfma4(lt[3], r[3], a1);
     return a0 + a1;
