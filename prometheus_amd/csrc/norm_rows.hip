@@ -70,7 +70,8 @@ __device__ __forceinline__ float row_sum8(const float (&y)[8]) {
 // ... and over a row of any D <= 256 by one wave: f(acc, d) adds element d's value to acc.
 // Below 128 elements lane l takes elements l and l + n in two sums, n the power of two at most D
 // (and 64); from there on it takes the four elements from 4 l on and from 4 (l + n) on in four,
-// n the power of two at most D / 4.
+// n the power of two at most D / 4.  (From 128 on with a remainder of D / 4 those operations' order
+// follows each row's alignment; this is the one of aligned rows.)
 template <typename F>
 __device__ __forceinline__ float row_sum_any(int D, int lane, F f) {
     const int n = 1 << min(6, 31 - __clz(D < 128 ? D : D / 4));

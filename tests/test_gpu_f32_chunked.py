@@ -19,7 +19,7 @@ import pytest
 import torch
 
 from oracle import delta_oracle as ref
-from prometheus_amd import _native, kernels, synth
+from prometheus_amd import _native, kernels, model, synth
 from tests.parity import assert_f32_parity
 
 pytestmark = pytest.mark.gpu
@@ -171,3 +171,27 @@ def test_f32_chunked_t0_and_empty_batch():
         o, s = kernels.chunked_delta_rule(q, k, v, b, s0)
     assert o.shape == (2, 0, 2, 64)
     assert torch.equal(s, s0)
+
+
+@pytest.mark.parametrize("tokens", [1, 16, 17, 33, 50, 70])
+@pytest.mark.parametrize("rule", ["delta", "model", "varlen"])
+def test_f32_chunked_widths_at_d64_give_the_same_bits(rule, tokens):
+    """At D = 64 a workgroup of 32 columns runs one chain wave to 16 of them, one of 16 columns two:
+    one chunk up to five, whole and partial, normalised rows and packed batches too."""
+    _, (q, k, v, b, s0) = _case((2, tokens, 3, 64), seed=tokens, s0_std=0.02)
+
+    def run():
+        if rule == "model":
+            return model.linear_attention(q, k, v, s0)
+        if rule == "delta":
+            return kernels.chunked_delta_rule(q, k, v, b, s0)
+        cu = torch.tensor([0, 0, tokens, 2 * tokens], dtype=torch.int32, device="cuda")
+        packed = [t.reshape(1, 2 * tokens, *t.shape[2:]) for t in (q, k, v, b)]
+        return kernels.chunked_delta_rule_varlen(*packed, cu)
+
+    with _path(2, 16):
+        narrow = run()
+    with _path(2, 32):
+        wide = run()
+    for a, e in zip(wide, narrow):
+        assert torch.equal(a, e) and a.isfinite().all()
