@@ -47,21 +47,21 @@
 //     its start state (dQ, dbeta, dK and dg but for what depends on G), then backwards from
 //     its end gradient (the rest).  S cannot be walked back as the ungated backward does
 //     (that divides by gC), hence the two walks; <S, G> needs S at every chunk's start again, which
-//     the way forwards keeps (in LDS at mid-span, else in the workspace: 64 KiB a chunk at D = 128,
-//     5% of the training pass).
+//     the way forwards keeps (the last one in registers, the middle one in LDS, the others in the
+//     workspace: 64 KiB a chunk at D = 128, 4% of the training pass).
 
 // Why chunks: the per-token kernels walk T tokens in sequence at about 500 (forward) and
 // 1,270 cycles (reverse) a token, bound by VALU issue; here a chunk of 16 tokens takes about
 // 2,800 to 4,100 cycles of the one sequential launch, and the rest is parallel over chunks.
-// Measured (backward alone), B4 T4096 H16 D128, bf16 q/k/v, per-head gate: 6.0 -> 1.55 ms (K10p
-// 122, K10s 515, K10c 910 us); B2, per-channel gate: 5.9 -> 0.93 ms (98, 345, 485); B3 T1000 H6
+// Measured (backward alone), B4 T4096 H16 D128, bf16 q/k/v, per-head gate: 6.0 -> 1.53 ms (K10p
+// 122, K10s 515, K10c 870 us); B2, per-channel gate: 5.9 -> 0.93 ms (97, 344, 480); B3 T1000 H6
 // D64 fp32: 1.11 -> 0.11 ms (11, 57, 39).  Against 64 bits the gradients of training inputs are at
 // 1.6e-7 to 2.5e-7 (the per-token kernels: 1.3e-7 to 1.9e-7).  What bounds it, by counters: K10s
-// the products of its recurrence waves (MFMA pipes busy 58% of the time at 64 pairs and 47% at 32,
+// the products of its recurrence waves (MFMA pipes busy 59% of the time at 64 pairs and 47% at 32,
 // where each chain wave has a SIMD to itself; the rest is the two exchanges and barriers of a
-// chunk), K10c the two together of the fp32 MFMA pipe (busy 44%, 41% per channel; its two waves
-// per SIMD wait to issue half of their time and at barriers a quarter) and of its workspace (3.5
-// GB in 910 us, 3.8 TB/s, where a copy reaches 4.7; 1.6 GB of it the states of the chunks).
+// chunk), K10c the two together of the fp32 MFMA pipe (busy 46%, 41% per channel; its two waves
+// per SIMD wait to issue half of their time and at barriers a quarter) and of its workspace (3.2
+// GB in 870 us, 3.7 TB/s, where a copy reaches 4.7; 1.3 GB of it the states of the chunks).
 
 #include <type_traits>
 
@@ -73,6 +73,9 @@ namespace pm {
 namespace {
 
 constexpr int kSpan = 8;  // chunks per span (128 tokens) at most
+// Chunks of a span whose start states K10c leaves in the workspace: not the first, the middle
+// and the last one's
+__host__ __device__ constexpr int kept_starts(int span_len) { return span_len > 2 ? span_len - 3 : 0; }
 
 __device__ __forceinline__ f32x4_t fma4(f32x4_t a, f32x4_t b, f32x4_t c) {
     const f32x4_t r = {fmaf(a[0], b[0], c[0]), fmaf(a[1], b[1], c[1]), fmaf(a[2], b[2], c[2]), fmaf(a[3], b[3], c[3])};
@@ -1219,10 +1222,10 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
             x[e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, off + 16 * e, (i * NT + w) * 1024, 0));
         return x;
     };
-    // this wave's S^T at the start of chunk m, left for the way back; m = 0 is in s_hist and m =
-    // span_len / 2 in LDS
+    // this wave's S^T at the start of chunk m, left for the way back; m = 0 is in s_hist, m =
+    // span_len / 2 in LDS, and the last chunk's stays in registers
     auto start_of = [=](int m) __attribute__((always_inline)) {
-        const size_t slot = (static_cast<size_t>(pair) * n_span + span) * (span_len - 2) + m - (m < span_len / 2 ? 1 : 2);
+        const size_t slot = (static_cast<size_t>(pair) * n_span + span) * kept_starts(span_len) + m - (m < span_len / 2 ? 1 : 2);
         return make_rsrc(s_ch + slot * D * D + w * NT * 256, NT * 1024);
     };
     f32x4_t St[NT];
@@ -1282,10 +1285,11 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
         const f32x4_t dQh = qa[0] + qa[1];          // dO S^T [4 g + v][16 w + r]
         const f32x4_t WS = wa[0] + wa[1];           // W S^T
         const f32x4_t kdk = -(b4 * WS);             // dL/dK^
-        if (m == span_len / 2) {
+        const bool last = m + 1 == nm;
+        if (m == span_len / 2 && !last) {
 #pragma unroll
             for (int i = 0; i < NT; ++i) st4(mid + 1024 * i, St[i]);
-        } else if (m != 0) {
+        } else if (m != 0 && !last) {
             const __amdgpu_buffer_rsrc_t rs = start_of(m);
 #pragma unroll
             for (int i = 0; i < NT; ++i)
@@ -1303,8 +1307,9 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
         f32x4_t wj;  // W at this lane's columns 16 w + r of d_v
 #pragma unroll
         for (int e = 0; e < 4; ++e) wj[e] = ix.colw(b + G::B_W, e, w, g);
-        // S^T = gC S^T + U^T K-, tiles i and i + 4 together (their reads pair up)
-        {
+        // S^T = gC S^T + U^T K-, tiles i and i + 4 together (their reads pair up); nothing reads the
+        // span's end state
+        if (!last) {
             constexpr int NP = NT > 4 ? 2 : 1;
             float uc[2][NP][4];
             auto rd = [&](int i) __attribute__((always_inline)) {
@@ -1346,7 +1351,7 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
         }
         // chunk m + 1's copies have landed (they are older than chunk m - 1's five stores, and those
         // of S^T above are the newest)
-        if (m != 0 && m != span_len / 2) wait_vm_n<4 + NT>();
+        if (m != 0 && m != span_len / 2 && !last) wait_vm_n<4 + NT>();
         else wait_vm_n<4>();
         lds_barrier();  // Z: totals in LDS, chunk m + 1 in its buffer, every wave done with chunk m's
         if (m + 2 < nm) issue(m + 2);
@@ -1475,18 +1480,19 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
         const unsigned char* b = buf(m);
         Own next = own;
         if (m > 0) next = load_own(m - 1, false);
-        f32x4_t Sm[NT];  // S^T at the chunk's start
-        if (m == 0) {
+        // S^T at the chunk's start
+        if (m + 1 == nm) {
+        } else if (m == 0) {
 #pragma unroll
-            for (int i = 0; i < NT; ++i) Sm[i] = gather(s_hist, i);
+            for (int i = 0; i < NT; ++i) St[i] = gather(s_hist, i);
         } else if (m == span_len / 2) {
 #pragma unroll
-            for (int i = 0; i < NT; ++i) Sm[i] = ld4(mid + 1024 * i);
+            for (int i = 0; i < NT; ++i) St[i] = ld4(mid + 1024 * i);
         } else {
             const __amdgpu_buffer_rsrc_t rs = start_of(m);
 #pragma unroll
             for (int i = 0; i < NT; ++i)
-                Sm[i] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rs, 16 * lane, 1024 * i, 0));
+                St[i] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rs, 16 * lane, 1024 * i, 0));
         }
         // U G^T
         f32x4_t ka[2] = {kZero4, kZero4};
@@ -1523,7 +1529,7 @@ __global__ __launch_bounds__(D * 4) void dec_span_kernel(
             rd(0);
 #pragma unroll
             for (int i = 0; i < NT; ++i) {
-                sg = fma4(Sm[i], Gt[i], sg);
+                sg = fma4(St[i], Gt[i], sg);
                 Gt[i] = Gt[i] * x.gc;
             }
             fence();
@@ -1622,7 +1628,7 @@ DecBwdWs dec_bwd_ws(long n_pairs, int T, int D) {
     w.w = al(w.g_hist + np * n_span * D * D * 4);
     w.u = al(w.w + tile);
     w.s_ch = al(w.u + tile);
-    w.bytes = w.s_ch + np * n_span * (sl - 2) * D * D * 4;  // (span starts and middles are kept elsewhere)
+    w.bytes = w.s_ch + np * n_span * kept_starts(static_cast<int>(sl)) * D * D * 4;
     return w;
 }
 
