@@ -427,6 +427,8 @@ int backward(const void* q, const void* k, const void* v, const float* beta, con
     const void* f32s[] = {beta, g, s0, go, gs, gbeta, gg, gs0, workspace, gq, gk, gv};
     for (int i = 0; i < (gt == kGradF32 ? 12 : 9); ++i)
         if (f32s[i] && !aligned(f32s[i], 4)) return fail(PM_E_ALIGN, "fp32 buffers must be 4-byte aligned");
+    for (int i = 9; i < 12; ++i)
+        if (f32s[i] && !aligned(f32s[i], 2)) return fail(PM_E_ALIGN, "bf16 gradients must be 2-byte aligned");
     const bool chunked16 = !gated && bwd_chunked(H, D, in_dtype);
     const bool chunked32 = !gated && bwd_chunked_f32(H, D, in_dtype);
     const bool chunked = chunked16 || chunked32;

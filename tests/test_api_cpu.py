@@ -610,3 +610,15 @@ def test_gated_backward_workspace_and_checks():
         assert rc == _native.E_UNSUPPORTED and b"per-token" in lib.pm_last_error()
     finally:
         _native.set_path(old)
+
+
+def test_bf16_gradient_buffers_are_checked_before_any_launch():
+    """pm_delta_bwd_bf16: a bf16 gradient at an odd address is refused, as an fp32 one off its four
+    bytes is, for each of gq, gk and gv and with and without gates."""
+    lib = _native.lib()
+    p, odd = ctypes.c_void_p(256), ctypes.c_void_p(257)
+    for g in (None, p):
+        for i in range(3):
+            out = [odd if j == i else p for j in range(3)]
+            rc = lib.pm_delta_bwd_bf16(p, p, p, p, g, None, p, p, *out, p, g, p, 1, 32, 1, 64, 0, p, 1 << 24, None)
+            assert rc == _native.E_ALIGN, i
