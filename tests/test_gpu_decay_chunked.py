@@ -251,15 +251,15 @@ def test_gate_gradient_of_strong_decays_in_long_spans(shape, chan):
 @pytest.mark.parametrize("chan", [False, True])
 @pytest.mark.parametrize("d,token", [(64, 105), (128, 96), (128, 111)])
 @pytest.mark.parametrize("value", [np.nan, np.inf])
-@pytest.mark.parametrize("what", ["q", "k", "v", "beta", "g", "go"])
+@pytest.mark.parametrize("what", ["q", "k", "v", "beta", "g", "go", "s0", "gs"])
 def test_infinities_and_nans_reach_what_they_reach_token_by_token(what, value, d, token, chan):
     """One infinity or NaN in an input: the outputs and gradients that the per-token kernels leave
     finite stay so (v: the tokens before it, and the other columns; q and dO: those after it),
     with their values, and no other becomes finite."""
     x, g, go, gs = _case((1, 200, 2, d), 5, chan, scale=0.1)
     x.q, x.k, x.v = x.q.copy(), x.k.copy(), x.v.copy()
-    a = {"q": x.q, "k": x.k, "v": x.v, "beta": x.beta, "g": g, "go": go}[what]
-    a[(0, token, 1, 7)[: a.ndim]] = value
+    a = {"q": x.q, "k": x.k, "v": x.v, "beta": x.beta, "g": g, "go": go, "s0": x.s0, "gs": gs}[what]
+    a[(0, 1, 7, token % d) if what in ("s0", "gs") else (0, token, 1, 7)[: a.ndim]] = value
     res = []
     for path in (0, 1):
         with _native.use_knobs(path, 0):
